@@ -143,17 +143,20 @@ struct dq_devmat {
     int tuned_rpt = 0, tuned_nt = -1, tuned_pipe = -1, tuned_lds = -1;
     // Row-tile order chosen by dq_spmv_tune (-1 = default round-robin, 0 = round-robin, 1 = XCD-contiguous).
     int tuned_xcd = -1;
-    // Fused-evolution term schedule, timed on the first evolution of this matrix (0 = not yet): rows per lane (2, 4,
-    // 8) and LDS x window (0, 1). A speed choice only: every schedule gives the same bits. Atomic: evolutions of one
+    // Fused-evolution term schedule, chosen on the first evolution of this matrix (0 = not yet): rows per lane (1, 2),
+    // non-temporal loads and LDS x window (0, 1). A speed choice only: every schedule gives the same bits. Atomic: evolutions of one
     // matrix may run from several threads, and the first ones may each time and store a choice.
-    mutable std::atomic<int> term_rpt{0}, term_lds{0};
-    // SpMV schedule for products that skip the matrix's all-zero blocks, chosen by dq_spmv_tune (0 / -1 = the
-    // library default): rows per lane, non-temporal loads, load schedule, LDS x window.
-    int skip_rpt = 0, skip_nt = -1, skip_pipe = -1, skip_lds = -1;
-    // The zero-block map (256-row blocks, zmap_words words per diagonal) dq_spmv_tune keeps when the matrix has
-    // all-zero blocks; a call that rewrites the values (dq_devmat_set_packed_device) recomputes it in place.
+    mutable std::atomic<int> term_rpt{0}, term_nt{0}, term_lds{0};
+    // Wave forms (dia_rows_wave) chosen by dq_spmv_tune: for products that read every block when it beat the row tiles
+    // above, and for products that skip the all-zero blocks (v = 0: no choice).
+    struct WaveSched {
+        int v = 0;  // rows per lane: 1 or 2
+        bool nt = true, lds = false;
+    };
+    WaveSched tuned_wave, skip_wave;
+    // The zero-block map (64-row blocks) dq_spmv_tune keeps when the matrix has all-zero blocks or parts; a call that
+    // rewrites the values (dq_devmat_set_packed_device) recomputes it in place.
     dq::DevBuf zmap;
-    int64_t zmap_words = 0;
     bool zmap_valid = false;
 
     int n() const { return static_cast<int>(offs.size()); }

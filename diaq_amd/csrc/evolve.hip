@@ -30,6 +30,9 @@
 
 namespace dq {
 
+// The blocks of a zero-block map word that hold a nonzero real or imaginary value.
+__device__ inline uint32_t any_part(uint2 w) { return w.x | w.y; }
+
 struct JobParam {
     double tau;      // sub-step length t / 2^s
     int32_t m;       // Taylor degree
@@ -57,7 +60,7 @@ __global__ __launch_bounds__(256) void horner_kernel(int64_t N, int n, const Dia
                                                      float *__restrict__ p32r, float *__restrict__ p32i,
                                                      const float *__restrict__ bin_r, const float *__restrict__ bin_i,
                                                      float *__restrict__ bout_r, float *__restrict__ bout_i,
-                                                     int64_t ntiles, int xcd, const uint32_t *__restrict__ zmask,
+                                                     int64_t ntiles, int xcd, const uint2 *__restrict__ zmask,
                                                      int64_t zwords) {
     const int j = blockIdx.y;
     const JobParam P = params[j];
@@ -102,7 +105,7 @@ __global__ __launch_bounds__(256) void horner_kernel(int64_t N, int n, const Dia
         // pass q of the tile covers block t*RPT + q of RPP rows; RPT divides 32, so the tile's bits share one word
         uint32_t live = (1u << RPT) - 1;
         if (zmask) {
-            const uint32_t w = zmask[(static_cast<int64_t>(j) * n + d) * zwords + ((t * RPT) >> 5)];
+            const uint32_t w = any_part(zmask[(static_cast<int64_t>(j) * n + d) * zwords + ((t * RPT) >> 5)]);
             live = (w >> ((t * RPT) & 31)) & ((1u << RPT) - 1);
             if (!live) continue;  // uniform: every value of the diagonal in this tile is zero
         }
@@ -177,7 +180,7 @@ __global__ __launch_bounds__(256) void horner4_kernel(int64_t N, int n, const Di
                                                       float *__restrict__ p32r, float *__restrict__ p32i,
                                                       const float *__restrict__ bin_r, const float *__restrict__ bin_i,
                                                       float *__restrict__ bout_r, float *__restrict__ bout_i,
-                                                      int64_t ntiles, int xcd, const uint32_t *__restrict__ zmask,
+                                                      int64_t ntiles, int xcd, const uint2 *__restrict__ zmask,
                                                       int64_t zwords) {
     static_assert(NS == 4 || NS == 8 || NS == 16, "four states per lane");
     constexpr int L = NS / 4;         // lanes per row
@@ -227,7 +230,7 @@ __global__ __launch_bounds__(256) void horner4_kernel(int64_t N, int n, const Di
             if (rhi <= tile || rlo >= tile + T) continue;  // uniform
             uint32_t live = (4 * RPT >= 32) ? ~0u : ((1u << (4 * RPT)) - 1);
             if (zmask) {
-                const uint32_t w = zmask[(static_cast<int64_t>(j) * n + d) * zwords + (blk0 >> 5)];
+                const uint32_t w = any_part(zmask[(static_cast<int64_t>(j) * n + d) * zwords + (blk0 >> 5)]);
                 live = (4 * RPT >= 32) ? w : ((w >> (blk0 & 31)) & ((1u << (4 * RPT)) - 1));
                 if (!live) continue;  // uniform: every value of the diagonal in this tile is zero
             }
@@ -323,7 +326,7 @@ __global__ __launch_bounds__(256) void probe_kernel(int64_t N, int n, const Diag
                                                     const float *__restrict__ p32r, const float *__restrict__ p32i,
                                                     const float *__restrict__ tin_r, const float *__restrict__ tin_i,
                                                     float *__restrict__ tout_r, float *__restrict__ tout_i,
-                                                    double *__restrict__ norms, const uint32_t *__restrict__ zmask,
+                                                    double *__restrict__ norms, const uint2 *__restrict__ zmask,
                                                     int64_t zwords) {
     const int j = blockIdx.y;
     const JobParam P = params[j];
@@ -344,7 +347,7 @@ __global__ __launch_bounds__(256) void probe_kernel(int64_t N, int n, const Diag
         uint32_t live = (1u << RPT) - 1;  // the zero-block map, as in horner_kernel
         if (zmask) {
             const int64_t b0 = static_cast<int64_t>(blockIdx.x) * RPT;
-            live = (zmask[(static_cast<int64_t>(j) * n + d) * zwords + (b0 >> 5)] >> (b0 & 31)) & ((1u << RPT) - 1);
+            live = (any_part(zmask[(static_cast<int64_t>(j) * n + d) * zwords + (b0 >> 5)]) >> (b0 & 31)) & ((1u << RPT) - 1);
             if (!live) continue;  // uniform
         }
         const TV *ar = hre + vb + md.rowbase;
@@ -390,7 +393,7 @@ __global__ __launch_bounds__(256) void probe4_kernel(int64_t N, int n, const Dia
                                                      const float *__restrict__ p32i, const float *__restrict__ tin_r,
                                                      const float *__restrict__ tin_i, float *__restrict__ tout_r,
                                                      float *__restrict__ tout_i, double *__restrict__ norms,
-                                                     const uint32_t *__restrict__ zmask, int64_t zwords) {
+                                                     const uint2 *__restrict__ zmask, int64_t zwords) {
     static_assert(NS == 4 || NS == 8 || NS == 16, "four states per lane");
     constexpr int L = NS / 4, WR = 64 / L, RPP = 4 * WR, T = RPP * R;
     const int j = blockIdx.y;
@@ -412,7 +415,7 @@ __global__ __launch_bounds__(256) void probe4_kernel(int64_t N, int n, const Dia
         if (hi_ <= tile || lo >= tile + T) continue;  // uniform
         uint32_t live = (4 * R >= 32) ? ~0u : ((1u << (4 * R)) - 1);
         if (zmask) {
-            const uint32_t w = zmask[(static_cast<int64_t>(j) * n + d) * zwords + (blk0 >> 5)];
+            const uint32_t w = any_part(zmask[(static_cast<int64_t>(j) * n + d) * zwords + (blk0 >> 5)]);
             live = (4 * R >= 32) ? w : ((w >> (blk0 & 31)) & ((1u << (4 * R)) - 1));
             if (!live) continue;  // uniform
         }
@@ -652,7 +655,7 @@ static void launch_level(const EvoClass &c, int64_t g, hipStream_t s) {
     float *bout_i = (g & 1) ? c.b1i.as<float>() : c.b0i.as<float>();
     const float *bin_r = (g & 1) ? c.b0r.as<float>() : c.b1r.as<float>();
     const float *bin_i = (g & 1) ? c.b0i.as<float>() : c.b1i.as<float>();
-    const uint32_t *zmask = g_evo_skip ? c.zmask.as<uint32_t>() : nullptr;
+    const uint2 *zmask = g_evo_skip ? c.zmask.as<uint2>() : nullptr;
     if constexpr (NS == 4 || NS == 8 || NS == 16) {
         if ((g_evo_vec >= 0 ? g_evo_vec : c.vec) == 1) {  // four states per lane (no LDS window)
             const int64_t rows4 = static_cast<int64_t>(1024 / NS) * rpt;
@@ -734,7 +737,7 @@ static void launch_probe(const EvoClass &c, int kstep, hipStream_t s) {
         hipLaunchKernelGGL((probe4_kernel<TV, NS, R>), grid4, dim3(256), 0, s, N, (int)c.offs.size(),
                            c.d_meta.as<DiagMeta>(), c.total, c.hre.as<TV>(), c.him.as<TV>(),
                            c.d_params.as<JobParam>(), kstep, c.p32r.as<float>(), c.p32i.as<float>(), tin_r, tin_i,
-                           tout_r, tout_i, c.d_probe.as<double>(), g_evo_skip ? c.zmask.as<uint32_t>() : nullptr,
+                           tout_r, tout_i, c.d_probe.as<double>(), g_evo_skip ? c.zmask.as<uint2>() : nullptr,
                            c.zwords);
         DQ_LAUNCH_CHECK();
         return;
@@ -743,7 +746,7 @@ static void launch_probe(const EvoClass &c, int kstep, hipStream_t s) {
     hipLaunchKernelGGL((probe_kernel<TV, NS, R>), grid, dim3(256), 0, s, N, (int)c.offs.size(),
                        c.d_meta.as<DiagMeta>(), c.total, c.hre.as<TV>(), c.him.as<TV>(), c.d_params.as<JobParam>(),
                        kstep, c.p32r.as<float>(), c.p32i.as<float>(), tin_r, tin_i, tout_r, tout_i,
-                       c.d_probe.as<double>(), g_evo_skip ? c.zmask.as<uint32_t>() : nullptr, c.zwords);
+                       c.d_probe.as<double>(), g_evo_skip ? c.zmask.as<uint2>() : nullptr, c.zwords);
     DQ_LAUNCH_CHECK();
 }
 
@@ -917,7 +920,7 @@ extern "C" int dq_evo_create(int n_jobs, dq_devmat *const *H, int n_states, int 
             const int nd = static_cast<int>(c.offs.size());
             const int64_t rpp = 256 / n_states;
             c.zwords = zero_block_words(c.N, static_cast<int>(rpp));
-            c.zmask = DevBuf(sizeof(uint32_t) * std::max<int64_t>(1, c.zwords * nd * c.jobs_n()));
+            c.zmask = DevBuf(sizeof(uint2) * std::max<int64_t>(1, c.zwords * nd * c.jobs_n()));
             if (nd == 0 || c.jobs_n() == 0) continue;
             const dim3 grid(static_cast<unsigned>(c.zwords), zero_map_grid_y(nd), static_cast<unsigned>(c.jobs_n()));
             dispatch(value_precision, n_states, [&](auto tv, auto ns) {
@@ -925,7 +928,7 @@ extern "C" int dq_evo_create(int n_jobs, dq_devmat *const *H, int n_states, int 
                 constexpr int RPP = 256 / decltype(ns)::value;
                 hipLaunchKernelGGL((zero_blocks_kernel<TV, RPP>), grid, dim3(256), 0, nullptr,
                                    static_cast<int64_t>(c.N), nd, c.d_meta.as<DiagMeta>(), c.total, c.hre.as<TV>(),
-                                   c.him.as<TV>(), c.zwords, c.zmask.as<uint32_t>());
+                                   c.him.as<TV>(), c.zwords, c.zmask.as<uint2>());
             });
             DQ_LAUNCH_CHECK();
         }

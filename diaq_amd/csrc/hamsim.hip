@@ -10,23 +10,29 @@
 // (Im h * s, -Re h * s) with s = dt/k, and adds term_k to the step's output; the first term reads psi directly and
 // writes out = psi + term_1, so the copies disappear. Per term: H read once, term_{k-1} read, term_k written and the
 // output read and written once (b*S + 4*b*N bytes). The same operation order as the reference per element:
-// row sums in slot order, then the scaling, then the add. The term kernel may stage the x window of each row tile in
-// LDS: the +-2^k offsets of a qubit Hamiltonian then share one copy of the term vector per tile. Its rows per lane
-// and LDS window are timed on the first evolution of a matrix and kept in the handle.
+// row sums in slot order, then the scaling, then the add. The row sums are dia_rows_wave's; the term kernel may stage
+// the x window of each row tile in LDS: the +-2^k offsets of a qubit Hamiltonian then share one copy of the term vector
+// per tile. Its schedule is timed on the first evolution of a matrix and kept in its handle.
 //
-// Each call first maps the 256-row blocks of every diagonal whose values are all zero (one read of H), and every term
-// skips them: such a block adds nothing to a row sum (the products it would add are zeros, exact in FP64 for finite
-// inputs), and a qubit Hamiltonian's flip diagonals are zero on alternate runs of 2^k rows (three runs in four for a
-// flip-flop term). H cannot change during the call, so the map stays valid for all of its terms.
+// Each call on a large matrix first maps, per 64-row block of every diagonal, whether its real and its imaginary
+// values are all zero (one read of H), and every term skips what is: a zero block adds nothing to a row sum (the
+// products it would add are zeros, exact in FP64 for finite inputs), a zero part is the constant 0. A qubit
+// Hamiltonian's flip diagonals are zero on alternate runs of 2^k rows (three runs in four for a flip-flop term) and
+// its imaginary part often everywhere. H cannot change during the call, so the map stays valid for all of its terms.
+//
+// Bound: reads of the live values. XXZ-20 (156 MB of nonzero real parts of 637 MB stored, and 67 MB of vectors per
+// term): 90.7 us per term with 256-row blocks, both parts read and a metadata chain per diagonal; 45 us now, 4.9 TB/s.
+// XXZ-10: 12.9 -> 5.8 us per term, the launch and three dependent round trips.
 #include <algorithm>
+#include <type_traits>
 
 #include "dia_rows.hpp"
 
 namespace dq {
 
 static int g_hamsim_skip = 1;  // "hamsim_skip_zero_blocks"
-static int g_hamsim_rpt = 0;   // "hamsim_rows_per_lane": 0 = the matrix's timed choice, else 2, 4 or 8
-static int g_hamsim_lds = -1;  // "hamsim_lds": -1 = the matrix's timed choice, else 0 or 1
+static int g_hamsim_rpt = 0;   // "hamsim_rows_per_lane": 0 = the matrix's choice; 2, 4 or 8: two adjacent rows per lane
+static int g_hamsim_lds = -1;  // "hamsim_lds": -1 = the matrix's choice, else 0 or 1 (with two rows per lane)
 
 bool hamsim_set_tuning(const std::string &key, int value) {
     if (key == "hamsim_skip_zero_blocks") {
@@ -51,7 +57,7 @@ bool hamsim_set_tuning(const std::string &key, int value) {
 // TO: the precision of the step output (and of psi, read by the first term). TO = T for an FP64 Hamiltonian. An FP32
 // Hamiltonian (the precision form) runs its terms in FP32 but adds them into an FP64 output; the step's last term
 // also writes the output rounded to FP32 (o32), the next step's FP32 input.
-template <typename T, typename TO, int RPT, bool LDS, bool ZM>
+template <typename T, typename TO, int V, bool NT, bool ZM, bool LDS>
 __global__ __launch_bounds__(256) void taylor_term_kernel(int64_t rows, int n, const DiagMeta *__restrict__ meta,
                                                           const T *__restrict__ are, const T *__restrict__ aim,
                                                           const T *__restrict__ tr, const T *__restrict__ ti,
@@ -59,39 +65,48 @@ __global__ __launch_bounds__(256) void taylor_term_kernel(int64_t rows, int n, c
                                                           TO *__restrict__ outr, TO *__restrict__ outi,
                                                           const TO *__restrict__ p0r, const TO *__restrict__ p0i,
                                                           T *__restrict__ o32r, T *__restrict__ o32i, double scale,
-                                                          int first, int64_t ntiles, int xcd,
-                                                          const uint32_t *__restrict__ zm, int64_t zwords) {
-    constexpr int TILE = 256 * RPT;
-    constexpr int HALO = LDS ? TILE / 2 : 0;
-    constexpr int W = LDS ? TILE + 2 * HALO : 1;
-    __shared__ T sr[W], si[W];
+                                                          int first, int64_t ntiles, int xcd, ZeroMap zm) {
+    constexpr int H = LDS ? 128 * V : 0;
+    __shared__ T sr[LDS ? 256 * V + 2 * H : 1], si[LDS ? 256 * V + 2 * H : 1];
     const int64_t t = tile_of_block(blockIdx.x, ntiles, xcd);
-    if (t >= ntiles) return;  // uniform: a surplus workgroup of the XCD-contiguous grid
-    const int64_t tile = t * TILE;
-    const int64_t tile_end = tile + TILE < rows ? tile + TILE : rows;
-    if constexpr (LDS) stage_x_window<T, RPT, HALO>(tile, rows, tr, ti, sr, si);
-    Acc<T> hr[RPT], hi[RPT];
-    dia_rows_tile<T, RPT, true, true, HALO, ZM>(tile, tile_end, n, meta, are, aim, tr, ti, 0, rows, hr, hi, sr, si,
-                                                zm, zwords);
+    if (t >= ntiles) return;  // uniform
+    if constexpr (LDS) stage_x_window<T, V, H>(t * 256 * V, rows, tr, ti, sr, si);
+    const int64_t row0 = wave_row0<V>(t);
+    if (row0 >= rows) return;  // uniform
+    const int64_t r = row0 + V * (threadIdx.x & 63);
+    // out = psi + term_1 at the first term (psi is the term_0 input), out += term_k after
+    TO orr[V], oii[V];
+    ld_rows(first ? p0r : outr, r, rows, orr);
+    ld_rows(first ? p0i : outi, r, rows, oii);
+    Acc<T> hr[V], hi[V];
+    dia_rows_wave<T, V, NT, ZM, H>(row0, n, meta, are, aim, tr, ti, 0, rows, hr, hi, zm, sr, si);
     const T s = static_cast<T>(scale);
+    T vr[V], vi[V];
 #pragma unroll
-    for (int j = 0; j < RPT; ++j) {
-        const int64_t r = tile + threadIdx.x + 256 * j;
-        if (r < rows) {
-            const T a = hr[j].get(), b = hi[j].get();
-            const T vr = b * s, vi = -a * s;  // (-i s)(a + ib)
-            nr[r] = vr;
-            ni[r] = vi;
-            // out = psi + term_1 at the first term (psi is the term_0 input), out += term_k after
-            const TO orr = (first ? p0r[r] : outr[r]) + static_cast<TO>(vr);
-            const TO oii = (first ? p0i[r] : outi[r]) + static_cast<TO>(vi);
-            outr[r] = orr;
-            outi[r] = oii;
-            if (o32r) {
-                o32r[r] = static_cast<T>(orr);
-                o32i[r] = static_cast<T>(oii);
-            }
+    for (int v = 0; v < V; ++v) {
+        vr[v] = hi[v].get() * s;  // (-i s)(a + ib)
+        vi[v] = -hr[v].get() * s;
+        if constexpr (std::is_same<T, TO>::value) {  // one rounding, spelled out so that every schedule has it
+            orr[v] = __builtin_fma(s, hi[v].get(), orr[v]);
+            oii[v] = __builtin_fma(s, -hr[v].get(), oii[v]);
+        } else {
+            orr[v] += static_cast<TO>(vr[v]);
+            oii[v] += static_cast<TO>(vi[v]);
         }
+    }
+    st_rows(nr, r, rows, vr);
+    st_rows(ni, r, rows, vi);
+    st_rows(outr, r, rows, orr);
+    st_rows(outi, r, rows, oii);
+    if (o32r) {
+        T fr[V], fi[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            fr[v] = static_cast<T>(orr[v]);
+            fi[v] = static_cast<T>(oii[v]);
+        }
+        st_rows(o32r, r, rows, fr);
+        st_rows(o32i, r, rows, fi);
     }
 }
 
@@ -119,72 +134,92 @@ static void convert2(int64_t n, const TS *ar, const TS *ai, TD *br, TD *bi, hipS
     DQ_LAUNCH_CHECK();
 }
 
-// One term: term_k = (-i scale) H in, out (+)= term_k, on tiles of 256 * RPT rows.
-template <typename T, typename TO, int RPT>
-static void launch_term(const dq_devmat &H, bool lds, const T *inr, const T *ini, T *nr, T *ni, TO *outr, TO *outi,
-                        const TO *p0r, const TO *p0i, T *o32r, T *o32i, double scale, int first, const uint32_t *zm,
-                        int64_t zwords, hipStream_t s) {
+// The term kernel's schedule: rows per lane (1 or 2) and non-temporal loads of H's values.
+struct TermSched {
+    int v = 1;
+    bool nt = true, lds = false;
+};
+
+// One term: term_k = (-i scale) H in, out (+)= term_k.
+template <typename T, typename TO>
+static void launch_term(const dq_devmat &H, const TermSched &c, const T *inr, const T *ini, T *nr, T *ni, TO *outr,
+                        TO *outi, const TO *p0r, const TO *p0i, T *o32r, T *o32i, double scale, int first,
+                        const ZeroMap &zm, hipStream_t s) {
     const int64_t N = H.rows;
-    const int64_t ntiles = (N + 256 * RPT - 1) / (256 * RPT);
+    const int64_t ntiles = (N + 256 * c.v - 1) / (256 * c.v);
     const int xcd = xcd_tiles_for(H);
     const dim3 grid(static_cast<unsigned>(grid_for_tiles(ntiles, xcd)));
     const DiagMeta *meta = H.d_meta.as<DiagMeta>();
     const T *are = static_cast<const T *>(H.re.p), *aim = static_cast<const T *>(H.im.p);
-#define DQ_TERM(L, Z)                                                                                             \
-    hipLaunchKernelGGL((taylor_term_kernel<T, TO, RPT, L, Z>), grid, dim3(256), 0, s, N, H.n(), meta, are, aim, inr, \
-                       ini, nr, ni, outr, outi, p0r, p0i, o32r, o32i, scale, first, ntiles, xcd, zm, zwords)
-    if (lds && zm) DQ_TERM(true, true);
-    else if (lds) DQ_TERM(true, false);
-    else if (zm) DQ_TERM(false, true);
-    else DQ_TERM(false, false);
+#define DQ_TERM(V, NT, Z, L)                                                                                          \
+    hipLaunchKernelGGL((taylor_term_kernel<T, TO, V, NT, Z, L>), grid, dim3(256), 0, s, N, H.n(), meta, are, aim, inr, \
+                       ini, nr, ni, outr, outi, p0r, p0i, o32r, o32i, scale, first, ntiles, xcd, zm)
+#define DQ_TERM_V(NT, Z)                                   \
+    do {                                                   \
+        if (c.v == 2 && c.lds) DQ_TERM(2, NT, Z, true);    \
+        else if (c.v == 2) DQ_TERM(2, NT, Z, false);       \
+        else DQ_TERM(1, NT, Z, false);                     \
+    } while (0)
+    if (c.nt && zm.w) DQ_TERM_V(true, true);
+    else if (c.nt) DQ_TERM_V(true, false);
+    else if (zm.w) DQ_TERM_V(false, true);
+    else DQ_TERM_V(false, false);
+#undef DQ_TERM_V
 #undef DQ_TERM
     DQ_LAUNCH_CHECK();
 }
 
-template <typename T, typename TO>
-using TermFn = void (*)(const dq_devmat &, bool, const T *, const T *, T *, T *, TO *, TO *, const TO *, const TO *,
-                        T *, T *, double, int, const uint32_t *, int64_t, hipStream_t);
+// The term kernel's schedule for H: rows per lane, LDS window (where some off-diagonal lies within half a tile) and
+// non-temporal loads. Below EVO_SMALL rows it is one row per lane with plain loads: the matrix is small, the launch
+// is what a term costs, and more and shorter waves shorten it (10 qubits: 5.8 us per term against 7.3 with two rows
+// per lane). Larger matrices time the candidates on two first terms (psi in, scratch out) the first time they are
+// evolved, and keep the choice in the handle: it depends on whether the live values stay in the 256 MB Infinity Cache
+// from term to term (XXZ-20, 156 MB of nonzero real parts: 45 us per term with plain loads, 53 non-temporal; XXZ-22:
+// 235 and 216). Every schedule adds the same products in the same order, so the choice changes the speed only.
+constexpr int64_t EVO_SMALL = int64_t(1) << 16;
 
 template <typename T, typename TO>
-static TermFn<T, TO> term_fn(int rpt) {
-    return rpt == 2 ? launch_term<T, TO, 2> : rpt == 4 ? launch_term<T, TO, 4> : launch_term<T, TO, 8>;
-}
-
-// The term kernel's schedule for H: rows per lane {2, 4, 8} x LDS window {off, on where some off-diagonal lies
-// within half a tile}, each timed on two first terms (psi in, scratch out) the first time H is evolved, and kept in
-// the handle. Every schedule adds the same products in the same order, so the choice changes the speed only.
-template <typename T, typename TO>
-static void term_schedule(const dq_devmat &H, const T *pr, const T *pi, const TO *p0r, const TO *p0i, TO *outr,
-                          TO *outi, T *tr, T *ti, const uint32_t *zm, int64_t zwords, hipStream_t s, int &rpt,
-                          bool &lds) {
-    if (H.term_rpt == 0 && (g_hamsim_rpt == 0 || g_hamsim_lds < 0)) {
+static TermSched term_schedule(const dq_devmat &H, const T *pr, const T *pi, const TO *p0r, const TO *p0i, TO *outr,
+                               TO *outi, T *tr, T *ti, const ZeroMap &zm, hipStream_t s) {
+    if (H.rows < EVO_SMALL) {
+        H.term_nt = 0;
+        H.term_lds = 0;
+        H.term_rpt = 1;
+    }
+    if (H.term_rpt == 0) {
         hipEvent_t e0, e1;
         DQ_HIP(hipEventCreate(&e0));
         DQ_HIP(hipEventCreate(&e1));
         float best = 1e30f;
-        int brpt = 8, blds = 0;
-        for (int r : {2, 4, 8}) {
-            for (int l = 0; l < 2; ++l) {
-                if (l && !lds_window_pays(H, r)) continue;
-                const TermFn<T, TO> f = term_fn<T, TO>(r);
-                f(H, l == 1, pr, pi, tr, ti, outr, outi, p0r, p0i, nullptr, nullptr, 0.1, 1, zm, zwords, s);  // warm
+        TermSched win;
+        for (int form = 0; form < 3; ++form) {
+            if (form == 2 && !lds_window_pays(H, 2)) continue;
+            for (int nt = 0; nt < 2; ++nt) {
+                const TermSched c{form == 0 ? 1 : 2, nt == 1, form == 2};
+                auto one = [&] {
+                    launch_term<T, TO>(H, c, pr, pi, tr, ti, outr, outi, p0r, p0i, nullptr, nullptr, 0.1, 1, zm, s);
+                };
+                one();  // warm
                 DQ_HIP(hipEventRecord(e0, s));
-                for (int q = 0; q < 2; ++q)
-                    f(H, l == 1, pr, pi, tr, ti, outr, outi, p0r, p0i, nullptr, nullptr, 0.1, 1, zm, zwords, s);
+                for (int q = 0; q < 2; ++q) one();
                 DQ_HIP(hipEventRecord(e1, s));
                 DQ_HIP(hipEventSynchronize(e1));
                 float ms = 0.f;
                 DQ_HIP(hipEventElapsedTime(&ms, e0, e1));
-                if (ms < best) { best = ms; brpt = r; blds = l; }
+                if (ms < best) { best = ms; win = c; }
             }
         }
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
-        H.term_lds = blds;  // before term_rpt, which marks the choice as made
-        H.term_rpt = brpt;
+        H.term_nt = win.nt ? 1 : 0;  // before term_rpt, which marks the choice as made
+        H.term_lds = win.lds ? 1 : 0;
+        H.term_rpt = win.v;
     }
-    rpt = g_hamsim_rpt ? g_hamsim_rpt : H.term_rpt.load();
-    lds = g_hamsim_lds >= 0 ? g_hamsim_lds == 1 : H.term_lds.load() == 1;
+    TermSched c;
+    c.v = g_hamsim_rpt ? 2 : H.term_rpt.load();
+    c.lds = g_hamsim_lds >= 0 ? g_hamsim_lds == 1 : H.term_lds.load() == 1;
+    c.nt = H.term_nt.load() == 1;
+    return c;
 }
 
 // One step out = sum_{k=0}^{m} (-i dt H)^k psi / k! (src/spHamSim_gpu_all_fused.cu:235-277). (pr, pi): psi in the
@@ -193,7 +228,7 @@ static void term_schedule(const dq_devmat &H, const T *pr, const T *pi, const TO
 template <typename T, typename TO>
 static void taylor_step(const dq_devmat &H, const T *pr, const T *pi, const TO *p0r, const TO *p0i, TO *outr,
                         TO *outi, T *o32r, T *o32i, T *t0r, T *t0i, T *t1r, T *t1i, double dt, int m,
-                        TermFn<T, TO> term, bool lds, const uint32_t *zm, int64_t zwords, hipStream_t s) {
+                        const TermSched &sched, const ZeroMap &zm, hipStream_t s) {
     const int64_t N = H.rows;
     if (m <= 0 || H.n() == 0) {  // out = psi (+ zero terms)
         hipLaunchKernelGGL(copy2_kernel<TO>, dim3(blocks_for(N, 256, 8192)), dim3(256), 0, s, N, p0r, p0i, outr,
@@ -210,8 +245,8 @@ static void taylor_step(const dq_devmat &H, const T *pr, const T *pi, const TO *
     T *bufr[2] = {t0r, t1r}, *bufi[2] = {t0i, t1i};
     for (int k = 1; k <= m; ++k) {
         T *nr = bufr[k & 1], *ni = bufi[k & 1];
-        term(H, lds, inr, ini, nr, ni, outr, outi, p0r, p0i, k == m ? o32r : nullptr, k == m ? o32i : nullptr,
-             dt / static_cast<double>(k), k == 1 ? 1 : 0, zm, zwords, s);
+        launch_term<T, TO>(H, sched, inr, ini, nr, ni, outr, outi, p0r, p0i, k == m ? o32r : nullptr,
+                           k == m ? o32i : nullptr, dt / static_cast<double>(k), k == 1 ? 1 : 0, zm, s);
         inr = nr;
         ini = ni;
     }
@@ -268,19 +303,17 @@ static void sumsq_parts(int64_t n, const double *re, const double *im, double *p
     DQ_LAUNCH_CHECK();
 }
 
-// The zero-block map of H (256-row blocks), read by every term of one evolution.
-template <typename T>
-static DevBuf zero_map(const dq_devmat &H, int m, int64_t zwords, hipStream_t s) {
-    DevBuf zmap;
-    if (g_hamsim_skip && H.n() > 0 && m > 0) {
-        zmap = DevBuf(sizeof(uint32_t) * zwords * H.n());
-        hipLaunchKernelGGL((zero_blocks_kernel<T, 256>), dim3(static_cast<unsigned>(zwords), zero_map_grid_y(H.n()), 1),
-                           dim3(256), 0, s, (int64_t)H.rows, H.n(), H.d_meta.as<DiagMeta>(), int64_t(0),
-                           static_cast<const T *>(H.re.p), static_cast<const T *>(H.im.p), zwords,
-                           zmap.as<uint32_t>());
-        DQ_LAUNCH_CHECK();
+// The zero-block map of H, read by every term of one evolution; `buf` keeps it. Below EVO_SMALL rows the look-up costs
+// a term more than the skipped loads (8 to 13 qubits: 0.9 to 1.5 us of 5 to 7), so none is made.
+static ZeroMap zero_map(const dq_devmat &H, int m, DevBuf &buf, hipStream_t s) {
+    ZeroMap z;
+    if (g_hamsim_skip && H.n() > 0 && m > 0 && H.rows >= EVO_SMALL) {
+        buf = DevBuf(zero_map_bytes(H, z.shift));
+        make_zero_map(H, z.shift, buf.as<uint2>(), s);
+        z.w = buf.as<uint2>();
+        z.words = zero_block_words(H.rows, 1 << z.shift);
     }
-    return zmap;
+    return z;
 }
 
 // Evolve the device state (pr, pi) in place over r steps of dt = t / r, all in H's precision.
@@ -291,18 +324,15 @@ static void evolve(const dq_devmat &H, T *pr, T *pi, double t, uint64_t r, int m
     const double dt = t / static_cast<double>(r);
     DevBuf br(N * sizeof(T)), bi(N * sizeof(T)), t0r(N * sizeof(T)), t0i(N * sizeof(T)), t1r(N * sizeof(T)),
         t1i(N * sizeof(T));
-    const int64_t zwords = zero_block_words(N, 256);
-    DevBuf zmap = zero_map<T>(H, m, zwords, s);
-    const uint32_t *zm = zmap.p ? zmap.as<uint32_t>() : nullptr;
+    DevBuf zmap;
+    const ZeroMap zm = zero_map(H, m, zmap, s);
     T *ar = pr, *ai = pi, *xr = br.as<T>(), *xi = bi.as<T>();
-    int rpt = 8;
-    bool lds = false;
+    TermSched sched;
     if (m > 0 && H.n() > 0)
-        term_schedule<T, T>(H, pr, pi, pr, pi, xr, xi, t0r.as<T>(), t0i.as<T>(), zm, zwords, s, rpt, lds);
-    const TermFn<T, T> term = term_fn<T, T>(rpt);
+        sched = term_schedule<T, T>(H, pr, pi, pr, pi, xr, xi, t0r.as<T>(), t0i.as<T>(), zm, s);
     for (uint64_t step = 0; step < r; ++step) {
         taylor_step<T, T>(H, ar, ai, ar, ai, xr, xi, nullptr, nullptr, t0r.as<T>(), t0i.as<T>(), t1r.as<T>(),
-                          t1i.as<T>(), dt, m, term, lds, zm, zwords, s);
+                          t1i.as<T>(), dt, m, sched, zm, s);
         std::swap(ar, xr);
         std::swap(ai, xi);
     }
@@ -327,20 +357,16 @@ static void evolve_mixed(const dq_devmat &H, double *pr, double *pi, double t, u
     double *part0 = parts.as<double>(), *part1 = part0 + RENORM_PARTS;
     sumsq_parts(N, pr, pi, part0, s);
     convert2<float, double>(N, pr, pi, p32r.as<float>(), p32i.as<float>(), s);
-    const int64_t zwords = zero_block_words(N, 256);
-    DevBuf zmap = zero_map<float>(H, m, zwords, s);
-    const uint32_t *zm = zmap.p ? zmap.as<uint32_t>() : nullptr;
+    DevBuf zmap;
+    const ZeroMap zm = zero_map(H, m, zmap, s);
     double *ar = pr, *ai = pi, *or_ = xr.as<double>(), *oi = xi.as<double>();
     float *in_r = p32r.as<float>(), *in_i = p32i.as<float>(), *nx_r = q32r.as<float>(), *nx_i = q32i.as<float>();
-    int rpt = 8;
-    bool lds = false;
+    TermSched sched;
     if (m > 0 && H.n() > 0)
-        term_schedule<float, double>(H, in_r, in_i, pr, pi, or_, oi, t0r.as<float>(), t0i.as<float>(), zm, zwords, s,
-                                     rpt, lds);
-    const TermFn<float, double> term = term_fn<float, double>(rpt);
+        sched = term_schedule<float, double>(H, in_r, in_i, pr, pi, or_, oi, t0r.as<float>(), t0i.as<float>(), zm, s);
     for (uint64_t step = 0; step < r; ++step) {
         taylor_step<float, double>(H, in_r, in_i, ar, ai, or_, oi, nx_r, nx_i, t0r.as<float>(), t0i.as<float>(),
-                                   t1r.as<float>(), t1i.as<float>(), dt, m, term, lds, zm, zwords, s);
+                                   t1r.as<float>(), t1i.as<float>(), dt, m, sched, zm, s);
         std::swap(ar, or_);
         std::swap(ai, oi);
         std::swap(in_r, nx_r);

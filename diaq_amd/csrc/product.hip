@@ -20,7 +20,7 @@
 // in parallel and leave each pair's row range and base pointers in LDS, then the pair loop reads them from there
 // (no chain of dependent metadata loads per pair).
 //
-// Zero blocks: for large operands the product first maps which 256-row blocks of each diagonal of A and B hold a
+// Zero blocks: for large operands the product first maps which 64-row blocks of each diagonal of A and B hold a
 // nonzero value (zero_blocks_kernel), and a pair whose A rows, or whose B rows, in the item's chunk are all zero is
 // dropped when its metadata is staged. Its products are all +-0, and a sum that starts at +0 is left unchanged by
 // adding +-0, so the result has the same bits; only a NaN or Inf facing a zero block is not propagated. A qubit
@@ -209,12 +209,12 @@ __device__ inline int64_t uniform64(int64_t v) {
     return static_cast<int64_t>((static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) | static_cast<uint32_t>(lo));
 }
 
-// Whether a 256-row block of the map row z (one diagonal; bit b of word w covers rows 256 (32 w + b) ..) that meets
-// rows [lo, hi) holds a nonzero value.
-__device__ inline bool blocks_live(const uint32_t *__restrict__ z, int64_t lo, int64_t hi) {
-    const int64_t b0 = lo >> 8, b1 = (hi - 1) >> 8;
+// Whether a block of diagonal k's map row that meets rows [lo, hi) holds a nonzero value.
+__device__ inline bool blocks_live(const ZeroMap &z, int64_t k, int64_t lo, int64_t hi) {
+    const uint2 *row = z.w + k * z.words;
+    const int64_t b0 = lo >> z.shift, b1 = (hi - 1) >> z.shift;
     for (int64_t w = b0 >> 5; w <= (b1 >> 5); ++w) {
-        uint32_t m = z[w];
+        uint32_t m = row[w].x | row[w].y;
         if (w == (b0 >> 5)) m &= 0xffffffffu << (b0 & 31);
         if (w == (b1 >> 5)) m &= 0xffffffffu >> (31 - (b1 & 31));
         if (m) return true;
@@ -231,8 +231,7 @@ __global__ __launch_bounds__(256) void product_kernel(const int2 *__restrict__ i
                                                       const T *__restrict__ aim, const T *__restrict__ bre,
                                                       const T *__restrict__ bim, T *__restrict__ cre,
                                                       T *__restrict__ cim, double divisor,
-                                                      const uint32_t *__restrict__ za, int64_t zwa,
-                                                      const uint32_t *__restrict__ zb, int64_t zwb) {
+                                                      ZeroMap za, ZeroMap zb) {
     constexpr int PROD_CHUNK = 256 * PROD_RPT;
     __shared__ int64_t s_abase[PROD_BATCH], s_bbase[PROD_BATCH];
     __shared__ int32_t s_lo[PROD_BATCH], s_hi[PROD_BATCH];
@@ -259,8 +258,8 @@ __global__ __launch_bounds__(256) void product_kernel(const int2 *__restrict__ i
             const int64_t lo = max(max(ta.rlo, tb.rlo - ta.off), r0);
             const int64_t hi = min(min(ta.rhi, tb.rhi - ta.off), r1);
             bool live = hi > lo;
-            if (live && za) live = blocks_live(za + static_cast<int64_t>(sa) * zwa, lo, hi);
-            if (live && zb) live = blocks_live(zb + static_cast<int64_t>(sb) * zwb, lo + ta.off, hi + ta.off);
+            if (live && za.w) live = blocks_live(za, sa, lo, hi);
+            if (live && zb.w) live = blocks_live(zb, sb, lo + ta.off, hi + ta.off);
             s_abase[threadIdx.x] = ta.rowbase;
             s_bbase[threadIdx.x] = tb.rowbase + ta.off;
             s_lo[threadIdx.x] = live ? static_cast<int32_t>(lo - q0) : 0;
@@ -397,26 +396,19 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
     DQ_HIP(hipMemcpyAsync(dsb.p, d.sb.data(), sizeof(int32_t) * d.sb.size(), hipMemcpyHostToDevice, s));
     // zero-block maps of A and B (a squaring maps its operand once; a map the handle keeps is used as it is)
     DevBuf zab, zbb;
-    const uint32_t *za = nullptr, *zb = nullptr;
-    const int64_t zwa = zero_block_words(A.rows, 256), zwb = zero_block_words(B.rows, 256);
+    ZeroMap za, zb;
     if (g_prod_skip && A.rows >= (int64_t(1) << 16) && A.n() > 0 && B.n() > 0) {
-        auto map_of = [&](const dq_devmat &M, int64_t zw, DevBuf &buf) -> const uint32_t * {
-            if (M.zmap_valid && M.zmap.p && M.zmap_words == zw) return M.zmap.as<uint32_t>();
-            buf = DevBuf(sizeof(uint32_t) * static_cast<size_t>(zw) * static_cast<size_t>(M.n()));
-            const dim3 g(static_cast<unsigned>(zw), zero_map_grid_y(M.n()), 1);
-            if (M.precision == DQ_F64)
-                hipLaunchKernelGGL((zero_blocks_kernel<double, 256>), g, dim3(256), 0, s, static_cast<int64_t>(M.rows),
-                                   M.n(), M.d_meta.as<DiagMeta>(), int64_t(0), M.re.as<double>(), M.im.as<double>(),
-                                   zw, buf.as<uint32_t>());
-            else
-                hipLaunchKernelGGL((zero_blocks_kernel<float, 256>), g, dim3(256), 0, s, static_cast<int64_t>(M.rows),
-                                   M.n(), M.d_meta.as<DiagMeta>(), int64_t(0), M.re.as<float>(), M.im.as<float>(), zw,
-                                   buf.as<uint32_t>());
-            DQ_LAUNCH_CHECK();
-            return buf.as<uint32_t>();
+        auto map_of = [&](const dq_devmat &M, DevBuf &buf) {
+            ZeroMap z = kept_zero_map(M);
+            if (z.w) return z;
+            buf = DevBuf(zero_map_bytes(M, z.shift));
+            make_zero_map(M, z.shift, buf.as<uint2>(), s);
+            z.w = buf.as<uint2>();
+            z.words = zero_block_words(M.rows, 1 << z.shift);
+            return z;
         };
-        za = map_of(A, zwa, zab);
-        zb = (&A == &B) ? za : map_of(B, zwb, zbb);
+        za = map_of(A, zab);
+        zb = (&A == &B) ? za : map_of(B, zbb);
     }
     hipLaunchKernelGGL(product_items_kernel, dim3(static_cast<unsigned>(std::min<int64_t>(n_chunks, 65536))),
                        dim3(256), 0, s, n_chunks, dfirst.as<int64_t>(), dclo.as<int32_t>(), dqof.as<int32_t>(),
@@ -427,7 +419,7 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
                        ditems.as<int2>(), dxcd.as<int64_t>(), dps.as<int64_t>(), dsa.as<int32_t>(),               \
                        dsb.as<int32_t>(), A.d_meta.as<DiagMeta>(), B.d_meta.as<DiagMeta>(), C->d_meta.as<DiagMeta>(), \
                        A.re.as<T>(), A.im.as<T>(), B.re.as<T>(), B.im.as<T>(), C->re.as<T>(), C->im.as<T>(), divisor, \
-                       za, zwa, zb, zwb)
+                       za, zb)
 #define DQ_PROD_LAUNCH(T, NTS)                                \
     do {                                                      \
         if (prod_rpt == 4) { DQ_PROD_LAUNCH_R(T, NTS, 4); }   \

@@ -3,8 +3,9 @@
 // Reference: spmv_single_diag_kernel / spmv_row_kernel / spmv_device (src/spMV_gpu.cu:17-168), spmv_host_vectors
 // (:171-183), spMV_ntimes_cuda (src/spMV_ntimes_gpu.cu:61-263).
 //
-// One kernel serves every diagonal count (the reference's one-diagonal kernel gives the same values: y is zero
-// except on the rows of the lone diagonal). A workgroup owns a tile of 256*RPT consecutive rows; lane l of the tile
+// Two kernels serve every diagonal count (the reference's one-diagonal kernel gives the same values: y is zero except
+// on the rows of the lone diagonal): row tiles for large matrices, and the wave form (spmv_wave_kernel) for matrices of
+// up to 2^21 rows and for every product that skips zero blocks (sched_for). In the row tiles a workgroup owns a tile of 256*RPT consecutive rows; lane l of the tile
 // handles rows tile + l + 256*j. For each diagonal (a uniform loop, metadata through scalar loads) the wave reads 64
 // consecutive values of the diagonal (one aligned 512-byte FP64 segment, row-aligned layout) and 64 consecutive
 // values of the shifted x window, so every access is a full, coalesced line. Each row sums its diagonals in slot
@@ -37,16 +38,13 @@ static int g_spmv_pipe = -1;  // load schedule: -1 = automatic, 0 = per-row pred
 static int g_spmv_lds = -1;   // LDS x window: -1 = automatic, 0 = off, 1 = on
 static int g_spmv_xcd = -1;   // tile order: -1 = automatic, 0 = round-robin over the XCDs, 1 = XCD-contiguous
 
-// ZM: zm is a zero-block map of A (256-row blocks, zwords words per diagonal) whose all-zero blocks are skipped: the
-// map dq_spmv_tune keeps in the handle (dropped when the values are rewritten), or one spMV_ntimes makes for a call.
-template <typename T, int RPT, bool NT, bool PIPE, bool LDS, bool ZM>
+template <typename T, int RPT, bool NT, bool PIPE, bool LDS>
 __global__ __launch_bounds__(256) void spmv_rows_kernel(int64_t rows, int64_t cols, int n,
                                                         const DiagMeta *__restrict__ meta, const T *__restrict__ are,
                                                         const T *__restrict__ aim, const T *__restrict__ xr,
                                                         const T *__restrict__ xi, T *__restrict__ yr,
                                                         T *__restrict__ yi, int64_t col_lo, int64_t col_hi,
-                                                        int accumulate, int64_t ntiles, int xcd,
-                                                        const uint32_t *__restrict__ zm, int64_t zwords) {
+                                                        int accumulate, int64_t ntiles, int xcd) {
     constexpr int TILE = 256 * RPT;
     constexpr int HALO = LDS ? TILE / 2 : 0;
     constexpr int W = LDS ? TILE + 2 * HALO : 1;
@@ -64,8 +62,7 @@ __global__ __launch_bounds__(256) void spmv_rows_kernel(int64_t rows, int64_t co
             if (r < rows) { ar[j].add(yr[r]); ai[j].add(yi[r]); }
         }
     }
-    dia_rows_tile<T, RPT, NT, PIPE, HALO, ZM>(tile, tile_end, n, meta, are, aim, xr, xi, col_lo, col_hi, ar, ai, sr,
-                                              si, zm, zwords);
+    dia_rows_tile<T, RPT, NT, PIPE, HALO>(tile, tile_end, n, meta, are, aim, xr, xi, col_lo, col_hi, ar, ai, sr, si);
 #pragma unroll
     for (int j = 0; j < RPT; ++j) {
         const int64_t r = tile + threadIdx.x + 256 * j;
@@ -73,37 +70,99 @@ __global__ __launch_bounds__(256) void spmv_rows_kernel(int64_t rows, int64_t co
     }
 }
 
+// V rows per lane on dia_rows_wave: waves of 64 V rows, four to a workgroup. ZM: zm is a zero-block map of A whose
+// all-zero blocks are skipped: the map dq_spmv_tune keeps in the handle (recomputed when the values are rewritten), or
+// one spMV_ntimes makes for a call.
+template <typename T, int V, bool NT, bool ZM, bool LDS>
+__global__ __launch_bounds__(256) void spmv_wave_kernel(int64_t rows, int64_t cols, int n,
+                                                        const DiagMeta *__restrict__ meta, const T *__restrict__ are,
+                                                        const T *__restrict__ aim, const T *__restrict__ xr,
+                                                        const T *__restrict__ xi, T *__restrict__ yr,
+                                                        T *__restrict__ yi, int64_t col_lo, int64_t col_hi,
+                                                        int accumulate, int64_t ntiles, int xcd, ZeroMap zm) {
+    constexpr int H = LDS ? 128 * V : 0;
+    __shared__ T sr[LDS ? 256 * V + 2 * H : 1], si[LDS ? 256 * V + 2 * H : 1];
+    const int64_t t = tile_of_block(blockIdx.x, ntiles, xcd);
+    if (t >= ntiles) return;  // uniform
+    if constexpr (LDS) stage_x_window<T, V, H>(t * 256 * V, cols, xr, xi, sr, si);
+    const int64_t row0 = wave_row0<V>(t);
+    if (row0 >= rows) return;  // uniform
+    const int64_t r = row0 + V * (threadIdx.x & 63);
+    Acc<T> ar[V], ai[V];
+    if (accumulate) {
+        T br[V], bi[V];
+        ld_rows(yr, r, rows, br);
+        ld_rows(yi, r, rows, bi);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            ar[v].add(br[v]);
+            ai[v].add(bi[v]);
+        }
+    }
+    dia_rows_wave<T, V, NT, ZM, H>(row0, n, meta, are, aim, xr, xi, col_lo, col_hi, ar, ai, zm, sr, si);
+    T outr[V], outi[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        outr[v] = ar[v].get();
+        outi[v] = ai[v].get();
+    }
+    st_rows(yr, r, rows, outr);
+    st_rows(yi, r, rows, outi);
+}
+
+// A complete SpMV schedule: rpt = 1 is the wave form (pipe and lds do not apply to it), 2 to 16 the row tiles.
+struct SpmvSched {
+    int rpt;
+    bool nt, pipe, lds;
+    int xcd;
+    int v = 1;
+};
+
 template <typename T>
-static void launch_rows(const dq_devmat &A, const T *xr, const T *xi, T *yr, T *yi, int rpt, bool nt, bool pipe,
-                        bool lds, int xcd, int64_t c0, int64_t c1, int accumulate, hipStream_t s,
-                        const uint32_t *zm = nullptr, int64_t zwords = 0) {
+static void launch_rows(const dq_devmat &A, const T *xr, const T *xi, T *yr, T *yi, const SpmvSched &c, int64_t c0,
+                        int64_t c1, int accumulate, hipStream_t s, const ZeroMap &zm) {
     const int64_t rows = A.rows, cols = A.cols;
     const DiagMeta *meta = A.d_meta.as<DiagMeta>();
     const T *are = static_cast<const T *>(A.re.p), *aim = static_cast<const T *>(A.im.p);
-    const int64_t ntiles = (rows + 256 * rpt - 1) / (256 * rpt);
-    const int64_t grid = grid_for_tiles(ntiles, xcd);
+    const int64_t ntiles = (rows + 256 * c.rpt - 1) / (256 * c.rpt);
+    const int64_t grid = grid_for_tiles(ntiles, c.xcd);
     if (grid > 0x7fffffffLL) throw ArgError("spmv: too many rows");
-#define DQ_SPMV_LAUNCH_Z(R, NT, PIPE, LDS, Z)                                                                    \
-    hipLaunchKernelGGL((spmv_rows_kernel<T, R, NT, PIPE, LDS, Z>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, \
-                       s, rows, cols, A.n(), meta, are, aim, xr, xi, yr, yi, c0, c1, accumulate, ntiles, xcd, zm,    \
-                       zwords)
-#define DQ_SPMV_LAUNCH(R, NT, PIPE, LDS)                           \
+    const dim3 g(static_cast<unsigned>(grid));
+    if (c.rpt == 1) {
+        const int64_t wtiles = (rows + 256 * c.v - 1) / (256 * c.v);
+        const dim3 wg(static_cast<unsigned>(grid_for_tiles(wtiles, c.xcd)));
+#define DQ_SPMV_WAVE_V(V, NT, Z, L)                                                                                  \
+    hipLaunchKernelGGL((spmv_wave_kernel<T, V, NT, Z, L>), wg, dim3(256), 0, s, rows, cols, A.n(), meta, are, aim, xr, \
+                       xi, yr, yi, c0, c1, accumulate, wtiles, c.xcd, zm)
+#define DQ_SPMV_WAVE(NT, Z)                                        \
     do {                                                           \
-        if (zm) { DQ_SPMV_LAUNCH_Z(R, NT, PIPE, LDS, true); }      \
-        else { DQ_SPMV_LAUNCH_Z(R, NT, PIPE, LDS, false); }        \
+        if (c.v == 2 && c.lds) DQ_SPMV_WAVE_V(2, NT, Z, true);     \
+        else if (c.v == 2) DQ_SPMV_WAVE_V(2, NT, Z, false);        \
+        else DQ_SPMV_WAVE_V(1, NT, Z, false);                      \
     } while (0)
-#define DQ_SPMV_SCHED(R, LDS)                                         \
-    if (nt && pipe) DQ_SPMV_LAUNCH(R, true, true, LDS);               \
-    else if (nt) DQ_SPMV_LAUNCH(R, true, false, LDS);                 \
-    else if (pipe) DQ_SPMV_LAUNCH(R, false, true, LDS);               \
+        if (c.nt && zm.w) DQ_SPMV_WAVE(true, true);
+        else if (c.nt) DQ_SPMV_WAVE(true, false);
+        else if (zm.w) DQ_SPMV_WAVE(false, true);
+        else DQ_SPMV_WAVE(false, false);
+#undef DQ_SPMV_WAVE
+#undef DQ_SPMV_WAVE_V
+        DQ_LAUNCH_CHECK();
+        return;
+    }
+#define DQ_SPMV_LAUNCH(R, NT, PIPE, LDS)                                                                             \
+    hipLaunchKernelGGL((spmv_rows_kernel<T, R, NT, PIPE, LDS>), g, dim3(256), 0, s, rows, cols, A.n(), meta, are, aim, \
+                       xr, xi, yr, yi, c0, c1, accumulate, ntiles, c.xcd)
+#define DQ_SPMV_SCHED(R, LDS)                                           \
+    if (c.nt && c.pipe) DQ_SPMV_LAUNCH(R, true, true, LDS);             \
+    else if (c.nt) DQ_SPMV_LAUNCH(R, true, false, LDS);                 \
+    else if (c.pipe) DQ_SPMV_LAUNCH(R, false, true, LDS);               \
     else DQ_SPMV_LAUNCH(R, false, false, LDS);
 #define DQ_SPMV_CASE(R)                                         \
     case R:                                                     \
-        if (lds) { DQ_SPMV_SCHED(R, true) }                     \
+        if (c.lds) { DQ_SPMV_SCHED(R, true) }                   \
         else { DQ_SPMV_SCHED(R, false) }                        \
         break;
-    switch (rpt) {
-        DQ_SPMV_CASE(1)
+    switch (c.rpt) {
         DQ_SPMV_CASE(2)
         DQ_SPMV_CASE(4)
         DQ_SPMV_CASE(8)
@@ -111,7 +170,6 @@ static void launch_rows(const dq_devmat &A, const T *xr, const T *xi, T *yr, T *
         default: throw ArgError("spmv: rows per lane must be 1, 2, 4, 8 or 16");
     }
 #undef DQ_SPMV_LAUNCH
-#undef DQ_SPMV_LAUNCH_Z
 #undef DQ_SPMV_SCHED
 #undef DQ_SPMV_CASE
     DQ_LAUNCH_CHECK();
@@ -157,25 +215,6 @@ bool lds_window_pays(const dq_devmat &A, int rpt) {
     return near >= 2;
 }
 
-// The schedule of SpMVs that skip A's zero blocks: fewer live diagonals per tile favour smaller tiles and
-// per-row loads (measured on a 24-qubit TFIM: 4 rows per lane, per-row predicated non-temporal loads, LDS window).
-static int skip_rpt_for(const dq_devmat &A) {
-    if (g_spmv_rpt > 0) return g_spmv_rpt;
-    return A.skip_rpt > 0 ? A.skip_rpt : 4;
-}
-static bool skip_nt_for(const dq_devmat &A) {
-    if (g_spmv_nt >= 0) return g_spmv_nt == 1;
-    return A.skip_nt >= 0 ? A.skip_nt == 1 : true;
-}
-static bool skip_pipe_for(const dq_devmat &A) {
-    if (g_spmv_pipe >= 0) return g_spmv_pipe == 1;
-    return A.skip_pipe >= 0 ? A.skip_pipe == 1 : false;
-}
-static bool skip_lds_for(const dq_devmat &A, int rpt) {
-    if (g_spmv_lds >= 0) return g_spmv_lds == 1;
-    return A.skip_lds >= 0 ? A.skip_lds == 1 : lds_window_pays(A, rpt);
-}
-
 int xcd_tiles_for(const dq_devmat &A) {
     if (g_spmv_xcd >= 0) return g_spmv_xcd;
     if (A.tuned_xcd >= 0) return A.tuned_xcd;
@@ -190,17 +229,55 @@ bool lds_window_for(const dq_devmat &A, int rpt) {
     return lds_window_pays(A, rpt);
 }
 
-// A complete SpMV schedule, for callers that choose one explicitly (the tuner's candidates).
-struct SpmvSched {
-    int rpt;
-    bool nt, pipe, lds;
-    int xcd;
-};
+// The untuned schedule for reading A's values from memory once per product. The wave form up to 2^21 rows: below
+// that a 2048-row tile leaves CUs idle or with one wave per SIMD, and each row tile pays a chain of dependent loads per
+// diagonal (TFIM-12: 24 -> 6 us; 100003 rows x 33 random diagonals: 46 -> 12 us; 2^18 rows, TFIM: 48 -> 27 us; at 10^6
+// rows 97 -> 90 us random, 84 -> 87 a band; at 4 10^6 rows the tiles win, 755 against 781 us). Two rows per lane
+// (16-byte loads) from 2^18 rows in FP64, where bytes count more than latency (2^18: equal; 2^20, TFIM: 151 -> 124 us
+// with the LDS window); in FP32 one row per lane (a band of 10^6 rows: 44 us against 55). With a map (fewer values to
+// read) the wave form at any size, FP32 with two rows per lane from 2^21 rows (TFIM-22: 2.00 -> 1.75 ms for 8
+// products). Non-temporal loads when the values exceed the Infinity Cache's 256 MiB (TFIM-18, 155 MB: 27 us plain, 34
+// non-temporal; TFIM-22: 613 and 567); with a map from 640 MiB stored, as about a third of it is live in a real
+// Hamiltonian.
+constexpr int64_t WAVE_ROWS = int64_t(1) << 21, WAVE2_ROWS = int64_t(1) << 18;
 
-// y = A x in n_bands column passes (0: automatic), skipping A's all-zero blocks when zm is given. The schedule is
+static SpmvSched wave_default(const dq_devmat &A, bool map) {
+    const bool f64 = A.precision == DQ_F64;
+    const int64_t bytes = 2 * A.total * elem_bytes(A.precision);
+    SpmvSched c{1, false, false, false, 0};
+    c.v = A.rows >= (f64 ? WAVE2_ROWS : WAVE_ROWS) ? 2 : 1;
+    c.lds = f64 && lds_window_pays(A, 2);
+    c.nt = bytes > (int64_t(map ? 640 : 256) << 20);
+    return c;
+}
+
+static SpmvSched sched_for(const dq_devmat &A, bool map) {
+    SpmvSched c{8, true, true, false, 0};
+    const dq_devmat::WaveSched &w = map ? A.skip_wave : A.tuned_wave;
+    const bool wave = map || (g_spmv_rpt > 0 ? g_spmv_rpt == 1 : A.tuned_rpt > 0 ? w.v > 0 : A.rows < WAVE_ROWS);
+    if (wave) {
+        c = wave_default(A, map);
+        if (w.v > 0) {
+            c.v = w.v;
+            c.nt = w.nt;
+            c.lds = w.lds;
+        }
+        if (g_spmv_nt >= 0) c.nt = g_spmv_nt == 1;
+        if (g_spmv_lds >= 0) c.lds = g_spmv_lds == 1;
+    } else {
+        c.rpt = auto_rpt(A);
+        c.nt = auto_nt(A);
+        c.pipe = auto_pipe(A);
+        c.lds = lds_window_for(A, c.rpt);
+    }
+    c.xcd = xcd_tiles_for(A);
+    return c;
+}
+
+// y = A x in n_bands column passes (0: automatic), skipping A's all-zero blocks when zm has a map. The schedule is
 // `force` if given, else the process-wide knobs, else A's tuned choice, else the defaults.
 void spmv_banded(const dq_devmat &A, const void *xr, const void *xi, void *yr, void *yi, int n_bands,
-                 hipStream_t s, const uint32_t *zm = nullptr, int64_t zwords = 0, const SpmvSched *force = nullptr) {
+                 hipStream_t s, const ZeroMap &zm = ZeroMap(), const SpmvSched *force = nullptr) {
     if (A.rows == 0) return;
     if (A.n() == 0) {  // no diagonals: y = 0 (a fill kernel, safe inside graph capture)
         const unsigned g = blocks_for(A.rows, 256, 4096);
@@ -215,74 +292,82 @@ void spmv_banded(const dq_devmat &A, const void *xr, const void *xi, void *yr, v
     }
     if (n_bands <= 0) n_bands = auto_bands(A);
     if (n_bands > static_cast<int>(A.cols)) n_bands = std::max<int>(1, A.cols);
-    const int rpt = force ? force->rpt : zm ? skip_rpt_for(A) : auto_rpt(A);
-    const bool nt = force ? force->nt : zm ? skip_nt_for(A) : auto_nt(A);
-    const bool pipe = force ? force->pipe : zm ? skip_pipe_for(A) : auto_pipe(A);
-    const bool lds = force ? force->lds : zm ? skip_lds_for(A, rpt) : lds_window_for(A, rpt);
-    const int xcd = force ? force->xcd : xcd_tiles_for(A);
+    const SpmvSched c = force ? *force : sched_for(A, zm.w != nullptr);
     const int64_t cols = A.cols;
     for (int b = 0; b < n_bands; ++b) {
         const int64_t c0 = cols * b / n_bands, c1 = cols * (b + 1) / n_bands;
         if (A.precision == DQ_F64)
-            launch_rows<double>(A, (const double *)xr, (const double *)xi, (double *)yr, (double *)yi, rpt, nt, pipe,
-                                lds, xcd, c0, c1, b > 0, s, zm, zwords);
+            launch_rows<double>(A, (const double *)xr, (const double *)xi, (double *)yr, (double *)yi, c, c0, c1, b > 0,
+                                s, zm);
         else
-            launch_rows<float>(A, (const float *)xr, (const float *)xi, (float *)yr, (float *)yi, rpt, nt, pipe, lds,
-                               xcd, c0, c1, b > 0, s, zm, zwords);
+            launch_rows<float>(A, (const float *)xr, (const float *)xi, (float *)yr, (float *)yi, c, c0, c1, b > 0, s,
+                               zm);
     }
 }
 
 static int g_spmv_skip = 1;  // "spmv_skip_zero_blocks"
 
 // Whether a sequence of n SpMVs on A's values should make its own zero-block map: not for a single product (the map
-// would cost about as much as the product saves), not when the handle already holds a valid one, nor with the skip
-// switched off.
+// would cost about as much as the product saves), not below 2^16 rows (a product is then a launch and a few round
+// trips, and the map's look-up costs it more than the skipped loads), not when the handle already holds a valid one,
+// nor with the skip switched off.
 static bool ntimes_uses_map(const dq_devmat &A, int n) {
-    return g_spmv_skip && n >= 2 && A.n() > 0 && A.rows > 0 && !A.zmap_valid;
+    return g_spmv_skip && n >= 2 && A.n() > 0 && A.rows >= (1u << 16) && !A.zmap_valid;
 }
 
 // The map a product with A may use without making one: the handle's, for FP64 matrices. (In FP64 a skipped block
 // changes no bit; a compensated FP32 sum would change in its last bits, and a single FP32 SpMV keeps the same bits
 // whether or not A was tuned.)
-static const uint32_t *handle_map(const dq_devmat &A) {
-    return (g_spmv_skip && A.zmap_valid && A.precision == DQ_F64) ? A.zmap.as<uint32_t>() : nullptr;
+static ZeroMap handle_map(const dq_devmat &A) {
+    return g_spmv_skip && A.precision == DQ_F64 ? kept_zero_map(A) : ZeroMap();
 }
 
 // The handle's map for a sequence of n products: a single product follows handle_map; two or more use the map in
 // any precision (their results are not compared with a single untuned SpMV's).
-static const uint32_t *sequence_map(const dq_devmat &A, int n) {
+static ZeroMap sequence_map(const dq_devmat &A, int n) {
     if (n == 1) return handle_map(A);
-    return (g_spmv_skip && A.zmap_valid) ? A.zmap.as<uint32_t>() : nullptr;
+    return g_spmv_skip ? kept_zero_map(A) : ZeroMap();
 }
 
-static size_t ntimes_map_bytes(const dq_devmat &A, int64_t &zwords) {
-    zwords = zero_block_words(A.rows, 256);
-    return sizeof(uint32_t) * static_cast<size_t>(zwords) * static_cast<size_t>(A.n());
+ZeroMap kept_zero_map(const dq_devmat &A) {
+    ZeroMap z;
+    if (!A.zmap_valid || !A.zmap.p) return z;
+    z.w = A.zmap.as<uint2>();
+    z.words = zero_block_words(A.rows, 1 << z.shift);
+    return z;
 }
 
-// Whether the map z of A shows a 256-row block, inside some diagonal's rows, whose values are all zero.
-static bool has_zero_blocks(const dq_devmat &A, const uint32_t *z, int64_t zwords, hipStream_t s) {
-    std::vector<uint32_t> h(static_cast<size_t>(zwords) * A.n());
-    DQ_HIP(hipMemcpyAsync(h.data(), z, h.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+size_t zero_map_bytes(const dq_devmat &A, int shift) {
+    return sizeof(uint2) * static_cast<size_t>(zero_block_words(A.rows, 1 << shift)) * static_cast<size_t>(A.n());
+}
+
+// Whether the map z of A shows a block, inside some diagonal's rows, whose real or imaginary values are all zero.
+static bool has_zero_blocks(const dq_devmat &A, const ZeroMap &z, hipStream_t s) {
+    std::vector<uint2> h(static_cast<size_t>(z.words) * A.n());
+    DQ_HIP(hipMemcpyAsync(h.data(), z.w, h.size() * sizeof(uint2), hipMemcpyDeviceToHost, s));
     DQ_HIP(hipStreamSynchronize(s));
     for (int k = 0; k < A.n(); ++k) {
         const DiagMeta &m = A.meta[k];
         if (m.rhi <= m.rlo) continue;
-        for (int64_t b = m.rlo / 256; b <= (m.rhi - 1) / 256; ++b)
-            if (!((h[static_cast<size_t>(k) * zwords + (b >> 5)] >> (b & 31)) & 1u)) return true;
+        for (int64_t b = m.rlo >> z.shift; b <= (m.rhi - 1) >> z.shift; ++b) {
+            const uint2 w = h[static_cast<size_t>(k) * z.words + (b >> 5)];
+            if (!((w.x & w.y) >> (b & 31) & 1u)) return true;
+        }
     }
     return false;
 }
 
-// A's zero-block map (256-row blocks) into z.
-static void ntimes_zero_map(const dq_devmat &A, int64_t zwords, uint32_t *z, hipStream_t s) {
-    const dim3 grid(static_cast<unsigned>(zwords), zero_map_grid_y(A.n()), 1);
-    if (A.precision == DQ_F64)
-        hipLaunchKernelGGL((zero_blocks_kernel<double, 256>), grid, dim3(256), 0, s, static_cast<int64_t>(A.rows),
-                           A.n(), A.d_meta.as<DiagMeta>(), int64_t(0), A.re.as<double>(), A.im.as<double>(), zwords, z);
-    else
-        hipLaunchKernelGGL((zero_blocks_kernel<float, 256>), grid, dim3(256), 0, s, static_cast<int64_t>(A.rows),
-                           A.n(), A.d_meta.as<DiagMeta>(), int64_t(0), A.re.as<float>(), A.im.as<float>(), zwords, z);
+void make_zero_map(const dq_devmat &A, int shift, uint2 *w, hipStream_t s) {
+    const int64_t words = zero_block_words(A.rows, 1 << shift);
+    const dim3 grid(static_cast<unsigned>(words), zero_map_grid_y(A.n()), 1);
+#define DQ_ZERO_MAP(T, BR)                                                                                          \
+    hipLaunchKernelGGL((zero_blocks_kernel<T, BR>), grid, dim3(256), 0, s, static_cast<int64_t>(A.rows), A.n(),      \
+                       A.d_meta.as<DiagMeta>(), int64_t(0), A.re.as<T>(), A.im.as<T>(), words, w)
+    if (A.precision == DQ_F64 && shift == 6) DQ_ZERO_MAP(double, 64);
+    else if (A.precision == DQ_F64) DQ_ZERO_MAP(double, 256);
+    else if (shift == 6) DQ_ZERO_MAP(float, 64);
+    else DQ_ZERO_MAP(float, 256);
+#undef DQ_ZERO_MAP
     DQ_LAUNCH_CHECK();
 }
 
@@ -291,13 +376,12 @@ static void ntimes_zero_map(const dq_devmat &A, int64_t zwords, uint32_t *z, hip
 // replay, and later SpMVs skip exactly the blocks that are zero now (none, if every block became nonzero).
 void refresh_zero_map(dq_devmat &A, hipStream_t s) {
     if (!A.zmap_valid || !A.zmap.p) return;
-    ntimes_zero_map(A, A.zmap_words, A.zmap.as<uint32_t>(), s);
+    make_zero_map(A, ZeroMap().shift, A.zmap.as<uint2>(), s);
 }
 
 // y = A x: the schedule of A, skipping its all-zero blocks when the handle holds their map (see handle_map).
 void spmv(const dq_devmat &A, const void *xr, const void *xi, void *yr, void *yi, hipStream_t s) {
-    const uint32_t *zm = handle_map(A);
-    spmv_banded(A, xr, xi, yr, yi, 0, s, zm, zm ? A.zmap_words : 0);
+    spmv_banded(A, xr, xi, yr, yi, 0, s, handle_map(A));
 }
 
 }  // namespace dq
@@ -363,12 +447,11 @@ extern "C" int dq_spmv_tune(dq_devmat *A, int repeats, uintptr_t stream, float *
             hipEvent_t a, b;
             ~Events() { (void)hipEventDestroy(a); (void)hipEventDestroy(b); }
         } ev{e0, e1};
-        const uint32_t *tz = nullptr;  // the zero-block map while the skip schedule is timed
-        int64_t tzw = 0;
+        ZeroMap tz;  // the zero-block map while the skip schedule is timed
         auto time_it = [&](const SpmvSched &c) {
-            spmv_banded(*A, xr.p, xi.p, yr.p, yi.p, 1, s, tz, tzw, &c);  // warm
+            spmv_banded(*A, xr.p, xi.p, yr.p, yi.p, 1, s, tz, &c);  // warm
             DQ_HIP(hipEventRecord(e0, s));
-            for (int r = 0; r < repeats; ++r) spmv_banded(*A, xr.p, xi.p, yr.p, yi.p, 1, s, tz, tzw, &c);
+            for (int r = 0; r < repeats; ++r) spmv_banded(*A, xr.p, xi.p, yr.p, yi.p, 1, s, tz, &c);
             DQ_HIP(hipEventRecord(e1, s));
             DQ_HIP(hipEventSynchronize(e1));
             float ms = 0.f;
@@ -393,31 +476,40 @@ extern "C" int dq_spmv_tune(dq_devmat *A, int repeats, uintptr_t stream, float *
         if (msx < best) { best = msx; win = wx; }
         A->tuned_rpt = win.rpt; A->tuned_nt = win.nt; A->tuned_pipe = win.pipe; A->tuned_lds = win.lds;
         A->tuned_xcd = win.xcd;
-        // third stage: when A has all-zero blocks, keep their map in the handle and time the schedules that skip
-        // them (used by A's FP64 SpMVs and by spMV_ntimes)
-        A->skip_rpt = win.rpt; A->skip_nt = win.nt; A->skip_pipe = win.pipe; A->skip_lds = win.lds;
+        // the wave forms, in the same order of tiles
+        auto time_waves = [&](float &limit, dq_devmat::WaveSched &to) {
+            to = dq_devmat::WaveSched();
+            for (int form = 0; form < 3; ++form) {
+                if (form == 2 && !lds_window_pays(*A, 2)) continue;
+                for (int nt = 0; nt <= 1; ++nt) {
+                    SpmvSched c{1, nt == 1, false, form == 2, win.xcd};
+                    c.v = form == 0 ? 1 : 2;
+                    const float ms = time_it(c);
+                    if (ms < limit) {
+                        limit = ms;
+                        to.v = c.v;
+                        to.nt = c.nt;
+                        to.lds = c.lds;
+                    }
+                }
+            }
+        };
+        A->tuned_wave = dq_devmat::WaveSched();
+        if (A->rows < 2 * WAVE_ROWS) time_waves(best, A->tuned_wave);  // beyond, the tiles read every block faster
+        // last stage: when A has all-zero blocks or parts and skipping them is faster, keep their map in the handle (used
+        // by A's FP64 SpMVs and by spMV_ntimes)
         A->zmap_valid = false;
+        A->skip_wave = dq_devmat::WaveSched();
         if (g_spmv_skip) {
-            const size_t zb = ntimes_map_bytes(*A, tzw);
+            const size_t zb = zero_map_bytes(*A, tz.shift);
             if (A->zmap.bytes != zb) A->zmap = DevBuf(zb);
-            A->zmap_words = tzw;
-            ntimes_zero_map(*A, tzw, A->zmap.as<uint32_t>(), s);
-            if (has_zero_blocks(*A, A->zmap.as<uint32_t>(), tzw, s)) {
-                tz = A->zmap.as<uint32_t>();
-                float zbest = 1e30f;
-                SpmvSched zw{4, true, false, false, win.xcd};
-                for (int lds = 0; lds <= 1; ++lds)
-                    for (int pipe = 0; pipe <= 1; ++pipe)
-                        for (int rpt : {1, 2, 4, 8, 16})
-                            for (int nt = 0; nt <= 1; ++nt) {
-                                if (lds && !lds_window_pays(*A, rpt)) continue;
-                                const SpmvSched c{rpt, nt == 1, pipe == 1, lds == 1, win.xcd};
-                                const float zms = time_it(c);
-                                if (zms < zbest) { zbest = zms; zw = c; }
-                            }
-                tz = nullptr;
-                A->skip_rpt = zw.rpt; A->skip_nt = zw.nt; A->skip_pipe = zw.pipe; A->skip_lds = zw.lds;
-                A->zmap_valid = true;
+            make_zero_map(*A, tz.shift, A->zmap.as<uint2>(), s);
+            tz.w = A->zmap.as<uint2>();
+            tz.words = zero_block_words(A->rows, 1 << tz.shift);
+            if (has_zero_blocks(*A, tz, s)) {
+                float zbest = best;
+                time_waves(zbest, A->skip_wave);
+                A->zmap_valid = A->skip_wave.v > 0;
             }
         }
         if (best_ms) *best_ms = best;
@@ -504,11 +596,11 @@ extern "C" int dq_spmv_host(const dq_devmat *A, const double *xr, const double *
 }
 
 // y = A^n x on device vectors (src/spMV_ntimes_gpu.cu:61-263 on resident data). `fixed_map` (may be null) is
-// device memory of fixed_words words the call may use for A's zero-block map instead of allocating one: the
+// device memory of fixed_bytes bytes the call may use for A's zero-block map instead of allocating one: the
 // allocation-free entry point passes its static scratch array; then the map is made even while the stream is being
 // captured (the array outlives every replay), and a map that would not fit is an error.
 static void ntimes_device(const dq_devmat *A, const void *xr, const void *xi, void *yr, void *yi, int n, void *work_r,
-                          void *work_i, hipStream_t s, uint32_t *fixed_map, int64_t fixed_words) {
+                          void *work_i, hipStream_t s, uint2 *fixed_map, size_t fixed_bytes) {
     if (!A) throw ArgError("matrix is NULL");
     if (n < 0) throw ArgError("spmv_ntimes_cuda: num_times must be >= 0");
     if (!xr || !xi || !yr || !yi) throw ArgError("spmv_ntimes_device: NULL vector");
@@ -537,21 +629,22 @@ static void ntimes_device(const dq_devmat *A, const void *xr, const void *xi, vo
     // dq_spmv_tune kept in the handle, or else, for two or more products, one made here -- in the caller's fixed
     // memory, or in stream-ordered memory so the call stays asynchronous. Without fixed memory no map is made while
     // the stream is being captured into a graph (a replay must not read memory this call has given back).
-    int64_t zwords = 0;
-    uint32_t *zmap = nullptr;
-    const uint32_t *zuse = sequence_map(*A, n);
-    if (zuse) zwords = A->zmap_words;
-    if (!zuse && ntimes_uses_map(*A, n)) {
-        const size_t bytes = ntimes_map_bytes(*A, zwords);
+    uint2 *zmap = nullptr;
+    ZeroMap z = sequence_map(*A, n);
+    if (!z.w && ntimes_uses_map(*A, n)) {
+        size_t bytes = zero_map_bytes(*A, z.shift);
+        uint2 *to = nullptr;
         if (fixed_map) {
-            if (static_cast<int64_t>(bytes / sizeof(uint32_t)) > fixed_words)
+            if (bytes > fixed_bytes) {  // blocks of 256 rows then
+                z.shift = 8;
+                bytes = zero_map_bytes(*A, z.shift);
+            }
+            if (bytes > fixed_bytes)
                 throw ArgError("spmv_ntimes_device_noalloc: the zero-block map of this matrix needs " +
-                               std::to_string(bytes) + " bytes, more than the " +
-                               std::to_string(fixed_words * sizeof(uint32_t)) +
+                               std::to_string(bytes) + " bytes, more than the " + std::to_string(fixed_bytes) +
                                " bytes of the library's static scratch (tune the matrix with dq_spmv_tune to keep "
                                "its map in the handle, or use dq_spmv_ntimes_device)");
-            ntimes_zero_map(*A, zwords, fixed_map, s);
-            zuse = fixed_map;
+            to = fixed_map;
         } else {
             hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
             DQ_HIP(hipStreamIsCapturing(s, &cap));
@@ -559,18 +652,21 @@ static void ntimes_device(const dq_devmat *A, const void *xr, const void *xi, vo
                 if (hipMallocAsync(reinterpret_cast<void **>(&zmap), bytes, s) != hipSuccess) {
                     (void)hipGetLastError();  // no stream-ordered memory: run without the map
                     zmap = nullptr;
-                } else {
-                    ntimes_zero_map(*A, zwords, zmap, s);
-                    zuse = zmap;
                 }
+                to = zmap;
             }
+        }
+        if (to) {
+            make_zero_map(*A, z.shift, to, s);
+            z.w = to;
+            z.words = zero_block_words(A->rows, 1 << z.shift);
         }
     }
     const void *sr = xr, *si = xi;
     for (int t = 0; t < n; ++t) {
         const bool to_y = (((n - 1 - t) % 2) == 0) != flip;
         void *dr = to_y ? yr : work_r, *di = to_y ? yi : work_i;
-        spmv_banded(*A, sr, si, dr, di, 0, s, zuse, zuse ? zwords : 0);
+        spmv_banded(*A, sr, si, dr, di, 0, s, z);
         sr = dr;
         si = di;
     }
@@ -586,18 +682,19 @@ extern "C" int dq_spmv_ntimes_device(const dq_devmat *A, const void *xr, const v
     return guard([&] { ntimes_device(A, xr, xi, yr, yi, n, work_r, work_i, as_stream(stream), nullptr, 0); });
 }
 
-// The allocation-free form's scratch: room for the zero-block map of a sequence (256-row blocks, one bit each, for
-// every diagonal), 16 MiB per GPU, held from the library's load until the process ends. In host code `scratch` only
-// stands in for the symbol; its device address comes from hipGetSymbolAddress, once per device.
+// The allocation-free form's scratch: room for the zero-block map of a sequence (64-row blocks, or 256-row blocks where
+// those would not fit; two bits each, for every diagonal), 32 MiB per GPU, held from the library's load until the
+// process ends. In host code `scratch` only stands in for the symbol; its device address comes from
+// hipGetSymbolAddress, once per device.
 constexpr int64_t NOALLOC_SCRATCH_WORDS = int64_t(1) << 22;
-static __device__ __align__(256) uint32_t scratch[NOALLOC_SCRATCH_WORDS];
+static __device__ __align__(256) uint2 scratch[NOALLOC_SCRATCH_WORDS];
 
 constexpr int NOALLOC_MAX_DEVICES = 64;
 static std::mutex g_scratch_mu;
-static uint32_t *g_scratch_ptr[NOALLOC_MAX_DEVICES] = {};
+static uint2 *g_scratch_ptr[NOALLOC_MAX_DEVICES] = {};
 
 // This device's copy of `scratch`, looked up on the first call on the device (with that device current).
-static uint32_t *noalloc_scratch() {
+static uint2 *noalloc_scratch() {
     int dev = 0;
     DQ_HIP(hipGetDevice(&dev));
     if (dev < 0 || dev >= NOALLOC_MAX_DEVICES) throw ArgError("spmv_ntimes_device_noalloc: device index out of range");
@@ -605,7 +702,7 @@ static uint32_t *noalloc_scratch() {
     if (!g_scratch_ptr[dev]) {
         void *p = nullptr;
         DQ_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-        g_scratch_ptr[dev] = static_cast<uint32_t *>(p);
+        g_scratch_ptr[dev] = static_cast<uint2 *>(p);
     }
     return g_scratch_ptr[dev];
 }
@@ -614,7 +711,7 @@ extern "C" int dq_spmv_ntimes_device_noalloc(const dq_devmat *A, const void *xr,
                                              int n, void *work_r, void *work_i, uintptr_t stream) {
     return guard([&] {
         ntimes_device(A, xr, xi, yr, yi, n, work_r, work_i, as_stream(stream), noalloc_scratch(),
-                      NOALLOC_SCRATCH_WORDS);
+                      sizeof(uint2) * NOALLOC_SCRATCH_WORDS);
     });
 }
 
@@ -640,18 +737,17 @@ extern "C" int dq_spmv_ntimes_host(const dq_devmat *A, const double *xr, const d
             throw ArgError("spmv_ntimes_cuda: repeated SpMV requires square matrix (M==N) for num_times > 1");
         DevVec a(N, A->precision), b(M, A->precision);
         a.put(xr, xi);
-        int64_t zwords = 0;
         DevBuf zmap;
-        const uint32_t *zuse = sequence_map(*A, n);
-        if (zuse) zwords = A->zmap_words;
-        if (!zuse && ntimes_uses_map(*A, n)) {
-            zmap = DevBuf(ntimes_map_bytes(*A, zwords));
-            ntimes_zero_map(*A, zwords, zmap.as<uint32_t>(), 0);
-            zuse = zmap.as<uint32_t>();
+        ZeroMap z = sequence_map(*A, n);
+        if (!z.w && ntimes_uses_map(*A, n)) {
+            zmap = DevBuf(zero_map_bytes(*A, z.shift));
+            make_zero_map(*A, z.shift, zmap.as<uint2>(), 0);
+            z.w = zmap.as<uint2>();
+            z.words = zero_block_words(A->rows, 1 << z.shift);
         }
         DevVec *in = &a, *out = &b;
         for (int t = 0; t < n; ++t) {
-            spmv_banded(*A, in->r.p, in->i.p, out->r.p, out->i.p, 0, 0, zuse, zuse ? zwords : 0);
+            spmv_banded(*A, in->r.p, in->i.p, out->r.p, out->i.p, 0, 0, z);
             if (t != n - 1) std::swap(in, out);
         }
         out->get(yr, yi);

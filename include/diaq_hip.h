@@ -125,24 +125,25 @@ int dq_spmv_device(const dq_devmat *A, const void *xr_dev, const void *xi_dev, v
 int dq_spmv_host(const dq_devmat *A, const double *xr, const double *xi, double *yr, double *yi);
 
 /* y = A^n x for host vectors, by n SpMVs on the device. Replaces spMV_ntimes_cuda (src/spMV_ntimes_gpu.cu:61-263).
- * For n >= 2 the products skip A's all-zero 256-row blocks (a map made once per call; the same bits in FP64). */
+ * For n >= 2 and at least 2^16 rows the products skip A's all-zero 64-row blocks, and the real or imaginary parts that
+ * are all zero (a map made once per call; the same bits in FP64). */
 int dq_spmv_ntimes_host(const dq_devmat *A, const double *xr, const double *xi, double *yr, double *yi, int n);
 
 /* y = A^num_times x on device vectors of A's precision, asynchronous on `stream`: the reference's spMV_ntimes
  * (src/spMV_ntimes_gpu.cu:61-263, same errors and num_times == 0 / no-diagonal rules) on data that stays resident.
  * work_r / work_i are one more vector of A.rows elements, needed when num_times > 1 or x == y (in place: the result
- * overwrites x); the products alternate between y and the work vectors. For num_times >= 2 the products skip A's
- * all-zero 256-row blocks through a map made once per call in stream-ordered memory (hipMallocAsync), with the
- * schedule dq_spmv_tune chose for that; while `stream` is being captured into a graph no map is made. The FP64 result
- * has the same bits either way. */
+ * overwrites x); the products alternate between y and the work vectors. For num_times >= 2 and at least 2^16 rows the
+ * products skip A's all-zero 64-row blocks and zero real or imaginary parts through a map made once per call in
+ * stream-ordered memory (hipMallocAsync), with the schedule dq_spmv_tune chose for that; while `stream` is being
+ * captured into a graph no map is made. The FP64 result has the same bits either way. */
 int dq_spmv_ntimes_device(const dq_devmat *A, const void *xr, const void *xi, void *yr, void *yi, int num_times,
                           void *work_r, void *work_i, uintptr_t stream);
 
 /* dq_spmv_ntimes_device without any device allocation: the same products, results and errors, but the zero-block map
- * a sequence of two or more products makes for an untuned matrix is written to a static 16 MiB device array of the
+ * a sequence of two or more products makes for an untuned matrix is written to a static 32 MiB device array of the
  * library (one per GPU, held until the process ends) instead of stream-ordered memory, and it is made even while
- * `stream` is being captured into a graph. A map that would not fit (more than 2^22 words: diagonals times
- * ceil(rows / 8192)) is an error; a matrix tuned by dq_spmv_tune uses the map kept in its handle and needs no scratch.
+ * `stream` is being captured into a graph. A map of 64-row blocks that would not fit takes 256-row blocks instead, and
+ * one that then does not fit (more than 2^22 words: diagonals times ceil(rows / 8192)) is an error; a matrix tuned by dq_spmv_tune uses the map kept in its handle and needs no scratch.
  * All calls on one GPU share the array: calls that overlap on one GPU (other streams, other threads) race, and a
  * captured graph that made its map there must not be replayed while another such call runs. No reference
  * counterpart: for callers that cannot allocate device memory (code under graph capture, serving loops). */
@@ -155,17 +156,19 @@ int dq_spmv_device_banded(const dq_devmat *A, const void *xr_dev, const void *xi
                           int n_bands, uintptr_t stream);
 
 /* SpMV autotuner: times every (load schedule, rows per lane, non-temporal loads, LDS x window) candidate `repeats`
- * times on scratch vectors and keeps the fastest in the matrix handle, used by every later SpMV with A. When A has
- * all-zero 256-row blocks it also keeps their map in the handle and the fastest schedule that skips them: later FP64
- * SpMVs with A and spMV_ntimes skip those blocks (the same bits; dq_devmat_set_packed_device recomputes the map for
+ * times on scratch vectors, and the wave forms (one or two rows per lane), and keeps the fastest in the matrix handle,
+ * used by every later SpMV with A. When A has all-zero 64-row blocks, or blocks whose real or imaginary parts are all
+ * zero, and skipping those is faster, it also keeps their map in the handle and the fastest schedule that skips them:
+ * later FP64 SpMVs with A and spMV_ntimes skip those blocks (the same bits; dq_devmat_set_packed_device recomputes the map for
  * the new values, in place and in stream order, so graphs captured earlier stay correct). best_ms (may be NULL)
  * receives the time of the schedule without the skip. The candidates are passed to the kernels directly: SpMVs of
  * other matrices meanwhile keep their schedules, but calls with A itself must not overlap its tuning. No reference
  * counterpart. */
 int dq_spmv_tune(dq_devmat *A, int repeats, uintptr_t stream, float *best_ms);
 
-/* The SpMV schedule A currently uses (after tuning or the defaults); any output pointer may be NULL. No reference
- * counterpart. */
+/* The row-tile schedule of A's SpMVs (after tuning or the defaults); any output pointer may be NULL. Products that run
+ * in the wave form instead (untuned: fewer than 2^21 rows, or a zero-block map; tuned: where it was faster) use its
+ * tile order only. No reference counterpart. */
 int dq_spmv_tuned_config(const dq_devmat *A, int *rows_per_lane, int *nontemporal, int *pipelined, int *lds_window,
                          int *xcd_tiles);
 
@@ -176,14 +179,14 @@ int dq_spmv_tuned_config(const dq_devmat *A, int *rows_per_lane, int *nontempora
 int dq_release_cached_memory(void);
 
 /* Process-wide tuning knobs for the autotuner and benchmarks: "spmv_rows_per_lane" (0 = automatic, or 1, 2, 4, 8,
- * 16), "spmv_bands" (0 = automatic, or the number of column bands), "spmv_nontemporal" (-1 = automatic, 0, 1:
+ * 16: 1 is the wave form, a wave's 64 rows with one metadata read per 64 diagonals), "spmv_bands" (0 = automatic, or the number of column bands), "spmv_nontemporal" (-1 = automatic, 0, 1:
  * stream the matrix values with non-temporal loads), "spmv_pipelined" (-1 = automatic, 0 = per-row predicated
  * loads, 1 = batched loads), "spmv_lds" (-1 = automatic, 0, 1: stage the x window of each row tile in LDS for the
  * diagonals within half a tile) and "spmv_xcd" (-1 = automatic, 0 = row tiles round-robin over the XCDs, 1 = each
  * XCD a contiguous eighth of the tiles) override a matrix's tuned SpMV schedule; "product_interleave" (0, 1 = default: row
  * chunks of a product interleaved over the XCDs) and "product_nt_store" (0, 1 = default: non-temporal stores of the
  * product's values), "product_rows_per_lane" (0 = default: 4 below 2^16 rows, else 8; or 4, 8, 16: row chunks of 256 x that) and
- * "product_skip_zero_blocks" (1 = default: for operands of at least 2^16 rows, map their all-zero 256-row blocks and
+ * "product_skip_zero_blocks" (1 = default: for operands of at least 2^16 rows, map their all-zero 64-row blocks and
  * drop the pairs whose rows in a chunk are all zero, same bits; 0 = read every pair) set the SpGEMM kernel's schedule; "evo_rows_per_lane" (0 = tuned, or 1, 2, 4, 8), "evo_xcd"
  * (-1 = tuned, 0, 1), "evo_lds" (-1 = tuned, 0, 1) and "evo_vec" (-1 = tuned, 0 = a lane per state, 1 = four states
  * per lane for 4, 8 or 16 states) and "evo_diag_batch" (0 = tuned, or 1, 2, 4: the diagonals whose loads the
@@ -193,7 +196,8 @@ int dq_release_cached_memory(void);
  * and "evo_skip_zero_blocks" (1 = default: skip the blocks of a diagonal whose values are all zero; 0 = read them);
  * "spmv_skip_zero_blocks" (1 = default, 0) and "hamsim_skip_zero_blocks" (1 = default, 0) do the same for the
  * SpMV (the map dq_spmv_tune keeps, and spMV_ntimes's own) and for the fused evolution's Taylor terms, whose schedule
- * "hamsim_rows_per_lane" (0 = timed per matrix, or 2, 4, 8) and "hamsim_lds" (-1 = timed, 0, 1) override;
+ * "hamsim_rows_per_lane" (0 = chosen per matrix; 2, 4 or 8 = two adjacent rows per lane) and "hamsim_lds" (-1 =
+ * chosen, 0, 1: with two rows per lane) override;
  * "spmm_tiled" (0 = not tiled, the default; 1, 2, 4 = LDS-tiled with that many elements per lane) and
  * "spmm_cols_per_lane" (0 = automatic: 2 for an even n_right, else 1; 1, 2, 4, 8; -1 = one C element per lane),
  * "spmm_rows_per_lane" (-1 = automatic: 2 for >= 32768 rows and an even n_right >= 64, else 0; 0 = off; 2, 4, 8: the
