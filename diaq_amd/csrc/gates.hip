@@ -1,14 +1,27 @@
 // Sequences of gates on a state vector (a Trotter step is one), applied in fused passes over HBM.
 //
 // Applying the gates one at a time (dq_kron_apply_device) streams the whole state through HBM once per gate. Here the
-// sequence is cut into passes. A pass loads tiles of 2^L amplitudes into LDS, applies every gate of its stretch of
-// the sequence to the tile in order, and writes the tile back: one HBM round trip for the whole stretch.
+// sequence is cut into passes. A pass loads tiles of 2^L amplitudes into registers, applies every gate of its stretch
+// of the sequence to the tile in order, and writes the tile back: one HBM round trip for the whole stretch.
 //
 // A tile is the set of amplitudes that agree on every qubit outside the pass's tile qubits T (|T| = L). T holds the
 // qubits of the stretch's non-diagonal gates, filled up with the lowest remaining qubits; the planner keeps qubits
-// 0..low-1 in T (low = 5 by default), so each tile is made of runs of at least 2^low contiguous amplitudes. A gate
-// whose only diagonal is the main one joins any pass: it multiplies each amplitude by the entry that the amplitude's
-// own index selects, wherever its qubits lie.
+// 0..low-1 in T, so each tile is made of runs of at least 2^low contiguous amplitudes. A gate whose only diagonal is
+// the main one joins any pass: it multiplies each amplitude by the entry that the amplitude's own index selects,
+// wherever its qubits lie.
+//
+// Layout. A workgroup of 256 lanes holds a tile, 2^R amplitudes per lane (R = L - 8), with a window of R consecutive
+// tile bits [a, a + R) in the register index and the other 8 bits in the lane index. A gate inside the window works on
+// the lane's own registers, with its entries in scalar registers; when the next gate lies outside, the planner puts a
+// step that moves the tile to another window through LDS (real parts, then imaginary parts, through one padded buffer
+// of 2^L values, 34 KB in FP64). A diagonal gate runs in any window: the lane's part of
+// its index is the same for all the lane's amplitudes, so it looks up one entry per value of the gate's qubits that lie
+// in the window (1, 2 or 4 for a two-qubit gate) and not one per amplitude.
+//
+// What bounds it: HBM for passes of few gates (28 qubits: 1.85 ms for 8 one-qubit gates, 4.6 TB/s; 2.42 ms when the tile's
+// runs lie 8 MB and more apart), vector issue for full ones (27 diagonal and 12 one-qubit gates: 3.37 ms, of which
+// 1.6 ms FP64 instructions). A first-order TFIM-28 step: 3 passes, 7.2 ms; 15.4 ms in 4 passes when the tiles lived in
+// LDS and every gate read and wrote them there.
 //
 // Each gate's arithmetic on each amplitude is the single-gate kernel's (each row adds its terms in the order of the
 // gate's diagonal slots, with the rounding sequence of dia_rows.hpp), and the order of the gates is kept, so the
@@ -16,6 +29,7 @@
 // plan copies the gates' values: the gates may be freed after planning.
 #include <algorithm>
 #include <cmath>
+#include <utility>
 #include <vector>
 
 #include "dia_rows.hpp"
@@ -23,378 +37,366 @@
 
 namespace dq {
 
-constexpr int GATES_MAX_K = 4;  // gates on up to four qubits (16 x 16)
-constexpr int PASS_MAX_GATES = 64, PASS_MAX_ROWPTR = 512, PASS_MAX_TERMS = 512;  // per pass, staged in LDS
+constexpr int GATES_MAX_K = 4;      // gates on up to four qubits (16 x 16)
+constexpr int PASS_MAX_GATES = 64;  // gates per pass
+constexpr int PASS_MAX_DIAG = 512;  // entries of a pass's diagonal gates, staged in LDS
+constexpr int GATE_MAX_TERMS = 512; // nonzero terms of one gate
 
-// A gate as the kernel sees it. Its terms are listed row by row: row r of the gate adds, in the order of the gate's
-// diagonal slots, value * x[c] for each term (c, value) in [rowptr[rp + r], rowptr[rp + r + 1]) (indexes local to the
-// pass). kind 0: a one- or two-qubit general gate on tile bits p .. p + k - 1; 1: main diagonal only, applied per
-// amplitude; 2: main diagonal only on qubits outside the tile, so one factor per tile. Non-diagonal gates on three or
-// four qubits get a pass of their own, run by the single-gate kernel (the fused kernel then needs no registers for
-// 8- and 16-row columns).
-struct GateOp {
-    int k, q, p, kind, rp;
+// One step of a pass. Non-diagonal gates on three or four qubits are no steps: they get a pass of their own, run by
+// the single-gate kernel.
+// Two kinds take several gates: where the code of different kinds meets the compiler copies every amplitude, so a stretch
+// of gates without a meeting point costs less than its steps one by one.
+enum { STEP_MOVE = 0, STEP_DIAG = 1, STEP_FULL2 = 2, STEP_ROWS2 = 3, STEP_ROWS4 = 4, STEP_RUN = 5, STEP_LAYER = 6,
+       STEP_FULL4 = 7, STEP_MASK2 = 8, STEP_MASK4 = 9 };
+struct GateStep {
+    int kind;
+    int a;     // STEP_MOVE: the new window; STEP_DIAG: which register bits the gate's qubits are (see diag_step)
+    int q, k;  // STEP_DIAG: first qubit, qubits
+    int j;     // the gate's first register bit; STEP_DIAG: the gate bit of register bit `a`
+    int at;    // STEP_DIAG: its first entry in the pass's LDS table; STEP_FULL*, STEP_MASK*: its entries (row-major,
+               // absent ones too) in terms;
+               // STEP_LAYER: the entries of full one-qubit gates on register bits 0 .. R - 1, one after the other
+    int end;   // STEP_ROWS*: its terms are [at, end); STEP_MASK*: bit r * rows + c: entry (r, c) is a term; STEP_RUN: this and the next end - 1 steps are diagonal gates on
+               // no register bit
+    int pad_;
 };
 
 struct PassHdr {
-    int n_gates, n_rowptr, n_terms, nc;
+    int n_steps, n_diag, nc, a0;  // steps; entries of the LDS table; qubits outside the tile; the first window
     int single, single_q;      // single >= 0: this pass is gate `single` of the plan's own copies, on qubits from single_q
     int tpos[16];              // tile bit i -> global qubit (ascending)
     int cpos[48];              // tile index bit m -> global qubit, for the qubits outside the tile (ascending)
-    int64_t gop, rowptr, term;  // first GateOp / rowptr entry / term of this pass in the plan's arrays
+    int64_t step, diag;        // first step / diagonal entry of this pass in the plan's arrays
 };
 
 template <typename T>
 struct GateTerm {
     T re, im;
-    int c, pad_;
+    int rc, pad_;  // row * rows + column
+};
+template <typename T>
+struct GateVal {
+    T re, im;
 };
 
-// A general gate on tile bits [p, p + k): columns of the tile as in the single-gate kernel, with 2^p in place of
-// 2^after. A lane takes CPT columns at a time so that each term read from LDS serves all of them; the rows' sums stay
-// in registers until every row of the column is done (the column is updated in place).
-template <typename T, int L, int GM>
-__device__ inline void tile_gate(const GateOp &G, const int *rowptr, const GateTerm<T> *terms, T *sr, T *si) {
-    constexpr int KG = GM == 2 ? 1 : GM == 4 ? 2 : GM == 8 ? 3 : 4;
-    constexpr int NCOL = 1 << (L - KG);
-    constexpr int CPT = NCOL >= 1024 ? 4 : NCOL >= 512 ? 2 : 1;
-    const int p = G.p;
-    for (int u0 = threadIdx.x; u0 < NCOL; u0 += 256 * CPT) {
-        int base[CPT];
+// f(0), .., f(N - 1) with constant arguments: the amplitude arrays stay in registers only if every index is a constant.
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_seq(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F &&f) {
+    static_for_seq(f, std::make_integer_sequence<int, N>{});
+}
+
+// Ends the code of one of several window variants: the variants' stores would otherwise be merged into one sequence
+// over a choice of addresses, which puts the amplitudes into memory.
+#define DQ_VARIANT_END(id) asm volatile("; variant %0" ::"n"(id))
+
+// LDS place of tile element e: one value of padding per 16, so that every window's lanes hit different banks. The
+// register and lane parts of e have no bit in common, so their places add up.
+__device__ inline int tile_place(int e) { return e + (e >> 4); }
+
+// Tile element of lane t with register index 0 in window a.
+template <int R>
+__device__ inline int lane_elem_of(int t, int a) {
+    return (t & ((1 << a) - 1)) | ((t >> a) << (a + R));
+}
+
+// Global index bits of lane t's part of the tile in window a.
+template <int R>
+__device__ inline int64_t lane_index(const PassHdr &P, int t, int a) {
+    int64_t v = 0;
 #pragma unroll
-        for (int i = 0; i < CPT; ++i) {
-            const int u = u0 + 256 * i;
-            base[i] = ((u >> p) << (p + KG)) | (u & ((1 << p) - 1));
+    for (int i = 0; i < 8; ++i) v |= static_cast<int64_t>((t >> i) & 1) << P.tpos[i < a ? i : i + R];
+    return v;
+}
+
+// Global index bits of register index m in window a (uniform).
+template <int R>
+__device__ inline int64_t reg_index(const PassHdr &P, int m, int a) {
+    int64_t v = 0;
+#pragma unroll
+    for (int b = 0; b < R; ++b) v |= static_cast<int64_t>((m >> b) & 1) << P.tpos[a + b];
+    return v;
+}
+
+// x = v x with the single-gate kernel's rounding, but for the sign of a zero: its sums start at +0, so its zeros are +0.
+// Signs of zeros change no other value, so one plus_zero before the store gives its bits.
+// The fmas write over x: left to itself the compiler accumulates into the product and copies the result back, two moves
+// per amplitude and gate.
+__device__ __forceinline__ void fma_over(double &x, double a, double c) {  // x = a x + c
+    asm("v_fma_f64 %0, %1, %0, %2" : "+v"(x) : "v"(a), "v"(c));
+}
+__device__ __forceinline__ void fma_over(float &x, float a, float c) {
+    asm("v_fma_f32 %0, %1, %0, %2" : "+v"(x) : "v"(a), "v"(c));
+}
+template <typename T>
+__device__ __forceinline__ void scale_amp(const GateVal<T> &v, T &xr, T &xi) {
+    const T nr = -(v.im * xi), ni = v.im * xr;
+    fma_over(xr, v.re, nr);
+    fma_over(xi, v.re, ni);
+}
+template <typename T>
+__device__ __forceinline__ T plus_zero(T v) {
+    return v + T(0);
+}
+
+// A diagonal gate. ct: the lane's part of the gate's index. S.a = 0: no register bit is one of its qubits; 1 + b:
+// register bit b alone is (its gate bit S.j); 1 + R + b: register bits b and b + 1 are gate bits 0 and 1; else
+// (a gate on three or four qubits) S.j holds, per register bit, 1 + its gate bit in 4 bits.
+template <typename T, int R, int B>
+__device__ __forceinline__ void diag_step(const GateStep &S, const GateVal<T> *tab, int ct, T (&xr)[1 << R],
+                                          T (&xi)[1 << R]) {
+    constexpr int E = 1 << R;
+    if constexpr (B < R) {
+        if (S.a == 1 + B) {
+            const GateVal<T> v0 = tab[ct], v1 = tab[ct | (1 << S.j)];
+            static_for<E>([&](auto m) { scale_amp((m >> B) & 1 ? v1 : v0, xr[m], xi[m]); });
+            DQ_VARIANT_END(B);
+        } else if (B + 1 < R && S.a == 1 + R + B) {
+            const GateVal<T> v0 = tab[ct], v1 = tab[ct | 1], v2 = tab[ct | 2], v3 = tab[ct | 3];
+            static_for<E>([&](auto m) {
+                constexpr int c = (m >> B) & 3;
+                scale_amp(c == 0 ? v0 : c == 1 ? v1 : c == 2 ? v2 : v3, xr[m], xi[m]);
+            });
+            DQ_VARIANT_END(16 + B);
+        } else {
+            diag_step<T, R, B + 1>(S, tab, ct, xr, xi);
         }
-        Acc<T> ar[CPT][GM], ai[CPT][GM];
-#pragma unroll
-        for (int r = 0; r < GM; ++r) {
-            const int t1 = rowptr[G.rp + r + 1];
-            for (int t = rowptr[G.rp + r]; t < t1; ++t) {
-                const GateTerm<T> w = terms[t];
-#pragma unroll
-                for (int i = 0; i < CPT; ++i) {
-                    if (u0 + 256 * i < NCOL) {
-                        const int a = base[i] + (w.c << p);
-                        cmac(ar[i][r], ai[i][r], w.re, w.im, sr[a], si[a]);
-                    }
-                }
+    } else if (S.a == 0) {
+        const GateVal<T> v = tab[ct];
+        static_for<E>([&](auto m) { scale_amp(v, xr[m], xi[m]); });
+        DQ_VARIANT_END(32);
+    } else {
+        static_for<E>([&](auto m) {
+            int c = ct;
+            for (int b = 0; b < R; ++b) {
+                const int g = (S.j >> (4 * b)) & 15;
+                if (((m >> b) & 1) && g) c |= 1 << (g - 1);
             }
-        }
-#pragma unroll
-        for (int i = 0; i < CPT; ++i) {
-            if (u0 + 256 * i < NCOL) {
-#pragma unroll
-                for (int r = 0; r < GM; ++r) {
-                    sr[base[i] + (r << p)] = ar[i][r].get();
-                    si[base[i] + (r << p)] = ai[i][r].get();
-                }
-            }
-        }
+            scale_amp(tab[c], xr[m], xi[m]);
+        });
+        DQ_VARIANT_END(33);
     }
 }
 
-template <typename T, int L>
-__global__ __launch_bounds__(256) void gates_pass_kernel(const PassHdr *__restrict__ hdr,
-                                                         const GateOp *__restrict__ gops,
-                                                         const int *__restrict__ rowptrs,
-                                                         const GateTerm<T> *__restrict__ terms_g, T *re, T *im,
-                                                         int64_t ntiles) {
-    constexpr int E = (1 << L) / 256;  // amplitudes per lane
-    __shared__ T sr[1 << L], si[1 << L];
-    __shared__ GateOp sg[PASS_MAX_GATES];
-    __shared__ int srp[PASS_MAX_ROWPTR];
-    __shared__ GateTerm<T> st[PASS_MAX_TERMS];
-    const PassHdr &P = *hdr;
-    const int ng = P.n_gates;
-    for (int i = threadIdx.x; i < ng; i += blockDim.x) sg[i] = gops[P.gop + i];
-    for (int i = threadIdx.x; i < P.n_rowptr; i += blockDim.x) srp[i] = rowptrs[P.rowptr + i];
-    for (int i = threadIdx.x; i < P.n_terms; i += blockDim.x) st[i] = terms_g[P.term + i];
-    // global offset of tile element e = deposit of e's bits at the tile qubits
-    int64_t off[E];
-#pragma unroll
-    for (int m = 0; m < E; ++m) {
-        const int e = threadIdx.x + 256 * m;
-        int64_t v = 0;
-#pragma unroll
-        for (int i = 0; i < L; ++i) v |= static_cast<int64_t>((e >> i) & 1) << P.tpos[i];
-        off[m] = v;
+// A one-qubit gate with all four entries g (row-major) on register bit B.
+template <typename T, int R, int B>
+__device__ __forceinline__ void full2_gate(const GateTerm<T> *__restrict__ g, T (&xr)[1 << R], T (&xi)[1 << R]) {
+    const T g0r = g[0].re, g0i = g[0].im, g1r = g[1].re, g1i = g[1].im;
+    const T g2r = g[2].re, g2i = g[2].im, g3r = g[3].re, g3i = g[3].im;
+    static_for<(1 << R) / 2>([&](auto c) {
+        constexpr int m = (c & ((1 << B) - 1)) | ((c >> B) << (B + 1)), n = m | (1 << B);
+        // a compensated FP32 sum of two terms is their plain sum
+        T ar, ai, br, bi, cr, ci, dr, di;
+        cmul(g0r, g0i, xr[m], xi[m], ar, ai);
+        cmul(g1r, g1i, xr[n], xi[n], br, bi);
+        cmul(g2r, g2i, xr[m], xi[m], cr, ci);
+        cmul(g3r, g3i, xr[n], xi[n], dr, di);
+        xr[m] = ar + br;
+        xi[m] = ai + bi;
+        xr[n] = cr + dr;
+        xi[n] = ci + di;
+    });
+}
+
+// The same on register bit j.
+template <typename T, int R, int B>
+__device__ __forceinline__ void full2_step(int j, const GateTerm<T> *__restrict__ g, T (&xr)[1 << R],
+                                           T (&xi)[1 << R]) {
+    if constexpr (B < R) {
+        if (j != B) {
+            full2_step<T, R, B + 1>(j, g, xr, xi);
+            return;
+        }
+        full2_gate<T, R, B>(g, xr, xi);
+        DQ_VARIANT_END(48 + B);
     }
+}
+
+// A gate of 2^K rows on register bits [j, j + K) whose rows take their terms in ascending column order: the entries g
+// are row-major, entry (r, c) is a term where bit r * rows + c of mask is set (FULL: all are). The lane's columns are
+// taken in two halves, whose sums fit beside the amplitudes.
+template <typename T, int R, int K, bool FULL, int B>
+__device__ __forceinline__ void grid_step(int j, int mask, const GateTerm<T> *__restrict__ g, T (&xr)[1 << R],
+                                          T (&xi)[1 << R]) {
+    if constexpr (B + K <= R) {
+        if (j != B) {
+            grid_step<T, R, K, FULL, B + 1>(j, mask, g, xr, xi);
+            return;
+        }
+        constexpr int G = 1 << K, NC = 1 << (R - K), H = NC < 2 ? NC : NC / 2;
+        static_for<NC / H>([&](auto half) {
+            Acc<T> ar[H][G], ai[H][G];
+            static_for<G>([&](auto r) {
+                static_for<G>([&](auto c) {
+                    if (FULL || ((mask >> (r * G + c)) & 1)) {  // uniform
+                        const T wr = g[r * G + c].re, wi = g[r * G + c].im;
+                        static_for<H>([&](auto u) {
+                            constexpr int col = half * H + u;
+                            constexpr int at = (col & ((1 << B) - 1)) | ((col >> B) << (B + K)) | (c << B);
+                            if constexpr (FULL && c == 0) {  // the first term: adding it to 0 changes a zero's sign only
+                                cmul(wr, wi, xr[at], xi[at], ar[u][r].s, ai[u][r].s);
+                            } else {
+                                cmac(ar[u][r], ai[u][r], wr, wi, xr[at], xi[at]);
+                            }
+                        });
+                        if constexpr (!FULL) DQ_VARIANT_END(4096 + 64 * half + r * G + c);
+                    }
+                });
+            });
+            static_for<H>([&](auto u) {
+                constexpr int col = half * H + u;
+                static_for<G>([&](auto r) {
+                    constexpr int at = (col & ((1 << B) - 1)) | ((col >> B) << (B + K)) | (r << B);
+                    xr[at] = ar[u][r].get();
+                    xi[at] = ai[u][r].get();
+                });
+            });
+        });
+        DQ_VARIANT_END(128 + 32 * K + 16 * (FULL ? 1 : 0) + B);
+    }
+}
+
+// A gate of 2^K rows on register bits [j, j + K), its terms [t0, t1) listed row by row in slot order: term (r, c, value)
+// adds value * x[c] to row r. The lane's columns are taken in two halves, whose sums fit beside the amplitudes.
+template <typename T, int R, int K, int B>
+__device__ __forceinline__ void rows_step(int j, int t0, int t1, const GateTerm<T> *__restrict__ terms,
+                                          T (&xr)[1 << R], T (&xi)[1 << R]) {
+    if constexpr (B + K <= R) {
+        if (j != B) {
+            rows_step<T, R, K, B + 1>(j, t0, t1, terms, xr, xi);
+            return;
+        }
+        constexpr int G = 1 << K, NC = 1 << (R - K), H = NC < 2 ? NC : NC / 2;  // H columns per half
+        static_for<NC / H>([&](auto half) {
+            Acc<T> ar[H][G], ai[H][G];
+            for (int t = t0; t < t1; ++t) {  // uniform
+                const int rc = terms[t].rc;
+                const T wr = terms[t].re, wi = terms[t].im;
+                static_for<G * G>([&](auto id) {
+                    if (rc == id) {  // uniform
+                        static_for<H>([&](auto u) {
+                            constexpr int col = half * H + u, r = id / G, c = id % G;
+                            constexpr int at = (col & ((1 << B) - 1)) | ((col >> B) << (B + K)) | (c << B);
+                            cmac(ar[u][r], ai[u][r], wr, wi, xr[at], xi[at]);
+                        });
+                        DQ_VARIANT_END(1024 + 256 * half + id);
+                    }
+                });
+            }
+            static_for<H>([&](auto u) {
+                constexpr int col = half * H + u;
+                static_for<G>([&](auto r) {
+                    constexpr int at = (col & ((1 << B) - 1)) | ((col >> B) << (B + K)) | (r << B);
+                    xr[at] = ar[u][r].get();
+                    xi[at] = ai[u][r].get();
+                });
+            });
+        });
+        DQ_VARIANT_END(64 + 16 * K + B);
+    }
+}
+
+// At least three waves per SIMD: 12-qubit tiles at 172 VGPRs had two, and the passes above took 3.69 and 2.62 ms.
+template <typename T, int L>
+__global__ __launch_bounds__(256, 3) void gates_pass_kernel(const PassHdr *__restrict__ hdr,
+                                                         const GateStep *__restrict__ steps,
+                                                         const GateTerm<T> *__restrict__ terms,
+                                                         const GateVal<T> *__restrict__ diag, T *re, T *im,
+                                                         int64_t ntiles) {
+    constexpr int R = L - 8, E = 1 << R;
+    __shared__ T buf[(1 << L) + (1 << L) / 16];
+    __shared__ GateVal<T> tab[PASS_MAX_DIAG];
+    const PassHdr &P = *hdr;
+    const int tid = threadIdx.x;
+    for (int i = tid; i < P.n_diag; i += 256) tab[i] = diag[P.diag + i];
+    const GateStep *__restrict__ st = steps + P.step;
     __syncthreads();
     for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
         int64_t base = 0;
         for (int i = 0; i < P.nc; ++i) base |= ((t >> i) & 1) << P.cpos[i];
-#pragma unroll
-        for (int m = 0; m < E; ++m) {
-            const int e = threadIdx.x + 256 * m;
-            sr[e] = re[base + off[m]];
-            si[e] = im[base + off[m]];
-        }
-        bool own = true;  // the LDS entries this lane last wrote are its own elements e = tid + 256 m
-        __syncthreads();
-        for (int j = 0; j < ng; ++j) {
-            const GateOp G = sg[j];
-            if (G.kind == 0) {
-                __syncthreads();
-                if (G.k == 1) tile_gate<T, L, 2>(G, srp, st, sr, si);
-                else tile_gate<T, L, 4>(G, srp, st, sr, si);
-                own = false;
-            } else {
-                // a run of diagonal gates: each amplitude goes through all of them in registers, gate by gate with
-                // the same rounding as one at a time (kind 2, qubits outside the tile: the index bits come from
-                // `base` alone, so c is the same for the whole tile)
-                if (!own) __syncthreads();
-                own = true;
-                int j2 = j;
-                while (j2 + 1 < ng && (sg[j2 + 1].kind == 1 || sg[j2 + 1].kind == 2)) ++j2;
-                T xr[E], xi[E];
-#pragma unroll
-                for (int m = 0; m < E; ++m) {
-                    xr[m] = sr[threadIdx.x + 256 * m];
-                    xi[m] = si[threadIdx.x + 256 * m];
-                }
-#pragma unroll 1
-                for (int jj = j; jj <= j2; ++jj) {
-                    const GateOp D = sg[jj];
-                    const GateTerm<T> *row = st + srp[D.rp];  // one term per row: row c's term is row[c]
-                    const int mask = (1 << D.k) - 1;
-#pragma unroll
-                    for (int m = 0; m < E; ++m) {
-                        const GateTerm<T> w = row[static_cast<int>(((base + off[m]) >> D.q) & mask)];
-                        Acc<T> ar, ai;
-                        cmac(ar, ai, w.re, w.im, xr[m], xi[m]);
-                        xr[m] = ar.get();
-                        xi[m] = ai.get();
-                    }
-                }
-#pragma unroll
-                for (int m = 0; m < E; ++m) {
-                    sr[threadIdx.x + 256 * m] = xr[m];
-                    si[threadIdx.x + 256 * m] = xi[m];
-                }
-                j = j2;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int m = 0; m < E; ++m) {
-            const int e = threadIdx.x + 256 * m;
-            re[base + off[m]] = sr[e];
-            im[base + off[m]] = si[e];
-        }
-        __syncthreads();  // the next tile reuses the LDS
-    }
-}
-
-// ------------------------------------------------------------------------------------------------------------------
-// Register layout: a lane keeps its E amplitudes of the tile (tile element e = threadIdx.x + 256 m) in registers for
-// the whole pass. Tile bits 0..5 are lane bits within a wave, 6..7 the wave, 8.. the register index m. A gate on lane
-// bits takes its partners by cross-lane shuffles, one on register bits from the lane's own registers, and only a
-// gate touching a wave bit exchanges through LDS. Each lane computes the rows of the amplitudes it owns, with the
-// same terms in the same order as the single-gate kernel, so the bits are the same.
-// ------------------------------------------------------------------------------------------------------------------
-// Row r of a gate over operands v[0..GM): the terms of the row in slot order.
-template <typename T, int GM>
-__device__ inline void gate_row(const int *rowptr, const GateTerm<T> *terms, int rp, int r, const T (&vr)[GM],
-                                const T (&vi)[GM], T &out_r, T &out_i) {
-    Acc<T> ar, ai;
-    const int t1 = rowptr[rp + r + 1];
-    for (int t = rowptr[rp + r]; t < t1; ++t) {
-        const GateTerm<T> w = terms[t];
-        T xr = vr[0], xi = vi[0];
-#pragma unroll
-        for (int c = 1; c < GM; ++c) {
-            if (w.c == c) {
-                xr = vr[c];
-                xi = vi[c];
-            }
-        }
-        cmac(ar, ai, w.re, w.im, xr, xi);
-    }
-    out_r = ar.get();
-    out_i = ai.get();
-}
-
-// A gate of 2^K rows on tile bits [p, p + K) inside the lane bits (p + K <= 6): partners by shuffles.
-template <typename T, int E, int K>
-__device__ inline void regs_gate_lanes(const GateOp &G, const int *rowptr, const GateTerm<T> *terms, T (&xr)[E],
-                                       T (&xi)[E]) {
-    constexpr int GM = 1 << K;
-    const int lane = threadIdx.x & 63;
-    const int r = (lane >> G.p) & (GM - 1);
-#pragma unroll
-    for (int m = 0; m < E; ++m) {
-        // partner d (d = c xor r, 1 <= d < GM) sits in lane lane ^ (d << p): one exchange per partner, the same
-        // masks for every lane
-        T wr[GM], wi[GM];
-        wr[0] = xr[m];
-        wi[0] = xi[m];
-#pragma unroll
-        for (int dd = 1; dd < GM; ++dd) {
-            wr[dd] = __shfl_xor(xr[m], dd << G.p);
-            wi[dd] = __shfl_xor(xi[m], dd << G.p);
-        }
-        T vr[GM], vi[GM];
-#pragma unroll
-        for (int c = 0; c < GM; ++c) {
-            vr[c] = wr[0];
-            vi[c] = wi[0];
-#pragma unroll
-            for (int dd = 1; dd < GM; ++dd) {
-                if ((c ^ r) == dd) {
-                    vr[c] = wr[dd];
-                    vi[c] = wi[dd];
-                }
-            }
-        }
-        gate_row<T, GM>(rowptr, terms, G.rp, r, vr, vi, xr[m], xi[m]);
-    }
-}
-
-// A gate of 2^K rows on register bits [RB, RB + K) of m: the partners are the lane's own registers.
-template <typename T, int E, int K, int RB>
-__device__ inline void regs_gate_regs(const GateOp &G, const int *rowptr, const GateTerm<T> *terms, T (&xr)[E],
-                                      T (&xi)[E]) {
-    constexpr int GM = 1 << K;
-    if constexpr (RB + K <= 31 && (E >> (RB + K)) >= 1) {
-#pragma unroll
-        for (int m0 = 0; m0 < E; ++m0) {
-            if (m0 & ((GM - 1) << RB)) continue;
-            T vr[GM], vi[GM], yr[GM], yi[GM];
-#pragma unroll
-            for (int c = 0; c < GM; ++c) {
-                vr[c] = xr[m0 | (c << RB)];
-                vi[c] = xi[m0 | (c << RB)];
-            }
-#pragma unroll
-            for (int r = 0; r < GM; ++r) gate_row<T, GM>(rowptr, terms, G.rp, r, vr, vi, yr[r], yi[r]);
-#pragma unroll
-            for (int c = 0; c < GM; ++c) {
-                xr[m0 | (c << RB)] = yr[c];
-                xi[m0 | (c << RB)] = yi[c];
-            }
-        }
-    }
-}
-
-template <typename T, int E, int K, int RB>
-__device__ inline void regs_gate_regs_dispatch(int rb, const GateOp &G, const int *rowptr, const GateTerm<T> *terms,
-                                               T (&xr)[E], T (&xi)[E]) {
-    if constexpr ((1 << (RB + K)) <= E) {
-        if (rb == RB) regs_gate_regs<T, E, K, RB>(G, rowptr, terms, xr, xi);
-        else regs_gate_regs_dispatch<T, E, K, RB + 1>(rb, G, rowptr, terms, xr, xi);
-    }
-}
-
-template <typename T, int L>
-__global__ __launch_bounds__(256) void gates_regs_kernel(const PassHdr *__restrict__ hdr,
-                                                         const GateOp *__restrict__ gops,
-                                                         const int *__restrict__ rowptrs,
-                                                         const GateTerm<T> *__restrict__ terms_g, T *re, T *im,
-                                                         int64_t ntiles) {
-    constexpr int E = (1 << L) / 256;  // amplitudes per lane
-    __shared__ T sr[1 << L], si[1 << L];  // only for gates that touch the wave bits 6 and 7
-    __shared__ GateOp sg[PASS_MAX_GATES];
-    __shared__ int srp[PASS_MAX_ROWPTR];
-    __shared__ GateTerm<T> st[PASS_MAX_TERMS];
-    const PassHdr &P = *hdr;
-    const int ng = P.n_gates;
-    for (int i = threadIdx.x; i < ng; i += blockDim.x) sg[i] = gops[P.gop + i];
-    for (int i = threadIdx.x; i < P.n_rowptr; i += blockDim.x) srp[i] = rowptrs[P.rowptr + i];
-    for (int i = threadIdx.x; i < P.n_terms; i += blockDim.x) st[i] = terms_g[P.term + i];
-    int64_t off[E];
-#pragma unroll
-    for (int m = 0; m < E; ++m) {
-        const int e = threadIdx.x + 256 * m;
-        int64_t v = 0;
-#pragma unroll
-        for (int i = 0; i < L; ++i) v |= static_cast<int64_t>((e >> i) & 1) << P.tpos[i];
-        off[m] = v;
-    }
-    __syncthreads();
-    for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-        int64_t base = 0;
-        for (int i = 0; i < P.nc; ++i) base |= ((t >> i) & 1) << P.cpos[i];
+        int a = P.a0;
+        asm volatile("" : "+s"(a));  // 2^R register offsets per window: made again per tile, not kept from tile to tile
+        int64_t idx = base | lane_index<R>(P, tid, a);
         T xr[E], xi[E];
-#pragma unroll
-        for (int m = 0; m < E; ++m) {
-            xr[m] = re[base + off[m]];
-            xi[m] = im[base + off[m]];
-        }
-        for (int j = 0; j < ng; ++j) {
-            const GateOp G = sg[j];
-            if (G.kind != 0) {  // diagonal: per amplitude, from its own index
-                const GateTerm<T> *row = st + srp[G.rp];
-                const int mask = (1 << G.k) - 1;
-#pragma unroll
-                for (int m = 0; m < E; ++m) {
-                    const GateTerm<T> w = row[static_cast<int>(((base + off[m]) >> G.q) & mask)];
-                    Acc<T> ar, ai;
-                    cmac(ar, ai, w.re, w.im, xr[m], xi[m]);
-                    xr[m] = ar.get();
-                    xi[m] = ai.get();
+        static_for<E>([&](auto m) {
+            const int64_t om = reg_index<R>(P, m, a);
+            xr[m] = (re + om)[idx];
+            xi[m] = (im + om)[idx];
+        });
+        for (int s = 0; s < P.n_steps; ++s) {  // uniform
+            const GateStep S = st[s];
+            if (S.kind == STEP_RUN) {
+                for (int i = 0; i < S.end; ++i) {  // uniform
+                    const GateStep D = st[s + i];
+                    const int ct = static_cast<int>(idx >> D.q) & ((1 << D.k) - 1);
+                    const GateVal<T> v = tab[D.at + ct];
+                    static_for<E>([&](auto m) { scale_amp(v, xr[m], xi[m]); });
                 }
-            } else if (G.p + G.k <= 6) {
-                if (G.k == 1) regs_gate_lanes<T, E, 1>(G, srp, st, xr, xi);
-                else regs_gate_lanes<T, E, 2>(G, srp, st, xr, xi);
-            } else if (G.p >= 8) {
-                if (G.k == 1) regs_gate_regs_dispatch<T, E, 1, 0>(G.p - 8, G, srp, st, xr, xi);
-                else regs_gate_regs_dispatch<T, E, 2, 0>(G.p - 8, G, srp, st, xr, xi);
-            } else {  // touches a wave bit: exchange through LDS
-                __syncthreads();  // earlier readers of the LDS copy are done
-#pragma unroll
-                for (int m = 0; m < E; ++m) {
-                    sr[threadIdx.x + 256 * m] = xr[m];
-                    si[threadIdx.x + 256 * m] = xi[m];
-                }
+                s += S.end - 1;
+                DQ_VARIANT_END(40);
+            } else if (S.kind == STEP_LAYER) {
+                static_for<R>([&](auto b) { full2_gate<T, R, b>(terms + S.at + 4 * b, xr, xi); });
+                DQ_VARIANT_END(41);
+            } else if (S.kind == STEP_DIAG) {
+                const int ct = static_cast<int>(idx >> S.q) & ((1 << S.k) - 1);
+                diag_step<T, R, 0>(S, tab + S.at, ct, xr, xi);
+            } else if (S.kind == STEP_FULL2) {
+                full2_step<T, R, 0>(S.j, terms + S.at, xr, xi);
+            } else if (S.kind == STEP_FULL4) {
+                grid_step<T, R, 2, true, 0>(S.j, 0, terms + S.at, xr, xi);
+            } else if (S.kind == STEP_MASK2) {
+                grid_step<T, R, 1, false, 0>(S.j, S.end, terms + S.at, xr, xi);
+            } else if (S.kind == STEP_MASK4) {
+                grid_step<T, R, 2, false, 0>(S.j, S.end, terms + S.at, xr, xi);
+            } else if (S.kind == STEP_MOVE) {
+                const int to = S.a;
+                const int w = tile_place(lane_elem_of<R>(tid, a)), r = tile_place(lane_elem_of<R>(tid, to));
+                static_for<E>([&](auto m) { buf[w + tile_place(m << a)] = xr[m]; });
                 __syncthreads();
-                const int GM = 1 << G.k;
-#pragma unroll
-                for (int m = 0; m < E; ++m) {
-                    const int e = threadIdx.x + 256 * m;
-                    const int r = (e >> G.p) & (GM - 1);
-                    Acc<T> ar, ai;
-                    const int t1 = srp[G.rp + r + 1];
-                    for (int tt = srp[G.rp + r]; tt < t1; ++tt) {
-                        const GateTerm<T> w = st[tt];
-                        const int a = e ^ ((w.c ^ r) << G.p);
-                        cmac(ar, ai, w.re, w.im, sr[a], si[a]);
-                    }
-                    xr[m] = ar.get();
-                    xi[m] = ai.get();
-                }
+                static_for<E>([&](auto m) { xr[m] = buf[r + tile_place(m << to)]; });
+                __syncthreads();
+                static_for<E>([&](auto m) { buf[w + tile_place(m << a)] = xi[m]; });
+                __syncthreads();
+                static_for<E>([&](auto m) { xi[m] = buf[r + tile_place(m << to)]; });
+                __syncthreads();  // the next move, of this tile or the next, writes the buffer again
+                a = to;
+                idx = base | lane_index<R>(P, tid, a);
+            } else if (S.kind == STEP_ROWS2) {
+                rows_step<T, R, 1, 0>(S.j, S.at, S.end, terms, xr, xi);
+            } else {
+                rows_step<T, R, 2, 0>(S.j, S.at, S.end, terms, xr, xi);
             }
         }
-#pragma unroll
-        for (int m = 0; m < E; ++m) {
-            re[base + off[m]] = xr[m];
-            im[base + off[m]] = xi[m];
-        }
-        __syncthreads();  // the next tile's LDS exchanges start after every lane is done with this one's
+        static_for<E>([&](auto m) {
+            const int64_t om = reg_index<R>(P, m, a);
+            (re + om)[idx] = plus_zero(xr[m]);
+            (im + om)[idx] = plus_zero(xi[m]);
+        });
     }
 }
 
 }  // namespace dq
 
-// A planned gate sequence: passes, gate ops, row pointers and terms (copies of the gates' values), built once and run
-// any number of times.
+// A planned gate sequence: passes, steps, terms and diagonal entries (copies of the gates' values), built
+// once and run any number of times.
 struct dq_gate_plan {
-    int n_qubits = 0, precision = DQ_F64, L = 11, kernel = 0;
+    int n_qubits = 0, precision = DQ_F64, L = 11;
     std::vector<dq::PassHdr> passes;
     std::vector<std::unique_ptr<dq_devmat>> big;  // copies of the non-diagonal gates on three or four qubits
-    dq::DevBuf d_passes, d_gops, d_rowptr, d_terms;
+    dq::DevBuf d_passes, d_steps, d_terms, d_diag;
 };
 
 namespace dq {
 
-static int g_gates_tile_qubits = 11;  // dq_set_tuning "gates_tile_qubits": 10, 11 or 12
-static int g_gates_low_qubits = 5;    // dq_set_tuning "gates_low_qubits": 4, 5 or 6 (qubits always in a tile)
-static int g_gates_kernel = 0;        // dq_set_tuning "gates_kernel": 0 = LDS tiles, 1 = register layout
+static int g_gates_tile_qubits = 0;  // dq_set_tuning "gates_tile_qubits": 10, 11 or 12; 0 (not set) = automatic
+static int g_gates_low_qubits = 0;   // dq_set_tuning "gates_low_qubits": 4, 5 or 6 (qubits always in a tile); 0: automatic
 
 bool gates_set_tuning(const std::string &key, int value) {
-    if (key == "gates_kernel") {
+    if (key == "gates_kernel") {  // kept for callers: there is one pass kernel
         if (value != 0 && value != 1) throw ArgError("gates_kernel must be 0 or 1");
-        g_gates_kernel = value;
         return true;
     }
     if (key == "gates_low_qubits") {
@@ -457,15 +459,62 @@ static HostGate host_gate(const dq_devmat &G, int k, int q) {
     return H;
 }
 
+// Where window [a, a + R) starts for a gate on tile bits [p, p + k), given the non-diagonal gates that follow it in the
+// pass (first tile bit, qubits): the place that holds the most of them, the highest of those (windows from bit 4 up
+// keep runs of 16 amplitudes in the lanes, so the pass can store from them).
+static int best_window(const std::vector<std::pair<int, int>> &gates, size_t i, int L, int R) {
+    const int p = gates[i].first, k = gates[i].second;
+    int best = -1, held = -1;
+    for (int a = std::max(0, p + k - R); a <= std::min(p, L - R); ++a) {
+        int n = 0;
+        for (size_t j = i; j < gates.size() && gates[j].first >= a && gates[j].first + gates[j].second <= a + R; ++j) ++n;
+        if (n >= held) {
+            held = n;
+            best = a;
+        }
+    }
+    return best;
+}
+
+// Turns stretches of the steps from `from` on into steps of several gates: diagonal gates on no register bit into
+// STEP_RUN, full one-qubit gates on register bits 0, 1, .. R - 1 in turn (whose entries follow each other) into STEP_LAYER.
+static void merge_steps(std::vector<GateStep> &steps, size_t from, int R) {
+    std::vector<GateStep> out;
+    for (size_t i = from; i < steps.size();) {
+        size_t e = i;
+        while (e < steps.size() && steps[e].kind == STEP_DIAG && steps[e].a == 0) ++e;
+        if (e > i) {
+            for (size_t j = i; j < e; ++j) out.push_back(steps[j]);
+            GateStep &first = out[out.size() - (e - i)];
+            first.kind = STEP_RUN;
+            first.end = static_cast<int>(e - i);
+            i = e;
+            continue;
+        }
+        while (e < steps.size() && e - i < static_cast<size_t>(R) && steps[e].kind == STEP_FULL2 &&
+               steps[e].j == static_cast<int>(e - i) && steps[e].at == steps[i].at + 4 * static_cast<int>(e - i))
+            ++e;
+        out.push_back(steps[i]);
+        if (e - i == static_cast<size_t>(R)) {
+            out.back().kind = STEP_LAYER;
+            i = e;
+        } else {
+            ++i;
+        }
+    }
+    steps.resize(from);
+    steps.insert(steps.end(), out.begin(), out.end());
+}
+
 // Greedy cut of the sequence into passes: a non-diagonal gate joins the current pass while the qubits of the pass's
-// non-diagonal gates, together with qubits 0..low-1, number at most L, and while the pass's tables fit in LDS.
+// non-diagonal gates, together with qubits 0..low-1, number at most L, and while the pass's diagonal entries fit in LDS.
 template <typename T>
-static void plan_passes(dq_gate_plan &P, const std::vector<HostGate> &gates,
+static void plan_passes(dq_gate_plan &P, int low_qubits, const std::vector<HostGate> &gates,
                         const std::vector<const dq_devmat *> &devgates) {
-    const int n = P.n_qubits, L = P.L;
-    std::vector<GateOp> ops;
-    std::vector<int> rowptr;
+    const int n = P.n_qubits, L = P.L, R = L - 8;
+    std::vector<GateStep> steps;
     std::vector<GateTerm<T>> terms;
+    std::vector<GateVal<T>> diag;
     auto close = [&](int g0, int g1, uint64_t S) {
         if (g1 <= g0) return;
         uint64_t Tm = S;
@@ -478,39 +527,109 @@ static void plan_passes(dq_gate_plan &P, const std::vector<HostGate> &gates,
             else D.cpos[c++] = b;
         }
         D.nc = c;
-        D.gop = static_cast<int64_t>(ops.size());
-        D.rowptr = static_cast<int64_t>(rowptr.size());
-        D.term = static_cast<int64_t>(terms.size());
-        int nrp = 0, nt = 0;
+        D.step = static_cast<int64_t>(steps.size());
+        D.diag = static_cast<int64_t>(diag.size());
+        std::vector<std::pair<int, int>> moving;  // the non-diagonal gates' tile bits (consecutive, as their qubits are)
+        for (int j = g0; j < g1; ++j) {
+            if (gates[j].diag) continue;
+            int pos = 0;
+            while (D.tpos[pos] != gates[j].q) ++pos;
+            moving.push_back({pos, gates[j].k});
+        }
+        const int stored = L - R;  // the last window
+        int a = stored;
+        if (!moving.empty()) {
+            const int w = best_window(moving, 0, L, R);
+            if (w >= 4) a = w;
+        }
+        D.a0 = a;
+        size_t im = 0;
         for (int j = g0; j < g1; ++j) {
             const HostGate &H = gates[j];
-            GateOp op{};
-            op.k = H.k;
-            op.q = H.q;
-            op.rp = nrp;
-            const uint64_t Q = ((uint64_t(1) << H.k) - 1) << H.q;
+            GateStep st{};
             if (H.diag) {
-                op.kind = (Q & Tm) ? 1 : 2;
+                st.kind = STEP_DIAG;
+                st.q = H.q;
+                st.k = H.k;
+                st.at = static_cast<int>(static_cast<int64_t>(diag.size()) - D.diag);
+                int bits = 0, first = -1, packed = 0;
+                for (int b = 0; b < R; ++b) {
+                    const int g = D.tpos[a + b] - H.q;  // gate bit of register bit b
+                    if (g < 0 || g >= H.k) continue;
+                    ++bits;
+                    if (first < 0) first = b;
+                    packed |= (g + 1) << (4 * b);
+                }
+                if (bits == 0) {
+                    st.a = 0;
+                } else if (bits == 1) {
+                    st.a = 1 + first;
+                    st.j = D.tpos[a + first] - H.q;
+                } else if (bits == 2 && H.k == 2) {  // tile bits ascend with the qubits: gate bits 0 and 1
+                    st.a = 1 + R + first;
+                } else {
+                    st.a = 1 + 2 * R;
+                    st.j = packed;
+                }
+                for (size_t t = 0; t < H.col.size(); ++t)
+                    diag.push_back(GateVal<T>{static_cast<T>(H.vre[t]), static_cast<T>(H.vim[t])});
             } else {
-                int pos = 0;
-                while (D.tpos[pos] != H.q) ++pos;
-                op.p = pos;  // the gate's qubits are consecutive, so are their tile bits
+                const auto [p, k] = moving[im];
+                if (p < a || p + k > a + R) {
+                    GateStep mv{};
+                    mv.kind = STEP_MOVE;
+                    mv.a = a = best_window(moving, im, L, R);
+                    steps.push_back(mv);
+                }
+                ++im;
+                st.j = p - a;
+                const int t0 = static_cast<int>(terms.size());
+                // rows whose terms ascend in column order (two terms add up to the same bits in either order) need no
+                // list of terms, only which entries they are
+                const int g = 1 << k;
+                bool ascending = true;
+                for (int r = 0; r < g; ++r)
+                    for (int t = H.rowptr[r] + 1; t < H.rowptr[r + 1]; ++t)
+                        ascending = ascending && H.col[t] != H.col[t - 1] && (k == 1 || H.col[t] > H.col[t - 1]);
+                for (int r = 0; r < g; ++r) ascending = ascending && H.rowptr[r + 1] - H.rowptr[r] <= g;
+                if (ascending) {
+                    terms.resize(terms.size() + static_cast<size_t>(g) * g, GateTerm<T>{T(0), T(0), 0, 0});
+                    int mask = 0;
+                    for (int r = 0; r < g; ++r)
+                        for (int t = H.rowptr[r]; t < H.rowptr[r + 1]; ++t) {
+                            mask |= 1 << (r * g + H.col[t]);
+                            terms[t0 + r * g + H.col[t]].re = static_cast<T>(H.vre[t]);
+                            terms[t0 + r * g + H.col[t]].im = static_cast<T>(H.vim[t]);
+                        }
+                    const bool full = mask == (1 << (g * g)) - 1;
+                    st.kind = k == 1 ? (full ? STEP_FULL2 : STEP_MASK2) : (full ? STEP_FULL4 : STEP_MASK4);
+                    st.end = mask;
+                } else {
+                    st.kind = k == 1 ? STEP_ROWS2 : STEP_ROWS4;
+                    for (int r = 0; r < g; ++r)
+                        for (int t = H.rowptr[r]; t < H.rowptr[r + 1]; ++t)
+                            terms.push_back(GateTerm<T>{static_cast<T>(H.vre[t]), static_cast<T>(H.vim[t]),
+                                                        r * g + H.col[t], 0});
+                    st.end = static_cast<int>(terms.size());
+                }
+                st.at = t0;
             }
-            for (int r : H.rowptr) rowptr.push_back(nt + r);
-            for (size_t t = 0; t < H.col.size(); ++t)
-                terms.push_back(GateTerm<T>{static_cast<T>(H.vre[t]), static_cast<T>(H.vim[t]), H.col[t], 0});
-            nrp += static_cast<int>(H.rowptr.size());
-            nt += static_cast<int>(H.col.size());
-            ops.push_back(op);
+            steps.push_back(st);
         }
-        D.n_gates = g1 - g0;
-        D.n_rowptr = nrp;
-        D.n_terms = nt;
+        merge_steps(steps, static_cast<size_t>(D.step), R);
+        if (a < 4 && a != stored) {  // back to a window whose lanes hold runs of 16 amplitudes
+            GateStep mv{};
+            mv.kind = STEP_MOVE;
+            mv.a = stored;
+            steps.push_back(mv);
+        }
+        D.n_steps = static_cast<int>(static_cast<int64_t>(steps.size()) - D.step);
+        D.n_diag = static_cast<int>(static_cast<int64_t>(diag.size()) - D.diag);
         P.passes.push_back(D);
     };
-    const uint64_t low = (uint64_t(1) << g_gates_low_qubits) - 1;
+    const uint64_t low = (uint64_t(1) << low_qubits) - 1;
     uint64_t S = 0;
-    int g0 = 0, nrp = 0, nt = 0;
+    int g0 = 0, nd = 0;
     for (int j = 0; j < static_cast<int>(gates.size()); ++j) {
         const HostGate &H = gates[j];
         if (!H.diag && H.k > 2) {  // a pass of its own: the single-gate kernel, on a copy the plan keeps
@@ -523,45 +642,38 @@ static void plan_passes(dq_gate_plan &P, const std::vector<HostGate> &gates,
             P.passes.push_back(D);
             g0 = j + 1;
             S = 0;
-            nrp = nt = 0;
+            nd = 0;
             continue;
         }
         const uint64_t Q = H.diag ? 0 : ((uint64_t(1) << H.k) - 1) << H.q;
-        const int hr = static_cast<int>(H.rowptr.size()), ht = static_cast<int>(H.col.size());
-        if (ht > PASS_MAX_TERMS) throw ArgError("gates: a gate has more than 512 nonzero terms");
-        if (j > g0 && (__builtin_popcountll(S | Q | low) > L || j - g0 >= PASS_MAX_GATES ||
-                       nrp + hr > PASS_MAX_ROWPTR || nt + ht > PASS_MAX_TERMS)) {
+        const int ht = static_cast<int>(H.col.size()), hd = H.diag ? ht : 0;
+        if (ht > GATE_MAX_TERMS) throw ArgError("gates: a gate has more than 512 nonzero terms");
+        if (j > g0 && (__builtin_popcountll(S | Q | low) > L || j - g0 >= PASS_MAX_GATES || nd + hd > PASS_MAX_DIAG)) {
             close(g0, j, S);
             g0 = j;
             S = 0;
-            nrp = nt = 0;
+            nd = 0;
         }
         S |= Q;
-        nrp += hr;
-        nt += ht;
+        nd += hd;
     }
     close(g0, static_cast<int>(gates.size()), S);
     DQ_HIP(hipDeviceSynchronize());  // the copies of the large gates are complete
-    P.d_passes = DevBuf(sizeof(PassHdr) * P.passes.size());
-    P.d_gops = DevBuf(sizeof(GateOp) * std::max<size_t>(1, ops.size()));
-    P.d_rowptr = DevBuf(sizeof(int) * std::max<size_t>(1, rowptr.size()));
-    P.d_terms = DevBuf(sizeof(GateTerm<T>) * std::max<size_t>(1, terms.size()));
-    DQ_HIP(hipMemcpy(P.d_passes.p, P.passes.data(), P.d_passes.bytes, hipMemcpyHostToDevice));
-    if (!ops.empty()) DQ_HIP(hipMemcpy(P.d_gops.p, ops.data(), sizeof(GateOp) * ops.size(), hipMemcpyHostToDevice));
-    if (!rowptr.empty())
-        DQ_HIP(hipMemcpy(P.d_rowptr.p, rowptr.data(), sizeof(int) * rowptr.size(), hipMemcpyHostToDevice));
-    if (!terms.empty())
-        DQ_HIP(hipMemcpy(P.d_terms.p, terms.data(), sizeof(GateTerm<T>) * terms.size(), hipMemcpyHostToDevice));
+    auto upload = [](DevBuf &buf, const auto &v) {
+        using E = typename std::decay_t<decltype(v)>::value_type;
+        buf = DevBuf(sizeof(E) * std::max<size_t>(1, v.size()));
+        if (!v.empty()) DQ_HIP(hipMemcpy(buf.p, v.data(), sizeof(E) * v.size(), hipMemcpyHostToDevice));
+    };
+    upload(P.d_passes, P.passes);
+    upload(P.d_steps, steps);
+    upload(P.d_terms, terms);
+    upload(P.d_diag, diag);
 }
 
 template <typename T>
 static void run_passes(const dq_gate_plan &P, void *re, void *im, hipStream_t s) {
     const int64_t ntiles = int64_t(1) << (P.n_qubits - P.L);
-    const unsigned grid = blocks_for(ntiles, 1, 2048);
-    const PassHdr *dp = P.d_passes.as<PassHdr>();
-    const GateOp *dg = P.d_gops.as<GateOp>();
-    const int *dr = P.d_rowptr.as<int>();
-    const GateTerm<T> *dt = P.d_terms.as<GateTerm<T>>();
+    const unsigned grid = blocks_for(ntiles, 1, 4096);
     for (size_t i = 0; i < P.passes.size(); ++i) {
         if (P.passes[i].single >= 0) {
             const dq_devmat &G = *P.big[P.passes[i].single];
@@ -571,20 +683,13 @@ static void run_passes(const dq_gate_plan &P, void *re, void *im, hipStream_t s)
             kron_apply(G, P.n_qubits - q - k, q, re, im, re, im, false, s);
             continue;
         }
-#define DQ_GATES_PASS(LL)                                                                                         \
-    if (P.kernel == 1)                                                                                            \
-        hipLaunchKernelGGL((gates_regs_kernel<T, LL>), dim3(grid), dim3(256), 0, s, dp + i, dg, dr, dt,            \
-                           static_cast<T *>(re), static_cast<T *>(im), ntiles);                                    \
-    else                                                                                                          \
-        hipLaunchKernelGGL((gates_pass_kernel<T, LL>), dim3(grid), dim3(256), 0, s, dp + i, dg, dr, dt,            \
-                           static_cast<T *>(re), static_cast<T *>(im), ntiles)
-        if (P.L == 10) {
-            DQ_GATES_PASS(10);
-        } else if (P.L == 12) {
-            DQ_GATES_PASS(12);
-        } else {
-            DQ_GATES_PASS(11);
-        }
+#define DQ_GATES_PASS(LL)                                                                                           \
+    hipLaunchKernelGGL((gates_pass_kernel<T, LL>), dim3(grid), dim3(256), 0, s, P.d_passes.as<PassHdr>() + i,        \
+                       P.d_steps.as<GateStep>(), P.d_terms.as<GateTerm<T>>(),                                       \
+                       P.d_diag.as<GateVal<T>>(), static_cast<T *>(re), static_cast<T *>(im), ntiles)
+        if (P.L == 10) DQ_GATES_PASS(10);
+        else if (P.L == 12) DQ_GATES_PASS(12);
+        else DQ_GATES_PASS(11);
 #undef DQ_GATES_PASS
         DQ_LAUNCH_CHECK();
     }
@@ -599,14 +704,19 @@ extern "C" int dq_gate_plan_create(int n_qubits, int n_gates, const dq_devmat *c
     return guard([&] {
         if (!out) throw ArgError("out is NULL");
         if (n_gates < 1 || !gates || !first_qubit) throw ArgError("gates: need at least one gate");
-        const int L = g_gates_tile_qubits;
-        if (n_qubits < L || n_qubits > 40)
-            throw ArgError("gates: n_qubits must be in [" + std::to_string(L) + ", 40] (smaller states: "
+        // Small states want many small tiles (a TFIM step on 14 qubits: 17, 20, 24 us with 10, 11, 12 tile qubits; 19
+        // two-qubit gates on 20 qubits: 69, 85, 94 us), large ones few passes (TFIM on 20: 52, 54, 46 us; on 22: 116,
+        // 111, 106; on 28: 10.3, 9.0, 7.2 ms). Four low qubits make runs of 16 amplitudes, whole 128-byte
+        // lines in FP64; a fifth costs tile qubits (28 qubits: 4 passes for 3, 8.3 ms; FP32 4.8 against 4.9 ms).
+        const int L = g_gates_tile_qubits ? g_gates_tile_qubits : n_qubits >= 21 ? 12 : n_qubits >= 19 ? 11 : 10;
+        const int low = g_gates_low_qubits ? g_gates_low_qubits : 4;
+        const int least = g_gates_tile_qubits ? g_gates_tile_qubits : 11;
+        if (n_qubits < least || n_qubits > 40)
+            throw ArgError("gates: n_qubits must be in [" + std::to_string(least) + ", 40] (smaller states: "
                            "dq_kron_apply_device per gate)");
         auto P = std::make_unique<dq_gate_plan>();
         P->n_qubits = n_qubits;
         P->L = L;
-        P->kernel = g_gates_kernel;
         std::vector<HostGate> hg;
         for (int j = 0; j < n_gates; ++j) {
             const dq_devmat *G = gates[j];
@@ -618,8 +728,8 @@ extern "C" int dq_gate_plan_create(int n_qubits, int n_gates, const dq_devmat *c
             hg.push_back(host_gate(*G, k, static_cast<int>(first_qubit[j])));
         }
         std::vector<const dq_devmat *> dg(gates, gates + n_gates);
-        if (P->precision == DQ_F64) plan_passes<double>(*P, hg, dg);
-        else plan_passes<float>(*P, hg, dg);
+        if (P->precision == DQ_F64) plan_passes<double>(*P, low, hg, dg);
+        else plan_passes<float>(*P, low, hg, dg);
         *out = P.release();
     });
 }

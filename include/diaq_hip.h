@@ -206,9 +206,9 @@ int dq_release_cached_memory(void);
  * exponential goes through a dense library GEMM); "dense_convert" (0 = automatic, 1 = per-row kernels, 2 = tiled
  * kernels) picks the kernels of dq_devmat_from_dense_device / dq_devmat_to_dense_device; "dense_convert_tile" (0 =
  * 32 x 64 tiles, the default, 1 = 64 x 32, 2 = 64 x 64, 3 = 128 x 32) their tiled kernels' tile; "gates_tile_qubits"
- * (10, 11 = default, 12) the tile of later gate plans, "gates_low_qubits" (4, 5 = default, 6) the low qubits that
- * every tile of theirs keeps (runs of 2^low contiguous amplitudes) and "gates_kernel" (0 = LDS tiles, the default;
- * 1 = amplitudes in registers with cross-lane shuffles) their pass kernel; "alloc_cache_mb" (-1 = an
+ * (10, 11, 12; unset: 10 below 19 qubits, 11 below 21, else 12) the tile of later gate plans, "gates_low_qubits" (4,
+ * 5, 6; unset: 4) the low qubits that every tile of theirs keeps (runs of 2^low contiguous amplitudes); "gates_kernel"
+ * (0, 1) is accepted and selects nothing: there is one pass kernel; "alloc_cache_mb" (-1 = an
  * eighth of the device memory, 0 = no cache) bounds the cache of freed device blocks. No reference counterpart. */
 int dq_set_tuning(const char *key, int value);
 
@@ -234,10 +234,11 @@ int dq_kron_apply_host(const dq_devmat *G, uint32_t before, uint32_t after, cons
 /* A planned sequence of gates (a Trotter step): gate j (a 2^k x 2^k device matrix, 1 <= k <= 4) acts on qubits
  * first_qubit[j] .. first_qubit[j] + k - 1 of an n_qubits state (qubit q = bit q of the amplitude index), i.e. it is
  * I_{2^(n - q - k)} (x) G_j (x) I_{2^q}. The plan cuts the sequence into passes that each stream the state through
- * HBM once and apply a stretch of gates to tiles of 2^11 amplitudes held in LDS (dq_set_tuning
- * "gates_tile_qubits": 10, 11 or 12). Running it is bitwise equal to applying the gates in order with
+ * HBM once and apply a stretch of gates to tiles of 2^10 to 2^12 amplitudes held in registers (dq_set_tuning
+ * "gates_tile_qubits"). Running it is bitwise equal to applying the gates in order with
  * dq_kron_apply_device(G_j, n - q - k, q, state, state, accumulate 0). All gates share one precision; the plan copies
- * their values (at most 512 nonzero entries per gate). n_qubits must be at least the tile qubits and at most 40.
+ * their values (at most 512 nonzero entries per gate). n_qubits must be at least 11 (the tile qubits where
+ * they are set) and at most 40.
  * No reference counterpart: the reference applies each gate in its own host loop (src/spKron.cpp:433-496), the step
  * that the diagonal-budgeted Trotterization workflow of the reference's README (README.md:340-352) builds on. */
 typedef struct dq_gate_plan dq_gate_plan;
