@@ -431,7 +431,12 @@ struct DiagTable {
     const uint32_t *bits() const { return reinterpret_cast<const uint32_t *>(buf.as<int64_t>() + nd); }
 };
 
-static unsigned tile_blocks(int64_t ntiles) { return static_cast<unsigned>((ntiles + CT_TPB - 1) / CT_TPB); }
+// Blocks of the tile kernels: CT_TPB tiles each where that makes at least TILE_BLOCKS blocks, else a tile each up to
+// that number (a 256 x 256 matrix, 32 tiles, took 200 us on the one block that its tiles made; 2048 x 2048 on 64).
+constexpr int64_t TILE_BLOCKS = 4096;
+static unsigned tile_blocks(int64_t ntiles) {
+    return static_cast<unsigned>(std::max((ntiles + CT_TPB - 1) / CT_TPB, std::min(ntiles, TILE_BLOCKS)));
+}
 
 
 template <typename T, int R, int C>
