@@ -24,6 +24,8 @@ bool dense_set_tuning(const std::string &key, int value) {
     return true;
 }
 
+bool dense_enabled() { return g_prod_dense == 1; }
+
 // The dense form pays when the pair work (at most nA * nB pairs of up to min(M, N) elements) reaches a quarter of
 // the dense product's M * K * N, and the dense operands stay small (every dimension <= 8192).
 bool dense_product_pays(const dq_devmat &A, const dq_devmat &B) {

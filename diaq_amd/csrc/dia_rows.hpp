@@ -178,6 +178,8 @@ struct ZeroMap {
 
 // Map A's values into w (zero_block_words(A.rows, 2^shift) words per diagonal; shift 6 or 8) on stream s.
 void make_zero_map(const dq_devmat &A, int shift, uint2 *w, hipStream_t s);
+// The same for A's diagonals in the order of `meta` (A.n() entries, on the device).
+void make_zero_map(const dq_devmat &A, const DiagMeta *meta, int shift, uint2 *w, hipStream_t s);
 size_t zero_map_bytes(const dq_devmat &A, int shift);
 // The map dq_spmv_tune keeps in A's handle (none if it keeps none).
 ZeroMap kept_zero_map(const dq_devmat &A);

@@ -221,6 +221,30 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
 // Dense path (dense.hip): expand to dense, the complex GEMM of gemm.hip, gather C's diagonals.
 std::unique_ptr<dq_devmat> product_dense(const dq_devmat &A, const dq_devmat &B, double divisor, hipStream_t s);
 bool dense_product_pays(const dq_devmat &A, const dq_devmat &B);
+bool dense_enabled();  // dq_set_tuning "product_dense"
+// The Taylor series of exp(X) over dense rows (expm_dense.hip), for a square X where dense_taylor_pays.
+bool dense_taylor_pays(const dq_devmat &X);
+struct TaylorRows {
+    TaylorRows(const dq_devmat &X, hipStream_t s);
+    // U = I + X + X^2 / 2! .. into `dense` (row-major interleaved complex double, N x N) and the structural offsets of
+    // the result; stop and warning as the series over pair products. max_iterations > 0. False where a term's norm is
+    // not finite: there the pair products, which skip the diagonals that a term does not hold, give other values.
+    bool series(int max_iterations, double tol, const char *who, DevBuf &dense, std::vector<int32_t> &offs);
+    // U <- U U for U = (the series' sum)^(2^j), with offsets `offs`; returns the square's offsets.
+    std::vector<int32_t> square(const std::vector<int32_t> &offs, DevBuf &U, int j);
+    int done = 0;  // terms added
+
+private:
+    int run(int k0, int n, const void *tin, const void *uin, void *tout, void *uout);
+    const dq_devmat &X;
+    hipStream_t s;
+    std::vector<DiagMeta> meta;
+    DevBuf dmeta, map, part, folded;
+    int64_t words = 0;
+};
+// Whether squaring a dense U with that many offsets beats pair products: where those would come to a quarter of the dense
+// work, and for any U of at most 512 rows.
+bool dense_square_pays(int64_t N, size_t n_offsets);
 // Dense side of the dense path (builders.hip): every element of the rows x cols interleaved complex double array
 // (leading dimension ld) from M's diagonals (zeros elsewhere), and M's stored elements back from such an array.
 void dia_to_dense(const dq_devmat &M, double *dense, int64_t ld, hipStream_t s);

@@ -168,12 +168,93 @@ __global__ __launch_bounds__(G_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)
         }
 }
 
+// The same product for matrices of few 128 x 128 tiles: a workgroup of 4 waves (2 x 2) owns 32 x 32 of C, a wave one
+// v_mfma_f64_16x16x4 tile, and K goes in steps of 16 (37 KB of LDS). The k-groups are added in the same order, so the
+// results have the same bits. Its tiles re-read A and B 4 times as often, so it runs at 45 TFLOP/s where the large tiles
+// reach 59 -- once they fill the chip: a 128 x 128 tile takes K x 0.57 us however few there are. us, large / small tiles:
+// 64^3 36 / 7, 256^3 147 / 21, 512^3 292 / 42, 1024^3 587 / 191.
+constexpr int GS_T = 32, GS_K = 16, GS_LD = GS_T + 4;
+constexpr int64_t GEMM_SMALL_TILES = 128;  // 128 x 128 tiles up to which the small kernel is used (even at about 170)
+
+__global__ __launch_bounds__(256) void zgemm_small_kernel(int64_t M, int64_t N, int64_t K, const d2 *__restrict__ A,
+                                                          const d2 *__restrict__ B, d2 *__restrict__ C, double divisor,
+                                                          int tiles_n) {
+    __shared__ double ar[2][GS_K][GS_LD], ai[2][GS_K][GS_LD], br[2][GS_K][GS_LD], bi[2][GS_K][GS_LD];
+    const int64_t m0 = static_cast<int64_t>(blockIdx.x / tiles_n) * GS_T;
+    const int64_t n0 = static_cast<int64_t>(blockIdx.x % tiles_n) * GS_T;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int wm = (wave >> 1) * 16, wn = (wave & 1) * 16, li = lane & 15, lk = lane >> 4;
+    const int arow = t / 8, ak = 2 * (t % 8), bk = t / 16, bc = 2 * (t % 16);
+    d2 ra[2], rb[2];
+    auto load = [&](int64_t k0) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            ra[e] = d2{0.0, 0.0};
+            rb[e] = d2{0.0, 0.0};
+            if (m0 + arow < M && k0 + ak + e < K) ra[e] = A[(m0 + arow) * K + k0 + ak + e];
+            if (k0 + bk < K && n0 + bc + e < N) rb[e] = B[(k0 + bk) * N + n0 + bc + e];
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            ar[buf][ak + e][arow] = ra[e].x;
+            ai[buf][ak + e][arow] = ra[e].y;
+            br[buf][bk][bc + e] = rb[e].x;
+            bi[buf][bk][bc + e] = rb[e].y;
+        }
+    };
+    d4 cr = d4{0.0, 0.0, 0.0, 0.0}, ci = cr;
+    load(0);
+    store(0);
+    __syncthreads();
+    const int64_t nk = (K + GS_K - 1) / GS_K;
+    for (int64_t ks = 0; ks < nk; ++ks) {
+        const int buf = static_cast<int>(ks & 1);
+        if (ks + 1 < nk) load((ks + 1) * GS_K);
+#pragma unroll
+        for (int kk = 0; kk < GS_K; kk += 4) {
+            const double a_r = ar[buf][kk + lk][wm + li], a_i = ai[buf][kk + lk][wm + li];
+            const double b_r = br[buf][kk + lk][wn + li], b_i = bi[buf][kk + lk][wn + li];
+            cr = __builtin_amdgcn_mfma_f64_16x16x4f64(a_r, b_r, cr, 0, 0, 0);
+            ci = __builtin_amdgcn_mfma_f64_16x16x4f64(a_r, b_i, ci, 0, 0, 0);
+            cr = __builtin_amdgcn_mfma_f64_16x16x4f64(-a_i, b_i, cr, 0, 0, 0);
+            ci = __builtin_amdgcn_mfma_f64_16x16x4f64(a_i, b_r, ci, 0, 0, 0);
+        }
+        if (ks + 1 < nk) {
+            store(buf ^ 1);
+            __syncthreads();
+        }
+    }
+    const int64_t c = n0 + wn + li;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int64_t r = m0 + wm + lk + 4 * v;
+        if (r < M && c < N) {
+            double vr = cr[v], vi = ci[v];
+            if (divisor != 1.0) {
+                vr = vr / divisor;
+                vi = vi / divisor;
+            }
+            C[r * N + c] = d2{vr, vi};
+        }
+    }
+}
+
 // C (M x N) = (A (M x K) B (K x N)) / divisor, complex interleaved row-major, on stream s.
 void zgemm_dense(int64_t M, int64_t N, int64_t K, const double *A, const double *B, double *C, double divisor,
                  hipStream_t s) {
     if (M <= 0 || N <= 0) return;
     const int64_t tm = (M + GB_M - 1) / GB_M, tn = (N + GB_N - 1) / GB_N;
     if (tm * tn > (int64_t(1) << 30)) throw ArgError("dense product: too many tiles");
+    if (tm * tn <= GEMM_SMALL_TILES) {
+        const int64_t sm = (M + GS_T - 1) / GS_T, sn = (N + GS_T - 1) / GS_T;
+        hipLaunchKernelGGL(zgemm_small_kernel, dim3(static_cast<unsigned>(sm * sn)), dim3(256), 0, s, M, N, K,
+                           reinterpret_cast<const d2 *>(A), reinterpret_cast<const d2 *>(B), reinterpret_cast<d2 *>(C),
+                           divisor, static_cast<int>(sn));
+        DQ_LAUNCH_CHECK();
+        return;
+    }
     const int tiles_m = static_cast<int>(tm), tiles_n = static_cast<int>(tn);
     const int per_xcd = (tiles_m * tiles_n + 7) / 8;
     hipLaunchKernelGGL(zgemm_mfma_kernel, dim3(static_cast<unsigned>(8 * per_xcd)), dim3(G_THREADS), 0, s, M, N, K,

@@ -97,6 +97,26 @@ static std::unique_ptr<dq_devmat> square_phase(std::unique_ptr<dq_devmat> U, int
     return convert_devmat(*P, DQ_F32, s);
 }
 
+// exp of the scaled matrix by the series, then sc squarings. Where it pays the series runs over dense rows, and as many
+// squarings as pay follow on the dense matrix, before the diagonals are gathered once.
+static std::unique_ptr<dq_devmat> series_and_squares(const dq_devmat &X, int max_iterations, double tol,
+                                                     const char *who, int *terms, int sc, hipStream_t s) {
+    if (max_iterations <= 0 || !dense_taylor_pays(X))
+        return square_phase(taylor(X, max_iterations, tol, who, terms, s), sc, s);
+    DevBuf U;
+    std::vector<int32_t> offs;
+    TaylorRows rows(X, s);
+    if (!rows.series(max_iterations, tol, who, U, offs))
+        return square_phase(taylor(X, max_iterations, tol, who, terms, s), sc, s);
+    if (terms) *terms = rows.done;
+    const int64_t N = X.rows;
+    for (int j = 0; sc > 0 && dense_square_pays(N, offs.size()); --sc, ++j) offs = rows.square(offs, U, j);
+    auto M = make_devmat(X.rows, X.rows, offs.data(), static_cast<int>(offs.size()), X.precision, s, false);
+    zero_gaps(*M, s);
+    dense_to_dia(*M, U.as<double>(), N, s);
+    return square_phase(std::move(M), sc, s);
+}
+
 static int scaling_exponent(double scaled_norm, double cutoff) {
     return (scaled_norm > cutoff) ? static_cast<int>(std::ceil(std::log2(scaled_norm / cutoff))) : 0;
 }
@@ -119,9 +139,8 @@ std::unique_ptr<dq_devmat> expm_negative(const dq_devmat &A, double t, int max_i
     const double tol_scaled = std::max(1e-15, tolerance * std::ldexp(1.0, -sc));
     auto X = make_devmat(A.rows, A.cols, A.offs.data(), A.n(), A.precision, s);
     if (-1.0 * scaled_t != 0.0) times_i_scale_copy(A, *X, -1.0 * scaled_t, s);
-    auto U = taylor(*X, max_iterations, tol_scaled, "expm_negative_taylor_cuda", terms, s);
     if (s_out) *s_out = sc;
-    return square_phase(std::move(U), sc, s);
+    return series_and_squares(*X, max_iterations, tol_scaled, "expm_negative_taylor_cuda", terms, sc, s);
 }
 
 std::unique_ptr<dq_devmat> expm(const dq_devmat &A, int max_iterations, double cutoff, double tolerance,
@@ -137,8 +156,7 @@ std::unique_ptr<dq_devmat> expm(const dq_devmat &A, int max_iterations, double c
     auto As = copy_devmat(A, s);
     scale_real(*As, inv_scale, s);
     const double tol_scaled = std::max(1e-15, tolerance * inv_scale);
-    auto U = taylor(*As, max_iterations, tol_scaled, "expm_taylor_cuda", nullptr, s);
-    return square_phase(std::move(U), sc, s);
+    return series_and_squares(*As, max_iterations, tol_scaled, "expm_taylor_cuda", nullptr, sc, s);
 }
 
 }  // namespace dq

@@ -358,11 +358,15 @@ static bool has_zero_blocks(const dq_devmat &A, const ZeroMap &z, hipStream_t s)
 }
 
 void make_zero_map(const dq_devmat &A, int shift, uint2 *w, hipStream_t s) {
+    make_zero_map(A, A.d_meta.as<DiagMeta>(), shift, w, s);
+}
+
+void make_zero_map(const dq_devmat &A, const DiagMeta *meta, int shift, uint2 *w, hipStream_t s) {
     const int64_t words = zero_block_words(A.rows, 1 << shift);
     const dim3 grid(static_cast<unsigned>(words), zero_map_grid_y(A.n()), 1);
 #define DQ_ZERO_MAP(T, BR)                                                                                          \
-    hipLaunchKernelGGL((zero_blocks_kernel<T, BR>), grid, dim3(256), 0, s, static_cast<int64_t>(A.rows), A.n(),      \
-                       A.d_meta.as<DiagMeta>(), int64_t(0), A.re.as<T>(), A.im.as<T>(), words, w)
+    hipLaunchKernelGGL((zero_blocks_kernel<T, BR>), grid, dim3(256), 0, s, static_cast<int64_t>(A.rows), A.n(), meta, \
+                       int64_t(0), A.re.as<T>(), A.im.as<T>(), words, w)
     if (A.precision == DQ_F64 && shift == 6) DQ_ZERO_MAP(double, 64);
     else if (A.precision == DQ_F64) DQ_ZERO_MAP(double, 256);
     else if (shift == 6) DQ_ZERO_MAP(float, 64);
