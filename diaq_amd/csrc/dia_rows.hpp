@@ -174,6 +174,7 @@ struct ZeroMap {
     const uint2 *w = nullptr;
     int64_t words = 0;
     int shift = 6;
+    int loads_only = 0;  // spare the loads of zeros, but add their products too (dia_rows_wave)
 };
 
 // Map A's values into w (zero_block_words(A.rows, 2^shift) words per diagonal; shift 6 or 8) on stream s.
@@ -437,7 +438,7 @@ __device__ inline void dia_rows_wave(int64_t row0, int n, const DiagMeta *__rest
                 for (int q = 1; q < V; ++q)
                     if ((64 * q) >> zm.shift) m2 |= 1u << ((64 * q) >> zm.shift);
                 parts = (((w.x >> b) & m2) ? RNG_RE : 0) | (((w.y >> b) & m2) ? RNG_IM : 0);
-                live = live && parts;
+                live = live && (parts || zm.loads_only);
             }
             vb = m.rowbase + row0;
             off = m.off;

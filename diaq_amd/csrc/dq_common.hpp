@@ -158,6 +158,9 @@ struct dq_devmat {
     // rewrites the values (dq_devmat_set_packed_device) recomputes it in place.
     dq::DevBuf zmap;
     bool zmap_valid = false;
+    // The map came with a product's result instead: it only spares the loads of zeros. A product with it still takes every
+    // stored element, so that a NaN or infinity of x meets the zeros as it does without a map.
+    bool zmap_loads_only = false;
 
     int n() const { return static_cast<int>(offs.size()); }
     int64_t stored() const {
@@ -216,8 +219,9 @@ bool evo_set_tuning(const std::string &key, int value);
 
 // C = (A B) / divisor with the structural dry-run (product.hip). allow_dense: a near-dense product may take the dense
 // path (dense.hip) -- same offsets, values equal up to the summation order; for pow and the matrix exponential.
+// keep_map: C may keep a zero-block map (dq_devmat::zmap_loads_only); the caller hands C out and changes no value of it.
 std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, double divisor, hipStream_t s,
-                                   bool allow_dense = false);
+                                   bool allow_dense = false, bool keep_map = false);
 // Dense path (dense.hip): expand to dense, the complex GEMM of gemm.hip, gather C's diagonals.
 std::unique_ptr<dq_devmat> product_dense(const dq_devmat &A, const dq_devmat &B, double divisor, hipStream_t s);
 bool dense_product_pays(const dq_devmat &A, const dq_devmat &B);

@@ -21,11 +21,17 @@
 // (no chain of dependent metadata loads per pair).
 //
 // Zero blocks: for large operands the product first maps which 64-row blocks of each diagonal of A and B hold a
-// nonzero value (zero_blocks_kernel), and a pair whose A rows, or whose B rows, in the item's chunk are all zero is
-// dropped when its metadata is staged. Its products are all +-0, and a sum that starts at +0 is left unchanged by
-// adding +-0, so the result has the same bits; only a NaN or Inf facing a zero block is not propagated. A qubit
-// Hamiltonian's +-2^k flip diagonals are zero on alternate runs of 2^k rows, so for k at least the chunk's log2 size
-// half of a far pair's chunks read nothing -- and far pairs' B rows are the reads no cache catches.
+// nonzero real or imaginary value (zero_blocks_kernel). A pair whose A rows, or whose B rows, in the item are all zero is
+// dropped when its metadata is staged: its products are all +-0, and a sum that starts at +0 is left unchanged by
+// adding +-0, so the result has the same bits; only a NaN or Inf facing such rows is not propagated. Of the pairs that
+// stay, each wave loads only the blocks and parts that hold a nonzero and multiplies zeros for the others, which gives
+// the same sums, NaN and Inf among them. A qubit Hamiltonian's +-2^k flip diagonals are zero on alternate runs of 2^k
+// rows, and its imaginary part often everywhere.
+//
+// Bound: the L2's and the memory's reads of A and B per pair against the stores of C (TFIM-20 H*H: 1681 pairs, 727
+// diagonals, 11 GB stored). Reading every part of a live pair: 4.00 ms; only the live blocks and parts: 3.06 ms.
+//
+// The items also write C's own zero-block map, by ballots on what they store; a large result keeps it (map_blocks).
 #include <algorithm>
 #include <atomic>
 #include <memory>
@@ -209,20 +215,49 @@ __device__ inline int64_t uniform64(int64_t v) {
     return static_cast<int64_t>((static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) | static_cast<uint32_t>(lo));
 }
 
-// Whether a block of diagonal k's map row that meets rows [lo, hi) holds a nonzero value.
-__device__ inline bool blocks_live(const ZeroMap &z, int64_t k, int64_t lo, int64_t hi) {
+// The bits of 32 consecutive blocks from block b0 (which may lie outside the map) of diagonal k: x real, y imaginary.
+__device__ inline uint2 map_window(const ZeroMap &z, int64_t k, int64_t b0) {
     const uint2 *row = z.w + k * z.words;
-    const int64_t b0 = lo >> z.shift, b1 = (hi - 1) >> z.shift;
-    for (int64_t w = b0 >> 5; w <= (b1 >> 5); ++w) {
-        uint32_t m = row[w].x | row[w].y;
-        if (w == (b0 >> 5)) m &= 0xffffffffu << (b0 & 31);
-        if (w == (b1 >> 5)) m &= 0xffffffffu >> (31 - (b1 & 31));
-        if (m) return true;
-    }
-    return false;
+    const int64_t w = b0 >> 5;
+    const int sh = static_cast<int>(b0 & 31);
+    const uint2 a = w >= 0 && w < z.words ? row[w] : make_uint2(0, 0);
+    if (sh == 0) return a;
+    const uint2 b = w + 1 >= 0 && w + 1 < z.words ? row[w + 1] : make_uint2(0, 0);
+    return make_uint2(a.x >> sh | b.x << (32 - sh), a.y >> sh | b.y << (32 - sh));
 }
 
-template <typename T, bool NTS, int PROD_RPT>
+// The same for the 32 blocks of 64 rows that start at row r0, which need not be a block's first row: a bit is set where
+// either block that holds some of the rows has it.
+__device__ inline uint2 map_rows(const ZeroMap &z, int64_t k, int64_t r0) {
+    uint2 m = map_window(z, k, r0 >> 6);
+    if (r0 & 63) {
+        const uint2 n = map_window(z, k, (r0 >> 6) + 1);
+        m.x |= n.x;
+        m.y |= n.y;
+    }
+    return m;
+}
+
+// Rows r + 256 j of p into v, R of them: a wave's 64 rows of pass j are block 4 j + wave of the item, and `live` has bit
+// 4 j set when they hold a nonzero. The others are zeros and are not loaded (uniform in the wave).
+template <typename T, int R>
+__device__ inline void ld_blocks(const T *p, uint32_t live, const uint32_t (&r)[R], T (&v)[R]) {
+    constexpr uint32_t ALL = R >= 8 ? 0x11111111u : 0x1111u;
+    if ((live & ALL) == ALL || (R > 8 && live)) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) v[j] = p[r[j]];
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) v[j] = T(0);
+    if (R > 8 || (live & ALL) == 0) return;
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+        if (live >> (4 * (j & 7)) & 1u) v[j] = p[r[j]];
+}
+
+// MAP: the operands have zero-block maps (za, zb).
+template <typename T, bool NTS, int PROD_RPT, bool MAP>
 __global__ __launch_bounds__(256) void product_kernel(const int2 *__restrict__ items, const int64_t *__restrict__ xcd_first,
                                                       const int64_t *__restrict__ pair_start,
                                                       const int32_t *__restrict__ pa, const int32_t *__restrict__ pb,
@@ -231,10 +266,14 @@ __global__ __launch_bounds__(256) void product_kernel(const int2 *__restrict__ i
                                                       const T *__restrict__ aim, const T *__restrict__ bre,
                                                       const T *__restrict__ bim, T *__restrict__ cre,
                                                       T *__restrict__ cim, double divisor,
-                                                      ZeroMap za, ZeroMap zb) {
+                                                      ZeroMap za, ZeroMap zb, uint2 *__restrict__ zc,
+                                                      int64_t zc_words) {
     constexpr int PROD_CHUNK = 256 * PROD_RPT;
     __shared__ int64_t s_abase[PROD_BATCH], s_bbase[PROD_BATCH];
     __shared__ int32_t s_lo[PROD_BATCH], s_hi[PROD_BATCH];
+    __shared__ uint4 s_live[MAP ? PROD_BATCH : 1];  // the item's blocks that hold a nonzero: A real, A imaginary, B real, B imaginary
+    constexpr int ZW = (PROD_RPT + 7) / 8;  // map words of an item's rows
+    __shared__ uint32_t s_zr[ZW], s_zi[ZW];
     // XCD-aware remap: the workgroups of XCD x (x = b mod 8) take the item range [xcd_first[x], xcd_first[x + 1]).
     const int64_t b = blockIdx.x;
     const int64_t w = xcd_first[b & 7] + (b >> 3);
@@ -244,6 +283,8 @@ __global__ __launch_bounds__(256) void product_kernel(const int2 *__restrict__ i
     const int64_t q0 = static_cast<int64_t>(it.x) * PROD_CHUNK;
     const int64_t r0 = max(m_c.rlo, q0), r1 = min(m_c.rhi, q0 + PROD_CHUNK);
     const int64_t p0 = pair_start[it.y], p1 = pair_start[it.y + 1];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (MAP && zc && threadIdx.x < ZW) s_zr[threadIdx.x] = s_zi[threadIdx.x] = 0;  // the first batch's barrier orders it
     T acc_r[PROD_RPT], acc_i[PROD_RPT];
 #pragma unroll
     for (int j = 0; j < PROD_RPT; ++j) { acc_r[j] = T(0); acc_i[j] = T(0); }
@@ -258,8 +299,19 @@ __global__ __launch_bounds__(256) void product_kernel(const int2 *__restrict__ i
             const int64_t lo = max(max(ta.rlo, tb.rlo - ta.off), r0);
             const int64_t hi = min(min(ta.rhi, tb.rhi - ta.off), r1);
             bool live = hi > lo;
-            if (live && za.w) live = blocks_live(za, sa, lo, hi);
-            if (live && zb.w) live = blocks_live(zb, sb, lo + ta.off, hi + ta.off);
+            uint4 m = make_uint4(~0u, ~0u, ~0u, ~0u);
+            if (MAP && live) {  // rows that a diagonal does not have are clear bits of its map
+                m = make_uint4(0, 0, 0, 0);
+#pragma unroll
+                for (int w8 = 0; w8 < ZW; ++w8) {
+                    const int64_t q = q0 + 2048 * w8;
+                    const uint2 a2 = map_rows(za, sa, q), b2 = map_rows(zb, sb, q + ta.off);
+                    m.x |= a2.x; m.y |= a2.y; m.z |= b2.x; m.w |= b2.y;
+                }
+                constexpr uint32_t IN = PROD_RPT < 8 ? 0xffffu : ~0u;  // the item's rows
+                live = ((m.x | m.y) & IN) && ((m.z | m.w) & IN);
+            }
+            if (MAP) s_live[threadIdx.x] = m;
             s_abase[threadIdx.x] = ta.rowbase;
             s_bbase[threadIdx.x] = tb.rowbase + ta.off;
             s_lo[threadIdx.x] = live ? static_cast<int32_t>(lo - q0) : 0;
@@ -271,26 +323,34 @@ __global__ __launch_bounds__(256) void product_kernel(const int2 *__restrict__ i
             const int64_t hi = q0 + __builtin_amdgcn_readfirstlane(s_hi[k]);
             if (hi <= lo) continue;  // uniform
             const int64_t abase = uniform64(s_abase[k]), bbase = uniform64(s_bbase[k]);
-            const T *apr = are + abase, *api = aim + abase;
-            const T *bpr = bre + bbase, *bpi = bim + bbase;
+            const T *apr = are + (abase + q0), *api = aim + (abase + q0);  // the item's first row
+            const T *bpr = bre + (bbase + q0), *bpi = bim + (bbase + q0);
+            uint32_t l_ar = ~0u, l_ai = ~0u, l_br = ~0u, l_bi = ~0u;
+            if constexpr (MAP) {
+                const uint4 m = s_live[k];
+                l_ar = __builtin_amdgcn_readfirstlane(m.x) >> wave;
+                l_ai = __builtin_amdgcn_readfirstlane(m.y) >> wave;
+                l_br = __builtin_amdgcn_readfirstlane(m.z) >> wave;
+                l_bi = __builtin_amdgcn_readfirstlane(m.w) >> wave;
+            }
+            const bool whole = lo == q0 && hi == q0 + PROD_CHUNK;  // uniform: the whole chunk, no per-row checks
             T va_r[PROD_RPT], va_i[PROD_RPT], vb_r[PROD_RPT], vb_i[PROD_RPT];
-            if (lo == q0 && hi == q0 + PROD_CHUNK) {  // uniform: the whole chunk, no per-row checks
+            uint32_t at[PROD_RPT];
+            const int32_t l0 = static_cast<int32_t>(lo - q0), h0 = static_cast<int32_t>(hi - q0);
+#pragma unroll
+            for (int j = 0; j < PROD_RPT; ++j) {
+                const int32_t r = static_cast<int32_t>(threadIdx.x) + 256 * j;
+                at[j] = whole ? r : (r < l0 ? l0 : (r >= h0 ? h0 - 1 : r));  // clamped to a valid row
+            }
+            ld_blocks(apr, l_ar, at, va_r);
+            ld_blocks(api, l_ai, at, va_i);
+            ld_blocks(bpr, l_br, at, vb_r);
+            ld_blocks(bpi, l_bi, at, vb_i);
+            if (!whole) {  // zero both operands of the rows outside [lo, hi)
 #pragma unroll
                 for (int j = 0; j < PROD_RPT; ++j) {
-                    const int64_t r = q0 + threadIdx.x + 256 * j;
-                    va_r[j] = apr[r]; va_i[j] = api[r]; vb_r[j] = bpr[r]; vb_i[j] = bpi[r];
-                }
-            } else {  // clamp to a valid row, zero both operands of the rows outside [lo, hi)
-#pragma unroll
-                for (int j = 0; j < PROD_RPT; ++j) {
-                    const int64_t r = q0 + threadIdx.x + 256 * j;
-                    const int64_t rc = r < lo ? lo : (r >= hi ? hi - 1 : r);
-                    va_r[j] = apr[rc]; va_i[j] = api[rc]; vb_r[j] = bpr[rc]; vb_i[j] = bpi[rc];
-                }
-#pragma unroll
-                for (int j = 0; j < PROD_RPT; ++j) {
-                    const int64_t r = q0 + threadIdx.x + 256 * j;
-                    if (r < lo || r >= hi) { va_r[j] = T(0); va_i[j] = T(0); vb_r[j] = T(0); vb_i[j] = T(0); }
+                    const int32_t r = static_cast<int32_t>(threadIdx.x) + 256 * j;
+                    if (r < l0 || r >= h0) { va_r[j] = T(0); va_i[j] = T(0); vb_r[j] = T(0); vb_i[j] = T(0); }
                 }
             }
 #pragma unroll
@@ -303,15 +363,17 @@ __global__ __launch_bounds__(256) void product_kernel(const int2 *__restrict__ i
         }
         __syncthreads();  // the next batch overwrites the staged pairs
     }
+    uint32_t zr[ZW] = {}, zi[ZW] = {};
 #pragma unroll
     for (int j = 0; j < PROD_RPT; ++j) {
         const int64_t r = q0 + threadIdx.x + 256 * j;
-        if (r >= r0 && r < r1) {
-            T vr = acc_r[j], vi = acc_i[j];
-            if (divisor != 1.0) {
-                vr = static_cast<T>(acc_r[j] / divisor);
-                vi = static_cast<T>(acc_i[j] / divisor);
-            }
+        const bool in = r >= r0 && r < r1;
+        T vr = acc_r[j], vi = acc_i[j];
+        if (divisor != 1.0) {
+            vr = static_cast<T>(acc_r[j] / divisor);
+            vi = static_cast<T>(acc_i[j] / divisor);
+        }
+        if (in) {
             if constexpr (NTS) {  // C is written once and not read here: keep it out of the caches
                 __builtin_nontemporal_store(vr, cre + m_c.rowbase + r);
                 __builtin_nontemporal_store(vi, cim + m_c.rowbase + r);
@@ -320,11 +382,58 @@ __global__ __launch_bounds__(256) void product_kernel(const int2 *__restrict__ i
                 cim[m_c.rowbase + r] = vi;
             }
         }
+        if (MAP && zc) {  // uniform; the wave's 64 rows of pass j are block 4 j + wave of the item
+            if (__ballot(in && !(vr == T(0)))) zr[j >> 3] |= 1u << (4 * (j & 7));
+            if (__ballot(in && !(vi == T(0)))) zi[j >> 3] |= 1u << (4 * (j & 7));
+        }
+    }
+    if (MAP && zc) {
+        if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+            for (int w8 = 0; w8 < ZW; ++w8) {
+                atomicOr(&s_zr[w8], zr[w8] << wave);
+                atomicOr(&s_zi[w8], zi[w8] << wave);
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x < ZW) {
+            uint2 *w = zc + it.y * zc_words + (q0 >> 11) + threadIdx.x;
+            if constexpr (PROD_RPT == 4) {  // half a word
+                uint16_t *h = reinterpret_cast<uint16_t *>(w) + ((q0 >> 10) & 1);
+                h[0] = static_cast<uint16_t>(s_zr[0]);
+                h[2] = static_cast<uint16_t>(s_zi[0]);
+            } else if ((q0 >> 11) + threadIdx.x < zc_words) {
+                *w = make_uint2(s_zr[threadIdx.x], s_zi[threadIdx.x]);
+            }
+        }
     }
 }
 
+// The set bits of a zero-block map, added to *out.
+__global__ __launch_bounds__(256) void map_bits_kernel(int64_t n, const uint2 *__restrict__ w,
+                                                       unsigned long long *__restrict__ out) {
+    unsigned c = 0;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        c += __popc(w[i].x) + __popc(w[i].y);
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(out, static_cast<unsigned long long>(c));
+}
+
+// The 64-row blocks of C's diagonals, when the product is to map them for the result's own products, else 0: FP64 values
+// beyond the Infinity Cache, where a product is bound by reading them (H*H of TFIM-20, 11 GB: SpMV 1.90 -> 0.94 ms). A
+// smaller result saves less than the map's fill, count and read-back (about 15 us).
+constexpr int64_t MAP_RESULT_BYTES = int64_t(256) << 20;
+
+static int64_t map_blocks(const dq_devmat &C) {
+    if (C.precision != DQ_F64 || C.rows < (1u << 16) || 16 * C.total <= MAP_RESULT_BYTES) return 0;
+    int64_t n = 0;
+    for (const DiagMeta &m : C.meta)
+        if (m.rhi > m.rlo) n += ((m.rhi - 1) >> 6) - (m.rlo >> 6) + 1;
+    return n;
+}
+
 std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, double divisor, hipStream_t s,
-                                   bool allow_dense) {
+                                   bool allow_dense, bool keep_map) {
     if (A.cols != B.rows) throw ArgError("diaQMatrix product_cuda: dimension mismatch.");
     if (A.precision != B.precision) throw ArgError("product: operands have different precisions");
     if (allow_dense && dense_product_pays(A, B)) return product_dense(A, B, divisor, s);
@@ -410,21 +519,37 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
         za = map_of(A, zab);
         zb = (&A == &B) ? za : map_of(B, zbb);
     }
+    // the result's own map, where a product with it may use one: kept when at least an eighth of its blocks are zero
+    const int64_t c_blocks = keep_map && za.w ? map_blocks(*C) : 0;
+    DevBuf zcb, dbits;
+    unsigned long long bits = 0;
+    if (c_blocks) {
+        zcb = DevBuf(zero_map_bytes(*C, ZeroMap().shift));
+        dbits = DevBuf(16);
+        zero_bytes(zcb.p, zcb.bytes, s);
+        zero_bytes(dbits.p, 8, s);
+    }
+    const int64_t zc_words = zero_block_words(C->rows, 64);
     hipLaunchKernelGGL(product_items_kernel, dim3(static_cast<unsigned>(std::min<int64_t>(n_chunks, 65536))),
                        dim3(256), 0, s, n_chunks, dfirst.as<int64_t>(), dclo.as<int32_t>(), dqof.as<int32_t>(),
                        ditems.as<int2>());
     DQ_LAUNCH_CHECK();
-#define DQ_PROD_LAUNCH_R(T, NTS, R)                                                                                \
-    hipLaunchKernelGGL((product_kernel<T, NTS, R>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, s,           \
+#define DQ_PROD_LAUNCH_M(T, NTS, R, M)                                                                             \
+    hipLaunchKernelGGL((product_kernel<T, NTS, R, M>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, s,        \
                        ditems.as<int2>(), dxcd.as<int64_t>(), dps.as<int64_t>(), dsa.as<int32_t>(),               \
                        dsb.as<int32_t>(), A.d_meta.as<DiagMeta>(), B.d_meta.as<DiagMeta>(), C->d_meta.as<DiagMeta>(), \
                        A.re.as<T>(), A.im.as<T>(), B.re.as<T>(), B.im.as<T>(), C->re.as<T>(), C->im.as<T>(), divisor, \
-                       za, zb)
-#define DQ_PROD_LAUNCH(T, NTS)                                \
-    do {                                                      \
-        if (prod_rpt == 4) { DQ_PROD_LAUNCH_R(T, NTS, 4); }   \
-        else if (prod_rpt == 16) { DQ_PROD_LAUNCH_R(T, NTS, 16); } \
-        else { DQ_PROD_LAUNCH_R(T, NTS, 8); }                 \
+                       za, zb, zcb.as<uint2>(), zc_words)
+#define DQ_PROD_LAUNCH_R(T, NTS, R)                          \
+    do {                                                     \
+        if (za.w) DQ_PROD_LAUNCH_M(T, NTS, R, true);         \
+        else DQ_PROD_LAUNCH_M(T, NTS, R, false);             \
+    } while (0)
+#define DQ_PROD_LAUNCH(T, NTS)                                     \
+    do {                                                           \
+        if (prod_rpt == 4) DQ_PROD_LAUNCH_R(T, NTS, 4);            \
+        else if (prod_rpt == 16) DQ_PROD_LAUNCH_R(T, NTS, 16);     \
+        else DQ_PROD_LAUNCH_R(T, NTS, 8);                          \
     } while (0)
     if (A.precision == DQ_F64) {
         if (g_prod_nt_store) DQ_PROD_LAUNCH(double, true);
@@ -435,8 +560,20 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
     }
 #undef DQ_PROD_LAUNCH
 #undef DQ_PROD_LAUNCH_R
+#undef DQ_PROD_LAUNCH_M
     DQ_LAUNCH_CHECK();
+    if (c_blocks) {
+        const int64_t words = static_cast<int64_t>(zcb.bytes / sizeof(uint2));
+        hipLaunchKernelGGL(map_bits_kernel, dim3(blocks_for(words, 256, 512)), dim3(256), 0, s, words, zcb.as<uint2>(),
+                           dbits.as<unsigned long long>());
+        DQ_LAUNCH_CHECK();
+        DQ_HIP(hipMemcpyAsync(&bits, dbits.p, sizeof(bits), hipMemcpyDeviceToHost, s));
+    }
     DQ_HIP(hipStreamSynchronize(s));  // before the work list is freed
+    if (c_blocks && static_cast<int64_t>(bits) <= 2 * c_blocks - c_blocks / 4) {
+        C->zmap = std::move(zcb);
+        C->zmap_valid = C->zmap_loads_only = true;
+    }
     return C;
 }
 
@@ -523,7 +660,7 @@ bool product_set_tuning(const std::string &key, int value) {
 extern "C" int dq_product_device(const dq_devmat *A, const dq_devmat *B, dq_devmat **out) {
     return guard([&] {
         if (!A || !B || !out) throw ArgError("NULL argument");
-        *out = product(*A, *B, 1.0, 0).release();
+        *out = product(*A, *B, 1.0, 0, false, true).release();
     });
 }
 

@@ -326,7 +326,9 @@ static ZeroMap handle_map(const dq_devmat &A) {
 // any precision (their results are not compared with a single untuned SpMV's).
 static ZeroMap sequence_map(const dq_devmat &A, int n) {
     if (n == 1) return handle_map(A);
-    return g_spmv_skip ? kept_zero_map(A) : ZeroMap();
+    ZeroMap z = g_spmv_skip ? kept_zero_map(A) : ZeroMap();
+    z.loads_only = 0;
+    return z;
 }
 
 ZeroMap kept_zero_map(const dq_devmat &A) {
@@ -334,6 +336,7 @@ ZeroMap kept_zero_map(const dq_devmat &A) {
     if (!A.zmap_valid || !A.zmap.p) return z;
     z.w = A.zmap.as<uint2>();
     z.words = zero_block_words(A.rows, 1 << z.shift);
+    z.loads_only = A.zmap_loads_only;
     return z;
 }
 
@@ -375,12 +378,24 @@ void make_zero_map(const dq_devmat &A, const DiagMeta *meta, int shift, uint2 *w
     DQ_LAUNCH_CHECK();
 }
 
-// After A's values were rewritten on stream s: recompute the zero-block map the handle keeps into the same buffer,
+__global__ void fill_map_kernel(int64_t n, uint2 *__restrict__ w) {
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        w[i] = make_uint2(~0u, ~0u);
+}
+
+// After A's values were rewritten on stream s: bring the zero-block map the handle keeps up to date in the same buffer,
 // ordered after the rewrite. A graph captured earlier that reads the handle's map then sees the new map on its next
-// replay, and later SpMVs skip exactly the blocks that are zero now (none, if every block became nonzero).
+// replay, and later SpMVs skip no block that is nonzero now. The map of a tuning is recomputed; a product's map, which
+// the caller did not ask for, is set to "every block nonzero" instead of reading all values again.
 void refresh_zero_map(dq_devmat &A, hipStream_t s) {
     if (!A.zmap_valid || !A.zmap.p) return;
-    make_zero_map(A, ZeroMap().shift, A.zmap.as<uint2>(), s);
+    if (!A.zmap_loads_only) {
+        make_zero_map(A, ZeroMap().shift, A.zmap.as<uint2>(), s);
+        return;
+    }
+    const int64_t n = static_cast<int64_t>(A.zmap.bytes / sizeof(uint2));
+    hipLaunchKernelGGL(fill_map_kernel, dim3(blocks_for(n, 256, 2048)), dim3(256), 0, s, n, A.zmap.as<uint2>());
+    DQ_LAUNCH_CHECK();
 }
 
 // y = A x: the schedule of A, skipping its all-zero blocks when the handle holds their map (see handle_map).
@@ -502,7 +517,7 @@ extern "C" int dq_spmv_tune(dq_devmat *A, int repeats, uintptr_t stream, float *
         if (A->rows < 2 * WAVE_ROWS) time_waves(best, A->tuned_wave);  // beyond, the tiles read every block faster
         // last stage: when A has all-zero blocks or parts and skipping them is faster, keep their map in the handle (used
         // by A's FP64 SpMVs and by spMV_ntimes)
-        A->zmap_valid = false;
+        A->zmap_valid = A->zmap_loads_only = false;
         A->skip_wave = dq_devmat::WaveSched();
         if (g_spmv_skip) {
             const size_t zb = zero_map_bytes(*A, tz.shift);

@@ -1,0 +1,92 @@
+"""The pair product's zero blocks (64 rows, real and imaginary part apart) and the map that a large result keeps: the bits
+of the forms that read every value, with odd rows, diagonals that end inside a block and offsets that are no multiple of
+a block; a NaN or infinity of x meets the result's zeros as without a map; new values replace the map."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from oracle import oracle as O  # noqa: E402
+
+ROWS = 130001
+
+
+def matrix(real):
+    """24 diagonals whose blocks are zero on runs of 64 to 4096 rows, in one part or both."""
+    rng = np.random.default_rng(5)
+    offs = sorted({0, 1, -1, 63, -64, 128, 200, -513, 1024, -2048, 4100, -8192, 16384, -16385, 32768, -40000, 50001, 60000,
+                   -60001, 129990, -129999, 7, 3000, -12345})
+    vals = []
+    for k, o in enumerate(offs):
+        n = O.diagonal_length(o, ROWS, ROWS)
+        r = np.arange(n) + max(0, -o)
+        v = rng.standard_normal(n) + (0j if real else 1j * rng.standard_normal(n))
+        if k % 3:
+            v = v * (r // (64 << (k % 7)) % 2)
+        if k % 5 == 4 and not real:
+            v = np.where(r // 128 % 2, v.real + 0j, 1j * v.imag)
+        vals.append(v)
+    return O.Dia(ROWS, ROWS, offs, vals)
+
+
+def tuning(key, value):
+    from diaq_amd import capi
+    capi.check(capi.lib().dq_set_tuning(key, value))
+
+
+def spmv(C, x):
+    import diaq_gpu as d
+    import torch
+    xr, xi = (torch.as_tensor(p, device="cuda").contiguous() for p in (x.real, x.imag))
+    yr, yi = torch.empty_like(xr), torch.empty_like(xi)
+    d.spmv_device(C, xr.data_ptr(), xi.data_ptr(), yr.data_ptr(), yi.data_ptr(), 0)
+    torch.cuda.synchronize()
+    return yr.cpu().numpy(), yi.cpu().numpy()
+
+
+@pytest.mark.parametrize("real", [True, False])
+def test_product_of_zero_blocks(real):
+    import diaq_amd  # noqa: F401
+    import diaq_gpu as d
+    import torch
+    from diaq_amd import capi
+    M = matrix(real)
+    D = d.to_device(d.diaQMatrix.from_diagonals([ROWS, ROWS], M.offsets, M.vals))
+    got = {}
+    try:
+        for rpt in (0, 4, 16):
+            tuning(b"product_rows_per_lane", rpt)
+            got[rpt] = d.product(D, D)
+        tuning(b"product_rows_per_lane", 0)
+        tuning(b"product_skip_zero_blocks", 0)
+        plain = d.product(D, D)
+    finally:
+        tuning(b"product_rows_per_lane", 0)
+        tuning(b"product_skip_zero_blocks", 1)
+    assert 16 * plain.stored > 1 << 28  # large enough to keep a map
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal(ROWS) + 1j * rng.standard_normal(ROWS)
+    bad = x.copy()
+    bad[[17, 30000, 129999]] = [np.nan, np.inf, -np.inf + 1j * np.inf]
+    want = {}
+    try:
+        tuning(b"spmv_skip_zero_blocks", 0)
+        want = {k: spmv(plain, v) for k, v in (("x", x), ("bad", bad))}
+    finally:
+        tuning(b"spmv_skip_zero_blocks", 1)
+    ref = O.spmv(M, O.spmv(M, x))
+    assert np.max(np.abs(want["x"][0] + 1j * want["x"][1] - ref)) < 1e-12 * np.max(np.abs(ref))
+    for rpt, C in got.items():
+        for k in plain.diagonals[:: 29]:
+            np.testing.assert_array_equal(np.asarray(C.get_diagonal(k)), np.asarray(plain.get_diagonal(k)))
+        for k, v in (("x", x), ("bad", bad)):
+            np.testing.assert_array_equal(spmv(C, v), want[k])
+    C = got[0]
+    ones = torch.ones(C.stored, dtype=torch.float64, device="cuda")
+    zeros = torch.zeros_like(ones)
+    capi.check(capi.lib().dq_devmat_set_packed_device(C.handle, ones.data_ptr(), zeros.data_ptr(), 0))
+    torch.cuda.synchronize()
+    E = O.Dia(ROWS, ROWS, list(C.diagonals), [np.ones(O.diagonal_length(o, ROWS, ROWS)) for o in C.diagonals])
+    y = O.spmv(E, x)
+    a, b = spmv(C, x)
+    assert np.max(np.abs(a + 1j * b - y)) < 1e-12 * np.max(np.abs(y))
