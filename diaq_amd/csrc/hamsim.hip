@@ -252,6 +252,154 @@ static void taylor_step(const dq_devmat &H, const T *pr, const T *pi, const TO *
     }
 }
 
+// Many steps of a small matrix in one workgroup: V rows per lane (row = lane + 1024 v), the rows' values of up to ND
+// diagonals in registers, the term vector in LDS (two buffers, a barrier per term), the step's output in registers.
+// Each buffer has `pad` zeros on either side, pad the largest |offset|, so that a row reads every diagonal at lane +
+// offset: one off a diagonal multiplies a zero by a zero, which leaves an FP64 sum that starts at +0 as it is (an FP32
+// sum is compensated and takes only the rows on the diagonal). Products, order and roundings are those of
+// taylor_term_kernel, so the result has the same bits.
+//
+// Bound: the LDS reads of x, 16 bytes per row, diagonal and term (10 qubits, 19 diagonals: 311 KB, 1.0 us at 128 bytes a
+// clock), where a launch per term costs its launch and the round trips to the L2. 10-qubit XXZ, 20 steps of 18 terms:
+// 2013 -> 553 us (1.5 us a term).
+constexpr int RES_LANES = 1024, RES_ND = 24;
+constexpr int RES_TERMS = 4096;  // terms of a launch: a few milliseconds
+
+template <typename T, typename TO, int V>
+__global__ __launch_bounds__(RES_LANES) void taylor_resident_kernel(int rows, int n, const DiagMeta *__restrict__ meta,
+                                                                    const T *__restrict__ are,
+                                                                    const T *__restrict__ aim, TO *__restrict__ pr,
+                                                                    TO *__restrict__ pi, double dt, int m, int steps,
+                                                                    int pad) {
+    struct alignas(2 * sizeof(T)) Cx {
+        T r, i;
+    };
+    extern __shared__ __align__(16) char smem[];
+    Cx *buf = reinterpret_cast<Cx *>(smem);
+    constexpr int G = sizeof(T) == 8 ? 3 : 2;  // diagonals whose x is read together: what the registers leave
+    static_assert(RES_ND % G == 0 && RES_ND <= 32, "whole groups, one bit per diagonal");
+    const int width = rows + 2 * pad;
+    T ar[V][RES_ND], ai[V][RES_ND];
+    uint32_t on[V];
+    int off[RES_ND];  // uniform
+#pragma unroll
+    for (int k = 0; k < RES_ND; ++k) off[k] = __builtin_amdgcn_readfirstlane(k < n ? meta[k].off : 0);
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const int r = static_cast<int>(threadIdx.x) + RES_LANES * v;
+        on[v] = 0;
+#pragma unroll
+        for (int k = 0; k < RES_ND; ++k) {
+            ar[v][k] = T(0);
+            ai[v][k] = T(0);
+            if (k < n) {  // uniform
+                const DiagMeta md = meta[k];
+                if (r >= md.rlo && r < md.rhi) {
+                    ar[v][k] = are[md.rowbase + r];
+                    ai[v][k] = aim[md.rowbase + r];
+                    on[v] |= 1u << k;
+                }
+            }
+        }
+    }
+    for (int e = threadIdx.x; e < 2 * width; e += blockDim.x) buf[e] = Cx{T(0), T(0)};
+    __syncthreads();
+    TO outr[V], outi[V];
+    int at[V];  // the row's place in a buffer; rows past the last one write nothing and read zeros or finite terms
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const int r = static_cast<int>(threadIdx.x) + RES_LANES * v;
+        at[v] = pad + min(r, rows - 1);
+        outr[v] = TO(0);
+        outi[v] = TO(0);
+        if (r < rows) {
+            outr[v] = pr[r];
+            outi[v] = pi[r];
+            buf[at[v]] = Cx{static_cast<T>(outr[v]), static_cast<T>(outi[v])};
+        }
+    }
+    __syncthreads();
+    int cur = 0;
+    for (int step = 0; step < steps; ++step) {
+        for (int k = 1; k <= m; ++k) {
+            const Cx *x = buf + cur * width;
+            Acc<T> hr[V], hi[V];
+#pragma unroll
+            for (int g = 0; g < RES_ND; g += G) {
+                if (g >= n) continue;  // uniform
+                Cx xv[V][G];
+#pragma unroll
+                for (int u = 0; u < G; ++u)
+#pragma unroll
+                    for (int v = 0; v < V; ++v) xv[v][u] = x[at[v] + off[g + u]];
+#pragma unroll
+                for (int u = 0; u < G; ++u)
+#pragma unroll
+                    for (int v = 0; v < V; ++v)
+                        if constexpr (sizeof(T) == 8) {
+                            if (g + u < n) cmac(hr[v], hi[v], ar[v][g + u], ai[v][g + u], xv[v][u].r, xv[v][u].i);
+                        } else if (on[v] >> (g + u) & 1u) {
+                            cmac(hr[v], hi[v], ar[v][g + u], ai[v][g + u], xv[v][u].r, xv[v][u].i);
+                        }
+            }
+            const T s = static_cast<T>(dt / static_cast<double>(k));
+            Cx *y = buf + (cur ^ 1) * width;
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                Cx t{hi[v].get() * s, -hr[v].get() * s};  // (-i s)(a + ib)
+                if constexpr (std::is_same<T, TO>::value) {
+                    outr[v] = __builtin_fma(s, hi[v].get(), outr[v]);
+                    outi[v] = __builtin_fma(s, -hr[v].get(), outi[v]);
+                } else {
+                    outr[v] += static_cast<TO>(t.r);
+                    outi[v] += static_cast<TO>(t.i);
+                }
+                if (k == m) t = Cx{static_cast<T>(outr[v]), static_cast<T>(outi[v])};  // the next step's input
+                if (static_cast<int>(threadIdx.x) + RES_LANES * v < rows) y[at[v]] = t;
+            }
+            cur ^= 1;
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const int r = static_cast<int>(threadIdx.x) + RES_LANES * v;
+        if (r < rows) {
+            pr[r] = outr[v];
+            pi[r] = outi[v];
+        }
+    }
+}
+
+// Whether H's evolution runs in taylor_resident_kernel: rows and diagonals whose values fit a workgroup's registers (96
+// of a lane's 128; FP32 values two rows per lane), and the two term buffers in 64 KB of LDS. A term then takes 0.7 us (6
+// qubits) to 1.6 us (10 qubits; FP32 10 qubits 1.9, 11 qubits 4.6), a launch of taylor_term_kernel 5.2 to 5.6 us at any
+// of these sizes.
+static bool resident_fits(const dq_devmat &H, int m, int *pad, size_t *lds) {
+    const int V = H.precision == DQ_F64 ? 1 : 2;
+    if (H.rows > static_cast<uint32_t>(RES_LANES * V) || H.n() > RES_ND || H.n() == 0 || m <= 0 || m > RES_TERMS)
+        return false;
+    int p = 0;
+    for (int32_t o : H.offs) p = std::max(p, o < 0 ? -o : o);
+    *pad = p;
+    *lds = 2 * (H.rows + 2 * static_cast<size_t>(p)) * 2 * elem_bytes(H.precision);
+    return *lds <= (size_t(64) << 10);
+}
+
+// r steps of dt on the state (pr, pi), in place.
+template <typename T, typename TO, int V>
+static void launch_resident(const dq_devmat &H, TO *pr, TO *pi, double dt, uint64_t r, int m, int pad, size_t lds,
+                            hipStream_t s) {
+    const unsigned lanes = std::min<unsigned>(RES_LANES, (H.rows + 63) / 64 * 64);
+    const uint64_t per = std::max<uint64_t>(1, RES_TERMS / m);
+    for (uint64_t done = 0; done < r; done += per) {
+        hipLaunchKernelGGL((taylor_resident_kernel<T, TO, V>), dim3(1), dim3(lanes), lds, s, static_cast<int>(H.rows),
+                           H.n(), H.d_meta.as<DiagMeta>(), H.re.as<T>(), H.im.as<T>(), pr, pi, dt, m,
+                           static_cast<int>(std::min(per, r - done)), pad);
+        DQ_LAUNCH_CHECK();
+    }
+}
+
 // ||v||^2 of an FP64 complex vector as RENORM_PARTS block partials (each block sums a fixed, grid-strided share of
 // the elements in a fixed order, so the partials -- and the fold of them -- have the same bits on every run).
 constexpr int RENORM_PARTS = 512;
@@ -303,6 +451,14 @@ static void sumsq_parts(int64_t n, const double *re, const double *im, double *p
     DQ_LAUNCH_CHECK();
 }
 
+// The state back to the norm that part0 holds.
+static void renormalise(int64_t N, double *pr, double *pi, const double *part0, double *part1, hipStream_t s) {
+    sumsq_parts(N, pr, pi, part1, s);
+    hipLaunchKernelGGL(renorm_kernel, dim3(blocks_for(N, 256, 8192)), dim3(256), 0, s, N, pr, pi, part0,
+                       (const double *)part1);
+    DQ_LAUNCH_CHECK();
+}
+
 // The zero-block map of H, read by every term of one evolution; `buf` keeps it. Below EVO_SMALL rows the look-up costs
 // a term more than the skipped loads (8 to 13 qubits: 0.9 to 1.5 us of 5 to 7), so none is made.
 static ZeroMap zero_map(const dq_devmat &H, int m, DevBuf &buf, hipStream_t s) {
@@ -322,6 +478,14 @@ static void evolve(const dq_devmat &H, T *pr, T *pi, double t, uint64_t r, int m
     const int64_t N = H.rows;
     if (r == 0 || N == 0) return;
     const double dt = t / static_cast<double>(r);
+    int pad = 0;
+    size_t lds = 0;
+    if (std::is_same<T, double>::value && resident_fits(H, m, &pad, &lds)) {
+        launch_resident<double, double, 1>(H, reinterpret_cast<double *>(pr), reinterpret_cast<double *>(pi), dt, r, m,
+                                           pad, lds, s);
+        DQ_HIP(hipStreamSynchronize(s));
+        return;
+    }
     DevBuf br(N * sizeof(T)), bi(N * sizeof(T)), t0r(N * sizeof(T)), t0i(N * sizeof(T)), t1r(N * sizeof(T)),
         t1i(N * sizeof(T));
     DevBuf zmap;
@@ -352,6 +516,18 @@ static void evolve_mixed(const dq_devmat &H, double *pr, double *pi, double t, u
     if (r == 0 || N == 0) return;
     const double dt = t / static_cast<double>(r);
     const size_t b32 = N * sizeof(float), b64 = N * sizeof(double);
+    int pad = 0;
+    size_t lds = 0;
+    if (resident_fits(H, m, &pad, &lds)) {
+        DevBuf parts(2 * RENORM_PARTS * sizeof(double));
+        double *part0 = parts.as<double>(), *part1 = part0 + RENORM_PARTS;
+        sumsq_parts(N, pr, pi, part0, s);
+        if (N <= RES_LANES) launch_resident<float, double, 1>(H, pr, pi, dt, r, m, pad, lds, s);
+        else launch_resident<float, double, 2>(H, pr, pi, dt, r, m, pad, lds, s);
+        renormalise(N, pr, pi, part0, part1, s);
+        DQ_HIP(hipStreamSynchronize(s));
+        return;
+    }
     DevBuf xr(b64), xi(b64), p32r(b32), p32i(b32), q32r(b32), q32i(b32), t0r(b32), t0i(b32), t1r(b32), t1i(b32);
     DevBuf parts(2 * RENORM_PARTS * sizeof(double));
     double *part0 = parts.as<double>(), *part1 = part0 + RENORM_PARTS;
@@ -377,10 +553,7 @@ static void evolve_mixed(const dq_devmat &H, double *pr, double *pi, double t, u
                            (const double *)ar, (const double *)ai, pr, pi);
         DQ_LAUNCH_CHECK();
     }
-    sumsq_parts(N, pr, pi, part1, s);
-    hipLaunchKernelGGL(renorm_kernel, dim3(blocks_for(N, 256, 8192)), dim3(256), 0, s, N, pr, pi,
-                       (const double *)part0, (const double *)part1);
-    DQ_LAUNCH_CHECK();
+    renormalise(N, pr, pi, part0, part1, s);
     DQ_HIP(hipStreamSynchronize(s));  // scratch buffers are freed on return
 }
 
