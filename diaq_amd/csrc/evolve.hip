@@ -166,27 +166,36 @@ __global__ __launch_bounds__(256) void horner_kernel(int64_t N, int n, const Dia
     }
 }
 
-// The same Horner level with four states per lane (NS = 4, 8 or 16: NS / 4 lanes per row): each diagonal's gather is
-// one 16-byte load of 4 adjacent states' real parts and one of their imaginary parts, and a lane's matrix value serves
-// its 4 states, so a wave issues a quarter of the vector memory instructions of horner_kernel for the same bytes. A
-// wave covers 256 / NS rows per pass -- exactly one block of the zero-block map -- and the workgroup RPT passes of
-// 1024 / NS rows. Each (row, state) sums its diagonals in the same order with the same operations as horner_kernel,
-// so the two kernels give the same bits.
-template <typename TV, int NS, int RPT, int DU = 1>
-__global__ __launch_bounds__(256) void horner4_kernel(int64_t N, int n, const DiagMeta *__restrict__ meta,
-                                                      int64_t total, const TV *__restrict__ hre,
-                                                      const TV *__restrict__ him, const JobParam *__restrict__ params,
-                                                      int64_t g, double *__restrict__ p64r, double *__restrict__ p64i,
-                                                      float *__restrict__ p32r, float *__restrict__ p32i,
-                                                      const float *__restrict__ bin_r, const float *__restrict__ bin_i,
-                                                      float *__restrict__ bout_r, float *__restrict__ bout_i,
-                                                      int64_t ntiles, int xcd, const uint2 *__restrict__ zmask,
-                                                      int64_t zwords) {
-    static_assert(NS == 4 || NS == 8 || NS == 16, "four states per lane");
-    constexpr int L = NS / 4;         // lanes per row
-    constexpr int WR = 64 / L;        // rows per wave and pass: one zero-map block (256 / NS rows)
-    constexpr int RPP = 4 * WR;       // rows per workgroup pass
-    constexpr int T = RPP * RPT;      // rows per tile: 4 RPT blocks, inside one 32-bit word of the map
+// The same Horner level in wave form: S = min(NS, 4) states per lane, L = NS / S lanes per row, 64 / L rows per wave and
+// pass, RPT passes of the workgroup's four waves. A diagonal's gather is one load of S adjacent states' real parts and one
+// of their imaginary parts, and a lane's matrix value serves its S states.
+//
+// The lanes of a wave first read 64 diagonals' metadata and map words at once, one diagonal each, and keep those that
+// hold a nonzero in the wave's rows as a ballot. The wave then walks the set bits, DU diagonals at a time with all of
+// their loads issued before the first product is added; a part (real, imaginary) that is all zero in the wave's rows
+// is not loaded. Each (row, state) sums its diagonals in the same order with the same operations as horner_kernel, so
+// the two kernels give the same bits.
+//
+// Bound: the round trips to the L2, one for the metadata and one per DU live diagonals; a chain metadata -> map word ->
+// value per diagonal took 22 us a level for two 15-qubit TFIM jobs of 8 states (5.6 ms in all), this 14 (3.6 ms).
+template <typename TV, int NS, int RPT, int DU>
+__global__ __launch_bounds__(256) void horner_wave_kernel(int64_t N, int n, const DiagMeta *__restrict__ meta,
+                                                          int64_t total, const TV *__restrict__ hre,
+                                                          const TV *__restrict__ him,
+                                                          const JobParam *__restrict__ params, int64_t g,
+                                                          double *__restrict__ p64r, double *__restrict__ p64i,
+                                                          float *__restrict__ p32r, float *__restrict__ p32i,
+                                                          const float *__restrict__ bin_r,
+                                                          const float *__restrict__ bin_i, float *__restrict__ bout_r,
+                                                          float *__restrict__ bout_i, int64_t ntiles, int xcd,
+                                                          const uint2 *__restrict__ zmask, int64_t zwords) {
+    constexpr int S = NS < 4 ? NS : 4;  // states per lane
+    constexpr int L = NS / S;           // lanes per row
+    constexpr int WR = 64 / L;          // rows per wave and pass, at most one block of the map (256 / NS rows)
+    constexpr int RPP = 4 * WR;         // rows per workgroup pass
+    constexpr int T = RPP * RPT;        // rows per tile: its blocks lie in one 32-bit word of the map
+    static_assert(T * NS / 256 <= 32 && T < 65536, "one map word, rows of a tile in 16 bits");
+    typedef float SV __attribute__((ext_vector_type(S), aligned(4 * S)));
     const int j = blockIdx.y;
     const JobParam P = params[j];
     if (g >= P.steps) return;
@@ -194,126 +203,125 @@ __global__ __launch_bounds__(256) void horner4_kernel(int64_t N, int n, const Di
     if (t >= ntiles) return;  // uniform: a surplus workgroup of the XCD-contiguous grid
     const int m = P.m;
     const int k = m - 1 - static_cast<int>(g % m);  // Horner level
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int h = lane % L;                          // states 4h .. 4h + 3 of the row
-    const int rw = lane / L;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h = S * (lane % L);                   // states h .. h + S - 1 of the row
     const int64_t tile = t * T;
-    const int64_t vb = static_cast<int64_t>(j) * total;
-    const int64_t sb = static_cast<int64_t>(j) * N * NS;
-    const float *xr = bin_r + sb;
-    const float *xi = bin_i + sb;
-    const int64_t blk0 = t * 4 * RPT;  // the tile's first map block
-    Acc<TV> hr[RPT][4], hi[RPT][4];
-    // DU diagonals per batch: their loads are all issued before the first of them is used (more loads in flight per
-    // wave); the products are still added diagonal after diagonal, in slot order
-    for (int d0 = 0; d0 < n; d0 += DU) {
-        TV va_r[DU][RPT], va_i[DU][RPT];
-        float4 vx_r[DU][RPT], vx_i[DU][RPT];
-        uint32_t lv[DU];
-        int64_t lo_[DU], hi_[DU];
+    const int64_t sb = static_cast<int64_t>(j) * N * NS + tile * NS;
+    const float *xr = bin_r + sb, *xi = bin_i + sb;
+    int row[RPT];  // the lane's rows in the tile
 #pragma unroll
-        for (int u = 0; u < DU; ++u) {
-            lv[u] = 0;
-            lo_[u] = 0;
-            hi_[u] = 0;
+    for (int q = 0; q < RPT; ++q) row[q] = RPP * q + WR * wave + lane / L;
+    // psi's entries, read before the sums so that they add no round trip after them
+    SV pr[RPT], pi[RPT];
 #pragma unroll
-            for (int q = 0; q < RPT; ++q) {
-                va_r[u][q] = TV(0);
-                va_i[u][q] = TV(0);
-                vx_r[u][q] = make_float4(0.f, 0.f, 0.f, 0.f);
-                vx_i[u][q] = vx_r[u][q];
-            }
-            const int d = d0 + u;
-            if (d >= n) continue;  // uniform
+    for (int q = 0; q < RPT; ++q) {
+        pr[q] = SV(0.f);
+        pi[q] = SV(0.f);
+        if (k > 0 && tile + row[q] < N) {
+            pr[q] = *reinterpret_cast<const SV *>(p32r + sb + row[q] * NS + h);
+            pi[q] = *reinterpret_cast<const SV *>(p32i + sb + row[q] * NS + h);
+        }
+    }
+    Acc<TV> hr[RPT][S], hi[RPT][S];
+    for (int k0 = 0; k0 < n; k0 += 64) {
+        int64_t vb = 0;
+        int off = 0, rng = 0, flags = 0;  // rng: the diagonal's rows in the tile, lo | hi << 16; flags: RPT live passes,
+        const int d = k0 + lane;          // bit 8 a real part, bit 9 an imaginary part
+        if (d < n) {
             const DiagMeta md = meta[d];
-            const int64_t rlo = md.rlo, rhi = md.rhi;
-            if (rhi <= tile || rlo >= tile + T) continue;  // uniform
-            uint32_t live = (4 * RPT >= 32) ? ~0u : ((1u << (4 * RPT)) - 1);
-            if (zmask) {
-                const uint32_t w = any_part(zmask[(static_cast<int64_t>(j) * n + d) * zwords + (blk0 >> 5)]);
-                live = (4 * RPT >= 32) ? w : ((w >> (blk0 & 31)) & ((1u << (4 * RPT)) - 1));
-                if (!live) continue;  // uniform: every value of the diagonal in this tile is zero
-            }
-            lv[u] = live;
-            lo_[u] = rlo;
-            hi_[u] = rhi;
-            const TV *ar = hre + vb + md.rowbase;
-            const TV *ai = him + vb + md.rowbase;
+            const int64_t lo = max(md.rlo - tile, int64_t(0)), hi_ = min(md.rhi - tile, int64_t(T));
+            if (lo < hi_) {
+                flags = ((1 << RPT) - 1) | 0x300;
+                if (zmask) {
+                    const int64_t b0 = tile * NS / 256;
+                    const uint2 w = zmask[(static_cast<int64_t>(j) * n + d) * zwords + (b0 >> 5)];
+                    flags = 0;
 #pragma unroll
-            for (int q = 0; q < RPT; ++q) {
-                if (!((live >> (4 * q + wave)) & 1u)) continue;  // uniform in the wave
-                const int64_t r = tile + RPP * q + WR * wave + rw;
-                const int64_t rc = r < rlo ? rlo : (r >= rhi ? rhi - 1 : r);  // stays inside the tile
-                va_r[u][q] = ar[rc];
-                va_i[u][q] = ai[rc];
-                const int64_t xo = (rc + md.off) * NS + 4 * h;
-                vx_r[u][q] = *reinterpret_cast<const float4 *>(xr + xo);
-                vx_i[u][q] = *reinterpret_cast<const float4 *>(xi + xo);
+                    for (int q = 0; q < RPT; ++q) {
+                        const int b = static_cast<int>(b0 & 31) + (RPP * q + WR * wave) * NS / 256;
+                        if (any_part(w) >> b & 1u) flags |= 1 << q;
+                        if (w.x >> b & 1u) flags |= 0x100;
+                        if (w.y >> b & 1u) flags |= 0x200;
+                    }
+                }
+                rng = static_cast<int>(lo) | static_cast<int>(hi_) << 16;
+                vb = static_cast<int64_t>(j) * total + md.rowbase + tile;
+                off = md.off;
             }
         }
+        uint64_t todo = __ballot(flags != 0);
+        while (todo) {  // uniform
+            TV va_r[DU][RPT], va_i[DU][RPT];
+            SV vx_r[DU][RPT], vx_i[DU][RPT];
+            int lo[DU], hi_[DU], lv[DU];
 #pragma unroll
-        for (int u = 0; u < DU; ++u) {
-            // rows off the diagonal add nothing (a compensated sum is not inert to zeros)
+            for (int u = 0; u < DU; ++u) {
+                lv[u] = 0;
+                lo[u] = hi_[u] = 0;
+                if (!todo) continue;
+                const int s = __builtin_ctzll(todo);
+                todo &= todo - 1;
+                const int64_t b = readlane64(vb, s);
+                const int64_t x0 = static_cast<int64_t>(__builtin_amdgcn_readlane(off, s)) * NS + h;
+                const int r2 = __builtin_amdgcn_readlane(rng, s);
+                lv[u] = __builtin_amdgcn_readlane(flags, s);
+                lo[u] = r2 & 0xffff;
+                hi_[u] = r2 >> 16;
 #pragma unroll
-            for (int q = 0; q < RPT; ++q) {
-                const int64_t r = tile + RPP * q + WR * wave + rw;
-                if (((lv[u] >> (4 * q + wave)) & 1u) && r >= lo_[u] && r < hi_[u]) {
-                    cmac(hr[q][0], hi[q][0], va_r[u][q], va_i[u][q], static_cast<TV>(vx_r[u][q].x),
-                         static_cast<TV>(vx_i[u][q].x));
-                    cmac(hr[q][1], hi[q][1], va_r[u][q], va_i[u][q], static_cast<TV>(vx_r[u][q].y),
-                         static_cast<TV>(vx_i[u][q].y));
-                    cmac(hr[q][2], hi[q][2], va_r[u][q], va_i[u][q], static_cast<TV>(vx_r[u][q].z),
-                         static_cast<TV>(vx_i[u][q].z));
-                    cmac(hr[q][3], hi[q][3], va_r[u][q], va_i[u][q], static_cast<TV>(vx_r[u][q].w),
-                         static_cast<TV>(vx_i[u][q].w));
+                for (int q = 0; q < RPT; ++q) {
+                    va_r[u][q] = TV(0);
+                    va_i[u][q] = TV(0);
+                    if (RPT > 1 && !(lv[u] >> q & 1)) continue;  // uniform
+                    const int rc = min(max(row[q], lo[u]), hi_[u] - 1);  // stays inside the tile
+                    if (lv[u] & 0x100) va_r[u][q] = (hre + b)[rc];  // uniform
+                    if (lv[u] & 0x200) va_i[u][q] = (him + b)[rc];
+                    vx_r[u][q] = *reinterpret_cast<const SV *>(xr + x0 + rc * NS);
+                    vx_i[u][q] = *reinterpret_cast<const SV *>(xi + x0 + rc * NS);
                 }
+            }
+#pragma unroll
+            for (int u = 0; u < DU; ++u) {
+                // rows off the diagonal add nothing (a compensated sum is not inert to zeros)
+#pragma unroll
+                for (int q = 0; q < RPT; ++q)
+                    if ((lv[u] >> q & 1) && row[q] >= lo[u] && row[q] < hi_[u]) {
+#pragma unroll
+                        for (int v = 0; v < S; ++v)
+                            cmac(hr[q][v], hi[q][v], va_r[u][q], va_i[u][q], static_cast<TV>(vx_r[u][q][v]),
+                                 static_cast<TV>(vx_i[u][q][v]));
+                    }
             }
         }
     }
 #pragma unroll
     for (int q = 0; q < RPT; ++q) {
-        const int64_t r = tile + RPP * q + WR * wave + rw;
-        if (r >= N) continue;
-        const int64_t o = sb + r * NS + 4 * h;
-        double a[4], b[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            a[v] = static_cast<double>(hr[q][v].get());
-            b[v] = static_cast<double>(hi[q][v].get());
-        }
+        if (tile + row[q] >= N) continue;
+        const int64_t o = sb + row[q] * NS + h;
+        SV outr, outi;
         if (k > 0) {  // b_k = psi + (Y/(k+1)) b_{k+1}, (Y/c) h = (tau/c) (Im h, -Re h)
             const double c = P.tau / static_cast<double>(k + 1);
-            const float4 pr = *reinterpret_cast<const float4 *>(p32r + o);
-            const float4 pi = *reinterpret_cast<const float4 *>(p32i + o);
-            float4 outr, outi;
-            outr.x = static_cast<float>(static_cast<double>(pr.x) + c * b[0]);
-            outr.y = static_cast<float>(static_cast<double>(pr.y) + c * b[1]);
-            outr.z = static_cast<float>(static_cast<double>(pr.z) + c * b[2]);
-            outr.w = static_cast<float>(static_cast<double>(pr.w) + c * b[3]);
-            outi.x = static_cast<float>(static_cast<double>(pi.x) - c * a[0]);
-            outi.y = static_cast<float>(static_cast<double>(pi.y) - c * a[1]);
-            outi.z = static_cast<float>(static_cast<double>(pi.z) - c * a[2]);
-            outi.w = static_cast<float>(static_cast<double>(pi.w) - c * a[3]);
-            *reinterpret_cast<float4 *>(bout_r + o) = outr;
-            *reinterpret_cast<float4 *>(bout_i + o) = outi;
-        } else {  // psi <- psi + Y b_1 in FP64; its FP32 copy goes to p32 (own entries) and to the next level's input
-            float nr32[4], ni32[4];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const double nr = p64r[o + v] + P.tau * b[v];
-                const double ni = p64i[o + v] - P.tau * a[v];
+            for (int v = 0; v < S; ++v) {
+                const double a = static_cast<double>(hr[q][v].get()), b = static_cast<double>(hi[q][v].get());
+                outr[v] = static_cast<float>(static_cast<double>(pr[q][v]) + c * b);
+                outi[v] = static_cast<float>(static_cast<double>(pi[q][v]) - c * a);
+            }
+        } else {  // psi <- psi + Y b_1 in FP64; its FP32 copy goes to p32 (own entries) and to the next level's input
+#pragma unroll
+            for (int v = 0; v < S; ++v) {
+                const double a = static_cast<double>(hr[q][v].get()), b = static_cast<double>(hi[q][v].get());
+                const double nr = p64r[o + v] + P.tau * b;
+                const double ni = p64i[o + v] - P.tau * a;
                 p64r[o + v] = nr;
                 p64i[o + v] = ni;
-                nr32[v] = static_cast<float>(nr);
-                ni32[v] = static_cast<float>(ni);
+                outr[v] = static_cast<float>(nr);
+                outi[v] = static_cast<float>(ni);
             }
-            const float4 fr = make_float4(nr32[0], nr32[1], nr32[2], nr32[3]);
-            const float4 fi = make_float4(ni32[0], ni32[1], ni32[2], ni32[3]);
-            *reinterpret_cast<float4 *>(p32r + o) = fr;
-            *reinterpret_cast<float4 *>(p32i + o) = fi;
-            *reinterpret_cast<float4 *>(bout_r + o) = fr;
-            *reinterpret_cast<float4 *>(bout_i + o) = fi;
+            *reinterpret_cast<SV *>(p32r + o) = outr;
+            *reinterpret_cast<SV *>(p32i + o) = outi;
         }
+        *reinterpret_cast<SV *>(bout_r + o) = outr;
+        *reinterpret_cast<SV *>(bout_i + o) = outi;
     }
 }
 
@@ -383,7 +391,7 @@ __global__ __launch_bounds__(256) void probe_kernel(int64_t N, int n, const Diag
     }
 }
 
-// The probe with four states per lane (NS = 4, 8 or 16), the gathers as 16-byte loads, as horner4_kernel; R rows per
+// The probe with four states per lane (NS = 4, 8 or 16), the gathers as 16-byte loads; R rows per
 // lane, tiles of 4 R zero-map blocks.
 template <typename TV, int NS, int R>
 __global__ __launch_bounds__(256) void probe4_kernel(int64_t N, int n, const DiagMeta *__restrict__ meta,
@@ -560,11 +568,13 @@ struct EvoClass {
     int64_t zwords = 0;
     std::vector<JobParam> params;
     int64_t G = 0;            // launches: max steps
-    int rpt = 4;              // tuned rows per lane
+    // the untuned schedule is the wave form's usual choice (16 jobs of 10 to 15 qubits x 8 states: 6.6 ms; a lane per
+    // state 8.8 ms with one row per lane, 11.9 with four)
+    int rpt = 1;              // tuned rows per lane
     int xcd = 0;              // tuned row-tile order: 0 round-robin over the XCDs, 1 XCD-contiguous
     int lds = 0;              // tuned: 1 = stage each tile's input window in LDS
-    int vec = 0;              // tuned: 1 = horner4_kernel (four states per lane; NS = 4, 8, 16, no LDS window)
-    int du = 1;               // tuned: horner4_kernel's diagonals per load batch (1, 2 or 4; 1 or 2 rows per lane)
+    int vec = 1;              // tuned: 1 = horner_wave_kernel (no LDS window)
+    int du = 4;               // tuned: horner_wave_kernel's diagonals per load batch (1, 2 or 4; 1 or 2 rows per lane)
     hipStream_t stream = nullptr;
     int jobs_n() const { return static_cast<int>(jobs.size()); }
 };
@@ -598,9 +608,9 @@ static int g_evo_rpt = 0;   // 0 = the class's, else 1, 2, 4 or 8
 static int g_evo_xcd = -1;  // -1 = the class's, else 0 or 1
 static int g_evo_lds = -1;  // -1 = the class's, else 0 or 1
 static int g_evo_skip = 1;  // skip the all-zero blocks of a diagonal ("evo_skip_zero_blocks")
-static int g_evo_vec = -1;  // -1 = the class's, else 0 (a lane per state) or 1 (four states per lane) ("evo_vec")
+static int g_evo_vec = -1;  // -1 = the class's, else 0 (a lane per state) or 1 (the wave form) ("evo_vec")
 static int g_evo_lanes = 4; // streams the classes are spread over in dq_evo_run; 0 = one per class ("evo_lanes")
-static int g_evo_du = 0;    // 0 = the class's, else the diagonals whose loads horner4_kernel issues together, for
+static int g_evo_du = 0;    // 0 = the class's, else the diagonals whose loads horner_wave_kernel issues together, for
                             // 1 or 2 rows per lane ("evo_diag_batch": 0, 1, 2 or 4)
 
 bool evo_set_tuning(const std::string &key, int value) {
@@ -656,32 +666,31 @@ static void launch_level(const EvoClass &c, int64_t g, hipStream_t s) {
     const float *bin_r = (g & 1) ? c.b0r.as<float>() : c.b1r.as<float>();
     const float *bin_i = (g & 1) ? c.b0i.as<float>() : c.b1i.as<float>();
     const uint2 *zmask = g_evo_skip ? c.zmask.as<uint2>() : nullptr;
-    if constexpr (NS == 4 || NS == 8 || NS == 16) {
-        if ((g_evo_vec >= 0 ? g_evo_vec : c.vec) == 1) {  // four states per lane (no LDS window)
-            const int64_t rows4 = static_cast<int64_t>(1024 / NS) * rpt;
-            const int64_t nt4 = (N + rows4 - 1) / rows4;
-            const dim3 grid4(static_cast<unsigned>(grid_for_tiles(nt4, xcd)), static_cast<unsigned>(c.jobs_n()));
+    if ((g_evo_vec >= 0 ? g_evo_vec : c.vec) == 1) {  // the wave form (no LDS window)
+        constexpr int WPP = 256 / (NS < 4 ? 1 : NS / 4);  // rows of a workgroup pass
+        const int64_t rows4 = static_cast<int64_t>(WPP) * rpt;
+        const int64_t nt4 = (N + rows4 - 1) / rows4;
+        const dim3 grid4(static_cast<unsigned>(grid_for_tiles(nt4, xcd)), static_cast<unsigned>(c.jobs_n()));
 #define DQ_HORNER4(R, DU)                                                                                          \
-    hipLaunchKernelGGL((horner4_kernel<TV, NS, R, DU>), grid4, dim3(256), 0, s, N, (int)c.offs.size(),              \
+    hipLaunchKernelGGL((horner_wave_kernel<TV, NS, R, DU>), grid4, dim3(256), 0, s, N, (int)c.offs.size(),          \
                        c.d_meta.as<DiagMeta>(), c.total, c.hre.as<TV>(), c.him.as<TV>(), c.d_params.as<JobParam>(), \
                        g, c.p64r.as<double>(), c.p64i.as<double>(), c.p32r.as<float>(), c.p32i.as<float>(), bin_r,   \
                        bin_i, bout_r, bout_i, nt4, xcd, zmask, c.zwords)
-            const int du = rpt <= 2 ? (g_evo_du > 0 ? g_evo_du : c.du) : 1;
-            switch (rpt * 8 + du) {
-                case 9: DQ_HORNER4(1, 1); break;
-                case 10: DQ_HORNER4(1, 2); break;
-                case 12: DQ_HORNER4(1, 4); break;
-                case 17: DQ_HORNER4(2, 1); break;
-                case 18: DQ_HORNER4(2, 2); break;
-                case 20: DQ_HORNER4(2, 4); break;
-                case 33: DQ_HORNER4(4, 1); break;
-                case 65: DQ_HORNER4(8, 1); break;
-                default: throw ArgError("evolve: rows per lane must be 1, 2, 4 or 8");
-            }
-#undef DQ_HORNER4
-            DQ_LAUNCH_CHECK();
-            return;
+        const int du = rpt <= 2 ? (g_evo_du > 0 ? g_evo_du : c.du) : 1;
+        switch (rpt * 8 + du) {
+            case 9: DQ_HORNER4(1, 1); break;
+            case 10: DQ_HORNER4(1, 2); break;
+            case 12: DQ_HORNER4(1, 4); break;
+            case 17: DQ_HORNER4(2, 1); break;
+            case 18: DQ_HORNER4(2, 2); break;
+            case 20: DQ_HORNER4(2, 4); break;
+            case 33: DQ_HORNER4(4, 1); break;
+            case 65: DQ_HORNER4(8, 1); break;
+            default: throw ArgError("evolve: rows per lane must be 1, 2, 4 or 8");
         }
+#undef DQ_HORNER4
+        DQ_LAUNCH_CHECK();
+        return;
     }
     const int64_t rows_per_block = static_cast<int64_t>(RPP) * rpt;
     const int64_t ntiles = (N + rows_per_block - 1) / rows_per_block;
@@ -900,7 +909,6 @@ extern "C" int dq_evo_create(int n_jobs, dq_devmat *const *H, int n_states, int 
             c.d_sq = DevBuf(sizeof(double) * nj * n_states);
             c.d_partial = DevBuf(sizeof(double) * nj * n_states * RENORM_BLOCKS);
             c.d_probe = DevBuf(sizeof(double) * nj * n_states * 2);
-            c.rpt = c.N >= (1u << 14) ? 4 : 1;
             DQ_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
         }
         // copy each Hamiltonian's values into its class slot (converted to the plan's precision: same layout)
@@ -1030,17 +1038,15 @@ extern "C" int dq_evo_tune(dq_evo *E, int *chosen_rpt, int *chosen_xcd, int *cho
             DevBuf fr(sv * 4), fi(sv * 4);
             DQ_HIP(hipMemcpy(fr.p, c.p32r.p, sv * 4, hipMemcpyDeviceToDevice));
             DQ_HIP(hipMemcpy(fi.p, c.p32i.p, sv * 4, hipMemcpyDeviceToDevice));
-            const bool vec_ok = E->n_states == 4 || E->n_states == 8 || E->n_states == 16;
             int bvec = c.vec, bdu = c.du;
             for (int cand = 0; cand < 28; ++cand) {
-                // 0-15: a lane per state (rows per lane x tile order x LDS window); 16-23: four states per lane;
-                // 24-27: four states per lane, 1 or 2 rows per lane, the loads of 2 diagonals batched (batches of
-                // 4 time about as well on a level with every job active but ran the 256-TFIM graph ~3 ms slower)
+                // 0-15: a lane per state (rows per lane x tile order x LDS window); 16-27: the wave form, rows per lane
+                // and diagonals per load batch as below x tile order
+                static constexpr int FORMS[6][2] = {{1, 4}, {1, 2}, {2, 4}, {2, 2}, {4, 1}, {8, 1}};
                 const int vec = cand >= 16 ? 1 : 0;
-                if (vec && !vec_ok) break;
-                const int rpt = cand >= 24 ? 1 << (cand & 1) : 1 << (cand & 3);
-                const int xcd = (cand >> (cand >= 24 ? 1 : 2)) & 1, lds = vec ? 0 : cand >> 3;
-                const int du = cand >= 24 ? 2 : 1;
+                const int rpt = vec ? FORMS[(cand - 16) >> 1][0] : 1 << (cand & 3);
+                const int xcd = vec ? cand & 1 : (cand >> 2) & 1, lds = vec ? 0 : cand >> 3;
+                const int du = vec ? FORMS[(cand - 16) >> 1][1] : 1;
                 c.rpt = rpt;
                 c.xcd = xcd;
                 c.lds = lds;

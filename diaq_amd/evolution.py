@@ -90,8 +90,8 @@ class BatchedEvolution:
 
     def tune(self):
         """Per class: (rows per lane, XCD-contiguous tile order, kernel form) chosen by timing. Form: 0 a lane per
-        state, 1 the same with the LDS window, 2 four states per lane, 3 and 4 four states per lane with the loads of
-        2 or 4 diagonals issued together."""
+        state, 1 the same with the LDS window, 2 the wave form, 3 and 4 the wave form with the loads of 2 or 4
+        diagonals issued together."""
         rpt = (ctypes.c_int * self.n_classes)()
         xcd = (ctypes.c_int * self.n_classes)()
         lds = (ctypes.c_int * self.n_classes)()

@@ -1,0 +1,65 @@
+"""The wave form of the batched evolution's Horner level against a lane per state: the same bits with 1, 2, 4, 8 and 16
+states, sizes that are no multiple of a wave, more than 64 diagonals, diagonals that end inside a wave, and blocks that are
+zero in one part or both; and the values against a Taylor series in NumPy (FP32 values: 2e-6)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from oracle import oracle as O  # noqa: E402
+
+
+def hamiltonian(rows, offs, seed):
+    rng = np.random.default_rng(seed)
+    vals = []
+    for k, o in enumerate(offs):
+        n = O.diagonal_length(o, rows, rows)
+        r = np.arange(n) + max(0, -o)
+        v = (rng.standard_normal(n) + 1j * rng.standard_normal(n)) / (2 * len(offs))
+        v = (v, v.real + 0j, 1j * v.imag, v * (r // (16 << k % 4) % 2))[k % 4]
+        vals.append(v.astype(np.complex64).astype(np.complex128))
+    return O.Dia(rows, rows, list(offs), vals)
+
+
+@pytest.mark.parametrize("n_states", [1, 2, 4, 8, 16])
+@pytest.mark.parametrize("rows,reach", [(65, 2), (300, 40), (1025, 3), (4100, 9)])
+def test_wave_form_has_the_same_bits(rows, reach, n_states):
+    import diaq_amd  # noqa: F401
+    import diaq_gpu as d
+    from diaq_amd import capi, evolution
+    L = capi.lib()
+    offs = sorted({*range(-reach, reach + 1), -rows + 1, rows - 2, rows // 2})
+    H = [hamiltonian(rows, offs, seed) for seed in (1, 2)]
+    B = evolution.BatchedEvolution([d.to_device(d.diaQMatrix.from_diagonals([rows, rows], M.offsets, M.vals)) for M in H],
+                                   n_states, "fp32")
+    t, m, s = [0.9, 0.5], [7, 9], [1, 2]
+    B.set_schedule(t, m, s)
+    rng = np.random.default_rng(4)
+    st = [rng.standard_normal((n_states, rows)) + 1j * rng.standard_normal((n_states, rows)) for _ in H]
+    st = [v / np.linalg.norm(v, axis=1, keepdims=True) for v in st]
+
+    def run(vec, rpt, du):
+        for key, v in ((b"evo_vec", vec), (b"evo_rows_per_lane", rpt), (b"evo_diag_batch", du)):
+            capi.check(L.dq_set_tuning(key, v))
+        for j, v in enumerate(st):
+            B.set_states(j, v)
+        B.run(use_graph=False, renormalize=False)
+        return [B.get_states(j, rows) for j in range(2)]
+
+    try:
+        base = run(0, 1, 0)
+        for rpt, du in ((1, 1), (1, 2), (1, 4), (2, 2), (2, 4), (4, 0), (8, 0)):
+            for a, b in zip(run(1, rpt, du), base):
+                np.testing.assert_array_equal(a, b, err_msg=f"rpt={rpt} du={du}")
+    finally:
+        for key, v in ((b"evo_vec", -1), (b"evo_rows_per_lane", 0), (b"evo_diag_batch", 0)):
+            capi.check(L.dq_set_tuning(key, v))
+    for j, M in enumerate(H):
+        for a, v in zip(base[j], st[j]):
+            tau = t[j] / 2 ** s[j]
+            for _ in range(2 ** s[j]):
+                term = v
+                for k in range(1, m[j] + 1):
+                    term = O.spmv(M, term) * (-1j * tau / k)
+                    v = v + term
+            assert np.linalg.norm(a - v) < 2e-6
