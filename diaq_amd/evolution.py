@@ -71,15 +71,12 @@ class BatchedEvolution:
     def set_states(self, job: int, states: np.ndarray):
         """states: (n_states, N) complex array."""
         st = np.ascontiguousarray(states, dtype=np.complex128)
-        re = np.ascontiguousarray(st.real)
-        im = np.ascontiguousarray(st.imag)
-        capi.check(capi.lib().dq_evo_set_states(self._h, job, capi.ptr(re), capi.ptr(im)))
+        capi.check(capi.lib().dq_evo_set_states_complex(self._h, job, capi.ptr(st)))
 
     def get_states(self, job: int, N: int) -> np.ndarray:
-        re = np.empty(self.n_states * N)
-        im = np.empty(self.n_states * N)
-        capi.check(capi.lib().dq_evo_get_states(self._h, job, capi.ptr(re), capi.ptr(im)))
-        return (re + 1j * im).reshape(self.n_states, N)
+        st = np.empty((self.n_states, N), np.complex128)
+        capi.check(capi.lib().dq_evo_get_states_complex(self._h, job, capi.ptr(st)))
+        return st
 
     def set_schedule(self, t, m, s):
         t = np.ascontiguousarray(t, np.float64)

@@ -380,6 +380,9 @@ int dq_evo_info(const dq_evo *E, int *n_classes, int *n_jobs, int *n_states);
 /* States of one job, state-major host arrays: state s, row r at [s*N + r]. */
 int dq_evo_set_states(dq_evo *E, int job, const double *re, const double *im);
 int dq_evo_get_states(const dq_evo *E, int job, double *re, double *im);
+/* The same with interleaved complex values, z[2 (s N + r)] + i z[2 (s N + r) + 1]. */
+int dq_evo_set_states_complex(dq_evo *E, int job, const double *z);
+int dq_evo_get_states_complex(const dq_evo *E, int job, double *z);
 
 /* Per job: evolve to t[j] by 2^s[j] sub-steps of a degree-m[j] Taylor polynomial (1 <= m <= 64, 0 <= s <= 24). */
 int dq_evo_set_schedule(dq_evo *E, const double *t, const int32_t *m, const int32_t *s);

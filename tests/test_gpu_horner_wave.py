@@ -63,3 +63,27 @@ def test_wave_form_has_the_same_bits(rows, reach, n_states):
                     term = O.spmv(M, term) * (-1j * tau / k)
                     v = v + term
             assert np.linalg.norm(a - v) < 2e-6
+
+
+@pytest.mark.parametrize("n_states", [1, 2, 16])
+@pytest.mark.parametrize("rows", [1, 3, 257])
+def test_states_cross_unchanged(rows, n_states):
+    """Split and interleaved states in and out of a job: the same values back through either pair, per job."""
+    import diaq_amd  # noqa: F401
+    import diaq_gpu as d
+    from diaq_amd import capi, evolution
+    L = capi.lib()
+    D = d.to_device(d.diaQMatrix.from_diagonals([rows, rows], [0], [np.ones(rows, complex)]))
+    B = evolution.BatchedEvolution([D, D], n_states, "fp32")
+    rng = np.random.default_rng(rows)
+    st = [rng.standard_normal((n_states, rows)) + 1j * rng.standard_normal((n_states, rows)) for _ in range(2)]
+    re, im = st[0].real.copy(), st[0].imag.copy()
+    capi.check(L.dq_evo_set_states(B._h, 0, capi.ptr(re), capi.ptr(im)))
+    B.set_states(1, st[1])
+    for j in range(2):
+        np.testing.assert_array_equal(B.get_states(j, rows), st[j])
+        a, b = np.empty((n_states, rows)), np.empty((n_states, rows))
+        capi.check(L.dq_evo_get_states(B._h, j, capi.ptr(a), capi.ptr(b)))
+        np.testing.assert_array_equal(a + 1j * b, st[j])
+    with pytest.raises(capi.DqError):
+        capi.check(L.dq_evo_set_states_complex(B._h, 2, capi.ptr(st[0])))
