@@ -325,6 +325,134 @@ __global__ __launch_bounds__(256) void horner_wave_kernel(int64_t N, int n, cons
     }
 }
 
+// All Horner levels of `subs` sub-steps of small Hamiltonians in one launch: a workgroup per (state, job), V rows per lane
+// (row = lane + 1024 v), the Horner vector in LDS (two buffers, a barrier per level), psi, its FP32 copy and the rows'
+// values, of up to RES_ND diagonals, in registers. A row takes exactly the diagonals that horner_kernel gives it -- those
+// it lies on whose zero-map block is live -- in the same order with the same operations, so the bits are the same.
+//
+// Bound: the compensated FP32 sums, 16 vector instructions per row, diagonal and level on one CU (10 qubits, 21
+// diagonals: 5376 clocks, 2.2 us). A launch per level costs its launch and three round trips to the L2 at least, 8 to 9
+// us, and a graph of many short nodes is enqueued at 2 to 3 us a node, which held back the large classes' streams:
+// TFIM jobs, 8 states each, wave form and this: 128 of 10 qubits 3.01 and 1.22 ms, 32 of 11 qubits 2.79 and 1.37 ms.
+constexpr int RES_LANES = 1024, RES_ND = 24;
+constexpr int RES_LEVELS = 4096;  // levels of a launch: 10 to 25 ms at most
+
+template <typename TV, int V>
+__global__ __launch_bounds__(RES_LANES) void horner_resident_kernel(int N, int n, int NS,
+                                                                    const DiagMeta *__restrict__ meta, int64_t total,
+                                                                    const TV *__restrict__ hre,
+                                                                    const TV *__restrict__ him,
+                                                                    const JobParam *__restrict__ params, int64_t sub0,
+                                                                    int subs, double *__restrict__ p64r,
+                                                                    double *__restrict__ p64i,
+                                                                    float *__restrict__ p32r,
+                                                                    float *__restrict__ p32i,
+                                                                    const uint2 *__restrict__ zmask, int64_t zwords) {
+    constexpr int G = V == 1 ? 4 : 2;  // diagonals whose x is read together: what the registers leave
+    __shared__ float2 x[2][RES_LANES * V];
+    __shared__ int s_off[RES_ND], s_base[RES_ND];
+    const int st = blockIdx.x, j = blockIdx.y;
+    const JobParam P = params[j];
+    const int64_t nsub = int64_t(1) << P.s;
+    if (P.steps == 0 || sub0 >= nsub) return;  // uniform: the job is done
+    const int todo = static_cast<int>(min(static_cast<int64_t>(subs), nsub - sub0));
+    const TV *ar = hre + j * total, *ai = him + j * total;
+    if (static_cast<int>(threadIdx.x) < n) {
+        s_off[threadIdx.x] = meta[threadIdx.x].off;
+        s_base[threadIdx.x] = static_cast<int>(meta[threadIdx.x].rowbase);
+    }
+    __syncthreads();
+    int row[V];
+    uint32_t on[V];  // a bit per diagonal that the row takes
+    TV rr[V][RES_ND], ri[V][RES_ND];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        row[v] = static_cast<int>(threadIdx.x) + RES_LANES * v;
+        on[v] = 0;
+        const int blk = row[v] * NS / 256;
+        for (int k = 0; k < n; ++k) {  // uniform
+            const int c = row[v] + s_off[k];
+            bool take = row[v] < N && c >= 0 && c < N;
+            if (take)
+                take = any_part(zmask[(static_cast<int64_t>(j) * n + k) * zwords + (blk >> 5)]) >> (blk & 31) & 1u;
+            if (take) on[v] |= 1u << k;
+        }
+#pragma unroll
+        for (int k = 0; k < RES_ND; ++k) {
+            const bool take = on[v] >> k & 1u;
+            const int e = take ? s_base[k] + row[v] : 0;
+            rr[v][k] = take ? ar[e] : TV(0);
+            ri[v][k] = take ? ai[e] : TV(0);
+        }
+    }
+    double sr[V], si[V];  // psi
+    float fr[V], fi[V];   // its FP32 copy
+    const int64_t o = static_cast<int64_t>(j) * N * NS + st;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        sr[v] = si[v] = 0.0;
+        fr[v] = fi[v] = 0.f;
+        if (row[v] < N) {
+            sr[v] = p64r[o + static_cast<int64_t>(row[v]) * NS];
+            si[v] = p64i[o + static_cast<int64_t>(row[v]) * NS];
+            fr[v] = p32r[o + static_cast<int64_t>(row[v]) * NS];
+            fi[v] = p32i[o + static_cast<int64_t>(row[v]) * NS];
+            x[0][row[v]] = make_float2(fr[v], fi[v]);
+        }
+    }
+    __syncthreads();
+    int cur = 0;
+    for (int sub = 0; sub < todo; ++sub) {
+        for (int k = P.m - 1; k >= 0; --k) {  // Horner level
+            const float2 *in = x[cur];
+            Acc<TV> hr[V], hi[V];
+#pragma unroll
+            for (int g = 0; g < RES_ND; g += G)
+                if (g < n) {  // uniform
+                    float2 xv[G][V];
+#pragma unroll
+                    for (int u = 0; u < G; ++u)
+#pragma unroll
+                        for (int v = 0; v < V; ++v)
+                            xv[u][v] = in[on[v] >> (g + u) & 1u ? row[v] + s_off[g + u] : 0];
+#pragma unroll
+                    for (int u = 0; u < G; ++u)
+#pragma unroll
+                        for (int v = 0; v < V; ++v)
+                            if (on[v] >> (g + u) & 1u)
+                                cmac(hr[v], hi[v], rr[v][g + u], ri[v][g + u], static_cast<TV>(xv[u][v].x),
+                                     static_cast<TV>(xv[u][v].y));
+                }
+            const double c = P.tau / static_cast<double>(k + 1);  // k = 0: tau itself
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                const double a = static_cast<double>(hr[v].get()), b = static_cast<double>(hi[v].get());
+                float br, bi;
+                if (k > 0) {  // b_k = psi + (Y/(k+1)) b_{k+1}, (Y/c) h = (tau/c) (Im h, -Re h); one rounding each
+                    br = static_cast<float>(__builtin_fma(c, b, static_cast<double>(fr[v])));
+                    bi = static_cast<float>(__builtin_fma(-c, a, static_cast<double>(fi[v])));
+                } else {  // psi <- psi + Y b_1 in FP64
+                    sr[v] = __builtin_fma(c, b, sr[v]);
+                    si[v] = __builtin_fma(-c, a, si[v]);
+                    br = fr[v] = static_cast<float>(sr[v]);
+                    bi = fi[v] = static_cast<float>(si[v]);
+                }
+                if (row[v] < N) x[cur ^ 1][row[v]] = make_float2(br, bi);
+            }
+            cur ^= 1;
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+        if (row[v] < N) {
+            p64r[o + static_cast<int64_t>(row[v]) * NS] = sr[v];
+            p64i[o + static_cast<int64_t>(row[v]) * NS] = si[v];
+            p32r[o + static_cast<int64_t>(row[v]) * NS] = fr[v];
+            p32i[o + static_cast<int64_t>(row[v]) * NS] = fi[v];
+        }
+}
+
 // Forward Taylor terms of the first sub-step for the a-posteriori estimate: t_k = (Y/k) t_{k-1}, t_0 = psi (FP32);
 // the squared norms of t_m and t_{m+1} of every state are accumulated into norms[(j*NS + state)*2 + (k - m)].
 template <typename TV, int NS, int RPT>
@@ -509,7 +637,16 @@ __global__ void fold_states_kernel(int nblocks, const double *__restrict__ parti
     const int j = blockIdx.x;
     for (int st = threadIdx.x; st < NS; st += blockDim.x) {
         double v = 0.0;
-        for (int b = 0; b < nblocks; ++b) v += partial[(static_cast<int64_t>(j) * nblocks + b) * NS + st];
+        const double *p = partial + static_cast<int64_t>(j) * nblocks * NS + st;
+        int b = 0;
+        for (; b + 16 <= nblocks; b += 16) {  // 16 loads in flight, added in order (256 partials: 47 us one by one)
+            double w[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) w[u] = p[(b + u) * NS];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v += w[u];
+        }
+        for (; b < nblocks; ++b) v += p[b * NS];
         out[static_cast<int64_t>(j) * NS + st] = v;
     }
 }
@@ -738,6 +875,45 @@ static void launch_level(const EvoClass &c, int64_t g, hipStream_t s) {
     DQ_LAUNCH_CHECK();
 }
 
+// Rows per lane of horner_resident_kernel for a class, 0: a launch per level. FP32 values up to 2048 rows, FP64 values
+// (twice the registers) up to 1024. TFIM, one job of one state, us a level here and with a launch each: 7 qubits 1.3 and
+// 4.7, 10 qubits 2.3 and 6.7, 11 qubits 5.3 and 7.1. At 4096 rows the values no longer fit, and reading them again each
+// level took 20 us against 7.5 to 14. An override of the Horner schedule asks for the launches.
+static int resident_rows(const EvoClass &c, int precision) {
+    if (g_evo_rpt > 0 || g_evo_xcd >= 0 || g_evo_lds >= 0 || g_evo_vec >= 0 || g_evo_du > 0 || !g_evo_skip) return 0;
+    const size_t n = c.offs.size();
+    if (n <= static_cast<size_t>(RES_ND) && c.N <= static_cast<uint32_t>(RES_LANES)) return 1;
+    return precision == DQ_F32 && n <= static_cast<size_t>(RES_ND) && c.N <= 2u * RES_LANES ? 2 : 0;
+}
+
+// The launches of a resident class: sub-steps of its longest job, RES_LEVELS levels or one sub-step at a time.
+static void launch_resident(const EvoClass &c, int precision, int NS, hipStream_t s) {
+    int64_t longest = 0;
+    int m = 1;
+    for (const JobParam &p : c.params) {
+        if (p.steps == 0) continue;
+        longest = std::max(longest, int64_t(1) << p.s);
+        m = std::max(m, p.m);
+    }
+    const int64_t per = std::max<int64_t>(1, RES_LEVELS / m);
+    const int V = resident_rows(c, precision);
+    const dim3 grid(static_cast<unsigned>(NS), static_cast<unsigned>(c.jobs_n()));
+    const dim3 lanes(std::min<unsigned>(RES_LANES, (c.N + 63) / 64 * 64));
+    for (int64_t sub = 0; sub < longest; sub += per) {
+        const int subs = static_cast<int>(std::min(per, longest - sub));
+#define DQ_RESIDENT(TV, V)                                                                                          \
+    hipLaunchKernelGGL((horner_resident_kernel<TV, V>), grid, lanes, 0, s, static_cast<int>(c.N),              \
+                       static_cast<int>(c.offs.size()), NS, c.d_meta.as<DiagMeta>(), c.total, c.hre.as<TV>(),       \
+                       c.him.as<TV>(), c.d_params.as<JobParam>(), sub, subs, c.p64r.as<double>(),                   \
+                       c.p64i.as<double>(), c.p32r.as<float>(), c.p32i.as<float>(), c.zmask.as<uint2>(), c.zwords)
+        if (precision != DQ_F32) DQ_RESIDENT(double, 1);
+        else if (V == 1) DQ_RESIDENT(float, 1);
+        else DQ_RESIDENT(float, 2);
+#undef DQ_RESIDENT
+        DQ_LAUNCH_CHECK();
+    }
+}
+
 constexpr int RENORM_BLOCKS = 256;
 
 template <int NS>
@@ -803,6 +979,11 @@ static void run_class_levels(dq_evo &E, EvoClass &c, hipStream_t s, bool renorm)
     dispatch(E.value_precision, E.n_states, [&](auto tv, auto ns) {
         using TV = decltype(tv);
         constexpr int NS = decltype(ns)::value;
+        if (resident_rows(c, E.value_precision)) {
+            launch_resident(c, E.value_precision, NS, s);
+            if (renorm) launch_renorm<NS>(c, s);
+            return;
+        }
         // prologue: the FP32 state into the input buffer of level 0 (b1: level g reads buffer (g+1) mod 2)
         const int64_t sv = static_cast<int64_t>(c.N) * NS * c.jobs_n();
         hipLaunchKernelGGL(copyf_kernel, dim3(blocks_for(sv, 256, 4096)), dim3(256), 0, s, sv, c.p32r.as<float>(),
@@ -837,6 +1018,11 @@ static std::vector<std::vector<int>> lane_plan(const dq_evo &E) {
             static_cast<double>(c.N) * (static_cast<double>(elem_bytes(E.value_precision)) *
                                             static_cast<double>(c.offs.size()) +
                                         24.0 * E.n_states);
+        if (const int V = resident_rows(c, E.value_precision)) {  // a workgroup per state, 2.3 us a level (V = 1)
+            const int64_t waves = (static_cast<int64_t>(c.jobs_n()) * E.n_states + 255) / 256;
+            cost[ci] = 0.0023 * V * static_cast<double>(c.G * waves);
+            continue;
+        }
         cost[ci] = 0.012 * static_cast<double>(c.G) + static_cast<double>(job_levels) * bytes_per_job_level / 3e9;
     }
     std::vector<int> order(nc);
@@ -860,7 +1046,14 @@ static std::vector<std::vector<int>> lane_plan(const dq_evo &E) {
 static std::vector<int64_t> graph_signature(const dq_evo &E, bool renorm) {
     std::vector<int64_t> sig{renorm ? 1 : 0, g_evo_rpt, g_evo_xcd, g_evo_lds, g_evo_skip, g_evo_vec, g_evo_lanes,
                              g_evo_du};
-    for (const auto &c : E.classes) sig.insert(sig.end(), {c.G, c.rpt, c.xcd, c.lds, c.vec, c.du});
+    for (const auto &c : E.classes) {
+        int64_t subs = 0, m = 0;  // what a resident class's launches depend on
+        for (const JobParam &p : c.params) {
+            subs = std::max<int64_t>(subs, p.steps ? int64_t(1) << p.s : 0);
+            m = std::max<int64_t>(m, p.m);
+        }
+        sig.insert(sig.end(), {c.G, c.rpt, c.xcd, c.lds, c.vec, c.du, subs, m});
+    }
     for (const auto &lane : lane_plan(E)) {
         sig.push_back(-1);
         sig.insert(sig.end(), lane.begin(), lane.end());

@@ -65,6 +65,42 @@ def test_wave_form_has_the_same_bits(rows, reach, n_states):
             assert np.linalg.norm(a - v) < 2e-6
 
 
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("rows,diags,n_states", [(1, 1, 1), (63, 24, 8), (64, 7, 2), (1023, 24, 4), (1024, 23, 16),
+                                                 (1024, 25, 8), (1025, 24, 1), (2048, 24, 8), (2049, 5, 1)])
+def test_many_levels_in_one_launch(rows, diags, n_states, precision):
+    """Small classes run all levels in one workgroup per state, up to 24 diagonals: the bits of a launch per level, also
+    across launches (more than 4096 levels), for jobs of different lengths, and on replays of the graph."""
+    import diaq_amd  # noqa: F401
+    import diaq_gpu as d
+    from diaq_amd import capi, evolution
+    L = capi.lib()
+    offs = sorted([0, *range(1, diags)], key=lambda k: (k * 7919) % 101)[:diags]
+    offs = sorted({o if k % 2 else -o for k, o in enumerate(offs) if o < rows} | ({rows - 1} if rows > diags else set()))
+    offs = offs[-diags:]
+    H = [hamiltonian(rows, offs, seed) for seed in (1, 2)]
+    B = evolution.BatchedEvolution([d.to_device(d.diaQMatrix.from_diagonals([rows, rows], M.offsets, M.vals)) for M in H],
+                                   n_states, precision)
+    B.set_schedule([0.7, 1.5], [7, 5], [3, 10])
+    rng = np.random.default_rng(4)
+    st = [rng.standard_normal((n_states, rows)) + 1j * rng.standard_normal((n_states, rows)) for _ in H]
+
+    def run(vec, graph):
+        capi.check(L.dq_set_tuning(b"evo_vec", vec))
+        for j, v in enumerate(st):
+            B.set_states(j, v)
+        B.run(use_graph=graph, renormalize=True)
+        return [B.get_states(j, rows) for j in range(2)]
+
+    try:
+        base = run(1, False)
+        for graph in (False, True, True):
+            for a, b in zip(run(-1, graph), base):
+                np.testing.assert_array_equal(a, b)
+    finally:
+        capi.check(L.dq_set_tuning(b"evo_vec", -1))
+
+
 @pytest.mark.parametrize("n_states", [1, 2, 16])
 @pytest.mark.parametrize("rows", [1, 3, 257])
 def test_states_cross_unchanged(rows, n_states):
