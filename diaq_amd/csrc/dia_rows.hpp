@@ -185,6 +185,11 @@ size_t zero_map_bytes(const dq_devmat &A, int shift);
 // The map dq_spmv_tune keeps in A's handle (none if it keeps none).
 ZeroMap kept_zero_map(const dq_devmat &A);
 
+// Several products with a band matrix per read of it (powers.hip): the launches for a sequence of n, n where one per
+// product is at least as good; and one launch, y = A^p x.
+int band_powers_launches(const dq_devmat &A, int n);
+void band_powers(const dq_devmat &A, const void *xr, const void *xi, void *yr, void *yi, int p, hipStream_t s);
+
 // PIPE = true: each diagonal's 4*RPT loads are issued together (full tiles unconditionally, boundary tiles with
 // clamped addresses), the schedule that keeps the most bytes in flight. Every schedule adds exactly the products of
 // the rows on the diagonal, in slot order, so a row's sum has the same bits whatever the schedule (a compensated

@@ -305,6 +305,8 @@ void spmv_banded(const dq_devmat &A, const void *xr, const void *xi, void *yr, v
     }
 }
 
+constexpr int64_t NOALLOC_SCRATCH_WORDS = int64_t(1) << 22;  // see `scratch` below
+
 static int g_spmv_skip = 1;  // "spmv_skip_zero_blocks"
 
 // Whether a sequence of n SpMVs on A's values should make its own zero-block map: not for a single product (the map
@@ -313,6 +315,22 @@ static int g_spmv_skip = 1;  // "spmv_skip_zero_blocks"
 // nor with the skip switched off.
 static bool ntimes_uses_map(const dq_devmat &A, int n) {
     return g_spmv_skip && n >= 2 && A.n() > 0 && A.rows >= (1u << 16) && !A.zmap_valid;
+}
+
+// The launches of a sequence of n products: several products each for a band matrix (band_powers_launches), else one.
+// At 1000 to 6 10^6 rows and 3 to 40 diagonals 2 products take 0.35 to 0.93 and 5 products 0.17 to 0.62 of a launch each.
+// Not where the tuner found that skipping A's zero blocks pays, nor under a process-wide schedule, nor for a matrix whose
+// map would not fit the allocation-free form's scratch (that form refuses the call).
+static int sequence_launches(const dq_devmat &A, int n) {
+    const bool forced = g_spmv_rpt > 0 || g_spmv_bands > 0 || g_spmv_nt >= 0 || g_spmv_pipe >= 0 || g_spmv_lds >= 0 ||
+                        g_spmv_xcd >= 0 || !g_spmv_skip;
+    if (forced || A.zmap_valid || zero_map_bytes(A, 8) > sizeof(uint2) * NOALLOC_SCRATCH_WORDS) return n;
+    return band_powers_launches(A, n);
+}
+
+// The products of launch i.
+static int sequence_products(int n, int launches, int i) {
+    return static_cast<int>(int64_t(n) * (i + 1) / launches - int64_t(n) * i / launches);
 }
 
 // The map a product with A may use without making one: the handle's, for FP64 matrices. (In FP64 a skipped block
@@ -643,14 +661,15 @@ static void ntimes_device(const dq_devmat *A, const void *xr, const void *xi, vo
         throw ArgError("spmv_ntimes_device: work vectors are needed for num_times > 1 or x == y");
     // destinations alternate between y and the work vectors so that the last product lands in y; with x == y and an
     // odd count the first product must not overwrite x, so the order flips and a copy ends the sequence
-    const bool flip = in_place && (n % 2 == 1);
+    const int launches = sequence_launches(*A, n);
+    const bool flip = in_place && (launches % 2 == 1);
     // the zero blocks of A, skipped by every product of the sequence (A cannot change during the call): the map
     // dq_spmv_tune kept in the handle, or else, for two or more products, one made here -- in the caller's fixed
     // memory, or in stream-ordered memory so the call stays asynchronous. Without fixed memory no map is made while
     // the stream is being captured into a graph (a replay must not read memory this call has given back).
     uint2 *zmap = nullptr;
     ZeroMap z = sequence_map(*A, n);
-    if (!z.w && ntimes_uses_map(*A, n)) {
+    if (launches == n && !z.w && ntimes_uses_map(*A, n)) {
         size_t bytes = zero_map_bytes(*A, z.shift);
         uint2 *to = nullptr;
         if (fixed_map) {
@@ -682,10 +701,11 @@ static void ntimes_device(const dq_devmat *A, const void *xr, const void *xi, vo
         }
     }
     const void *sr = xr, *si = xi;
-    for (int t = 0; t < n; ++t) {
-        const bool to_y = (((n - 1 - t) % 2) == 0) != flip;
+    for (int t = 0; t < launches; ++t) {
+        const bool to_y = (((launches - 1 - t) % 2) == 0) != flip;
         void *dr = to_y ? yr : work_r, *di = to_y ? yi : work_i;
-        spmv_banded(*A, sr, si, dr, di, 0, s, z);
+        if (launches < n) band_powers(*A, sr, si, dr, di, sequence_products(n, launches, t), s);
+        else spmv_banded(*A, sr, si, dr, di, 0, s, z);
         sr = dr;
         si = di;
     }
@@ -705,7 +725,6 @@ extern "C" int dq_spmv_ntimes_device(const dq_devmat *A, const void *xr, const v
 // those would not fit; two bits each, for every diagonal), 32 MiB per GPU, held from the library's load until the
 // process ends. In host code `scratch` only stands in for the symbol; its device address comes from
 // hipGetSymbolAddress, once per device.
-constexpr int64_t NOALLOC_SCRATCH_WORDS = int64_t(1) << 22;
 static __device__ __align__(256) uint2 scratch[NOALLOC_SCRATCH_WORDS];
 
 constexpr int NOALLOC_MAX_DEVICES = 64;
@@ -758,16 +777,18 @@ extern "C" int dq_spmv_ntimes_host(const dq_devmat *A, const double *xr, const d
         a.put(xr, xi);
         DevBuf zmap;
         ZeroMap z = sequence_map(*A, n);
-        if (!z.w && ntimes_uses_map(*A, n)) {
+        const int launches = sequence_launches(*A, n);
+        if (launches == n && !z.w && ntimes_uses_map(*A, n)) {
             zmap = DevBuf(zero_map_bytes(*A, z.shift));
             make_zero_map(*A, z.shift, zmap.as<uint2>(), 0);
             z.w = zmap.as<uint2>();
             z.words = zero_block_words(A->rows, 1 << z.shift);
         }
         DevVec *in = &a, *out = &b;
-        for (int t = 0; t < n; ++t) {
-            spmv_banded(*A, in->r.p, in->i.p, out->r.p, out->i.p, 0, 0, z);
-            if (t != n - 1) std::swap(in, out);
+        for (int t = 0; t < launches; ++t) {
+            if (launches < n) band_powers(*A, in->r.p, in->i.p, out->r.p, out->i.p, sequence_products(n, launches, t), 0);
+            else spmv_banded(*A, in->r.p, in->i.p, out->r.p, out->i.p, 0, 0, z);
+            if (t != launches - 1) std::swap(in, out);
         }
         out->get(yr, yi);
     });
