@@ -23,7 +23,6 @@
 #include <algorithm>
 #include <cmath>
 #include <map>
-#include <numeric>
 #include <vector>
 
 #include "dia_rows.hpp"
@@ -979,11 +978,6 @@ static void run_class_levels(dq_evo &E, EvoClass &c, hipStream_t s, bool renorm)
     dispatch(E.value_precision, E.n_states, [&](auto tv, auto ns) {
         using TV = decltype(tv);
         constexpr int NS = decltype(ns)::value;
-        if (resident_rows(c, E.value_precision)) {
-            launch_resident(c, E.value_precision, NS, s);
-            if (renorm) launch_renorm<NS>(c, s);
-            return;
-        }
         // prologue: the FP32 state into the input buffer of level 0 (b1: level g reads buffer (g+1) mod 2)
         const int64_t sv = static_cast<int64_t>(c.N) * NS * c.jobs_n();
         hipLaunchKernelGGL(copyf_kernel, dim3(blocks_for(sv, 256, 4096)), dim3(256), 0, s, sv, c.p32r.as<float>(),
@@ -994,7 +988,16 @@ static void run_class_levels(dq_evo &E, EvoClass &c, hipStream_t s, bool renorm)
     });
 }
 
-// Which classes run on which stream, in order. Branches of a graph share the process's few hardware queues, and a
+// A resident class's levels.
+static void run_class_resident(const dq_evo &E, const EvoClass &c, hipStream_t s, bool renorm) {
+    dispatch(E.value_precision, E.n_states, [&](auto, auto ns) {
+        constexpr int NS = decltype(ns)::value;
+        launch_resident(c, E.value_precision, NS, s);
+        if (renorm) launch_renorm<NS>(c, s);
+    });
+}
+
+// Which classes with a launch per level run on which stream, in order. Branches of a graph share the process's few hardware queues, and a
 // queue runs what it is given in order, so with a stream per class the classes mostly ran one after another, the
 // longest often late (256-TFIM batch: one kernel in flight 79 % of the graph's time). Instead the classes go to
 // g_evo_lanes streams by longest-first list scheduling on an estimate of their time -- per level a launch cost, per
@@ -1003,8 +1006,12 @@ static void run_class_levels(dq_evo &E, EvoClass &c, hipStream_t s, bool renorm)
 static std::vector<std::vector<int>> lane_plan(const dq_evo &E) {
     const int nc = static_cast<int>(E.classes.size());
     std::vector<std::vector<int>> plan;
+    std::vector<int> order;
+    for (int ci = 0; ci < nc; ++ci)
+        if (!resident_rows(E.classes[ci], E.value_precision)) order.push_back(ci);
+    if (order.empty()) return plan;
     if (g_evo_lanes == 0) {
-        for (int ci = 0; ci < nc; ++ci) plan.push_back({ci});
+        for (int ci : order) plan.push_back({ci});
         return plan;
     }
     std::vector<double> cost(nc, 0.0);
@@ -1018,17 +1025,10 @@ static std::vector<std::vector<int>> lane_plan(const dq_evo &E) {
             static_cast<double>(c.N) * (static_cast<double>(elem_bytes(E.value_precision)) *
                                             static_cast<double>(c.offs.size()) +
                                         24.0 * E.n_states);
-        if (const int V = resident_rows(c, E.value_precision)) {  // a workgroup per state, 2.3 us a level (V = 1)
-            const int64_t waves = (static_cast<int64_t>(c.jobs_n()) * E.n_states + 255) / 256;
-            cost[ci] = 0.0023 * V * static_cast<double>(c.G * waves);
-            continue;
-        }
         cost[ci] = 0.012 * static_cast<double>(c.G) + static_cast<double>(job_levels) * bytes_per_job_level / 3e9;
     }
-    std::vector<int> order(nc);
-    std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost[a] > cost[b]; });
-    const int k = std::min(g_evo_lanes, std::max(1, nc));
+    const int k = std::min(g_evo_lanes, static_cast<int>(order.size()));
     plan.assign(k, {});
     std::vector<double> load(k, 0.0);
     for (int ci : order) {
@@ -1046,14 +1046,7 @@ static std::vector<std::vector<int>> lane_plan(const dq_evo &E) {
 static std::vector<int64_t> graph_signature(const dq_evo &E, bool renorm) {
     std::vector<int64_t> sig{renorm ? 1 : 0, g_evo_rpt, g_evo_xcd, g_evo_lds, g_evo_skip, g_evo_vec, g_evo_lanes,
                              g_evo_du};
-    for (const auto &c : E.classes) {
-        int64_t subs = 0, m = 0;  // what a resident class's launches depend on
-        for (const JobParam &p : c.params) {
-            subs = std::max<int64_t>(subs, p.steps ? int64_t(1) << p.s : 0);
-            m = std::max<int64_t>(m, p.m);
-        }
-        sig.insert(sig.end(), {c.G, c.rpt, c.xcd, c.lds, c.vec, c.du, subs, m});
-    }
+    for (const auto &c : E.classes) sig.insert(sig.end(), {c.G, c.rpt, c.xcd, c.lds, c.vec, c.du});
     for (const auto &lane : lane_plan(E)) {
         sig.push_back(-1);
         sig.insert(sig.end(), lane.begin(), lane.end());
@@ -1188,10 +1181,10 @@ static void put_states(dq_evo *E, int job, const double *re, const double *im, c
     DevBuf in(static_cast<size_t>(n) * 16);
     double *d = in.as<double>();
     if (both) {
-        DQ_HIP(hipMemcpyAsync(d, both, n * 16, hipMemcpyHostToDevice, 0));
+        DQ_HIP(hipMemcpy(d, both, n * 16, hipMemcpyHostToDevice));
     } else {
-        DQ_HIP(hipMemcpyAsync(d, re, n * 8, hipMemcpyHostToDevice, 0));
-        DQ_HIP(hipMemcpyAsync(d + n, im, n * 8, hipMemcpyHostToDevice, 0));
+        DQ_HIP(hipMemcpy(d, re, n * 8, hipMemcpyHostToDevice));
+        DQ_HIP(hipMemcpy(d + n, im, n * 8, hipMemcpyHostToDevice));
     }
     hipLaunchKernelGGL(states_in_kernel, dim3(blocks_for(n, 256, 4096)), dim3(256), 0, 0, N, E->n_states, d,
                        both ? d + 1 : d + n, both ? 2 : 1, c->p64r.as<double>() + at, c->p64i.as<double>() + at,
@@ -1335,8 +1328,9 @@ extern "C" int dq_evo_tune(dq_evo *E, int *chosen_rpt, int *chosen_xcd, int *cho
     });
 }
 
-// Evolve every job by its schedule. use_graph: capture all classes (one stream each, forked from and joined to
-// `stream`) into one graph on the first call and replay it afterwards; otherwise launch directly. renormalize: end
+// Evolve every job by its schedule. Resident classes, a few launches each, run on their own streams, forked from and
+// joined to `stream`. The others: use_graph captures them (on the streams of the lane plan) into one graph on the first
+// call and replays it afterwards; otherwise they are launched directly. renormalize: end
 // with the FP64 renormalisation of every state. ms_out (may be NULL): elapsed GPU time.
 extern "C" int dq_evo_run(dq_evo *E, int use_graph, int renormalize, uintptr_t stream, float *ms_out) {
     return guard([&] {
@@ -1366,7 +1360,24 @@ extern "C" int dq_evo_run(dq_evo *E, int use_graph, int renormalize, uintptr_t s
                 DQ_HIP(hipStreamWaitEvent(base, joins[li], 0));
             }
         };
-        if (use_graph) {
+        std::vector<hipEvent_t> res_events;  // the fork, then a join per resident class
+        auto start_resident = [&] {
+            auto event = [&] {
+                hipEvent_t e;
+                DQ_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+                res_events.push_back(e);
+                return e;
+            };
+            const hipEvent_t start = event();
+            DQ_HIP(hipEventRecord(start, s0));
+            for (const EvoClass &c : E->classes) {
+                if (!resident_rows(c, E->value_precision)) continue;
+                DQ_HIP(hipStreamWaitEvent(c.stream, start, 0));
+                run_class_resident(*E, c, c.stream, renormalize != 0);
+                DQ_HIP(hipEventRecord(event(), c.stream));
+            }
+        };
+        if (use_graph && !plan.empty()) {
             std::vector<int64_t> sig = graph_signature(*E, renormalize != 0);
             if (E->exec && E->graph_sig != sig) {
                 (void)hipGraphExecDestroy(E->exec); E->exec = nullptr;
@@ -1391,18 +1402,21 @@ extern "C" int dq_evo_run(dq_evo *E, int use_graph, int renormalize, uintptr_t s
                 E->graph_sig = std::move(sig);
             }
             DQ_HIP(hipEventRecord(e0, s0));
+            start_resident();
             DQ_HIP(hipGraphLaunch(E->exec, s0));
-            DQ_HIP(hipEventRecord(e1, s0));
         } else {
             DQ_HIP(hipEventRecord(e0, s0));
-            body(s0);
-            DQ_HIP(hipEventRecord(e1, s0));
+            start_resident();
+            if (!plan.empty()) body(s0);
         }
+        for (size_t i = 1; i < res_events.size(); ++i) DQ_HIP(hipStreamWaitEvent(s0, res_events[i], 0));
+        DQ_HIP(hipEventRecord(e1, s0));
         DQ_HIP(hipEventSynchronize(e1));
         float ms = 0.f;
         DQ_HIP(hipEventElapsedTime(&ms, e0, e1));
         if (ms_out) *ms_out = ms;
         for (auto &j : joins) (void)hipEventDestroy(j);
+        for (auto &e : res_events) (void)hipEventDestroy(e);
         (void)hipEventDestroy(fork);
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
