@@ -34,6 +34,7 @@
 // The items also write C's own zero-block map, by ballots on what they store; a large result keeps it (map_blocks).
 #include <algorithm>
 #include <atomic>
+#include <cstring>
 #include <memory>
 #include <numeric>
 
@@ -419,6 +420,10 @@ __global__ __launch_bounds__(256) void map_bits_kernel(int64_t n, const uint2 *_
     if ((threadIdx.x & 63) == 0) atomicAdd(out, static_cast<unsigned long long>(c));
 }
 
+// Pair lists up to this size join the other work lists in one upload; longer ones are copied from where they are, as
+// gathering them first would take about as long as a copy of their own.
+constexpr size_t UPLOAD_PAIR_BYTES = size_t(1) << 18;
+
 // The 64-row blocks of C's diagonals, when the product is to map them for the result's own products, else 0: FP64 values
 // beyond the Infinity Cache, where a product is bound by reading them (H*H of TFIM-20, 11 GB: SpMV 1.90 -> 0.94 ms). A
 // smaller result saves less than the map's fill, count and read-back (about 15 us).
@@ -492,17 +497,44 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
     for (int x = 0; x < 8; ++x) per_xcd = std::max(per_xcd, xcd_first[x + 1] - xcd_first[x]);
     const int64_t grid = per_xcd * 8;
     if (grid > 0x7fffffffLL) throw ArgError("product: too many work items");
-    DevBuf dfirst(sizeof(int64_t) * first.size()), dclo(sizeof(int32_t) * c_lo.size()),
-        dqof(sizeof(int32_t) * q_of.size()), dxcd(sizeof(int64_t) * xcd_first.size()),
-        ditems(sizeof(int2) * static_cast<size_t>(n_work)), dps(sizeof(int64_t) * d.pair_start.size()),
-        dsa(sizeof(int32_t) * std::max<size_t>(1, d.sa.size())), dsb(sizeof(int32_t) * std::max<size_t>(1, d.sb.size()));
-    DQ_HIP(hipMemcpyAsync(dfirst.p, first.data(), dfirst.bytes, hipMemcpyHostToDevice, s));
-    DQ_HIP(hipMemcpyAsync(dclo.p, c_lo.data(), dclo.bytes, hipMemcpyHostToDevice, s));
-    DQ_HIP(hipMemcpyAsync(dqof.p, q_of.data(), dqof.bytes, hipMemcpyHostToDevice, s));
-    DQ_HIP(hipMemcpyAsync(dxcd.p, xcd_first.data(), dxcd.bytes, hipMemcpyHostToDevice, s));
-    DQ_HIP(hipMemcpyAsync(dps.p, d.pair_start.data(), dps.bytes, hipMemcpyHostToDevice, s));
-    DQ_HIP(hipMemcpyAsync(dsa.p, d.sa.data(), sizeof(int32_t) * d.sa.size(), hipMemcpyHostToDevice, s));
-    DQ_HIP(hipMemcpyAsync(dsb.p, d.sb.data(), sizeof(int32_t) * d.sb.size(), hipMemcpyHostToDevice, s));
+    // one block for the work lists and, but for long pair lists, one copy: seven of each cost a small product more than
+    // its kernel (2048 rows, 11-qubit Pauli sum squared, with the conversion to dense: 172 -> 158 us; 1024 rows, TFIM-10 squared and applied: 113 -> 81)
+    size_t lists = 0;
+    auto place = [&](size_t bytes) {
+        const size_t at = lists;
+        lists += (bytes + 15) / 16 * 16;
+        return at;
+    };
+    const size_t at_first = place(sizeof(int64_t) * first.size()), at_clo = place(sizeof(int32_t) * c_lo.size()),
+                 at_qof = place(sizeof(int32_t) * q_of.size()), at_xcd = place(sizeof(int64_t) * xcd_first.size()),
+                 at_ps = place(sizeof(int64_t) * d.pair_start.size()), small = lists,
+                 at_sa = place(sizeof(int32_t) * d.sa.size()), at_sb = place(sizeof(int32_t) * d.sb.size()),
+                 whole = lists, at_items = place(sizeof(int2) * static_cast<size_t>(n_work));
+    DevBuf work(lists);
+    char *const dev = work.as<char>();
+    const bool pairs_too = whole - small <= UPLOAD_PAIR_BYTES;
+    std::vector<char> host(pairs_too ? whole : small);
+    auto put = [&](size_t at, const auto &v) {
+        if (!v.empty()) std::memcpy(host.data() + at, v.data(), sizeof(v[0]) * v.size());
+    };
+    put(at_first, first);
+    put(at_clo, c_lo);
+    put(at_qof, q_of);
+    put(at_xcd, xcd_first);
+    put(at_ps, d.pair_start);
+    if (pairs_too) {
+        put(at_sa, d.sa);
+        put(at_sb, d.sb);
+    } else {
+        DQ_HIP(hipMemcpyAsync(dev + at_sa, d.sa.data(), sizeof(int32_t) * d.sa.size(), hipMemcpyHostToDevice, s));
+        DQ_HIP(hipMemcpyAsync(dev + at_sb, d.sb.data(), sizeof(int32_t) * d.sb.size(), hipMemcpyHostToDevice, s));
+    }
+    DQ_HIP(hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, s));
+    const auto *dfirst = reinterpret_cast<const int64_t *>(dev + at_first), *dxcd = reinterpret_cast<const int64_t *>(dev + at_xcd),
+               *dps = reinterpret_cast<const int64_t *>(dev + at_ps);
+    const auto *dclo = reinterpret_cast<const int32_t *>(dev + at_clo), *dqof = reinterpret_cast<const int32_t *>(dev + at_qof),
+               *dsa = reinterpret_cast<const int32_t *>(dev + at_sa), *dsb = reinterpret_cast<const int32_t *>(dev + at_sb);
+    auto *ditems = reinterpret_cast<int2 *>(dev + at_items);
     // zero-block maps of A and B (a squaring maps its operand once; a map the handle keeps is used as it is)
     DevBuf zab, zbb;
     ZeroMap za, zb;
@@ -531,13 +563,11 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
     }
     const int64_t zc_words = zero_block_words(C->rows, 64);
     hipLaunchKernelGGL(product_items_kernel, dim3(static_cast<unsigned>(std::min<int64_t>(n_chunks, 65536))),
-                       dim3(256), 0, s, n_chunks, dfirst.as<int64_t>(), dclo.as<int32_t>(), dqof.as<int32_t>(),
-                       ditems.as<int2>());
+                       dim3(256), 0, s, n_chunks, dfirst, dclo, dqof, ditems);
     DQ_LAUNCH_CHECK();
 #define DQ_PROD_LAUNCH_M(T, NTS, R, M)                                                                             \
     hipLaunchKernelGGL((product_kernel<T, NTS, R, M>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, s,        \
-                       ditems.as<int2>(), dxcd.as<int64_t>(), dps.as<int64_t>(), dsa.as<int32_t>(),               \
-                       dsb.as<int32_t>(), A.d_meta.as<DiagMeta>(), B.d_meta.as<DiagMeta>(), C->d_meta.as<DiagMeta>(), \
+                       ditems, dxcd, dps, dsa, dsb, A.d_meta.as<DiagMeta>(), B.d_meta.as<DiagMeta>(), C->d_meta.as<DiagMeta>(), \
                        A.re.as<T>(), A.im.as<T>(), B.re.as<T>(), B.im.as<T>(), C->re.as<T>(), C->im.as<T>(), divisor, \
                        za, zb, zcb.as<uint2>(), zc_words)
 #define DQ_PROD_LAUNCH_R(T, NTS, R)                          \
