@@ -673,7 +673,9 @@ static void plan_passes(dq_gate_plan &P, int low_qubits, const std::vector<HostG
 template <typename T>
 static void run_passes(const dq_gate_plan &P, void *re, void *im, hipStream_t s) {
     const int64_t ntiles = int64_t(1) << (P.n_qubits - P.L);
-    const unsigned grid = blocks_for(ntiles, 1, 4096);
+    // four tiles or more per workgroup of a large state: with sixteen the last workgroups left a tenth of the chip idle
+    // (28 qubits 7.15 -> 7.07 ms, FP32 4.91 -> 4.79, 25 qubits 804 -> 781 us)
+    const unsigned grid = blocks_for(ntiles, 1, 16384);
     for (size_t i = 0; i < P.passes.size(); ++i) {
         if (P.passes[i].single >= 0) {
             const dq_devmat &G = *P.big[P.passes[i].single];
