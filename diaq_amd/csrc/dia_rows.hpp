@@ -175,7 +175,13 @@ struct ZeroMap {
     int64_t words = 0;
     int shift = 6;
     int loads_only = 0;  // spare the loads of zeros, but add their products too (dia_rows_wave)
+    // Or, in place of w, the map that the first product of a sequence leaves (dia_rows_wave, MK): per 64-row block and 64
+    // diagonals a word of real and one of imaginary bits (`words` then holds the rows).
+    const ulonglong2 *by_block = nullptr;
+    __host__ __device__ bool any() const { return w || by_block; }
 };
+
+inline int64_t map_by_block_bytes(int64_t rows, int n) { return ((rows + 63) / 64) * ((n + 63) / 64) * 16; }
 
 // Map A's values into w (zero_block_words(A.rows, 2^shift) words per diagonal; shift 6 or 8) on stream s.
 void make_zero_map(const dq_devmat &A, int shift, uint2 *w, hipStream_t s);
@@ -335,11 +341,14 @@ constexpr int RNG_HI = 10, RNG_MASK = (1 << RNG_HI) - 1, RNG_RE = 1 << 20, RNG_I
 // and add nothing). Lane s holds diagonal s: vb (element index of its value in the wave's first row), off and rng.
 // ZM: a part whose rng bit is clear is zero in these rows and is not loaded. H > 0: (sr, si) is the workgroup's x
 // window at the wave's first row, and the diagonals with |off| <= H read x from there.
-template <typename T, int V, int DB, bool NT, bool ZM, int H, bool PART>
+// MK: the values' nonzero parts go to `bits` of the diagonal's lane, one bit per 64-row block and part (block q of the
+// wave: real 1 << 2 q, imaginary 2 << 2 q), and a diagonal that is zero in all of the wave's rows adds nothing, as with a map.
+template <typename T, int V, int DB, bool NT, bool ZM, int H, bool PART, bool MK>
 __device__ inline void wave_batch(uint64_t &todo, int cnt, int lane, int64_t vb, int off, int rng,
                                   const T *__restrict__ are, const T *__restrict__ aim, const T *__restrict__ xr,
                                   const T *__restrict__ xi, Acc<T> (&ar)[V], Acc<T> (&ai)[V], const T *sr,
-                                  const T *si) {
+                                  const T *si, int &bits) {
+    int from[DB];
     T va_r[DB][V], va_i[DB][V], vx_r[DB][V], vx_i[DB][V];
     int lo[DB], hi[DB];
     bool full = true;  // every row of the wave lies on every diagonal of the batch
@@ -350,6 +359,7 @@ __device__ inline void wave_batch(uint64_t &todo, int cnt, int lane, int64_t vb,
             s = __builtin_ctzll(todo);
             todo &= todo - 1;
         }
+        from[u] = s;
         const int64_t b = readlane64(vb, s);
         const int x = __builtin_amdgcn_readlane(off, s);
         const bool near = H > 0 && x >= -H && x <= H;  // uniform
@@ -390,10 +400,35 @@ __device__ inline void wave_batch(uint64_t &todo, int cnt, int lane, int64_t vb,
             }
         }
     }
+    bool live[DB];  // uniform
+#pragma unroll
+    for (int u = 0; u < DB; ++u) live[u] = !PART || u < cnt;
+    if constexpr (MK) {
+#pragma unroll
+        for (int u = 0; u < DB; ++u) {
+            bool r = false, i = false;  // a lane's V rows lie in one block
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                const bool in = live[u] && V * lane + v >= lo[u] && V * lane + v < hi[u];
+                r = r || (in && !(va_r[u][v] == T(0)));
+                i = i || (in && !(va_i[u][v] == T(0)));
+            }
+            const uint64_t nr = __ballot(r), ni = __ballot(i);
+            live[u] = nr || ni;
+            int found = 0;
+#pragma unroll
+            for (int q = 0; q < V; ++q) {
+                constexpr uint64_t BLOCK = V == 1 ? ~uint64_t(0) : (uint64_t(1) << (64 / V)) - 1;
+                if ((nr >> (q * (64 / V) % 64)) & BLOCK) found |= 1 << (2 * q);
+                if ((ni >> (q * (64 / V) % 64)) & BLOCK) found |= 2 << (2 * q);
+            }
+            if (found && lane == from[u]) bits = found;
+        }
+    }
     if (full) {  // uniform
 #pragma unroll
         for (int u = 0; u < DB; ++u)
-            if (!PART || u < cnt) {
+            if (live[u]) {
 #pragma unroll
                 for (int v = 0; v < V; ++v) cmac(ar[v], ai[v], va_r[u][v], va_i[u][v], vx_r[u][v], vx_i[u][v]);
             }
@@ -403,19 +438,20 @@ __device__ inline void wave_batch(uint64_t &todo, int cnt, int lane, int64_t vb,
     for (int u = 0; u < DB; ++u)  // rows off the diagonal add nothing (not even a zero)
 #pragma unroll
         for (int v = 0; v < V; ++v)
-            if ((!PART || u < cnt) && V * lane + v >= lo[u] && V * lane + v < hi[u])
+            if (live[u] && V * lane + v >= lo[u] && V * lane + v < hi[u])
                 cmac(ar[v], ai[v], va_r[u][v], va_i[u][v], vx_r[u][v], vx_i[u][v]);
 }
 
 // The sums of rows row0 + V lane + v (row0 a multiple of 64 V, below the matrix's rows). With a map its blocks are at
 // least a wave's rows or whole parts of them. H > 0: the caller has staged the x window of the workgroup's 256 V rows
 // with stage_x_window (halo H on both sides) in (sr, si).
-template <typename T, int V, bool NT, bool ZM, int H = 0>
+// MK: no map yet; the wave writes its blocks' words of zm.by_block (passed as `made`) from what it reads.
+template <typename T, int V, bool NT, bool ZM, int H = 0, bool MK = false>
 __device__ inline void dia_rows_wave(int64_t row0, int n, const DiagMeta *__restrict__ meta,
                                      const T *__restrict__ are, const T *__restrict__ aim, const T *__restrict__ xr,
                                      const T *__restrict__ xi, int64_t col_lo, int64_t col_hi, Acc<T> (&ar)[V],
                                      Acc<T> (&ai)[V], const ZeroMap &zm, const T *sr = nullptr,
-                                     const T *si = nullptr) {
+                                     const T *si = nullptr, ulonglong2 *made = nullptr, int64_t rows = 0) {
     constexpr int DB = 8 / V;
     const int lane = threadIdx.x & 63;
     xr += row0;
@@ -435,7 +471,20 @@ __device__ inline void dia_rows_wave(int64_t row0, int n, const DiagMeta *__rest
             const int64_t hi = min(min(m.rhi, col_hi - m.off) - row0, int64_t(64 * V));
             live = lo < hi;
             int parts = RNG_RE | RNG_IM;
-            if constexpr (ZM) {  // the 2^shift-row block that holds the wave's rows, or the blocks that they are
+            if (ZM && zm.by_block) {  // the wave's blocks (the last ones may lie past the rows: live is false there)
+                const int64_t words = (n + 63) >> 6;
+                const int64_t blk = (row0 >> 6) * words + (k0 >> 6);
+                ulonglong2 w = zm.by_block[blk];
+#pragma unroll
+                for (int q = 1; q < V; ++q)
+                    if (row0 + 64 * q < zm.words) {  // words: the rows of a map by block
+                        const ulonglong2 o = zm.by_block[blk + q * words];
+                        w.x |= o.x;
+                        w.y |= o.y;
+                    }
+                parts = ((w.x >> lane) & 1 ? RNG_RE : 0) | ((w.y >> lane) & 1 ? RNG_IM : 0);
+                live = live && parts;
+            } else if constexpr (ZM) {  // the 2^shift-row block that holds the wave's rows, or the blocks that they are
                 const uint2 w = zm.w[static_cast<int64_t>(k) * zm.words + (row0 >> (zm.shift + 5))];
                 const int b = static_cast<int>((row0 >> zm.shift) & 31);
                 uint32_t m2 = 1u;
@@ -450,14 +499,25 @@ __device__ inline void dia_rows_wave(int64_t row0, int n, const DiagMeta *__rest
             rng = live ? static_cast<int>(lo) | static_cast<int>(hi) << RNG_HI | parts : 0;
         }
         uint64_t todo = __ballot(live);
-        int cnt = __popcll(todo);
+        int cnt = __popcll(todo), bits = 0;
         for (; cnt >= DB; cnt -= DB)
-            wave_batch<T, V, DB, NT, ZM, H, false>(todo, DB, lane, vb, off, rng, are, aim, xr, xi, ar, ai, sr, si);
+            wave_batch<T, V, DB, NT, ZM, H, false, MK>(todo, DB, lane, vb, off, rng, are, aim, xr, xi, ar, ai, sr, si, bits);
         if (cnt >= DB / 2) {
-            wave_batch<T, V, DB / 2, NT, ZM, H, false>(todo, DB / 2, lane, vb, off, rng, are, aim, xr, xi, ar, ai, sr, si);
+            wave_batch<T, V, DB / 2, NT, ZM, H, false, MK>(todo, DB / 2, lane, vb, off, rng, are, aim, xr, xi, ar, ai, sr,
+                                                           si, bits);
             cnt -= DB / 2;
         }
-        if (cnt) wave_batch<T, V, DB / 2, NT, ZM, H, true>(todo, cnt, lane, vb, off, rng, are, aim, xr, xi, ar, ai, sr, si);
+        if (cnt)
+            wave_batch<T, V, DB / 2, NT, ZM, H, true, MK>(todo, cnt, lane, vb, off, rng, are, aim, xr, xi, ar, ai, sr, si,
+                                                          bits);
+        if constexpr (MK) {
+#pragma unroll
+            for (int q = 0; q < V; ++q) {
+                const uint64_t re = __ballot((bits >> (2 * q)) & 1), im = __ballot((bits >> (2 * q)) & 2);
+                if (lane == 0 && row0 + 64 * q < rows)
+                    made[((row0 >> 6) + q) * ((n + 63) >> 6) + (k0 >> 6)] = make_ulonglong2(re, im);
+            }
+        }
     }
 }
 

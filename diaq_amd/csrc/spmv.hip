@@ -71,15 +71,17 @@ __global__ __launch_bounds__(256) void spmv_rows_kernel(int64_t rows, int64_t co
 }
 
 // V rows per lane on dia_rows_wave: waves of 64 V rows, four to a workgroup. ZM: zm is a zero-block map of A whose
-// all-zero blocks are skipped: the map dq_spmv_tune keeps in the handle (recomputed when the values are rewritten), or
-// one spMV_ntimes makes for a call.
-template <typename T, int V, bool NT, bool ZM, bool LDS>
+// all-zero blocks are skipped: the map dq_spmv_tune keeps in the handle (recomputed when the values are rewritten), a
+// product's own, or one that spMV_ntimes makes for a call.
+// MK: A has no map, and the product leaves one in `made` (map_by_block_bytes) for the products that follow.
+template <typename T, int V, bool NT, bool ZM, bool LDS, bool MK>
 __global__ __launch_bounds__(256) void spmv_wave_kernel(int64_t rows, int64_t cols, int n,
                                                         const DiagMeta *__restrict__ meta, const T *__restrict__ are,
                                                         const T *__restrict__ aim, const T *__restrict__ xr,
                                                         const T *__restrict__ xi, T *__restrict__ yr,
                                                         T *__restrict__ yi, int64_t col_lo, int64_t col_hi,
-                                                        int accumulate, int64_t ntiles, int xcd, ZeroMap zm) {
+                                                        int accumulate, int64_t ntiles, int xcd, ZeroMap zm,
+                                                        ulonglong2 *__restrict__ made) {
     constexpr int H = LDS ? 128 * V : 0;
     __shared__ T sr[LDS ? 256 * V + 2 * H : 1], si[LDS ? 256 * V + 2 * H : 1];
     const int64_t t = tile_of_block(blockIdx.x, ntiles, xcd);
@@ -99,7 +101,7 @@ __global__ __launch_bounds__(256) void spmv_wave_kernel(int64_t rows, int64_t co
             ai[v].add(bi[v]);
         }
     }
-    dia_rows_wave<T, V, NT, ZM, H>(row0, n, meta, are, aim, xr, xi, col_lo, col_hi, ar, ai, zm, sr, si);
+    dia_rows_wave<T, V, NT, ZM, H, MK>(row0, n, meta, are, aim, xr, xi, col_lo, col_hi, ar, ai, zm, sr, si, made, rows);
     T outr[V], outi[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) {
@@ -120,7 +122,7 @@ struct SpmvSched {
 
 template <typename T>
 static void launch_rows(const dq_devmat &A, const T *xr, const T *xi, T *yr, T *yi, const SpmvSched &c, int64_t c0,
-                        int64_t c1, int accumulate, hipStream_t s, const ZeroMap &zm) {
+                        int64_t c1, int accumulate, hipStream_t s, const ZeroMap &zm, ulonglong2 *made) {
     const int64_t rows = A.rows, cols = A.cols;
     const DiagMeta *meta = A.d_meta.as<DiagMeta>();
     const T *are = static_cast<const T *>(A.re.p), *aim = static_cast<const T *>(A.im.p);
@@ -131,19 +133,21 @@ static void launch_rows(const dq_devmat &A, const T *xr, const T *xi, T *yr, T *
     if (c.rpt == 1) {
         const int64_t wtiles = (rows + 256 * c.v - 1) / (256 * c.v);
         const dim3 wg(static_cast<unsigned>(grid_for_tiles(wtiles, c.xcd)));
-#define DQ_SPMV_WAVE_V(V, NT, Z, L)                                                                                  \
-    hipLaunchKernelGGL((spmv_wave_kernel<T, V, NT, Z, L>), wg, dim3(256), 0, s, rows, cols, A.n(), meta, are, aim, xr, \
-                       xi, yr, yi, c0, c1, accumulate, wtiles, c.xcd, zm)
-#define DQ_SPMV_WAVE(NT, Z)                                        \
-    do {                                                           \
-        if (c.v == 2 && c.lds) DQ_SPMV_WAVE_V(2, NT, Z, true);     \
-        else if (c.v == 2) DQ_SPMV_WAVE_V(2, NT, Z, false);        \
-        else DQ_SPMV_WAVE_V(1, NT, Z, false);                      \
+#define DQ_SPMV_WAVE_V(V, NT, Z, L, MK)                                                                              \
+    hipLaunchKernelGGL((spmv_wave_kernel<T, V, NT, Z, L, MK>), wg, dim3(256), 0, s, rows, cols, A.n(), meta, are, aim, \
+                       xr, xi, yr, yi, c0, c1, accumulate, wtiles, c.xcd, zm, made)
+#define DQ_SPMV_WAVE(NT, Z, MK)                                        \
+    do {                                                               \
+        if (c.v == 2 && c.lds) DQ_SPMV_WAVE_V(2, NT, Z, true, MK);     \
+        else if (c.v == 2) DQ_SPMV_WAVE_V(2, NT, Z, false, MK);        \
+        else DQ_SPMV_WAVE_V(1, NT, Z, false, MK);                      \
     } while (0)
-        if (c.nt && zm.w) DQ_SPMV_WAVE(true, true);
-        else if (c.nt) DQ_SPMV_WAVE(true, false);
-        else if (zm.w) DQ_SPMV_WAVE(false, true);
-        else DQ_SPMV_WAVE(false, false);
+        if (made && c.nt) DQ_SPMV_WAVE(true, false, true);
+        else if (made) DQ_SPMV_WAVE(false, false, true);
+        else if (c.nt && zm.any()) DQ_SPMV_WAVE(true, true, false);
+        else if (c.nt) DQ_SPMV_WAVE(true, false, false);
+        else if (zm.any()) DQ_SPMV_WAVE(false, true, false);
+        else DQ_SPMV_WAVE(false, false, false);
 #undef DQ_SPMV_WAVE
 #undef DQ_SPMV_WAVE_V
         DQ_LAUNCH_CHECK();
@@ -275,9 +279,11 @@ static SpmvSched sched_for(const dq_devmat &A, bool map) {
 }
 
 // y = A x in n_bands column passes (0: automatic), skipping A's all-zero blocks when zm has a map. The schedule is
-// `force` if given, else the process-wide knobs, else A's tuned choice, else the defaults.
+// `force` if given, else the process-wide knobs, else A's tuned choice, else the defaults. made: the product, in one
+// pass, leaves a map by block there.
 void spmv_banded(const dq_devmat &A, const void *xr, const void *xi, void *yr, void *yi, int n_bands,
-                 hipStream_t s, const ZeroMap &zm = ZeroMap(), const SpmvSched *force = nullptr) {
+                 hipStream_t s, const ZeroMap &zm = ZeroMap(), const SpmvSched *force = nullptr,
+                 ulonglong2 *made = nullptr) {
     if (A.rows == 0) return;
     if (A.n() == 0) {  // no diagonals: y = 0 (a fill kernel, safe inside graph capture)
         const unsigned g = blocks_for(A.rows, 256, 4096);
@@ -292,16 +298,16 @@ void spmv_banded(const dq_devmat &A, const void *xr, const void *xi, void *yr, v
     }
     if (n_bands <= 0) n_bands = auto_bands(A);
     if (n_bands > static_cast<int>(A.cols)) n_bands = std::max<int>(1, A.cols);
-    const SpmvSched c = force ? *force : sched_for(A, zm.w != nullptr);
+    const SpmvSched c = force ? *force : sched_for(A, zm.any() || made);
     const int64_t cols = A.cols;
     for (int b = 0; b < n_bands; ++b) {
         const int64_t c0 = cols * b / n_bands, c1 = cols * (b + 1) / n_bands;
         if (A.precision == DQ_F64)
             launch_rows<double>(A, (const double *)xr, (const double *)xi, (double *)yr, (double *)yi, c, c0, c1, b > 0,
-                                s, zm);
+                                s, zm, made);
         else
             launch_rows<float>(A, (const float *)xr, (const float *)xi, (float *)yr, (float *)yi, c, c0, c1, b > 0, s,
-                               zm);
+                               zm, made);
     }
 }
 
@@ -632,6 +638,19 @@ extern "C" int dq_spmv_host(const dq_devmat *A, const double *xr, const double *
     });
 }
 
+// A product of a sequence: with `made`, the first one leaves A's map by block there and the others skip by it. It reads
+// every value anyway, and a map from a pass of its own costs as much as a product (10^6 rows, 33 random diagonals, FP64, two
+// products: 274 -> 198 us; TFIM-20, five: 418 -> 373).
+static void sequence_product(const dq_devmat &A, const void *xr, const void *xi, void *yr, void *yi, hipStream_t s,
+                             const ZeroMap &map, ulonglong2 *made, bool first) {
+    ZeroMap z = map;
+    if (made && !first) {
+        z.by_block = made;
+        z.words = A.rows;
+    }
+    spmv_banded(A, xr, xi, yr, yi, 0, s, z, nullptr, first ? made : nullptr);
+}
+
 // y = A^n x on device vectors (src/spMV_ntimes_gpu.cu:61-263 on resident data). `fixed_map` (may be null) is
 // device memory of fixed_bytes bytes the call may use for A's zero-block map instead of allocating one: the
 // allocation-free entry point passes its static scratch array; then the map is made even while the stream is being
@@ -667,36 +686,46 @@ static void ntimes_device(const dq_devmat *A, const void *xr, const void *xi, vo
     // dq_spmv_tune kept in the handle, or else, for two or more products, one made here -- in the caller's fixed
     // memory, or in stream-ordered memory so the call stays asynchronous. Without fixed memory no map is made while
     // the stream is being captured into a graph (a replay must not read memory this call has given back).
-    uint2 *zmap = nullptr;
+    // (Where a map by block fits, the first product leaves it as it goes; else the map is made by a pass of its own.)
+    void *stream_mem = nullptr;
+    ulonglong2 *made = nullptr;
     ZeroMap z = sequence_map(*A, n);
     if (launches == n && !z.w && ntimes_uses_map(*A, n)) {
-        size_t bytes = zero_map_bytes(*A, z.shift);
-        uint2 *to = nullptr;
+        size_t bytes = map_by_block_bytes(M, A->n());
+        bool by_block = g_spmv_bands <= 1;
+        void *to = nullptr;
         if (fixed_map) {
-            if (bytes > fixed_bytes) {  // blocks of 256 rows then
-                z.shift = 8;
+            by_block = by_block && bytes <= fixed_bytes;
+            if (!by_block) {
                 bytes = zero_map_bytes(*A, z.shift);
+                if (bytes > fixed_bytes) {  // blocks of 256 rows then
+                    z.shift = 8;
+                    bytes = zero_map_bytes(*A, z.shift);
+                }
+                if (bytes > fixed_bytes)
+                    throw ArgError("spmv_ntimes_device_noalloc: the zero-block map of this matrix needs " +
+                                   std::to_string(bytes) + " bytes, more than the " + std::to_string(fixed_bytes) +
+                                   " bytes of the library's static scratch (tune the matrix with dq_spmv_tune to keep "
+                                   "its map in the handle, or use dq_spmv_ntimes_device)");
             }
-            if (bytes > fixed_bytes)
-                throw ArgError("spmv_ntimes_device_noalloc: the zero-block map of this matrix needs " +
-                               std::to_string(bytes) + " bytes, more than the " + std::to_string(fixed_bytes) +
-                               " bytes of the library's static scratch (tune the matrix with dq_spmv_tune to keep "
-                               "its map in the handle, or use dq_spmv_ntimes_device)");
             to = fixed_map;
         } else {
+            if (!by_block) bytes = zero_map_bytes(*A, z.shift);
             hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
             DQ_HIP(hipStreamIsCapturing(s, &cap));
             if (cap == hipStreamCaptureStatusNone) {
-                if (hipMallocAsync(reinterpret_cast<void **>(&zmap), bytes, s) != hipSuccess) {
+                if (hipMallocAsync(&stream_mem, bytes, s) != hipSuccess) {
                     (void)hipGetLastError();  // no stream-ordered memory: run without the map
-                    zmap = nullptr;
+                    stream_mem = nullptr;
                 }
-                to = zmap;
+                to = stream_mem;
             }
         }
-        if (to) {
-            make_zero_map(*A, z.shift, to, s);
-            z.w = to;
+        if (to && by_block) {
+            made = static_cast<ulonglong2 *>(to);
+        } else if (to) {
+            make_zero_map(*A, z.shift, static_cast<uint2 *>(to), s);
+            z.w = static_cast<uint2 *>(to);
             z.words = zero_block_words(A->rows, 1 << z.shift);
         }
     }
@@ -705,11 +734,11 @@ static void ntimes_device(const dq_devmat *A, const void *xr, const void *xi, vo
         const bool to_y = (((launches - 1 - t) % 2) == 0) != flip;
         void *dr = to_y ? yr : work_r, *di = to_y ? yi : work_i;
         if (launches < n) band_powers(*A, sr, si, dr, di, sequence_products(n, launches, t), s);
-        else spmv_banded(*A, sr, si, dr, di, 0, s, z);
+        else sequence_product(*A, sr, si, dr, di, s, z, made, t == 0);
         sr = dr;
         si = di;
     }
-    if (zmap) DQ_HIP(hipFreeAsync(zmap, s));
+    if (stream_mem) DQ_HIP(hipFreeAsync(stream_mem, s));
     if (flip) {
         DQ_HIP(hipMemcpyAsync(yr, work_r, M * eb, hipMemcpyDeviceToDevice, s));
         DQ_HIP(hipMemcpyAsync(yi, work_i, M * eb, hipMemcpyDeviceToDevice, s));
@@ -776,18 +805,24 @@ extern "C" int dq_spmv_ntimes_host(const dq_devmat *A, const double *xr, const d
         DevVec a(N, A->precision), b(M, A->precision);
         a.put(xr, xi);
         DevBuf zmap;
+        ulonglong2 *made = nullptr;
         ZeroMap z = sequence_map(*A, n);
         const int launches = sequence_launches(*A, n);
         if (launches == n && !z.w && ntimes_uses_map(*A, n)) {
-            zmap = DevBuf(zero_map_bytes(*A, z.shift));
-            make_zero_map(*A, z.shift, zmap.as<uint2>(), 0);
-            z.w = zmap.as<uint2>();
-            z.words = zero_block_words(A->rows, 1 << z.shift);
+            const bool by_block = g_spmv_bands <= 1;
+            zmap = DevBuf(by_block ? map_by_block_bytes(M, A->n()) : zero_map_bytes(*A, z.shift));
+            if (by_block) {
+                made = zmap.as<ulonglong2>();
+            } else {
+                make_zero_map(*A, z.shift, zmap.as<uint2>(), 0);
+                z.w = zmap.as<uint2>();
+                z.words = zero_block_words(A->rows, 1 << z.shift);
+            }
         }
         DevVec *in = &a, *out = &b;
         for (int t = 0; t < launches; ++t) {
             if (launches < n) band_powers(*A, in->r.p, in->i.p, out->r.p, out->i.p, sequence_products(n, launches, t), 0);
-            else spmv_banded(*A, in->r.p, in->i.p, out->r.p, out->i.p, 0, 0, z);
+            else sequence_product(*A, in->r.p, in->i.p, out->r.p, out->i.p, 0, z, made, t == 0);
             if (t != launches - 1) std::swap(in, out);
         }
         out->get(yr, yi);

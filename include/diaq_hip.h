@@ -133,8 +133,8 @@ int dq_spmv_ntimes_host(const dq_devmat *A, const double *xr, const double *xi, 
  * (src/spMV_ntimes_gpu.cu:61-263, same errors and num_times == 0 / no-diagonal rules) on data that stays resident.
  * work_r / work_i are one more vector of A.rows elements, needed when num_times > 1 or x == y (in place: the result
  * overwrites x); the products alternate between y and the work vectors. For num_times >= 2 and at least 2^16 rows the
- * products skip A's all-zero 64-row blocks and zero real or imaginary parts through a map made once per call in
- * stream-ordered memory (hipMallocAsync), with the schedule dq_spmv_tune chose for that; while `stream` is being
+ * products after the first skip A's all-zero 64-row blocks and zero real or imaginary parts through a map that the
+ * first one leaves in stream-ordered memory (hipMallocAsync), with the schedule dq_spmv_tune chose for that; while `stream` is being
  * captured into a graph no map is made. The FP64 result has the same bits either way. Products with a band matrix of up
  * to 40 diagonals, in every spMV_ntimes form, run several to a launch instead, which read A once and need no map. */
 int dq_spmv_ntimes_device(const dq_devmat *A, const void *xr, const void *xi, void *yr, void *yi, int num_times,
