@@ -14,7 +14,8 @@
 // next to psi -- carries FP32 rounding, so the error per sub-step is FP32 eps times ||Y b_1||, not times ||psi||.
 //
 // Launch g of a class advances every job of the class by one Horner level (jobs that are done return at once); the
-// class needs max_j m_j 2^{s_j} launches, captured once into a graph with one branch per class on its own stream.
+// class needs max_j m_j 2^{s_j} launches, captured once into a graph whose branches are the streams of a lane plan. A
+// class of small Hamiltonians runs all its levels in one launch or a few instead (horner_resident_kernel), beside the graph.
 // A final FP64 pass renormalises every state.
 //
 // A-posteriori check: the probe runs the forward Taylor terms t_k = (Y/k) t_{k-1} of the first sub-step from the

@@ -498,7 +498,8 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
     const int64_t grid = per_xcd * 8;
     if (grid > 0x7fffffffLL) throw ArgError("product: too many work items");
     // one block for the work lists and, but for long pair lists, one copy: seven of each cost a small product more than
-    // its kernel (2048 rows, 11-qubit Pauli sum squared, with the conversion to dense: 172 -> 158 us; 1024 rows, TFIM-10 squared and applied: 113 -> 81)
+    // its kernel (1024 rows, TFIM-10 squared and applied: 113 -> 81 us; 2048 rows, 11-qubit Pauli sum squared, with the
+    // conversion to dense: 172 -> 158)
     size_t lists = 0;
     auto place = [&](size_t bytes) {
         const size_t at = lists;
