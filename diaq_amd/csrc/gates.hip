@@ -51,7 +51,7 @@ enum { STEP_MOVE = 0, STEP_DIAG = 1, STEP_FULL2 = 2, STEP_ROWS2 = 3, STEP_ROWS4 
 struct GateStep {
     int kind;
     int a;     // STEP_MOVE: the new window; STEP_DIAG: which register bits the gate's qubits are (see diag_step)
-    int q, k;  // STEP_DIAG: first qubit, qubits
+    int q, k;  // STEP_DIAG: first qubit, qubits; STEP_LAYER: k = 1 where all are cross gates
     int j;     // the gate's first register bit; STEP_DIAG: the gate bit of register bit `a`
     int at;    // STEP_DIAG: its first entry in the pass's LDS table; STEP_FULL*, STEP_MASK*: its entries (row-major,
                // absent ones too) in terms;
@@ -201,6 +201,36 @@ __device__ __forceinline__ void full2_gate(const GateTerm<T> *__restrict__ g, T 
     });
 }
 
+// A cross gate: real diagonal entries, imaginary others (a rotation about X). The products with the zero parts, which
+// full2_gate adds as zeros, are left out: 12 instructions for a pair of amplitudes against 20, with the same roundings and,
+// for finite amplitudes, the same values (a TFIM step of 28 qubits 7.13 -> 6.81 ms, of 25 789 -> 744 us).
+template <typename T, int R, int B>
+__device__ __forceinline__ void cross_gate(const GateTerm<T> *__restrict__ g, T (&xr)[1 << R], T (&xi)[1 << R]) {
+#pragma clang fp contract(off)
+    const T c0 = g[0].re, s1 = g[1].im, s2 = g[2].im, c3 = g[3].re;
+    static_for<(1 << R) / 2>([&](auto c) {
+#pragma clang fp contract(off)
+        constexpr int m = (c & ((1 << B) - 1)) | ((c >> B) << (B + 1)), n = m | (1 << B);
+        const T ar = c0 * xr[m], ai = c0 * xi[m], br = s1 * xi[n], bi = s1 * xr[n];
+        const T cr = s2 * xi[m], ci = s2 * xr[m], dr = c3 * xr[n], di = c3 * xi[n];
+        xr[m] = ar - br;
+        xi[m] = ai + bi;
+        xr[n] = dr - cr;
+        xi[n] = ci + di;
+    });
+}
+
+// Whether every amplitude of the wave is finite: a NaN or an infinity leaves the sum of zeros.
+template <typename T, int E>
+__device__ __forceinline__ bool all_finite(const T (&xr)[E], const T (&xi)[E]) {
+    T a = T(0), b = T(0);
+    static_for<E>([&](auto m) {
+        a = __builtin_fma(xr[m], T(0), a);
+        b = __builtin_fma(xi[m], T(0), b);
+    });
+    return !__any(!(a + b == T(0)));
+}
+
 // The same on register bit j.
 template <typename T, int R, int B>
 __device__ __forceinline__ void full2_step(int j, const GateTerm<T> *__restrict__ g, T (&xr)[1 << R],
@@ -338,8 +368,13 @@ __global__ __launch_bounds__(256, 3) void gates_pass_kernel(const PassHdr *__res
                 s += S.end - 1;
                 DQ_VARIANT_END(40);
             } else if (S.kind == STEP_LAYER) {
-                static_for<R>([&](auto b) { full2_gate<T, R, b>(terms + S.at + 4 * b, xr, xi); });
-                DQ_VARIANT_END(41);
+                if (S.k && all_finite(xr, xi)) {  // uniform in the wave
+                    static_for<R>([&](auto b) { cross_gate<T, R, b>(terms + S.at + 4 * b, xr, xi); });
+                    DQ_VARIANT_END(42);
+                } else {
+                    static_for<R>([&](auto b) { full2_gate<T, R, b>(terms + S.at + 4 * b, xr, xi); });
+                    DQ_VARIANT_END(41);
+                }
             } else if (S.kind == STEP_DIAG) {
                 const int ct = static_cast<int>(idx >> S.q) & ((1 << S.k) - 1);
                 diag_step<T, R, 0>(S, tab + S.at, ct, xr, xi);
@@ -478,7 +513,13 @@ static int best_window(const std::vector<std::pair<int, int>> &gates, size_t i, 
 
 // Turns stretches of the steps from `from` on into steps of several gates: diagonal gates on no register bit into
 // STEP_RUN, full one-qubit gates on register bits 0, 1, .. R - 1 in turn (whose entries follow each other) into STEP_LAYER.
-static void merge_steps(std::vector<GateStep> &steps, size_t from, int R) {
+// A layer of cross gates alone (cross_gate) has k = 1.
+template <typename T>
+static void merge_steps(std::vector<GateStep> &steps, size_t from, int R, const std::vector<GateTerm<T>> &terms) {
+    auto cross = [&](int at) {
+        const GateTerm<T> *g = terms.data() + at;
+        return g[0].im == T(0) && g[3].im == T(0) && g[1].re == T(0) && g[2].re == T(0);
+    };
     std::vector<GateStep> out;
     for (size_t i = from; i < steps.size();) {
         size_t e = i;
@@ -497,6 +538,9 @@ static void merge_steps(std::vector<GateStep> &steps, size_t from, int R) {
         out.push_back(steps[i]);
         if (e - i == static_cast<size_t>(R)) {
             out.back().kind = STEP_LAYER;
+            out.back().k = 1;
+            for (int b = 0; b < R; ++b)
+                if (!cross(out.back().at + 4 * b)) out.back().k = 0;
             i = e;
         } else {
             ++i;
@@ -616,7 +660,7 @@ static void plan_passes(dq_gate_plan &P, int low_qubits, const std::vector<HostG
             }
             steps.push_back(st);
         }
-        merge_steps(steps, static_cast<size_t>(D.step), R);
+        merge_steps(steps, static_cast<size_t>(D.step), R, terms);
         if (a < 4 && a != stored) {  // back to a window whose lanes hold runs of 16 amplitudes
             GateStep mv{};
             mv.kind = STEP_MOVE;
