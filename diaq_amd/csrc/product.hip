@@ -29,7 +29,8 @@
 // rows, and its imaginary part often everywhere.
 //
 // Bound: the L2's and the memory's reads of A and B per pair against the stores of C (TFIM-20 H*H: 1681 pairs, 727
-// diagonals, 11 GB stored). Reading every part of a live pair: 4.00 ms; only the live blocks and parts: 3.06 ms.
+// diagonals, 11 GB stored). Reading every part of a live pair: 4.00 ms; only the live blocks and parts: 3.03 ms; eight
+// items of a workgroup together: 2.23 ms.
 //
 // The items also write C's own zero-block map, by ballots on what they store; a large result keeps it (map_blocks).
 #include <algorithm>
@@ -161,6 +162,7 @@ static std::shared_ptr<const DryRun> dryrun_reused(uint32_t rows, uint32_t cols,
 }
 
 constexpr int PROD_BATCH = 256;
+constexpr int PROD_GROUP = 8;  // at most as many items of a workgroup
 
 // Process-wide knobs (dq_set_tuning): chunk order across XCDs and non-temporal stores of C.
 static int g_prod_interleave = 1;
@@ -268,58 +270,99 @@ __global__ __launch_bounds__(256) void product_kernel(const int2 *__restrict__ i
                                                       const T *__restrict__ bim, T *__restrict__ cre,
                                                       T *__restrict__ cim, double divisor,
                                                       ZeroMap za, ZeroMap zb, uint2 *__restrict__ zc,
-                                                      int64_t zc_words) {
+                                                      int64_t zc_words, int group) {
     constexpr int PROD_CHUNK = 256 * PROD_RPT;
     __shared__ int64_t s_abase[PROD_BATCH], s_bbase[PROD_BATCH];
     __shared__ int32_t s_lo[PROD_BATCH], s_hi[PROD_BATCH];
-    __shared__ uint4 s_live[MAP ? PROD_BATCH : 1];  // the item's blocks that hold a nonzero: A real, A imaginary, B real, B imaginary
+    __shared__ uint4 s_live[MAP ? PROD_BATCH : 1];  // the item's blocks that hold a nonzero: A real, A imaginary, B real,
+                                                    // B imaginary
     constexpr int ZW = (PROD_RPT + 7) / 8;  // map words of an item's rows
-    __shared__ uint32_t s_zr[ZW], s_zi[ZW];
+    __shared__ uint32_t s_zr[2][4][ZW], s_zi[2][4][ZW];  // by parity of the item and wave
+    // the workgroup's items: result diagonal, first row, its rows [r0, r1) as offsets from that, its pairs
+    __shared__ int64_t s_q0[PROD_GROUP], s_cbase[PROD_GROUP], s_p0[PROD_GROUP];
+    __shared__ int32_t s_c[PROD_GROUP], s_r0[PROD_GROUP], s_r1[PROD_GROUP], s_cnt[PROD_GROUP];
     // XCD-aware remap: the workgroups of XCD x (x = b mod 8) take the item range [xcd_first[x], xcd_first[x + 1]).
     const int64_t b = blockIdx.x;
-    const int64_t w = xcd_first[b & 7] + (b >> 3);
-    if (w >= xcd_first[(b & 7) + 1]) return;  // uniform
-    const int2 it = items[w];
-    const DiagMeta m_c = mc[it.y];
-    const int64_t q0 = static_cast<int64_t>(it.x) * PROD_CHUNK;
-    const int64_t r0 = max(m_c.rlo, q0), r1 = min(m_c.rhi, q0 + PROD_CHUNK);
-    const int64_t p0 = pair_start[it.y], p1 = pair_start[it.y + 1];
+    const int64_t w = xcd_first[b & 7] + (b >> 3) * group, w_end = xcd_first[(b & 7) + 1];
+    if (w >= w_end) return;  // uniform
+    const int ng = MAP ? static_cast<int>(min<int64_t>(group, w_end - w)) : 1;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (MAP && zc && threadIdx.x < ZW) s_zr[threadIdx.x] = s_zi[threadIdx.x] = 0;  // the first batch's barrier orders it
-    T acc_r[PROD_RPT], acc_i[PROD_RPT];
-#pragma unroll
-    for (int j = 0; j < PROD_RPT; ++j) { acc_r[j] = T(0); acc_i[j] = T(0); }
-    for (int64_t pbat = p0; pbat < p1; pbat += PROD_BATCH) {
-        const int nb = static_cast<int>(min<int64_t>(PROD_BATCH, p1 - pbat));
-        if (static_cast<int>(threadIdx.x) < nb) {
-            const int64_t p = pbat + threadIdx.x;
-            const int32_t sa = pa[p], sb = pb[p];
-            const DiagMeta ta = ma[sa];
-            const DiagMeta tb = mb[sb];
-            // rows r of this item with r on A's diagonal and r + dA on B's: [lo, hi), as offsets from q0
-            const int64_t lo = max(max(ta.rlo, tb.rlo - ta.off), r0);
-            const int64_t hi = min(min(ta.rhi, tb.rhi - ta.off), r1);
-            bool live = hi > lo;
-            uint4 m = make_uint4(~0u, ~0u, ~0u, ~0u);
-            if (MAP && live) {  // rows that a diagonal does not have are clear bits of its map
-                m = make_uint4(0, 0, 0, 0);
-#pragma unroll
-                for (int w8 = 0; w8 < ZW; ++w8) {
-                    const int64_t q = q0 + 2048 * w8;
-                    const uint2 a2 = map_rows(za, sa, q), b2 = map_rows(zb, sb, q + ta.off);
-                    m.x |= a2.x; m.y |= a2.y; m.z |= b2.x; m.w |= b2.y;
-                }
-                constexpr uint32_t IN = PROD_RPT < 8 ? 0xffffu : ~0u;  // the item's rows
-                live = ((m.x | m.y) & IN) && ((m.z | m.w) & IN);
-            }
-            if (MAP) s_live[threadIdx.x] = m;
-            s_abase[threadIdx.x] = ta.rowbase;
-            s_bbase[threadIdx.x] = tb.rowbase + ta.off;
-            s_lo[threadIdx.x] = live ? static_cast<int32_t>(lo - q0) : 0;
-            s_hi[threadIdx.x] = live ? static_cast<int32_t>(hi - q0) : 0;
+    struct Item {
+        int64_t q0, cbase, p0;
+        int32_t c, r0, r1, cnt;
+    };
+    auto load_item = [&](int64_t i) {
+        const int2 it = items[i];
+        const DiagMeta m_c = mc[it.y];
+        const int64_t q0 = static_cast<int64_t>(it.x) * PROD_CHUNK, p0 = pair_start[it.y];
+        return Item{q0, m_c.rowbase, p0, it.y, static_cast<int32_t>(max(m_c.rlo, q0) - q0),
+                    static_cast<int32_t>(min(m_c.rhi, q0 + PROD_CHUNK) - q0),
+                    static_cast<int32_t>(pair_start[it.y + 1] - p0)};
+    };
+    Item only{};  // without maps: the one item, uniform
+    if constexpr (MAP) {
+        if (static_cast<int>(threadIdx.x) < ng) {
+            const Item it = load_item(w + threadIdx.x);
+            s_q0[threadIdx.x] = it.q0;
+            s_cbase[threadIdx.x] = it.cbase;
+            s_p0[threadIdx.x] = it.p0;
+            s_c[threadIdx.x] = it.c;
+            s_r0[threadIdx.x] = it.r0;
+            s_r1[threadIdx.x] = it.r1;
+            s_cnt[threadIdx.x] = it.cnt;
         }
         __syncthreads();
-        for (int k = 0; k < nb; ++k) {
+    } else {
+        only = load_item(w);
+    }
+    int base = 0, staged = 0, first = 0;  // the staged pairs [base, staged) of the workgroup's, and the item's first one
+    for (int g = 0; g < ng; ++g) {  // uniform
+        const int64_t q0 = MAP ? uniform64(s_q0[g]) : only.q0;
+        const int cnt = MAP ? __builtin_amdgcn_readfirstlane(s_cnt[g]) : only.cnt;
+        T acc_r[PROD_RPT], acc_i[PROD_RPT];
+#pragma unroll
+        for (int j = 0; j < PROD_RPT; ++j) { acc_r[j] = T(0); acc_i[j] = T(0); }
+        for (int pk = first; pk < first + cnt; ++pk) {
+            if (pk == staged) {  // uniform: the next batch of pairs
+                __syncthreads();  // the last one is done with
+                int of = 0, at = staged + static_cast<int>(threadIdx.x);  // the lane's pair: number `at` of item `of`
+                if constexpr (MAP) {
+                    while (of < ng && at >= s_cnt[of]) at -= s_cnt[of++];
+                } else {
+                    of = at >= only.cnt;
+                }
+                if (of < ng) {
+                    const int64_t p = (MAP ? s_p0[of] : only.p0) + at, q0 = MAP ? s_q0[of] : only.q0;
+                    const int32_t sa = pa[p], sb = pb[p];
+                    const DiagMeta ta = ma[sa];
+                    const DiagMeta tb = mb[sb];
+                    // rows r of the item with r on A's diagonal and r + dA on B's: [lo, hi), as offsets from q0
+                    const int64_t lo = max(max(ta.rlo, tb.rlo - ta.off), q0 + (MAP ? s_r0[of] : only.r0));
+                    const int64_t hi = min(min(ta.rhi, tb.rhi - ta.off), q0 + (MAP ? s_r1[of] : only.r1));
+                    bool live = hi > lo;
+                    uint4 m = make_uint4(~0u, ~0u, ~0u, ~0u);
+                    if (MAP && live) {  // rows that a diagonal does not have are clear bits of its map
+                        m = make_uint4(0, 0, 0, 0);
+#pragma unroll
+                        for (int w8 = 0; w8 < ZW; ++w8) {
+                            const int64_t q = q0 + 2048 * w8;
+                            const uint2 a2 = map_rows(za, sa, q), b2 = map_rows(zb, sb, q + ta.off);
+                            m.x |= a2.x; m.y |= a2.y; m.z |= b2.x; m.w |= b2.y;
+                        }
+                        constexpr uint32_t IN = PROD_RPT < 8 ? 0xffffu : ~0u;  // the item's rows
+                        live = ((m.x | m.y) & IN) && ((m.z | m.w) & IN);
+                    }
+                    if (MAP) s_live[threadIdx.x] = m;
+                    s_abase[threadIdx.x] = ta.rowbase;
+                    s_bbase[threadIdx.x] = tb.rowbase + ta.off;
+                    s_lo[threadIdx.x] = live ? static_cast<int32_t>(lo - q0) : 0;
+                    s_hi[threadIdx.x] = live ? static_cast<int32_t>(hi - q0) : 0;
+                }
+                base = staged;
+                staged += PROD_BATCH;
+                __syncthreads();
+            }
+            const int k = pk - base;
             const int64_t lo = q0 + __builtin_amdgcn_readfirstlane(s_lo[k]);
             const int64_t hi = q0 + __builtin_amdgcn_readfirstlane(s_hi[k]);
             if (hi <= lo) continue;  // uniform
@@ -362,49 +405,54 @@ __global__ __launch_bounds__(256) void product_kernel(const int2 *__restrict__ i
                 acc_i[j] += im;
             }
         }
-        __syncthreads();  // the next batch overwrites the staged pairs
-    }
-    uint32_t zr[ZW] = {}, zi[ZW] = {};
+        first += cnt;
+        const int32_t r0 = MAP ? s_r0[g] : only.r0, r1 = MAP ? s_r1[g] : only.r1;
+        const int64_t cbase = (MAP ? uniform64(s_cbase[g]) : only.cbase) + q0;
+        uint32_t zr[ZW] = {}, zi[ZW] = {};
 #pragma unroll
-    for (int j = 0; j < PROD_RPT; ++j) {
-        const int64_t r = q0 + threadIdx.x + 256 * j;
-        const bool in = r >= r0 && r < r1;
-        T vr = acc_r[j], vi = acc_i[j];
-        if (divisor != 1.0) {
-            vr = static_cast<T>(acc_r[j] / divisor);
-            vi = static_cast<T>(acc_i[j] / divisor);
-        }
-        if (in) {
-            if constexpr (NTS) {  // C is written once and not read here: keep it out of the caches
-                __builtin_nontemporal_store(vr, cre + m_c.rowbase + r);
-                __builtin_nontemporal_store(vi, cim + m_c.rowbase + r);
-            } else {
-                cre[m_c.rowbase + r] = vr;
-                cim[m_c.rowbase + r] = vi;
+        for (int j = 0; j < PROD_RPT; ++j) {
+            const int32_t r = static_cast<int32_t>(threadIdx.x) + 256 * j;
+            const bool in = r >= r0 && r < r1;
+            T vr = acc_r[j], vi = acc_i[j];
+            if (divisor != 1.0) {
+                vr = static_cast<T>(acc_r[j] / divisor);
+                vi = static_cast<T>(acc_i[j] / divisor);
+            }
+            if (in) {
+                if constexpr (NTS) {  // C is written once and not read here: keep it out of the caches
+                    __builtin_nontemporal_store(vr, cre + cbase + r);
+                    __builtin_nontemporal_store(vi, cim + cbase + r);
+                } else {
+                    cre[cbase + r] = vr;
+                    cim[cbase + r] = vi;
+                }
+            }
+            if (MAP && zc) {  // uniform; the wave's 64 rows of pass j are block 4 j + wave of the item
+                if (__ballot(in && !(vr == T(0)))) zr[j >> 3] |= 1u << (4 * (j & 7));
+                if (__ballot(in && !(vi == T(0)))) zi[j >> 3] |= 1u << (4 * (j & 7));
             }
         }
-        if (MAP && zc) {  // uniform; the wave's 64 rows of pass j are block 4 j + wave of the item
-            if (__ballot(in && !(vr == T(0)))) zr[j >> 3] |= 1u << (4 * (j & 7));
-            if (__ballot(in && !(vi == T(0)))) zi[j >> 3] |= 1u << (4 * (j & 7));
-        }
-    }
-    if (MAP && zc) {
-        if ((threadIdx.x & 63) == 0) {
+        if (MAP && zc) {
+            uint32_t (&gr)[4][ZW] = s_zr[g & 1], (&gi)[4][ZW] = s_zi[g & 1];
+            if ((threadIdx.x & 63) == 0) {
 #pragma unroll
-            for (int w8 = 0; w8 < ZW; ++w8) {
-                atomicOr(&s_zr[w8], zr[w8] << wave);
-                atomicOr(&s_zi[w8], zi[w8] << wave);
+                for (int w8 = 0; w8 < ZW; ++w8) {
+                    gr[wave][w8] = zr[w8] << wave;
+                    gi[wave][w8] = zi[w8] << wave;
+                }
             }
-        }
-        __syncthreads();
-        if (threadIdx.x < ZW) {
-            uint2 *w = zc + it.y * zc_words + (q0 >> 11) + threadIdx.x;
-            if constexpr (PROD_RPT == 4) {  // half a word
-                uint16_t *h = reinterpret_cast<uint16_t *>(w) + ((q0 >> 10) & 1);
-                h[0] = static_cast<uint16_t>(s_zr[0]);
-                h[2] = static_cast<uint16_t>(s_zi[0]);
-            } else if ((q0 >> 11) + threadIdx.x < zc_words) {
-                *w = make_uint2(s_zr[threadIdx.x], s_zi[threadIdx.x]);
+            __syncthreads();  // the item after the next writes here again, behind the next item's barrier
+            if (threadIdx.x < ZW) {
+                const uint32_t br = gr[0][threadIdx.x] | gr[1][threadIdx.x] | gr[2][threadIdx.x] | gr[3][threadIdx.x];
+                const uint32_t bi = gi[0][threadIdx.x] | gi[1][threadIdx.x] | gi[2][threadIdx.x] | gi[3][threadIdx.x];
+                uint2 *to = zc + s_c[g] * zc_words + (q0 >> 11) + threadIdx.x;
+                if constexpr (PROD_RPT == 4) {  // half a word
+                    uint16_t *h = reinterpret_cast<uint16_t *>(to) + ((q0 >> 10) & 1);
+                    h[0] = static_cast<uint16_t>(br);
+                    h[2] = static_cast<uint16_t>(bi);
+                } else if ((q0 >> 11) + threadIdx.x < zc_words) {
+                    *to = make_uint2(br, bi);
+                }
             }
         }
     }
@@ -419,6 +467,12 @@ __global__ __launch_bounds__(256) void map_bits_kernel(int64_t n, const uint2 *_
     for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
     if ((threadIdx.x & 63) == 0) atomicAdd(out, static_cast<unsigned long long>(c));
 }
+
+// Items of a workgroup, for operands with maps (2^16 rows or more): they share the round trips of their metadata, which take
+// a good part of an item's time, while enough workgroups remain. us, 1 / 2 / 8 items: 280 000 items (TFIM-20 squared and
+// applied) 4036 / 3629 / 3388, 29 000 (TFIM-17) 572 / 552 / 567. Smaller products have few items and run them one by one,
+// without the barrier that sharing takes.
+constexpr int64_t MANY_ITEMS = int64_t(1) << 17;
 
 // Pair lists up to this size join the other work lists in one upload; longer ones are copied from where they are, as
 // gathering them first would take about as long as a copy of their own.
@@ -494,7 +548,9 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
     // chunks in the order above; with fewer chunks than XCDs a chunk's items spread over several
     for (int x = 0; x <= 8; ++x) xcd_first[x] = n_work * x / 8;
     int64_t per_xcd = 0;
-    for (int x = 0; x < 8; ++x) per_xcd = std::max(per_xcd, xcd_first[x + 1] - xcd_first[x]);
+    const bool maps = g_prod_skip && A.rows >= (uint32_t(1) << 16) && A.n() > 0 && B.n() > 0;
+    const int group = !maps ? 1 : n_work >= MANY_ITEMS ? PROD_GROUP : 2;
+    for (int x = 0; x < 8; ++x) per_xcd = std::max(per_xcd, (xcd_first[x + 1] - xcd_first[x] + group - 1) / group);
     const int64_t grid = per_xcd * 8;
     if (grid > 0x7fffffffLL) throw ArgError("product: too many work items");
     // one block for the work lists and, but for long pair lists, one copy: seven of each cost a small product more than
@@ -539,7 +595,7 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
     // zero-block maps of A and B (a squaring maps its operand once; a map the handle keeps is used as it is)
     DevBuf zab, zbb;
     ZeroMap za, zb;
-    if (g_prod_skip && A.rows >= (int64_t(1) << 16) && A.n() > 0 && B.n() > 0) {
+    if (maps) {
         auto map_of = [&](const dq_devmat &M, DevBuf &buf) {
             ZeroMap z = kept_zero_map(M);
             if (z.w) return z;
@@ -570,7 +626,7 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
     hipLaunchKernelGGL((product_kernel<T, NTS, R, M>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, s,        \
                        ditems, dxcd, dps, dsa, dsb, A.d_meta.as<DiagMeta>(), B.d_meta.as<DiagMeta>(), C->d_meta.as<DiagMeta>(), \
                        A.re.as<T>(), A.im.as<T>(), B.re.as<T>(), B.im.as<T>(), C->re.as<T>(), C->im.as<T>(), divisor, \
-                       za, zb, zcb.as<uint2>(), zc_words)
+                       za, zb, zcb.as<uint2>(), zc_words, group)
 #define DQ_PROD_LAUNCH_R(T, NTS, R)                          \
     do {                                                     \
         if (za.w) DQ_PROD_LAUNCH_M(T, NTS, R, true);         \
