@@ -465,7 +465,10 @@ __global__ __launch_bounds__(256) void map_bits_kernel(int64_t n, const uint2 *_
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         c += __popc(w[i].x) + __popc(w[i].y);
     for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(out, static_cast<unsigned long long>(c));
+    __shared__ unsigned part[4];
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(out, static_cast<unsigned long long>(part[0]) + part[1] + part[2] + part[3]);
 }
 
 // Items of a workgroup, for operands with maps (2^16 rows or more): they share the round trips of their metadata, which take
@@ -651,7 +654,7 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
     DQ_LAUNCH_CHECK();
     if (c_blocks) {
         const int64_t words = static_cast<int64_t>(zcb.bytes / sizeof(uint2));
-        hipLaunchKernelGGL(map_bits_kernel, dim3(blocks_for(words, 256, 512)), dim3(256), 0, s, words, zcb.as<uint2>(),
+        hipLaunchKernelGGL(map_bits_kernel, dim3(blocks_for(words, 1024, 128)), dim3(256), 0, s, words, zcb.as<uint2>(),
                            dbits.as<unsigned long long>());
         DQ_LAUNCH_CHECK();
         DQ_HIP(hipMemcpyAsync(&bits, dbits.p, sizeof(bits), hipMemcpyDeviceToHost, s));
