@@ -239,7 +239,7 @@ struct TaylorRows {
     int done = 0;  // terms added
 
 private:
-    int run(int k0, int n, const void *tin, const void *uin, void *tout, void *uout);
+    void run(int k0, int n, const void *tin, const void *uin, void *tout, void *uout, bool norms);
     const dq_devmat &X;
     hipStream_t s;
     std::vector<DiagMeta> meta;

@@ -26,8 +26,10 @@
 #include <cmath>
 #include <cstdio>
 #include <numeric>
+#include <stdexcept>
 
 #include "dia_rows.hpp"
+#include "taylor_shape.hpp"
 
 namespace dq {
 
@@ -116,7 +118,8 @@ __device__ __forceinline__ void taylor_columns(uint64_t todo, int lane, int64_t 
 }
 
 // Terms k0 + 1 .. k0 + terms of rows blockIdx.x * RB ..; Tin / Uin (null: T_0 = U_0 = I), Tout (may be null) / Uout
-// row-major complex N x N. part[j * gridDim.x + block]: the block's share of the squared Frobenius norm of term k0 + 1 + j.
+// row-major complex N x N. part[j * gridDim.x + block]: the block's share of the squared Frobenius norm of term k0 + 1 + j
+// (null: no norms, for any number of terms).
 template <typename T, int THREADS, int CPT, int RB>
 __global__ __launch_bounds__(THREADS) void taylor_rows_kernel(int N, TaylorSlots X, const T *__restrict__ xre,
                                                               const T *__restrict__ xim, int k0, int terms,
@@ -196,11 +199,13 @@ __global__ __launch_bounds__(THREADS) void taylor_rows_kernel(int N, TaylorSlots
                 const double x = static_cast<double>(t.x), y = static_cast<double>(t.y);
                 if (c < N && r0 + b < N) sq += x * x + y * y;
             }
+        if (part) {  // uniform
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
-        if (lane == 0) red[wave] = sq;
+            for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
+            if (lane == 0) red[wave] = sq;
+        }
         __syncthreads();  // the new term and the waves' sums
-        if (tid == 0) {
+        if (part && tid == 0) {
             double v = 0.0;
             for (int w = 0; w < THREADS / 64; ++w) v += red[w];
             part[static_cast<int64_t>(j) * gridDim.x + blockIdx.x] = v;
@@ -280,27 +285,28 @@ std::vector<int32_t> series_offsets(const dq_devmat &X, int terms) {
 
 template <typename T>
 void launch_rows(int N, const TaylorSlots &S, const dq_devmat &X, int k0, int terms, const c64 *Tin, const c64 *Uin,
-                 c64 *Tout, c64 *Uout, double *part, int &grid, hipStream_t s) {
+                 c64 *Tout, c64 *Uout, double *part, hipStream_t s) {
     const T *xre = X.re.as<T>(), *xim = X.im.as<T>();
-#define DQ_TAYLOR(TH, CPT, RB)                                                                                         \
-    do {                                                                                                               \
-        grid = (N + (RB)-1) / (RB);                                                                                    \
-        if (terms > 0)                                                                                                 \
-            hipLaunchKernelGGL((taylor_rows_kernel<T, TH, CPT, RB>), dim3(static_cast<unsigned>(grid)), dim3(TH), 0, s, \
-                               N, S, xre, xim, k0, terms, Tin, Uin, Tout, Uout, part);                                 \
-    } while (0)
-    // a row per workgroup while that fills the chip, then as many as 128 KB of LDS hold
-    if (N <= 256) DQ_TAYLOR(256, 1, 1);
-    else if (N <= 512) DQ_TAYLOR(512, 1, 2);
-    else if (N <= 1024) DQ_TAYLOR(1024, 1, 4);
-    else if (N <= 2048) DQ_TAYLOR(1024, 2, 4);
-    else if (N <= 4096) DQ_TAYLOR(1024, 4, 2);
-    else DQ_TAYLOR(1024, 8, 1);
+    const dim3 grid(static_cast<unsigned>(taylor_grid(N)));
+#define DQ_TAYLOR(I)                                                                                               \
+    case I:                                                                                                        \
+        hipLaunchKernelGGL(                                                                                        \
+            (taylor_rows_kernel<T, TAYLOR_SHAPES[I].threads, TAYLOR_SHAPES[I].cols, TAYLOR_SHAPES[I].rows>), grid, \
+            dim3(TAYLOR_SHAPES[I].threads), 0, s, N, S, xre, xim, k0, terms, Tin, Uin, Tout, Uout, part);          \
+        break;
+    switch (taylor_shape(N)) {
+        DQ_TAYLOR(0)
+        DQ_TAYLOR(1)
+        DQ_TAYLOR(2)
+        DQ_TAYLOR(3)
+        DQ_TAYLOR(4)
+        DQ_TAYLOR(5)
+    }
 #undef DQ_TAYLOR
     DQ_LAUNCH_CHECK();
 }
 
-constexpr int FIRST_TERMS = 6, MAX_BATCH = 32;
+constexpr int FIRST_TERMS = 6;
 constexpr double ACTION_COST = 5.0;
 }  // namespace
 
@@ -311,7 +317,7 @@ constexpr double ACTION_COST = 5.0;
 // a tridiagonal X 1.79 / 1.93).
 bool dense_taylor_pays(const dq_devmat &X) {
     const int64_t N = X.rows;
-    if (!dense_enabled() || N < 1 || N > 8192 || X.n() == 0) return false;
+    if (!dense_enabled() || N < 1 || N > TAYLOR_MAX_N || X.n() == 0) return false;
     if (N <= 1024) return true;
     if (4 * static_cast<int64_t>(X.n()) > N) return false;
     if (N <= 2048) return true;
@@ -333,21 +339,23 @@ TaylorRows::TaylorRows(const dq_devmat &X_, hipStream_t s_) : X(X_), s(s_) {
     map = DevBuf(sizeof(uint2) * static_cast<size_t>(words) * X.n());
     DQ_HIP(hipMemcpyAsync(dmeta.p, meta.data(), dmeta.bytes, hipMemcpyHostToDevice, s));
     make_zero_map(X, dmeta.as<DiagMeta>(), 6, map.as<uint2>(), s);
-    part = DevBuf(sizeof(double) * MAX_BATCH * static_cast<size_t>(N));
-    folded = DevBuf(sizeof(double) * MAX_BATCH);
+    part = DevBuf(sizeof(double) * static_cast<size_t>(taylor_parts_room(N)));
+    folded = DevBuf(sizeof(double) * TAYLOR_BATCH);
 }
 
-int TaylorRows::run(int k0, int n, const void *tin, const void *uin, void *tout, void *uout) {
+void TaylorRows::run(int k0, int n, const void *tin, const void *uin, void *tout, void *uout, bool norms) {
     const TaylorSlots S{dmeta.as<DiagMeta>(), map.as<uint2>(), words, X.n()};
     const int N = static_cast<int>(X.rows);
-    int grid = 0;
+    if (n < 1) return;
+    if (N > TAYLOR_MAX_N || taylor_parts(N, n, norms) > static_cast<int64_t>(part.bytes / sizeof(double)))
+        throw std::logic_error("expm: a launch of the series outgrows its workspace");
+    double *const parts = norms ? part.as<double>() : nullptr;
     if (X.precision == DQ_F64)
         launch_rows<double>(N, S, X, k0, n, static_cast<const c64 *>(tin), static_cast<const c64 *>(uin),
-                            static_cast<c64 *>(tout), static_cast<c64 *>(uout), part.as<double>(), grid, s);
+                            static_cast<c64 *>(tout), static_cast<c64 *>(uout), parts, s);
     else
         launch_rows<float>(N, S, X, k0, n, static_cast<const c64 *>(tin), static_cast<const c64 *>(uin),
-                           static_cast<c64 *>(tout), static_cast<c64 *>(uout), part.as<double>(), grid, s);
-    return grid;
+                           static_cast<c64 *>(tout), static_cast<c64 *>(uout), parts, s);
 }
 
 bool TaylorRows::series(int max_iterations, double tol, const char *who, DevBuf &dense, std::vector<int32_t> &offs) {
@@ -366,15 +374,14 @@ bool TaylorRows::series(int max_iterations, double tol, const char *who, DevBuf 
             do {
                 ++want;
                 p *= rho / (done + want);
-            } while (p >= tol && want < MAX_BATCH);
+            } while (p >= tol && want < TAYLOR_BATCH);
         }
         want = std::min(want, max_iterations - done);
-        double sq[MAX_BATCH];
+        double sq[TAYLOR_BATCH];
         for (;;) {
-            const int grid = run(done, want, done ? Tb[cur].p : nullptr, done ? Ub[cur].p : nullptr, Tb[cur ^ 1].p,
-                                 Ub[cur ^ 1].p);
-            hipLaunchKernelGGL(fold_parts_kernel, dim3(static_cast<unsigned>(want)), dim3(256), 0, s, grid,
-                               part.as<double>(), folded.as<double>());
+            run(done, want, done ? Tb[cur].p : nullptr, done ? Ub[cur].p : nullptr, Tb[cur ^ 1].p, Ub[cur ^ 1].p, true);
+            hipLaunchKernelGGL(fold_parts_kernel, dim3(static_cast<unsigned>(want)), dim3(256), 0, s,
+                               static_cast<int>(taylor_grid(X.rows)), part.as<double>(), folded.as<double>());
             DQ_LAUNCH_CHECK();
             DQ_HIP(hipMemcpyAsync(sq, folded.p, sizeof(double) * want, hipMemcpyDeviceToHost, s));
             DQ_HIP(hipStreamSynchronize(s));
@@ -416,7 +423,7 @@ std::vector<int32_t> TaylorRows::square(const std::vector<int32_t> &offs, DevBuf
     const double action = std::ldexp(static_cast<double>(done) * X.n(), j);
     if (X.precision == DQ_F64 && ACTION_COST * action < static_cast<double>(N)) {
         for (int64_t i = 0; i < (int64_t(1) << j); ++i) {
-            run(0, done, U.p, U.p, nullptr, P.p);
+            run(0, done, U.p, U.p, nullptr, P.p, false);  // `done` may exceed TAYLOR_BATCH; no norms are needed
             std::swap(U, P);
         }
     } else {

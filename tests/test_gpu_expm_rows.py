@@ -127,3 +127,29 @@ def test_small_products(n):
     # three products of length n: n eps times the product of the absolute values
     bound = np.linalg.matrix_power(np.abs(M), 4)
     assert np.all(np.abs(got - ref) <= 16 * n * 2.0 ** -53 * bound + 1e-300)
+
+
+@pytest.mark.parametrize("n,near,a,cutoff,batches", [(4100, (1, 7, 49, 343, 1201, 2401), 11.0, 15.0, 1),
+                                                     (4096, (1, 7, 61, 500, 1777), 20.0, 30.0, 2)])
+def test_squaring_by_more_terms_than_a_batch(n, near, a, cutoff, batches):
+    """A large cutoff leaves exp(-iAt/2) more terms than a batch of 32 (one row to a workgroup) or two (two rows), and the
+    squaring applies them all at once: U V against SciPy's action of the exponential on V."""
+    import diaq_gpu as d
+    import scipy.sparse as sp
+    from scipy.sparse.linalg import expm_multiply
+    offs = sorted({0, *near, *(-o for o in near)})
+    vals = [np.full(n - abs(o), 1.0 / len(offs)) for o in offs]
+    A = d.to_device(d.diaQMatrix.from_diagonals([n, n], offs, [v + 0j for v in vals]), "fp64")
+    (uo, uv), m, s = expm(A, 1, 2 * a, tolerance=1e-10, cutoff=cutoff)
+    assert s == 1 and m > 32 * batches and 5 * m * len(offs) < n  # by terms, past the batches
+    V = np.random.default_rng(n).choice([-1.0, 1.0], size=(n, 4))
+    got, at = np.zeros((n, 4), complex), 0
+    for o in uo:
+        k = n - abs(o)
+        r, c = max(0, -o), max(0, o)
+        got[r:r + k] += (uv[0][at:at + k] + 1j * uv[1][at:at + k])[:, None] * V[c:c + k]
+        at += k
+    ref = expm_multiply(sp.diags(vals, offs, format="csr") * (-2j * a), V)
+    # term k of a row carries k (diagonals + 3) roundings of a^k / k!: a (diagonals + 3) e^a eps for the series, twice that
+    # through the second application, and its own; the truncation is below the tolerance
+    assert np.max(np.abs(got - ref)) < 3 * a * (len(offs) + 3) * np.exp(a) * 2.0 ** -53 + 1e-9
