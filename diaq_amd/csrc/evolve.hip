@@ -1040,6 +1040,18 @@ static std::vector<std::vector<int>> lane_plan(const dq_evo &E) {
     return plan;
 }
 
+// Whether a lane is a branch of the graph: from GRAPH_KERNELS kernels on. A graph whose four branches held four short
+// kernels each has ended in a segmentation fault of the host, cause unknown; with 16 to a branch and more they have run
+// throughout. A shorter lane is launched directly beside the graph, which costs no more than its nodes would (16 classes of
+// 2100 rows and one level: 0.42 ms as a graph of 4 lanes, 0.32 launched directly on a stream each).
+constexpr int64_t GRAPH_KERNELS = 16;
+
+static bool lane_in_graph(const dq_evo &E, const std::vector<int> &lane, bool renorm) {
+    int64_t kernels = 0;
+    for (int ci : lane) kernels += 1 + E.classes[ci].G + (renorm ? 3 : 0);
+    return kernels >= GRAPH_KERNELS;
+}
+
 // What a captured graph's launches depend on: the renormalisation flag, the process-wide Horner overrides, per class
 // its number of levels and its tuned schedule, and the lane plan. The kernels read each job's (tau, m, s) from
 // d_params when they run, so a new schedule that keeps every class's number of levels and the plan replays the same
@@ -1329,10 +1341,10 @@ extern "C" int dq_evo_tune(dq_evo *E, int *chosen_rpt, int *chosen_xcd, int *cho
     });
 }
 
-// Evolve every job by its schedule. Resident classes, a few launches each, run on their own streams, forked from and
-// joined to `stream`. The others: use_graph captures them (on the streams of the lane plan) into one graph on the first
-// call and replays it afterwards; otherwise they are launched directly. renormalize: end
-// with the FP64 renormalisation of every state. ms_out (may be NULL): elapsed GPU time.
+// Evolve every job by its schedule. Resident classes, a few launches each, run on their own streams, the others on the
+// streams of the lane plan, forked from and joined to `stream`. use_graph captures the lanes of GRAPH_KERNELS or more
+// kernels into one graph on the first call and replays it afterwards; the rest is launched directly. renormalize: end with
+// the FP64 renormalisation of every state. ms_out (may be NULL): elapsed GPU time.
 extern "C" int dq_evo_run(dq_evo *E, int use_graph, int renormalize, uintptr_t stream, float *ms_out) {
     return guard([&] {
         if (!E) throw ArgError("plan is NULL");
@@ -1348,37 +1360,49 @@ extern "C" int dq_evo_run(dq_evo *E, int use_graph, int renormalize, uintptr_t s
                 DQ_HIP(hipStreamCreateWithFlags(&l, hipStreamNonBlocking));
                 E->lanes.push_back(l);
             }
-        std::vector<hipEvent_t> joins(plan.size());
-        for (auto &j : joins) DQ_HIP(hipEventCreateWithFlags(&j, hipEventDisableTiming));
-        auto body = [&](hipStream_t base) {
+        auto lane_stream = [&](size_t li) { return g_evo_lanes > 0 ? E->lanes[li] : E->classes[plan[li][0]].stream; };
+        std::vector<size_t> captured, direct;  // lanes
+        for (size_t li = 0; li < plan.size(); ++li)
+            if (!plan[li].empty())
+                (use_graph && lane_in_graph(*E, plan[li], renormalize != 0) ? captured : direct).push_back(li);
+        std::vector<hipEvent_t> events;
+        auto event = [&] {
+            hipEvent_t e;
+            DQ_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            events.push_back(e);
+            return e;
+        };
+        auto capture = [&](hipStream_t base) {
             DQ_HIP(hipEventRecord(fork, base));
-            for (size_t li = 0; li < plan.size(); ++li) {
-                if (plan[li].empty()) continue;
-                hipStream_t ls = g_evo_lanes > 0 ? E->lanes[li] : E->classes[plan[li][0]].stream;
+            for (size_t li : captured) {
+                const hipStream_t ls = lane_stream(li);
                 DQ_HIP(hipStreamWaitEvent(ls, fork, 0));
                 for (int ci : plan[li]) run_class_levels(*E, E->classes[ci], ls, renormalize != 0);
-                DQ_HIP(hipEventRecord(joins[li], ls));
-                DQ_HIP(hipStreamWaitEvent(base, joins[li], 0));
+                const hipEvent_t join = event();
+                DQ_HIP(hipEventRecord(join, ls));
+                DQ_HIP(hipStreamWaitEvent(base, join, 0));
             }
         };
-        std::vector<hipEvent_t> res_events;  // the fork, then a join per resident class
-        auto start_resident = [&] {
-            auto event = [&] {
-                hipEvent_t e;
-                DQ_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-                res_events.push_back(e);
-                return e;
-            };
+        std::vector<hipEvent_t> joins;  // of what start_direct launched
+        auto start_direct = [&] {
             const hipEvent_t start = event();
             DQ_HIP(hipEventRecord(start, s0));
             for (const EvoClass &c : E->classes) {
                 if (!resident_rows(c, E->value_precision)) continue;
                 DQ_HIP(hipStreamWaitEvent(c.stream, start, 0));
                 run_class_resident(*E, c, c.stream, renormalize != 0);
-                DQ_HIP(hipEventRecord(event(), c.stream));
+                joins.push_back(event());
+                DQ_HIP(hipEventRecord(joins.back(), c.stream));
+            }
+            for (size_t li : direct) {
+                const hipStream_t ls = lane_stream(li);
+                DQ_HIP(hipStreamWaitEvent(ls, start, 0));
+                for (int ci : plan[li]) run_class_levels(*E, E->classes[ci], ls, renormalize != 0);
+                joins.push_back(event());
+                DQ_HIP(hipEventRecord(joins.back(), ls));
             }
         };
-        if (use_graph && !plan.empty()) {
+        if (!captured.empty()) {
             std::vector<int64_t> sig = graph_signature(*E, renormalize != 0);
             if (E->exec && E->graph_sig != sig) {
                 (void)hipGraphExecDestroy(E->exec); E->exec = nullptr;
@@ -1389,7 +1413,7 @@ extern "C" int dq_evo_run(dq_evo *E, int use_graph, int renormalize, uintptr_t s
                 DQ_HIP(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
                 DQ_HIP(hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal));
                 try {
-                    body(cap);
+                    capture(cap);
                 } catch (...) {
                     hipGraph_t g = nullptr;
                     (void)hipStreamEndCapture(cap, &g);
@@ -1403,21 +1427,19 @@ extern "C" int dq_evo_run(dq_evo *E, int use_graph, int renormalize, uintptr_t s
                 E->graph_sig = std::move(sig);
             }
             DQ_HIP(hipEventRecord(e0, s0));
-            start_resident();
+            start_direct();
             DQ_HIP(hipGraphLaunch(E->exec, s0));
         } else {
             DQ_HIP(hipEventRecord(e0, s0));
-            start_resident();
-            if (!plan.empty()) body(s0);
+            start_direct();
         }
-        for (size_t i = 1; i < res_events.size(); ++i) DQ_HIP(hipStreamWaitEvent(s0, res_events[i], 0));
+        for (const hipEvent_t j : joins) DQ_HIP(hipStreamWaitEvent(s0, j, 0));
         DQ_HIP(hipEventRecord(e1, s0));
         DQ_HIP(hipEventSynchronize(e1));
         float ms = 0.f;
         DQ_HIP(hipEventElapsedTime(&ms, e0, e1));
         if (ms_out) *ms_out = ms;
-        for (auto &j : joins) (void)hipEventDestroy(j);
-        for (auto &e : res_events) (void)hipEventDestroy(e);
+        for (auto &e : events) (void)hipEventDestroy(e);
         (void)hipEventDestroy(fork);
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);

@@ -402,8 +402,8 @@ int dq_evo_probe(dq_evo *E, double *est);
 
 /* Evolve every job by its schedule; the classes run on evo_lanes streams (see dq_set_tuning), forked from and joined
  * to `stream`. Classes of small Hamiltonians (up to 2048 rows with FP32 values, 1024 with FP64, and 24 diagonals) run
- * all their levels in one or a few launches. use_graph != 0 captures the others into a HIP graph on the first call and
- * replays it; renormalize != 0 ends with an FP64 renormalisation of every state. ms_out (may be NULL) receives the GPU time. The
+ * all their levels in one or a few launches. use_graph != 0 captures the others, but for streams of fewer than 16
+ * launches, into a HIP graph on the first call and replays it; renormalize != 0 ends with an FP64 renormalisation of every state. ms_out (may be NULL) receives the GPU time. The
  * graph is captured again only when what its launches depend on changed: a class's number of Horner levels (max over
  * its jobs of m 2^s), the tuned schedule, the evo_* tuning keys, the classes' assignment to streams or renormalize.
  * A new schedule that keeps those replays the same graph (the kernels read t, m and s from device memory). */

@@ -123,3 +123,45 @@ def test_states_cross_unchanged(rows, n_states):
         np.testing.assert_array_equal(a + 1j * b, st[j])
     with pytest.raises(capi.DqError):
         capi.check(L.dq_evo_set_states_complex(B._h, 2, capi.ptr(st[0])))
+
+
+@pytest.mark.parametrize("forced", [False, True])
+@pytest.mark.parametrize("levels", [(1, 1), (1, 13), (11, 12), (12, 11), (13, 30)])
+def test_lanes_of_few_kernels_beside_the_graph(levels, forced):
+    """Two classes, of 2049 and 300 rows, with levels at both sides of what a graph takes (16 kernels: 12 levels and the
+    norm), the small one also in the wave form (evo_vec = 1): on replays the bits of the launches without a graph, also after the levels of both have changed places."""
+    import diaq_amd  # noqa: F401
+    import diaq_gpu as d
+    from diaq_amd import capi, evolution
+    L = capi.lib()
+    rows = (2049, 300)
+    H = [hamiltonian(n, sorted({0, 1, -1, n // 3, -(n // 3)}), n) for n in rows]
+    B = evolution.BatchedEvolution([d.to_device(d.diaQMatrix.from_diagonals([n, n], M.offsets, M.vals))
+                                    for n, M in zip(rows, H)], 2, "fp32")
+    assert B.n_classes == 2
+    rng = np.random.default_rng(6)
+    st = [rng.standard_normal((2, n)) + 1j * rng.standard_normal((2, n)) for n in rows]
+
+    def run(graph):
+        for j, v in enumerate(st):
+            B.set_states(j, v)
+        B.run(use_graph=graph, renormalize=True)
+        return [B.get_states(j, n) for j, n in enumerate(rows)]
+
+    try:
+        capi.check(L.dq_set_tuning(b"evo_vec", 1 if forced else -1))
+        for m in (levels, levels[::-1]):
+            B.set_schedule([0.4, 0.7], m, [0, 0])
+            base = run(False)
+            for _ in range(3):
+                for a, b in zip(run(True), base):
+                    np.testing.assert_array_equal(a, b)
+        for a, v, M, t, k in zip(base, st, H, (0.4, 0.7), m):
+            for x, y in zip(a, v):
+                term = want = y
+                for i in range(1, k + 1):
+                    term = O.spmv(M, term) * (-1j * t / i)
+                    want = want + term
+                assert np.linalg.norm(x - want / np.linalg.norm(want)) < 2e-6
+    finally:
+        capi.check(L.dq_set_tuning(b"evo_vec", -1))
