@@ -426,8 +426,8 @@ struct dq_gate_plan {
 
 namespace dq {
 
-static int g_gates_tile_qubits = 0;  // dq_set_tuning "gates_tile_qubits": 10, 11 or 12; 0 (not set) = automatic
-static int g_gates_low_qubits = 0;   // dq_set_tuning "gates_low_qubits": 4, 5 or 6 (qubits always in a tile); 0: automatic
+static int g_gates_tile_qubits = 0;  // dq_set_tuning "gates_tile_qubits": 10, 11 or 12; 0 = automatic
+static int g_gates_low_qubits = 0;   // dq_set_tuning "gates_low_qubits": 4, 5 or 6 (qubits always in a tile); 0 = automatic
 
 bool gates_set_tuning(const std::string &key, int value) {
     if (key == "gates_kernel") {  // kept for callers: there is one pass kernel
@@ -435,12 +435,13 @@ bool gates_set_tuning(const std::string &key, int value) {
         return true;
     }
     if (key == "gates_low_qubits") {
-        if (value < 4 || value > 6) throw ArgError("gates_low_qubits must be 4, 5 or 6");
+        if (value != 0 && (value < 4 || value > 6)) throw ArgError("gates_low_qubits must be 0 (automatic), 4, 5 or 6");
         g_gates_low_qubits = value;
         return true;
     }
     if (key != "gates_tile_qubits") return false;
-    if (value < 10 || value > 12) throw ArgError("gates_tile_qubits must be 10, 11 or 12");
+    if (value != 0 && (value < 10 || value > 12))
+        throw ArgError("gates_tile_qubits must be 0 (automatic), 10, 11 or 12");
     g_gates_tile_qubits = value;
     return true;
 }

@@ -10,3 +10,13 @@ if ROOT not in sys.path:
 
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (gfx950) GPU and the built HIP library")
+
+
+@pytest.fixture(autouse=True)
+def automatic_gate_tiles():
+    """Gate plans choose their tile for each test, whatever an earlier one left set: the tuning is the process's."""
+    yield
+    capi = sys.modules.get("diaq_amd.capi")
+    if capi:
+        for key in (b"gates_tile_qubits", b"gates_low_qubits"):
+            capi.check(capi.lib().dq_set_tuning(key, 0))

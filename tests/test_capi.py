@@ -250,3 +250,13 @@ def test_host_dia_sparsity_dense_and_scaled_add():
     dA.addMatrixScaled(dB, 0.5, -2.0)
     np.testing.assert_allclose(d.to_numpy(dA), A + (0.5 - 2j) * B, rtol=0, atol=1e-15)
     assert list(dA.dIndices) == sorted(set(O.from_dense(A).offsets) | set(O.from_dense(B).offsets))
+
+
+def test_gate_tile_knobs_take_automatic():
+    L = capi.lib()
+    for key, good, bad in ((b"gates_tile_qubits", (0, 10, 11, 12, 0), (-1, 1, 9, 13)),
+                           (b"gates_low_qubits", (0, 4, 5, 6, 0), (-1, 3, 7))):
+        for v in good:
+            assert L.dq_set_tuning(key, v) == capi.DQ_OK, (key, v)
+        for v in bad:
+            assert L.dq_set_tuning(key, v) == capi.DQ_ERR_ARG and key in L.dq_last_error()

@@ -71,3 +71,20 @@ def test_gate_windows_bitwise(n, precision):
     bits = torch.int64 if precision == "fp64" else torch.int32
     for v, w in zip(a, b):
         assert torch.equal(v.view(bits), w.view(bits))
+
+
+def test_the_automatic_tile_comes_back():
+    """0 sets both knobs back to automatic. A layer on 26 qubits: 12, 8 and 6 of them to a pass with 12-qubit tiles and four
+    low qubits, which is the automatic choice; 11, 7, 7 and 1 with 11-qubit tiles; 12, 6, 6 and 2 with six low qubits."""
+    import diaq_amd  # noqa: F401
+    import diaq_gpu as d
+    from diaq_amd import capi
+    L = capi.lib()
+    rng = np.random.default_rng(0)
+    seq = [(gate(unitary(rng, 2), "fp64"), q) for q in range(26)]
+    got = []
+    for tile, low in ((0, 0), (11, 0), (0, 0), (0, 6), (0, 0)):
+        capi.check(L.dq_set_tuning(b"gates_tile_qubits", tile))
+        capi.check(L.dq_set_tuning(b"gates_low_qubits", low))
+        got.append(d.GatePlan(26, seq).n_passes)
+    assert got == [3, 4, 3, 4, 3]
