@@ -374,8 +374,9 @@ __global__ __launch_bounds__(RES_LANES) void taylor_resident_kernel(int rows, in
 // Whether H's evolution runs in taylor_resident_kernel: rows and diagonals whose values fit a workgroup's registers (96
 // of a lane's 128; FP32 values two rows per lane), and the two term buffers in 64 KB of LDS. A term then takes 0.7 us (6
 // qubits) to 1.6 us (10 qubits; FP32 10 qubits 1.9, 11 qubits 4.6), a launch of taylor_term_kernel 4.6 to 6.1 us at these
-// sizes.
+// sizes. An override of the terms' schedule asks for those launches.
 static bool resident_fits(const dq_devmat &H, int m, int *pad, size_t *lds) {
+    if (g_hamsim_rpt > 0 || g_hamsim_lds >= 0 || !g_hamsim_skip) return false;
     const int V = H.precision == DQ_F64 ? 1 : 2;
     if (H.rows > static_cast<uint32_t>(RES_LANES * V) || H.n() > RES_ND || H.n() == 0 || m <= 0 || m > RES_TERMS)
         return false;

@@ -198,7 +198,8 @@ int dq_release_cached_memory(void);
  * "spmv_skip_zero_blocks" (1 = default, 0) and "hamsim_skip_zero_blocks" (1 = default, 0) do the same for the
  * SpMV (the map dq_spmv_tune keeps, and spMV_ntimes's own) and for the fused evolution's Taylor terms, whose schedule
  * "hamsim_rows_per_lane" (0 = chosen per matrix; 2, 4 or 8 = two adjacent rows per lane) and "hamsim_lds" (-1 =
- * chosen, 0, 1: with two rows per lane) override;
+ * chosen, 0, 1: with two rows per lane) override (any of the three also asks for a launch per term where a small matrix
+ * would take them all in one);
  * "spmm_tiled" (0 = not tiled, the default; 1, 2, 4 = LDS-tiled with that many elements per lane) and
  * "spmm_cols_per_lane" (0 = automatic: 2 for an even n_right, else 1; 1, 2, 4, 8; -1 = one C element per lane),
  * "spmm_rows_per_lane" (-1 = automatic: 2 for >= 32768 rows and an even n_right >= 64, else 0; 0 = off; 2, 4, 8: the

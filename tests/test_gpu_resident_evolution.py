@@ -55,3 +55,33 @@ def test_small_evolution(case, precision):
     torch.cuda.synchronize()
     got = (pr + 1j * pi).cpu().numpy()
     assert np.linalg.norm(got - want) < (1e-12 if precision == "fp64" else 1e-6)
+
+
+@pytest.mark.parametrize("key,value", [(b"hamsim_lds", 0), (b"hamsim_rows_per_lane", 2), (b"hamsim_skip_zero_blocks", 0)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("case", [(1, 1), (65, 23), (1000, 24), (1024, 13), (1999, 21), (2048, 24)])
+def test_an_override_asks_for_a_launch_per_term(case, precision, key, value):
+    """The terms' own schedule, which each override selects, and one workgroup for all of them: the same bits, also where the
+    steps take several launches (more than 4096 terms)."""
+    import diaq_amd  # noqa: F401
+    import diaq_gpu as d
+    import torch
+    from diaq_amd import capi
+    rows, diags = case
+    H = hamiltonian(rows, diags, np.complex64 if precision == "fp32" else np.complex128)
+    D = d.to_device(d.diaQMatrix.from_diagonals([rows, rows], H.offsets, H.vals), precision)
+    rng = np.random.default_rng(5)
+    psi = rng.standard_normal(rows) + 1j * rng.standard_normal(rows)
+    L, off = capi.lib(), {b"hamsim_lds": -1, b"hamsim_rows_per_lane": 0, b"hamsim_skip_zero_blocks": 1}[key]
+    out = []
+    for steps, m in ((2, 7), (600, 7)):
+        for v in (off, value):
+            pr, pi = (torch.as_tensor(p, device="cuda").contiguous() for p in (psi.real, psi.imag))
+            try:
+                capi.check(L.dq_set_tuning(key, v))
+                d.hamsim_device_fp64_state(D, pr.data_ptr(), pi.data_ptr(), 0.01 * steps, steps, m, 0)
+            finally:
+                capi.check(L.dq_set_tuning(key, off))
+            torch.cuda.synchronize()
+            out.append((pr.cpu().numpy(), pi.cpu().numpy()))
+        np.testing.assert_array_equal(out[-1], out[-2])
