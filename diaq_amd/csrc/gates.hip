@@ -29,6 +29,7 @@
 // plan copies the gates' values: the gates may be freed after planning.
 #include <algorithm>
 #include <cmath>
+#include <limits>
 #include <utility>
 #include <vector>
 
@@ -67,6 +68,10 @@ struct PassHdr {
     int tpos[16];              // tile bit i -> global qubit (ascending)
     int cpos[48];              // tile index bit m -> global qubit, for the qubits outside the tile (ascending)
     int64_t step, diag;        // first step / diagonal entry of this pass in the plan's arrays
+    // Where a wave's amplitudes may leave the finite ones (stay_finite) it takes the "wild" steps, n_steps further on: every
+    // gate by itself, by its terms (STEP_ROWS*). check = 0: no step needs finite amplitudes, there are no others.
+    int check, pad_;
+    double limit;              // the bound of stay_finite
 };
 
 template <typename T>
@@ -188,7 +193,7 @@ __device__ __forceinline__ void full2_gate(const GateTerm<T> *__restrict__ g, T 
     const T g2r = g[2].re, g2i = g[2].im, g3r = g[3].re, g3i = g[3].im;
     static_for<(1 << R) / 2>([&](auto c) {
         constexpr int m = (c & ((1 << B) - 1)) | ((c >> B) << (B + 1)), n = m | (1 << B);
-        // a compensated FP32 sum of two terms is their plain sum
+        // a compensated FP32 sum of two finite terms is their plain sum
         T ar, ai, br, bi, cr, ci, dr, di;
         cmul(g0r, g0i, xr[m], xi[m], ar, ai);
         cmul(g1r, g1i, xr[n], xi[n], br, bi);
@@ -203,7 +208,7 @@ __device__ __forceinline__ void full2_gate(const GateTerm<T> *__restrict__ g, T 
 
 // A cross gate: real diagonal entries, imaginary others (a rotation about X). The products with the zero parts, which
 // full2_gate adds as zeros, are left out: 12 instructions for a pair of amplitudes against 20, with the same roundings and,
-// for finite amplitudes, the same values (a TFIM step of 28 qubits 7.13 -> 6.81 ms, of 25 789 -> 744 us).
+// while every amplitude is finite, the same values (a TFIM step of 28 qubits 7.13 -> 6.81 ms, of 25 789 -> 744 us).
 template <typename T, int R, int B>
 __device__ __forceinline__ void cross_gate(const GateTerm<T> *__restrict__ g, T (&xr)[1 << R], T (&xi)[1 << R]) {
 #pragma clang fp contract(off)
@@ -220,15 +225,31 @@ __device__ __forceinline__ void cross_gate(const GateTerm<T> *__restrict__ g, T 
     });
 }
 
-// Whether every amplitude of the wave is finite: a NaN or an infinity leaves the sum of zeros.
+// Whether a lane's amplitudes and all that a pass makes of them stay finite: then zeros may be left out of a sum, and
+// a compensated sum of two terms is their plain sum (it is NaN where the first one is infinite). A gate makes the largest
+// real or imaginary part at most as many times larger as the entries of a row add up to (absolute real and imaginary
+// parts); `limit` is the largest finite value over the product of these factors, with room for the roundings. False for a
+// NaN. A wave looks when it has loaded a tile and after each move: FP64 2^(R+1) additions, FP32 half as many maxima. It
+// replaces a look per cross layer (FP32, 28 qubits: a TFIM step 4.79 -> 4.72 ms) and is new to passes of general gates in
+// FP32 (14 gates on every other qubit in 2 passes 2.01 -> 2.09 ms).
 template <typename T, int E>
-__device__ __forceinline__ bool all_finite(const T (&xr)[E], const T (&xi)[E]) {
+__device__ __forceinline__ bool stay_finite(const T (&xr)[E], const T (&xi)[E], T limit) {
     T a = T(0), b = T(0);
-    static_for<E>([&](auto m) {
-        a = __builtin_fma(xr[m], T(0), a);
-        b = __builtin_fma(xi[m], T(0), b);
+    static_for<E / 2>([&](auto h) {
+        constexpr int m = 2 * h;
+        const T w = __builtin_elementwise_abs(xr[m]), x = __builtin_elementwise_abs(xi[m]);
+        const T y = __builtin_elementwise_abs(xr[m + 1]), z = __builtin_elementwise_abs(xi[m + 1]);
+        if constexpr (sizeof(T) == 4) {  // the largest (NaN if one is), two values an instruction
+            a = __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, w), x);
+            b = __builtin_elementwise_maximum(__builtin_elementwise_maximum(b, y), z);
+        } else {
+            a += w;
+            b += x;
+            a += y;
+            b += z;
+        }
     });
-    return !__any(!(a + b == T(0)));
+    return a + b < limit;
 }
 
 // The same on register bit j.
@@ -343,6 +364,7 @@ __global__ __launch_bounds__(256, 3) void gates_pass_kernel(const PassHdr *__res
     const int tid = threadIdx.x;
     for (int i = tid; i < P.n_diag; i += 256) tab[i] = diag[P.diag + i];
     const GateStep *__restrict__ st = steps + P.step;
+    const T limit = static_cast<T>(P.limit);
     __syncthreads();
     for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
         int64_t base = 0;
@@ -356,8 +378,10 @@ __global__ __launch_bounds__(256, 3) void gates_pass_kernel(const PassHdr *__res
             xr[m] = (re + om)[idx];
             xi[m] = (im + om)[idx];
         });
+        // 0, or n_steps: the wave takes the wild steps, until a move brings it other amplitudes
+        int wild = P.check && __any(!stay_finite(xr, xi, limit)) ? P.n_steps : 0;
         for (int s = 0; s < P.n_steps; ++s) {  // uniform
-            const GateStep S = st[s];
+            const GateStep S = st[s + wild];
             if (S.kind == STEP_RUN) {
                 for (int i = 0; i < S.end; ++i) {  // uniform
                     const GateStep D = st[s + i];
@@ -368,13 +392,14 @@ __global__ __launch_bounds__(256, 3) void gates_pass_kernel(const PassHdr *__res
                 s += S.end - 1;
                 DQ_VARIANT_END(40);
             } else if (S.kind == STEP_LAYER) {
-                if (S.k && all_finite(xr, xi)) {  // uniform in the wave
+                if (S.k) {
                     static_for<R>([&](auto b) { cross_gate<T, R, b>(terms + S.at + 4 * b, xr, xi); });
                     DQ_VARIANT_END(42);
                 } else {
                     static_for<R>([&](auto b) { full2_gate<T, R, b>(terms + S.at + 4 * b, xr, xi); });
                     DQ_VARIANT_END(41);
                 }
+                s += R - 1;
             } else if (S.kind == STEP_DIAG) {
                 const int ct = static_cast<int>(idx >> S.q) & ((1 << S.k) - 1);
                 diag_step<T, R, 0>(S, tab + S.at, ct, xr, xi);
@@ -399,6 +424,7 @@ __global__ __launch_bounds__(256, 3) void gates_pass_kernel(const PassHdr *__res
                 __syncthreads();  // the next move, of this tile or the next, writes the buffer again
                 a = to;
                 idx = base | lane_index<R>(P, tid, a);
+                wild = P.check && __any(!stay_finite(xr, xi, limit)) ? P.n_steps : 0;
             } else if (S.kind == STEP_ROWS2) {
                 rows_step<T, R, 1, 0>(S.j, S.at, S.end, terms, xr, xi);
             } else {
@@ -512,43 +538,38 @@ static int best_window(const std::vector<std::pair<int, int>> &gates, size_t i, 
     return best;
 }
 
-// Turns stretches of the steps from `from` on into steps of several gates: diagonal gates on no register bit into
-// STEP_RUN, full one-qubit gates on register bits 0, 1, .. R - 1 in turn (whose entries follow each other) into STEP_LAYER.
-// A layer of cross gates alone (cross_gate) has k = 1.
+// Makes stretches of the steps from `from` on one step of several gates, which the pass skips to the end of: diagonal gates
+// on no register bit a STEP_RUN, full one-qubit gates on register bits 0, 1, .. R - 1 in turn (whose entries follow each
+// other) a STEP_LAYER. A layer of cross gates alone (cross_gate) has k = 1.
 template <typename T>
 static void merge_steps(std::vector<GateStep> &steps, size_t from, int R, const std::vector<GateTerm<T>> &terms) {
     auto cross = [&](int at) {
         const GateTerm<T> *g = terms.data() + at;
         return g[0].im == T(0) && g[3].im == T(0) && g[1].re == T(0) && g[2].re == T(0);
     };
-    std::vector<GateStep> out;
     for (size_t i = from; i < steps.size();) {
+        GateStep &first = steps[i];
         size_t e = i;
         while (e < steps.size() && steps[e].kind == STEP_DIAG && steps[e].a == 0) ++e;
         if (e > i) {
-            for (size_t j = i; j < e; ++j) out.push_back(steps[j]);
-            GateStep &first = out[out.size() - (e - i)];
             first.kind = STEP_RUN;
             first.end = static_cast<int>(e - i);
             i = e;
             continue;
         }
         while (e < steps.size() && e - i < static_cast<size_t>(R) && steps[e].kind == STEP_FULL2 &&
-               steps[e].j == static_cast<int>(e - i) && steps[e].at == steps[i].at + 4 * static_cast<int>(e - i))
+               steps[e].j == static_cast<int>(e - i) && steps[e].at == first.at + 4 * static_cast<int>(e - i))
             ++e;
-        out.push_back(steps[i]);
         if (e - i == static_cast<size_t>(R)) {
-            out.back().kind = STEP_LAYER;
-            out.back().k = 1;
+            first.kind = STEP_LAYER;
+            first.k = 1;
             for (int b = 0; b < R; ++b)
-                if (!cross(out.back().at + 4 * b)) out.back().k = 0;
+                if (!cross(first.at + 4 * b)) first.k = 0;
             i = e;
         } else {
             ++i;
         }
     }
-    steps.resize(from);
-    steps.insert(steps.end(), out.begin(), out.end());
 }
 
 // Greedy cut of the sequence into passes: a non-diagonal gate joins the current pass while the qubits of the pass's
@@ -560,6 +581,16 @@ static void plan_passes(dq_gate_plan &P, int low_qubits, const std::vector<HostG
     std::vector<GateStep> steps;
     std::vector<GateTerm<T>> terms;
     std::vector<GateVal<T>> diag;
+    // the most by which the largest real or imaginary part can grow
+    auto growth = [](const HostGate &H) {
+        double most = 1.0;
+        for (size_t r = 0; r + 1 < H.rowptr.size(); ++r) {
+            double row = 0.0;
+            for (int t = H.rowptr[r]; t < H.rowptr[r + 1]; ++t) row += std::fabs(H.vre[t]) + std::fabs(H.vim[t]);
+            if (!(row <= most)) most = row;  // a NaN stays
+        }
+        return most;
+    };
     auto close = [&](int g0, int g1, uint64_t S) {
         if (g1 <= g0) return;
         uint64_t Tm = S;
@@ -588,6 +619,9 @@ static void plan_passes(dq_gate_plan &P, int low_qubits, const std::vector<HostG
             if (w >= 4) a = w;
         }
         D.a0 = a;
+        std::vector<GateStep> wild;          // the pass's steps for tiles that may leave the finite amplitudes
+        std::vector<GateTerm<T>> listed;     // and their terms, in slot order
+        bool needs_finite = false;
         size_t im = 0;
         for (int j = g0; j < g1; ++j) {
             const HostGate &H = gates[j];
@@ -625,19 +659,30 @@ static void plan_passes(dq_gate_plan &P, int low_qubits, const std::vector<HostG
                     mv.kind = STEP_MOVE;
                     mv.a = a = best_window(moving, im, L, R);
                     steps.push_back(mv);
+                    wild.push_back(mv);
                 }
                 ++im;
                 st.j = p - a;
-                const int t0 = static_cast<int>(terms.size());
-                // rows whose terms ascend in column order (two terms add up to the same bits in either order) need no
-                // list of terms, only which entries they are
+                const int t0 = static_cast<int>(terms.size()), l0 = static_cast<int>(listed.size());
+                // rows whose terms ascend in column order (finite sums of two terms have the same bits in either order)
+                // need no list of terms, only which entries they are
                 const int g = 1 << k;
-                bool ascending = true;
-                for (int r = 0; r < g; ++r)
-                    for (int t = H.rowptr[r] + 1; t < H.rowptr[r + 1]; ++t)
-                        ascending = ascending && H.col[t] != H.col[t - 1] && (k == 1 || H.col[t] > H.col[t - 1]);
-                for (int r = 0; r < g; ++r) ascending = ascending && H.rowptr[r + 1] - H.rowptr[r] <= g;
-                if (ascending) {
+                bool distinct = true, ascending = true;
+                for (int r = 0; r < g; ++r) {
+                    for (int t = H.rowptr[r]; t < H.rowptr[r + 1]; ++t) {
+                        listed.push_back(GateTerm<T>{static_cast<T>(H.vre[t]), static_cast<T>(H.vim[t]),
+                                                     r * g + H.col[t], 0});
+                        if (t == H.rowptr[r]) continue;
+                        distinct = distinct && H.col[t] != H.col[t - 1];
+                        ascending = ascending && H.col[t] > H.col[t - 1];
+                    }
+                    distinct = distinct && H.rowptr[r + 1] - H.rowptr[r] <= g;
+                }
+                GateStep by_terms = st;
+                by_terms.kind = k == 1 ? STEP_ROWS2 : STEP_ROWS4;
+                by_terms.at = l0;
+                by_terms.end = static_cast<int>(listed.size());
+                if (distinct && (k == 1 || ascending)) {
                     terms.resize(terms.size() + static_cast<size_t>(g) * g, GateTerm<T>{T(0), T(0), 0, 0});
                     int mask = 0;
                     for (int r = 0; r < g; ++r)
@@ -648,17 +693,18 @@ static void plan_passes(dq_gate_plan &P, int low_qubits, const std::vector<HostG
                         }
                     const bool full = mask == (1 << (g * g)) - 1;
                     st.kind = k == 1 ? (full ? STEP_FULL2 : STEP_MASK2) : (full ? STEP_FULL4 : STEP_MASK4);
+                    st.at = t0;
                     st.end = mask;
+                    needs_finite = needs_finite || (sizeof(T) == 4 && (full || !ascending));
                 } else {
-                    st.kind = k == 1 ? STEP_ROWS2 : STEP_ROWS4;
-                    for (int r = 0; r < g; ++r)
-                        for (int t = H.rowptr[r]; t < H.rowptr[r + 1]; ++t)
-                            terms.push_back(GateTerm<T>{static_cast<T>(H.vre[t]), static_cast<T>(H.vim[t]),
-                                                        r * g + H.col[t], 0});
+                    st = by_terms;
+                    st.at = t0;
+                    terms.insert(terms.end(), listed.begin() + l0, listed.end());
                     st.end = static_cast<int>(terms.size());
                 }
-                st.at = t0;
+                wild.push_back(by_terms);
             }
+            if (H.diag) wild.push_back(st);
             steps.push_back(st);
         }
         merge_steps(steps, static_cast<size_t>(D.step), R, terms);
@@ -667,9 +713,26 @@ static void plan_passes(dq_gate_plan &P, int low_qubits, const std::vector<HostG
             mv.kind = STEP_MOVE;
             mv.a = stored;
             steps.push_back(mv);
+            wild.push_back(mv);
         }
         D.n_steps = static_cast<int>(static_cast<int64_t>(steps.size()) - D.step);
         D.n_diag = static_cast<int>(static_cast<int64_t>(diag.size()) - D.diag);
+        for (size_t i = D.step; i < steps.size(); ++i)
+            needs_finite = needs_finite || (steps[i].kind == STEP_LAYER && steps[i].k);
+        if (needs_finite) {
+            for (GateStep &w : wild)
+                if (w.kind == STEP_ROWS2 || w.kind == STEP_ROWS4) {
+                    w.at += static_cast<int>(terms.size());
+                    w.end += static_cast<int>(terms.size());
+                }
+            terms.insert(terms.end(), listed.begin(), listed.end());
+            D.check = 1;
+            steps.insert(steps.end(), wild.begin(), wild.end());
+            double grows = 32.0;
+            for (int j = g0; j < g1; ++j) grows *= growth(gates[j]);
+            const bool finite = grows < std::numeric_limits<double>::infinity();  // false for a NaN
+            D.limit = finite ? static_cast<double>(std::numeric_limits<T>::max()) / grows : 0.0;
+        }
         P.passes.push_back(D);
     };
     const uint64_t low = (uint64_t(1) << low_qubits) - 1;
