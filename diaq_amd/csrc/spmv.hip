@@ -680,7 +680,10 @@ static void ntimes_device(const dq_devmat *A, const void *xr, const void *xi, vo
         throw ArgError("spmv_ntimes_device: work vectors are needed for num_times > 1 or x == y");
     // destinations alternate between y and the work vectors so that the last product lands in y; with x == y and an
     // odd count the first product must not overwrite x, so the order flips and a copy ends the sequence
-    const int launches = sequence_launches(*A, n);
+    int launches = sequence_launches(*A, n);
+    // x may be the work vector for an odd n: the first product goes to y, and x is not read again. An even number of
+    // launches would write over x while it is read.
+    if (launches < n && launches % 2 == 0 && (work_r == xr || work_i == xi)) launches = n;
     const bool flip = in_place && (launches % 2 == 1);
     // the zero blocks of A, skipped by every product of the sequence (A cannot change during the call): the map
     // dq_spmv_tune kept in the handle, or else, for two or more products, one made here -- in the caller's fixed

@@ -62,3 +62,32 @@ def test_band_powers(rows, band, precision):
         ref = O.spmv(M, ref)
     err = np.max(np.abs(got[1][0] + 1j * got[1][1] - ref))
     assert err <= (1e-12 if precision == "fp64" else 2e-6) * max(np.max(np.abs(ref)), 1e-30)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [3, 5, 7, 9, 11, 15])
+def test_x_as_the_work_vector(n, precision):
+    """An odd count needs x for its first product only, so x may also be the work vector, however many launches it takes."""
+    import diaq_amd  # noqa: F401
+    import diaq_gpu as d
+    import torch
+    from diaq_amd import capi
+    L = capi.lib()
+    rows = 200003
+    rng = np.random.default_rng(n)
+    for band in ("tri", "wide", "gaps"):
+        offs = BANDS[band]
+        vals = [rng.standard_normal(rows - abs(o)) / len(offs) + 0j for o in offs]
+        D = d.to_device(d.diaQMatrix.from_diagonals([rows, rows], offs, vals), precision)
+        dt = torch.float64 if precision == "fp64" else torch.float32
+        x = rng.standard_normal((2, rows))
+        out = []
+        for shared in (False, True):
+            xr, xi = (torch.as_tensor(p, device="cuda").to(dt).contiguous() for p in x)
+            yr, yi = torch.empty_like(xr), torch.empty_like(xi)
+            wr, wi = (xr, xi) if shared else (torch.empty_like(xr), torch.empty_like(xi))
+            capi.check(L.dq_spmv_ntimes_device(D.handle, xr.data_ptr(), xi.data_ptr(), yr.data_ptr(), yi.data_ptr(), n,
+                                               wr.data_ptr(), wi.data_ptr(), 0))
+            torch.cuda.synchronize()
+            out.append((yr.cpu().numpy(), yi.cpu().numpy()))
+        np.testing.assert_array_equal(out[0], out[1], err_msg=band)
