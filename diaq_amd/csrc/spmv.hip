@@ -410,7 +410,8 @@ __global__ void fill_map_kernel(int64_t n, uint2 *__restrict__ w) {
 // After A's values were rewritten on stream s: bring the zero-block map the handle keeps up to date in the same buffer,
 // ordered after the rewrite. A graph captured earlier that reads the handle's map then sees the new map on its next
 // replay, and later SpMVs skip no block that is nonzero now. The map of a tuning is recomputed; a product's map, which
-// the caller did not ask for, is set to "every block nonzero" instead of reading all values again.
+// the caller did not ask for, is set to "every block nonzero" for those graphs instead of reading all values again, and the
+// handle has none from then on: a sequence makes its own.
 void refresh_zero_map(dq_devmat &A, hipStream_t s) {
     if (!A.zmap_valid || !A.zmap.p) return;
     if (!A.zmap_loads_only) {
@@ -420,6 +421,7 @@ void refresh_zero_map(dq_devmat &A, hipStream_t s) {
     const int64_t n = static_cast<int64_t>(A.zmap.bytes / sizeof(uint2));
     hipLaunchKernelGGL(fill_map_kernel, dim3(blocks_for(n, 256, 2048)), dim3(256), 0, s, n, A.zmap.as<uint2>());
     DQ_LAUNCH_CHECK();
+    A.zmap_valid = A.zmap_loads_only = false;
 }
 
 // y = A x: the schedule of A, skipping its all-zero blocks when the handle holds their map (see handle_map).
