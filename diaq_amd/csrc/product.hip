@@ -270,7 +270,9 @@ __global__ __launch_bounds__(256) void product_kernel(const int2 *__restrict__ i
                                                       const T *__restrict__ bim, T *__restrict__ cre,
                                                       T *__restrict__ cim, double divisor,
                                                       ZeroMap za, ZeroMap zb, uint2 *__restrict__ zc,
-                                                      int64_t zc_words, int group) {
+                                                      int64_t zc_words, int group,
+                                                      const unsigned long long *__restrict__ live,
+                                                      unsigned long long sparse, int sparse_group) {
     constexpr int PROD_CHUNK = 256 * PROD_RPT;
     __shared__ int64_t s_abase[PROD_BATCH], s_bbase[PROD_BATCH];
     __shared__ int32_t s_lo[PROD_BATCH], s_hi[PROD_BATCH];
@@ -283,6 +285,7 @@ __global__ __launch_bounds__(256) void product_kernel(const int2 *__restrict__ i
     __shared__ int32_t s_c[PROD_GROUP], s_r0[PROD_GROUP], s_r1[PROD_GROUP], s_cnt[PROD_GROUP];
     // XCD-aware remap: the workgroups of XCD x (x = b mod 8) take the item range [xcd_first[x], xcd_first[x + 1]).
     const int64_t b = blockIdx.x;
+    if (MAP && live && *live <= sparse) group = sparse_group;  // uniform; the last workgroups then find nothing to do
     const int64_t w = xcd_first[b & 7] + (b >> 3) * group, w_end = xcd_first[(b & 7) + 1];
     if (w >= w_end) return;  // uniform
     const int ng = MAP ? static_cast<int>(min<int64_t>(group, w_end - w)) : 1;
@@ -471,11 +474,33 @@ __global__ __launch_bounds__(256) void map_bits_kernel(int64_t n, const uint2 *_
     if (threadIdx.x == 0) atomicAdd(out, static_cast<unsigned long long>(part[0]) + part[1] + part[2] + part[3]);
 }
 
-// Items of a workgroup, for operands with maps (2^16 rows or more): they share the round trips of their metadata, which take
-// a good part of an item's time, while enough workgroups remain. us, 1 / 2 / 8 items: 280 000 items (TFIM-20 squared and
-// applied) 4036 / 3629 / 3388, 29 000 (TFIM-17) 572 / 552 / 567. Smaller products have few items and run them one by one,
-// without the barrier that sharing takes.
-constexpr int64_t MANY_ITEMS = int64_t(1) << 17;
+// The blocks of a zero-block map that hold a nonzero, added to *out.
+__global__ __launch_bounds__(256) void live_blocks_kernel(int64_t n, const uint2 *__restrict__ w,
+                                                          unsigned long long *__restrict__ out) {
+    unsigned c = 0;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        c += __popc(w[i].x | w[i].y);
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+    __shared__ unsigned part[4];
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(out, static_cast<unsigned long long>(part[0]) + part[1] + part[2] + part[3]);
+}
+
+// Items of a workgroup, for operands with maps: they share the round trips of their metadata, but take turns where workgroups
+// of one item run side by side and find each other's operands in the L2. Where most pairs are dead, as in a qubit
+// Hamiltonian, the metadata is a good part of an item; where all are live, sharing costs up to half of the speed. us for
+// 1 / 2 / 4 / 8 items:
+//   TFIM-20 squared, 372 000 items            3080 / 2680 / 2490 / 2430
+//   TFIM-16 squared times itself, 503 000     9690 / 8160 / 7650 / 7930;  times the TFIM, 110 000: 1090 / 975 / 925 / 967
+//   33 diagonals side by side, 133 000        8740 / 8900 / 13230 / 17460;  24 far apart, 253 000: 3700 / 3590 / 3650 / 3940
+// So from MANY_ITEMS on the product counts the live blocks of its operands' maps (two launches, 10 us) and its workgroups
+// read the count: 4 items, from 4 MANY_ITEMS on 8, where a quarter of the blocks is zero or more. The grid is made for the
+// other case; the workgroups that have nothing to do then are its last ones. There and from SOME_ITEMS on it is two items
+// where a result diagonal has fewer than FEW_PAIRS pairs (TFIM-17, 33 000 items: 318 / 300; 16 diagonals far apart, 53 000:
+// 739 / 731; 5 side by side, 9 200: 241 / 244), else one (9 side by side, 8 700: 283 / 293). Smaller products have few
+// workgroups: 16 diagonals, 3 360 items 90 / 99, 9 diagonals, 544 items 53 / 57.
+constexpr int64_t SOME_ITEMS = int64_t(1) << 12, MANY_ITEMS = int64_t(1) << 16, FEW_PAIRS = 3;
 
 // Pair lists up to this size join the other work lists in one upload; longer ones are copied from where they are, as
 // gathering them first would take about as long as a copy of their own.
@@ -486,12 +511,16 @@ constexpr size_t UPLOAD_PAIR_BYTES = size_t(1) << 18;
 // smaller result saves less than the map's fill, count and read-back (about 15 us).
 constexpr int64_t MAP_RESULT_BYTES = int64_t(256) << 20;
 
-static int64_t map_blocks(const dq_devmat &C) {
-    if (C.precision != DQ_F64 || C.rows < (1u << 16) || 16 * C.total <= MAP_RESULT_BYTES) return 0;
+static int64_t blocks_of(const dq_devmat &M) {
     int64_t n = 0;
-    for (const DiagMeta &m : C.meta)
+    for (const DiagMeta &m : M.meta)
         if (m.rhi > m.rlo) n += ((m.rhi - 1) >> 6) - (m.rlo >> 6) + 1;
     return n;
+}
+
+static int64_t map_blocks(const dq_devmat &C) {
+    if (C.precision != DQ_F64 || C.rows < (1u << 16) || 16 * C.total <= MAP_RESULT_BYTES) return 0;
+    return blocks_of(C);
 }
 
 std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, double divisor, hipStream_t s,
@@ -552,7 +581,10 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
     for (int x = 0; x <= 8; ++x) xcd_first[x] = n_work * x / 8;
     int64_t per_xcd = 0;
     const bool maps = g_prod_skip && A.rows >= (uint32_t(1) << 16) && A.n() > 0 && B.n() > 0;
-    const int group = !maps ? 1 : n_work >= MANY_ITEMS ? PROD_GROUP : 2;
+    const bool few_pairs = static_cast<int64_t>(d.sa.size()) < FEW_PAIRS * nc;
+    const bool by_zeros = maps && n_work >= MANY_ITEMS;
+    const int group = maps && n_work >= SOME_ITEMS && few_pairs ? 2 : 1;
+    const int sparse_group = n_work >= 4 * MANY_ITEMS ? PROD_GROUP : 4;
     for (int x = 0; x < 8; ++x) per_xcd = std::max(per_xcd, (xcd_first[x + 1] - xcd_first[x] + group - 1) / group);
     const int64_t grid = per_xcd * 8;
     if (grid > 0x7fffffffLL) throw ArgError("product: too many work items");
@@ -611,6 +643,23 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
         za = map_of(A, zab);
         zb = (&A == &B) ? za : map_of(B, zbb);
     }
+    DevBuf dlive;
+    unsigned long long sparse = 0;
+    if (by_zeros) {
+        dlive = DevBuf(16);
+        zero_bytes(dlive.p, 8, s);
+        int64_t blocks = 0;
+        auto count = [&](const dq_devmat &M, const ZeroMap &z) {
+            const int64_t words = z.words * M.n();
+            hipLaunchKernelGGL(live_blocks_kernel, dim3(blocks_for(words, 1024, 128)), dim3(256), 0, s, words, z.w,
+                               dlive.as<unsigned long long>());
+            DQ_LAUNCH_CHECK();
+            blocks += blocks_of(M);
+        };
+        count(A, za);
+        if (&A != &B) count(B, zb);
+        sparse = static_cast<unsigned long long>(blocks - blocks / 4);
+    }
     // the result's own map, where a product with it may use one: kept when at least an eighth of its blocks are zero
     const int64_t c_blocks = keep_map && za.w ? map_blocks(*C) : 0;
     DevBuf zcb, dbits;
@@ -629,7 +678,7 @@ std::unique_ptr<dq_devmat> product(const dq_devmat &A, const dq_devmat &B, doubl
     hipLaunchKernelGGL((product_kernel<T, NTS, R, M>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, s,        \
                        ditems, dxcd, dps, dsa, dsb, A.d_meta.as<DiagMeta>(), B.d_meta.as<DiagMeta>(), C->d_meta.as<DiagMeta>(), \
                        A.re.as<T>(), A.im.as<T>(), B.re.as<T>(), B.im.as<T>(), C->re.as<T>(), C->im.as<T>(), divisor, \
-                       za, zb, zcb.as<uint2>(), zc_words, group)
+                       za, zb, zcb.as<uint2>(), zc_words, group, dlive.as<unsigned long long>(), sparse, sparse_group)
 #define DQ_PROD_LAUNCH_R(T, NTS, R)                          \
     do {                                                     \
         if (za.w) DQ_PROD_LAUNCH_M(T, NTS, R, true);         \

@@ -90,3 +90,45 @@ def test_product_of_zero_blocks(real):
     y = O.spmv(E, x)
     a, b = spmv(C, x)
     assert np.max(np.abs(a + 1j * b - y)) < 1e-12 * np.max(np.abs(y))
+
+
+@pytest.mark.parametrize("zeros", [False, True])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("diags", [4, 16, 24])
+def test_items_of_a_workgroup(diags, precision, zeros):
+    """2^18 + 77 rows: 1 700, 26 000 and more than 65 536 items, one, two or four to a workgroup by their number and by how
+    many blocks of the operands are zero; near diagonals with many pairs a result and far ones with few. The same values as
+    without maps, where each workgroup has one."""
+    import diaq_amd  # noqa: F401
+    import diaq_gpu as d
+    import torch
+    from diaq_amd import capi
+    rows = (1 << 18) + 77
+    rng = np.random.default_rng(diags)
+    for offs in (sorted(int(o) for o in rng.choice(np.arange(-rows // 2, rows // 2), diags, replace=False)),
+                 list(range(-diags // 2, diags // 2))):
+        vals = []
+        for o in offs:
+            n = rows - abs(o)
+            v = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+            if zeros:
+                v[(np.arange(n) + max(0, -o)) // 256 % 2 == 1] = 0
+            vals.append(v)
+        A = d.to_device(d.diaQMatrix.from_diagonals([rows, rows], offs, vals), precision)
+        C = d.product(A, A)
+        try:
+            tuning(b"product_skip_zero_blocks", 0)
+            plain = d.product(A, A)
+        finally:
+            tuning(b"product_skip_zero_blocks", 1)
+        assert C.diagonals == plain.diagonals
+        dt = torch.float64 if precision == "fp64" else torch.float32
+        x = [torch.randn(rows, dtype=dt, device="cuda") for _ in range(2)]
+        y = [[torch.empty_like(v) for v in x] for _ in range(2)]
+        for M, (yr, yi) in zip((C, plain), y):
+            capi.check(capi.lib().dq_spmv_device(M.handle, x[0].data_ptr(), x[1].data_ptr(), yr.data_ptr(), yi.data_ptr(), 0))
+        torch.cuda.synchronize()
+        assert torch.equal(y[0][0], y[1][0]) and torch.equal(y[0][1], y[1][1])
+        for k in plain.diagonals[:: max(1, len(plain.diagonals) // 6)]:
+            np.testing.assert_array_equal(np.asarray(C.get_diagonal(k)), np.asarray(plain.get_diagonal(k)))
+        del C, plain
