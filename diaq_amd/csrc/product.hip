@@ -507,9 +507,11 @@ constexpr int64_t SOME_ITEMS = int64_t(1) << 12, MANY_ITEMS = int64_t(1) << 16, 
 constexpr size_t UPLOAD_PAIR_BYTES = size_t(1) << 18;
 
 // The 64-row blocks of C's diagonals, when the product is to map them for the result's own products, else 0: FP64 values
-// beyond the Infinity Cache, where a product is bound by reading them (H*H of TFIM-20, 11 GB: SpMV 1.90 -> 0.94 ms). A
-// smaller result saves less than the map's fill, count and read-back (about 15 us).
-constexpr int64_t MAP_RESULT_BYTES = int64_t(256) << 20;
+// of 1 GiB or more, far beyond the Infinity Cache, where a product is bound by reading them. One SpMV with H*H, us, without
+// and with the map: TFIM-20 (10.2 GiB) 1904 / 946, XXZ-18 (1.9 GiB) 392 / 260, TFIM-17 (0.9 GiB) 211 / 246, XXZ-16 (0.4 GiB)
+// 99 / 119: there the look-ups cost more than the loads that they spare, and the product itself pays for the map's fill,
+// stores, count and read-back (3 diagonals, 2^21 rows: 139 -> 119 without).
+constexpr int64_t MAP_RESULT_BYTES = int64_t(1) << 30;
 
 static int64_t blocks_of(const dq_devmat &M) {
     int64_t n = 0;

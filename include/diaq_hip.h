@@ -264,7 +264,7 @@ int dq_product_dryrun(uint32_t rows, uint32_t cols, int32_t n_a, const int32_t *
                       const int32_t *offs_b, int32_t *n_res, int64_t *n_pairs, int32_t *res_offsets,
                       int64_t *res_pair_start, int32_t *pair_slot_a, int32_t *pair_slot_b);
 
-/* C = A B on the device, without pruning. A result of more than 256 MiB keeps a map of its all-zero 64-row blocks, which
+/* C = A B on the device, without pruning. An FP64 result of more than 1 GiB keeps a map of its all-zero 64-row blocks, which
  * spares its SpMVs the loads of zeros (the same results; new values set with dq_devmat_set_packed_device clear it).
  * Replaces product_device (src/deviceMatrix_gpu.hpp:78, src/spGEMM_gpu.cu:84-151). */
 int dq_product_device(const dq_devmat *A, const dq_devmat *B, dq_devmat **out);

@@ -94,16 +94,16 @@ def test_product_of_zero_blocks(real):
 
 @pytest.mark.parametrize("zeros", [False, True])
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
-@pytest.mark.parametrize("diags", [4, 16, 24])
+@pytest.mark.parametrize("diags", [4, 16, 36])
 def test_items_of_a_workgroup(diags, precision, zeros):
-    """2^18 + 77 rows: 1 700, 26 000 and more than 65 536 items, one, two or four to a workgroup by their number and by how
+    """2^19 + 77 rows: 2 300, 25 000 and more than 65 536 items, one, two or four to a workgroup by their number and by how
     many blocks of the operands are zero; near diagonals with many pairs a result and far ones with few. The same values as
     without maps, where each workgroup has one."""
     import diaq_amd  # noqa: F401
     import diaq_gpu as d
     import torch
     from diaq_amd import capi
-    rows = (1 << 18) + 77
+    rows = (1 << 19) + 77
     rng = np.random.default_rng(diags)
     for offs in (sorted(int(o) for o in rng.choice(np.arange(-rows // 2, rows // 2), diags, replace=False)),
                  list(range(-diags // 2, diags // 2))):
@@ -122,6 +122,7 @@ def test_items_of_a_workgroup(diags, precision, zeros):
         finally:
             tuning(b"product_skip_zero_blocks", 1)
         assert C.diagonals == plain.diagonals
+        assert diags < 36 or offs[1] - offs[0] == 1 or len(C.diagonals) * (rows // 2048) > 1 << 16
         dt = torch.float64 if precision == "fp64" else torch.float32
         x = [torch.randn(rows, dtype=dt, device="cuda") for _ in range(2)]
         y = [[torch.empty_like(v) for v in x] for _ in range(2)]
@@ -132,3 +133,54 @@ def test_items_of_a_workgroup(diags, precision, zeros):
         for k in plain.diagonals[:: max(1, len(plain.diagonals) // 6)]:
             np.testing.assert_array_equal(np.asarray(C.get_diagonal(k)), np.asarray(plain.get_diagonal(k)))
         del C, plain
+
+
+def test_a_large_result_keeps_its_map():
+    """A result above 1 GiB with many zero blocks: its SpMV takes a NaN and infinities to the zeros as without the map, a
+    sequence has its FP64 bits, and new values without zeros, and then with other zeros, are not read by the old map."""
+    import diaq_amd  # noqa: F401
+    import diaq_gpu as d
+    import torch
+    from diaq_amd import capi
+    L = capi.lib()
+    rows = (1 << 19) + 77
+    rng = np.random.default_rng(11)
+    offs = sorted(int(o) for o in rng.choice(np.arange(-rows // 2, rows // 2), 24, replace=False))
+    vals = []
+    for k, o in enumerate(offs):
+        n = rows - abs(o)
+        v = (rng.standard_normal(n) + (k % 2) * 1j * rng.standard_normal(n)) / 20
+        v[(np.arange(n) + max(0, -o)) // (512 << k % 3) % 2 == 1] = 0
+        vals.append(v)
+    A = d.to_device(d.diaQMatrix.from_diagonals([rows, rows], offs, vals))
+    C = d.product(A, A)
+    assert 16 * C.stored > 1 << 30
+    x = rng.standard_normal(rows) + 1j * rng.standard_normal(rows)
+    bad = x.copy()
+    bad[[17, 30000, 129999]] = [np.nan, np.inf, -np.inf + 1j * np.inf]
+
+    def ntimes(M, v, n):
+        t = [torch.as_tensor(p, device="cuda").contiguous() for p in (v.real, v.imag)]
+        y, w = [torch.empty_like(p) for p in t], [torch.empty_like(p) for p in t]
+        capi.check(L.dq_spmv_ntimes_device(M.handle, t[0].data_ptr(), t[1].data_ptr(), y[0].data_ptr(), y[1].data_ptr(), n,
+                                           w[0].data_ptr(), w[1].data_ptr(), 0))
+        torch.cuda.synchronize()
+        return [p.cpu().numpy() for p in y]
+
+    def compare(inputs):
+        got = [(spmv(C, v), ntimes(C, x, 3)) for v in inputs]
+        try:
+            tuning(b"spmv_skip_zero_blocks", 0)
+            want = [(spmv(C, v), ntimes(C, x, 3)) for v in inputs]
+        finally:
+            tuning(b"spmv_skip_zero_blocks", 1)
+        for a, b in zip(got, want):
+            np.testing.assert_array_equal(a, b)
+
+    compare((x, bad))
+    one = torch.ones(C.stored, dtype=torch.float64, device="cuda") / 1000
+    for keep in (one > 0, torch.arange(C.stored, device="cuda") // 4096 % 2 == 0):
+        re, im = one * keep, one * ~keep
+        capi.check(L.dq_devmat_set_packed_device(C.handle, re.data_ptr(), im.data_ptr(), 0))
+        torch.cuda.synchronize()
+        compare((x, bad))
