@@ -5,7 +5,8 @@
 //
 // Two kernels serve every diagonal count (the reference's one-diagonal kernel gives the same values: y is zero except
 // on the rows of the lone diagonal): row tiles for large matrices, and the wave form (spmv_wave_kernel) for matrices of
-// up to 2^21 rows and for every product that skips zero blocks (sched_for). In the row tiles a workgroup owns a tile of 256*RPT consecutive rows; lane l of the tile
+// fewer than 1.8 10^6 rows (2^20 in FP32) and for every product that skips zero blocks (sched_for). In the row tiles a
+// workgroup owns a tile of 256*RPT consecutive rows; lane l of the tile
 // handles rows tile + l + 256*j. For each diagonal (a uniform loop, metadata through scalar loads) the wave reads 64
 // consecutive values of the diagonal (one aligned 512-byte FP64 segment, row-aligned layout) and 64 consecutive
 // values of the shifted x window, so every access is a full, coalesced line. Each row sums its diagonals in slot
@@ -233,23 +234,26 @@ bool lds_window_for(const dq_devmat &A, int rpt) {
     return lds_window_pays(A, rpt);
 }
 
-// The untuned schedule for reading A's values from memory once per product. The wave form up to 2^21 rows: below
-// that a 2048-row tile leaves CUs idle or with one wave per SIMD, and each row tile pays a chain of dependent loads per
-// diagonal (TFIM-12: 24 -> 6 us; 100003 rows x 33 random diagonals: 46 -> 12 us; 2^18 rows, TFIM: 48 -> 27 us; at 10^6
-// rows 97 -> 90 us random, 84 -> 87 a band; at 4 10^6 rows the tiles win, 755 against 781 us). Two rows per lane
+// The untuned schedule for reading A's values from memory once per product. The wave form for matrices of few rows, where
+// a 2048-row tile leaves CUs idle or with one wave per SIMD, and each row tile pays a chain of dependent loads per
+// diagonal (TFIM-12: 24 -> 6 us; 100003 rows x 33 random diagonals: 46 -> 12 us; 2^18 rows, TFIM: 48 -> 27 us). The line,
+// us, tiles / wave form, 33 diagonals side by side and at random: FP64 2^20 rows 89 / 90 and 101 / 97, 1.5 10^6 140 / 135
+// and 146 / 143, 2^21 184 / 190 and 196 / 204, 4 10^6 755 / 781 random; FP32 700 000 rows 54 / 31 and 49 / 31, 2^20 50 / 57
+// and 55 / 54 (TFIM-20 63 / 69), 1.5 10^6 67 / 85 and 75 / 75, 2^21 96 / 113 and 99 / 99. Two rows per lane
 // (16-byte loads) from 2^18 rows in FP64, where bytes count more than latency (2^18: equal; 2^20, TFIM: 151 -> 124 us
 // with the LDS window); in FP32 one row per lane (a band of 10^6 rows: 44 us against 55). With a map (fewer values to
 // read) the wave form at any size, FP32 with two rows per lane from 2^21 rows (TFIM-22: 2.00 -> 1.75 ms for 8
 // products). Non-temporal loads when the values exceed the Infinity Cache's 256 MiB (TFIM-18, 155 MB: 27 us plain, 34
 // non-temporal; TFIM-22: 613 and 567); with a map from 640 MiB stored, as about a third of it is live in a real
 // Hamiltonian.
-constexpr int64_t WAVE_ROWS = int64_t(1) << 21, WAVE2_ROWS = int64_t(1) << 18;
+constexpr int64_t WAVE_ROWS_F64 = int64_t(7) << 18, WAVE_ROWS_F32 = int64_t(1) << 20;
+constexpr int64_t WAVE2_ROWS_F64 = int64_t(1) << 18, WAVE2_ROWS_F32 = int64_t(1) << 21;
 
 static SpmvSched wave_default(const dq_devmat &A, bool map) {
     const bool f64 = A.precision == DQ_F64;
     const int64_t bytes = 2 * A.total * elem_bytes(A.precision);
     SpmvSched c{1, false, false, false, 0};
-    c.v = A.rows >= (f64 ? WAVE2_ROWS : WAVE_ROWS) ? 2 : 1;
+    c.v = A.rows >= (f64 ? WAVE2_ROWS_F64 : WAVE2_ROWS_F32) ? 2 : 1;
     c.lds = f64 && lds_window_pays(A, 2);
     c.nt = bytes > (int64_t(map ? 640 : 256) << 20);
     return c;
@@ -258,7 +262,8 @@ static SpmvSched wave_default(const dq_devmat &A, bool map) {
 static SpmvSched sched_for(const dq_devmat &A, bool map) {
     SpmvSched c{8, true, true, false, 0};
     const dq_devmat::WaveSched &w = map ? A.skip_wave : A.tuned_wave;
-    const bool wave = map || (g_spmv_rpt > 0 ? g_spmv_rpt == 1 : A.tuned_rpt > 0 ? w.v > 0 : A.rows < WAVE_ROWS);
+    const bool few_rows = A.rows < (A.precision == DQ_F64 ? WAVE_ROWS_F64 : WAVE_ROWS_F32);
+    const bool wave = map || (g_spmv_rpt > 0 ? g_spmv_rpt == 1 : A.tuned_rpt > 0 ? w.v > 0 : few_rows);
     if (wave) {
         c = wave_default(A, map);
         if (w.v > 0) {
@@ -540,7 +545,7 @@ extern "C" int dq_spmv_tune(dq_devmat *A, int repeats, uintptr_t stream, float *
             }
         };
         A->tuned_wave = dq_devmat::WaveSched();
-        if (A->rows < 2 * WAVE_ROWS) time_waves(best, A->tuned_wave);  // beyond, the tiles read every block faster
+        if (A->rows < (1u << 22)) time_waves(best, A->tuned_wave);  // beyond, the tiles read every block faster
         // last stage: when A has all-zero blocks or parts and skipping them is faster, keep their map in the handle (used
         // by A's FP64 SpMVs and by spMV_ntimes)
         A->zmap_valid = A->zmap_loads_only = false;

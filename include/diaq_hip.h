@@ -168,7 +168,7 @@ int dq_spmv_device_banded(const dq_devmat *A, const void *xr_dev, const void *xi
 int dq_spmv_tune(dq_devmat *A, int repeats, uintptr_t stream, float *best_ms);
 
 /* The row-tile schedule of A's SpMVs (after tuning or the defaults); any output pointer may be NULL. Products that run
- * in the wave form instead (untuned: fewer than 2^21 rows, or a zero-block map; tuned: where it was faster) use its
+ * in the wave form instead (untuned: fewer than 1.8 10^6 rows, 2^20 in FP32, or a zero-block map; tuned: where it was faster) use its
  * tile order only. No reference counterpart. */
 int dq_spmv_tuned_config(const dq_devmat *A, int *rows_per_lane, int *nontemporal, int *pipelined, int *lds_window,
                          int *xcd_tiles);
