@@ -20,8 +20,9 @@
 // so the prediction does not overshoot), and a batch that did run past the stop is run again with the right count.
 //
 // Bound: the L2's reads of X, once per RB rows and term, and the latency between them (a workgroup per CU: its rows fill
-// the LDS). TFIM-12 (4096 rows, 25 diagonals): 0.21 ms per term. exp(-iHt) as a whole, ms, before / now: TFIM-8 2.7 /
-// 0.34, TFIM-12 39 / 7.1, XXZ-13 212 / 82.
+// the LDS). TFIM-12 (4096 rows, 25 diagonals): 14 terms of the series and 14 of the squaring in 4 launches, 0.25 ms per term
+// with the launches' reads and writes of T and U. exp(-iHt) as a whole, ms, before / now: TFIM-8 2.7 / 0.25, TFIM-12 39 / 7.1,
+// XXZ-13 212 / 82.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -414,7 +415,7 @@ bool dense_square_pays(int64_t N, size_t n_offsets) {
 }
 
 // U holds p(X)^(2^j) for the series' polynomial p: its square is p(X) applied to it 2^j times, at `done` terms of X's
-// diagonals each, or one dense product. Measured, ms: TFIM-12 (16 terms of 25
+// diagonals each, or one dense product. Measured, ms: TFIM-12 (14 terms of 25
 // diagonals) 3.3 by terms, 9.4 by the product; a term and diagonal costs as much as ACTION_COST rows of the product where
 // X's values are complex, less where a part is zero.
 std::vector<int32_t> TaylorRows::square(const std::vector<int32_t> &offs, DevBuf &U, int j) {

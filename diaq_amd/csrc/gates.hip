@@ -18,9 +18,9 @@
 // its index is the same for all the lane's amplitudes, so it looks up one entry per value of the gate's qubits that lie
 // in the window (1, 2 or 4 for a two-qubit gate) and not one per amplitude.
 //
-// What bounds it: HBM for passes of few gates (28 qubits: 1.85 ms for 8 one-qubit gates, 4.6 TB/s; 2.42 ms when the tile's
-// runs lie 8 MB and more apart), vector issue for full ones (27 diagonal and 12 one-qubit gates: 3.37 ms, of which
-// 1.6 ms FP64 instructions). A first-order TFIM-28 step: 3 passes, 7.2 ms; 15.4 ms in 4 passes when the tiles lived in
+// What bounds it: HBM for passes of few gates (28 qubits: 1.69 ms for 8 one-qubit gates, 5.1 TB/s; 2.24 ms when the tile's
+// runs lie 8 MB and more apart), vector issue for full ones (27 diagonal gates and 12 rotations about X: 2.74 ms, with 12
+// general one-qubit gates 3.07). A first-order TFIM-28 step: 3 passes, 6.8 ms; 15.4 ms in 4 passes when the tiles lived in
 // LDS and every gate read and wrote them there.
 //
 // Each gate's arithmetic on each amplitude is the single-gate kernel's (each row adds its terms in the order of the
@@ -57,8 +57,8 @@ struct GateStep {
     int at;    // STEP_DIAG: its first entry in the pass's LDS table; STEP_FULL*, STEP_MASK*: its entries (row-major,
                // absent ones too) in terms;
                // STEP_LAYER: the entries of full one-qubit gates on register bits 0 .. R - 1, one after the other
-    int end;   // STEP_ROWS*: its terms of a row, from `at` on; STEP_MASK*: bit r * rows + c: entry (r, c) is a term; STEP_RUN: this and the next end - 1 steps are diagonal gates on
-               // no register bit
+    int end;   // STEP_ROWS*: its terms of a row, from `at` on; STEP_MASK*: bit r * rows + c: entry (r, c) is a term;
+               // STEP_RUN: this and the next end - 1 steps are diagonal gates on no register bit
     int pad_;
 };
 
@@ -823,10 +823,10 @@ extern "C" int dq_gate_plan_create(int n_qubits, int n_gates, const dq_devmat *c
     return guard([&] {
         if (!out) throw ArgError("out is NULL");
         if (n_gates < 1 || !gates || !first_qubit) throw ArgError("gates: need at least one gate");
-        // Small states want many small tiles (a TFIM step on 14 qubits: 17, 20, 24 us with 10, 11, 12 tile qubits; 19
-        // two-qubit gates on 20 qubits: 69, 85, 94 us), large ones few passes (TFIM on 20: 52, 54, 46 us; on 22: 116,
-        // 111, 106; on 28: 10.3, 9.0, 7.2 ms). Four low qubits make runs of 16 amplitudes, whole 128-byte
-        // lines in FP64; a fifth costs tile qubits (28 qubits: 4 passes for 3, 8.3 ms; FP32 4.8 against 4.9 ms).
+        // Small states want many small tiles (a TFIM step on 14 qubits: 18, 20, 24 us with 10, 11, 12 tile qubits; 19
+        // two-qubit gates on 20 qubits: 65, 68, 80 us), large ones few passes (TFIM on 20: 58, 58, 46 us; on 22: 120,
+        // 121, 104; on 28: 9.7, 8.8, 6.8 ms). Four low qubits make runs of 16 amplitudes, whole 128-byte
+        // lines in FP64; a fifth costs tile qubits (28 qubits: 4 passes for 3, 8.0 ms; FP32 4.6 against 4.7 ms).
         const int L = g_gates_tile_qubits ? g_gates_tile_qubits : n_qubits >= 21 ? 12 : n_qubits >= 19 ? 11 : 10;
         const int low = g_gates_low_qubits ? g_gates_low_qubits : 4;
         const int least = g_gates_tile_qubits ? g_gates_tile_qubits : 11;

@@ -6,7 +6,8 @@
 // them. A workgroup takes L = R + (p - 1)(hl + hh) rows, one per lane, loads their values into registers once, the x
 // window into LDS, and computes p products: after product s the rows within p - s halos of its R hold A^s x, the
 // others hold values that no kept row reads. Every row sums its diagonals in slot order with the operations of
-// dia_rows_tile, so the rows have the same bits (a zero block is read like any other).
+// dia_rows_tile, so the rows have the bits of products that read every block. (A zero block is read like any other: a
+// compensated FP32 sum that skips it, as products with a map do, may differ in its last bits.)
 //
 // Bound: the values' reads, L / (R p) of a pass each, against the sums: a compensated FP32 sum is 16 vector instructions
 // per element, 13 us per product of 33 10^6 elements on the whole chip. 512 lanes and, in FP32, at most 128 registers leave
